@@ -670,12 +670,15 @@ int plan_create(Plan **out, const ksw2_pair_t *pairs, const int *idx, int nidx, 
         auto longest_first = [&](std::vector<int> &m) {
             std::stable_sort(m.begin(), m.end(), [&](int x, int y) { return pair_steps(p->jobs[x]) > pair_steps(p->jobs[y]); });
         };
-        for (int grp = 0; grp < kGroups; ++grp) {
+        for (int part = 0; part < 2 * kGroups; ++part) {
+            const int grp = part / 2;
+            const bool lut = part % 2 == 0;
+            auto mine = [&](int k) { return grp_of[k] == grp && (p->jobs[k].lut != 0) == lut; };
             // every wide pair of the group in one launch, each on its own
             // number of workgroups
             std::vector<int> members;
             for (int k = 0; k < p->n_fast; ++k)
-                if (grp_of[k] == grp && wide(k)) members.push_back(k);
+                if (mine(k) && wide(k)) members.push_back(k);
             if (!members.empty()) {
                 longest_first(members);
                 const int wf = (int)p->h_wfirst.size();
@@ -687,7 +690,7 @@ int plan_create(Plan **out, const ksw2_pair_t *pairs, const int *idx, int nidx, 
                 }
                 p->h_wfirst.push_back(blocks);
                 // team: the largest, for a one-workgroup launch of spread pairs
-                p->launches.push_back({grp, tmax, (int)order.size(), (int)members.size(), 0, 1, p->n_wide, wf});
+                p->launches.push_back({grp, tmax, (int)order.size(), (int)members.size(), 0, 1, p->n_wide, wf, lut});
                 p->n_wide += (int)members.size();
                 order.insert(order.end(), members.begin(), members.end());
             }
@@ -696,10 +699,10 @@ int plan_create(Plan **out, const ksw2_pair_t *pairs, const int *idx, int nidx, 
             members.clear();
             int tmax = 0;
             for (int k = 0; k < p->n_fast; ++k)
-                if (grp_of[k] == grp && !wide(k)) members.push_back(k), tmax = std::max(tmax, team[k]);
+                if (mine(k) && !wide(k)) members.push_back(k), tmax = std::max(tmax, team[k]);
             if (!members.empty()) {
                 longest_first(members);
-                p->launches.push_back({grp, tmax, (int)order.size(), (int)members.size(), grp % Plan::kLanes, 0, 0, 0});
+                p->launches.push_back({grp, tmax, (int)order.size(), (int)members.size(), grp % Plan::kLanes, 0, 0, 0, lut});
                 order.insert(order.end(), members.begin(), members.end());
             }
         }
@@ -995,10 +998,10 @@ static void plan_capture(Plan *p)
         sa.order = p->d_order + l.off, sa.njobs = l.count;
         if (ok && use_queue(qmode, p, l) && nq < kMaxQueueHeads) {
             ok = clear_queue_heads(p->d_qhead + nq, 1, st) == hipSuccess &&
-                 launch_stripe_queue(sa, l.grp, p->R, p->d_qhead + nq, st) == hipSuccess;
+                 launch_stripe_queue(sa, l.grp, p->R, l.lut, p->d_qhead + nq, st) == hipSuccess;
             ++nq;
         } else if (ok) {
-            ok = launch_stripe(sa, l.grp, l.team, p->R, st) == hipSuccess;
+            ok = launch_stripe(sa, l.grp, l.team, p->R, l.lut, st) == hipSuccess;
         }
     }
     for (int k = 0; k < Plan::kLanes; ++k)
@@ -1125,8 +1128,8 @@ int plan_launch(Plan *p, const Progress *prog)
                     if (!l.wide) continue;
                     sa.order = p->d_order + l.off, sa.njobs = l.count;
                     sa.wctl = p->d_wctl + (int64_t)l.woff * kWideCtl, sa.wfirst = p->d_wfirst + l.wf;
-                    const int half = std::max(1, stripe_wide_capacity(l.grp, p->R) / 2);
-                    KSW_HIP_TRY(launch_stripe_wide(sa, l.grp, p->R, p->h_wfirst.data() + l.wf, half, st));
+                    const int half = std::max(1, stripe_wide_capacity(l.grp, p->R, l.lut) / 2);
+                    KSW_HIP_TRY(launch_stripe_wide(sa, l.grp, p->R, l.lut, p->h_wfirst.data() + l.wf, half, st));
                 }
                 if (!wait_slots_release(st, q)) return KSW2_HIP_EDEVICE;
             }
@@ -1134,8 +1137,8 @@ int plan_launch(Plan *p, const Progress *prog)
         for (const Plan::Launch &l : p->launches) {
             if (!l.wide) continue;
             sa.order = p->d_order + l.off, sa.njobs = l.count, sa.wctl = p->d_wctl + (int64_t)l.woff * kWideCtl;
-            if (wide_now) KSW_HIP_TRY(launch_stripe_wide_epilogue(sa, l.grp, p->R, st));
-            else KSW_HIP_TRY(launch_stripe(sa, l.grp, l.team, p->R, st));  // one-workgroup teams
+            if (wide_now) KSW_HIP_TRY(launch_stripe_wide_epilogue(sa, l.grp, p->R, l.lut, st));
+            else KSW_HIP_TRY(launch_stripe(sa, l.grp, l.team, p->R, l.lut, st));  // one-workgroup teams
         }
     }
     // one-wave teams run as persistent workers over the launch's job list (a
@@ -1151,10 +1154,10 @@ int plan_launch(Plan *p, const Progress *prog)
         if (use_queue(qmode, p, l) && nq < kMaxQueueHeads) {
             // its head zeroed on the launch's own stream, before the workers
             KSW_HIP_TRY(clear_queue_heads(p->d_qhead + nq, 1, st));
-            KSW_HIP_TRY(launch_stripe_queue(sa, l.grp, p->R, p->d_qhead + nq, st));
+            KSW_HIP_TRY(launch_stripe_queue(sa, l.grp, p->R, l.lut, p->d_qhead + nq, st));
             ++nq;
         } else {
-            KSW_HIP_TRY(launch_stripe(sa, l.grp, l.team, p->R, st));
+            KSW_HIP_TRY(launch_stripe(sa, l.grp, l.team, p->R, l.lut, st));
         }
     }
     for (int k = 0; k < Plan::kLanes; ++k)

@@ -131,13 +131,15 @@ hipError_t launch_general_walk(const GenWalkArgs &a, hipStream_t st);
 enum StripeGroup { kGroupLeft = 0, kGroupRight = 1, kGroupScoreOnly = 2, kGroupTracks = 3, kGroups = 4 };
 
 // Stripe kernel: one workgroup of `team` waves (1..kMaxTeam) per job, R
-// rows per lane (8 or 4; the jobs' layouts must use the same R).
-hipError_t launch_stripe(const StripeArgs &a, int group, int team, int R, hipStream_t st);
+// rows per lane (8 or 4; the jobs' layouts must use the same R); lut: score
+// candidates from a byte table (every job's lut must be the same: the two
+// forms are kernels of their own, which keeps each within its registers).
+hipError_t launch_stripe(const StripeArgs &a, int group, int team, int R, bool lut, hipStream_t st);
 // Persistent one-wave workers (as many as fit on the device, at most one per
 // job) claiming the launch's jobs in list order from a device queue head
 // (*qhead, zero at launch: clear_queue_heads); every job runs as a one-wave
 // team.  A drop-in for launch_stripe with team 1.
-hipError_t launch_stripe_queue(const StripeArgs &a, int group, int R, int32_t *qhead, hipStream_t st);
+hipError_t launch_stripe_queue(const StripeArgs &a, int group, int R, bool lut, int32_t *qhead, hipStream_t st);
 hipError_t clear_queue_heads(int32_t *qhead, int n, hipStream_t st);
 int stripe_queue_workers(int group, int R);
 
@@ -155,11 +157,11 @@ constexpr int kWideGroup = 4;       // waves per workgroup: one per SIMD of a CU
 constexpr int kWideCtlStride = 16;  // dwords between two waves' progress counts
 constexpr int kWideCtlLate = kMaxWide * kWideCtlStride;  // raised when a wait gave up
 constexpr int kWideCtl = kWideCtlLate + 64;              // dwords per job
-hipError_t launch_stripe_wide(const StripeArgs &a, int group, int R, const int32_t *h_wfirst, int max_wgs,
+hipError_t launch_stripe_wide(const StripeArgs &a, int group, int R, bool lut, const int32_t *h_wfirst, int max_wgs,
                               hipStream_t st);
 // Workgroups of the wide stripe kernel the device holds at once.
-int stripe_wide_capacity(int group, int R);
-hipError_t launch_stripe_wide_epilogue(const StripeArgs &a, int group, int R, hipStream_t st);
+int stripe_wide_capacity(int group, int R, bool lut);
+hipError_t launch_stripe_wide_epilogue(const StripeArgs &a, int group, int R, bool lut, hipStream_t st);
 // Zeroes a plan's wide redo count (kWideCtl dwords at werr).
 hipError_t clear_wide_err(int32_t *werr, hipStream_t st);
 // Waves of the stripe kernel that fit on the device at once.

@@ -171,7 +171,7 @@ struct Plan {
     std::vector<int> order;          // plan slot -> caller index
     std::vector<uint64_t> cig_off;   // plan slot -> uint32 offset in the cig arena
     // Per job group (0 left-aligned traceback, 1 right-aligned, 2 score-only,
-    // 3 Singletrack tracks): one wide launch and one launch of one-workgroup
+    // 3 Singletrack tracks) and score form (lut): one wide launch and one launch of one-workgroup
     // teams (`team` = the largest; each pair's own size is in its KswJob).
     // `off`/`count` index d_order.
     // wide: a wide launch (each pair on its own number of kWideGroup-wave
@@ -179,6 +179,7 @@ struct Plan {
     // whose first-workgroup table starts at entry `wf` of h_wfirst/d_wfirst.
     struct Launch {
         int grp, team, off, count, lane, wide, woff, wf;
+        bool lut;
     };
     std::vector<Launch> launches;
     struct GLaunch {

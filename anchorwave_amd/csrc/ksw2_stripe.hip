@@ -31,14 +31,16 @@
 //    workgroups on different CUs; the counts and column-buffer entries are
 //    then device-scope accesses, and the epilogue runs in a launch of its
 //    own.
-//  * Scaled, negated state.  Every difference value w is kept as -8*w plus a
-//    3-bit tag, so a chain of v_pk_min_i16 yields both the maximum of the
-//    five candidates (s, a, b, a2, b2) and the index the reference's strict
-//    '>' (or '>=' for right alignment) chain would pick: ties resolve to the
-//    smallest (left) or largest (right) index through the tag.  With
-//    T = (x+v) + 8e - 8z (tag-free), the new x is min(T, 0) and the
-//    continuation flag is the sign of T (left); right alignment keeps x
-//    biased by -8 so that the sign of T is its '>= 0' flag.
+//  * Cells (ksw2_cell.h): negated values on packed halves, with a scale and a
+//    tag where direction bytes are wanted, plain for scores and tracks.
+//    VALU issue bounds the kernel: a middle pass of eight rows takes 248
+//    VALU instructions per step (16 cells per lane), 297 before the
+//    three-input minimum, the constant-free candidates, the flag bits taken
+//    two rows at a time and the score tables that travel between lanes.  The
+//    fixed batch (4,096 x 2 kbp, bytes and walk) went from 12.76 to 9.15 ms a
+//    launch, score only from 8.99 to 6.43, tracks (2,048 pairs) from 6.63 to
+//    4.95; a lone 5 kbp pair on four rows per lane from 4.84 to 2.74 ms, the
+//    plain blocks' unrolled steps helping it most.
 //  * Exactness.  The reference computes on int8 lanes.  The host only routes
 //    a call here when every in-band intermediate provably stays inside int8
 //    (then 16-bit arithmetic gives the same values), the match score is 0
@@ -55,7 +57,9 @@
 #include <stdint.h>
 
 #include <algorithm>
+#include <type_traits>
 
+#include "ksw2_cell.h"
 #include "ksw2_common.h"
 #include "ksw2_kernels.h"
 #include "ksw2_walk.h"
@@ -64,7 +68,7 @@ namespace kswhip {
 
 namespace {
 
-constexpr int kDppWaveShl1 = 0x130;
+constexpr int kDppWaveShl1 = 0x130, kDppWaveShr1 = 0x138;
 constexpr int kDppWaveRor1 = 0x13C;
 constexpr int kLag = kWave;      // steps the high stripe trails the low one
 constexpr int kAhead = 16;       // steps before a block its boundary entries are loaded
@@ -72,136 +76,55 @@ constexpr int kAhead = 16;       // steps before a block its boundary entries ar
 // What a pass stores per cell.
 enum Mode { kDirs = 0, kScoreOnly = 1, kTracks = 2 };
 
-typedef short v2s __attribute__((ext_vector_type(2)));
-typedef unsigned short v2u __attribute__((ext_vector_type(2)));
+using cell::bfi;
+using cell::hi16;
+using cell::lo16;
+using cell::perm;
+using cell::splat;
 
-__device__ __forceinline__ int bits(v2s v) { return __builtin_bit_cast(int, v); }
-__device__ __forceinline__ v2s vec(int x) { return __builtin_bit_cast(v2s, x); }
-__device__ __forceinline__ v2s splat(int x) { return (v2s){(short)x, (short)x}; }
-__device__ __forceinline__ v2s vmin(v2s a, v2s b) { return __builtin_elementwise_min(a, b); }
-__device__ __forceinline__ int lo16(int x) { return (int)(int16_t)(x & 0xffff); }
-__device__ __forceinline__ int hi16(int x) { return x >> 16; }
+// The cell of a mode and how far its sums are scaled (as a shift).
+template <bool RIGHT, int MODE> struct CellOf {
+    typedef cell::RawCell type;
+    static constexpr int shift = 0;
+};
+template <bool RIGHT> struct CellOf<RIGHT, kDirs> {
+    typedef cell::DirCell<RIGHT> type;
+    static constexpr int shift = 3;
+};
 
-// (a & m) | (b & ~m): one v_bfi_b32
-__device__ __forceinline__ int bfi(int m, int a, int b) { return (a & m) | (b & ~m); }
-
-// (a & m) | b as one v_and_or_b32
-__device__ __forceinline__ int and_or(int a, int m, int b)
+// Lane k takes lane k+1's value (lane 63 `old`), lane k takes lane k-1's
+// (lane 0 `old`), lane k takes lane k-1's (lane 0 lane 63's).
+__device__ __forceinline__ uint32_t dpp_shl1(uint32_t old, uint32_t src)
 {
-    int r;
-    asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "s"(m), "v"(b));
-    return r;
+    return (uint32_t)__builtin_amdgcn_update_dpp((int)old, (int)src, kDppWaveShl1, 0xF, 0xF, false);
 }
-
-__device__ __forceinline__ int dpp_shl1(int old, int src)
+__device__ __forceinline__ uint32_t dpp_shr1(uint32_t old, uint32_t src)
 {
-    return __builtin_amdgcn_update_dpp(old, src, kDppWaveShl1, 0xF, 0xF, false);
+    return (uint32_t)__builtin_amdgcn_update_dpp((int)old, (int)src, kDppWaveShr1, 0xF, 0xF, false);
+}
+__device__ __forceinline__ uint32_t dpp_ror1(uint32_t src)
+{
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)src, kDppWaveRor1, 0xF, 0xF, false);
 }
 
 // The value from the cell above for every lane: lane k takes lane k-1's
 // (both halves); lane 0 takes lane 63's low half of the previous step into
 // its high half, and the low stripe's boundary value (the high half of b_hi)
-// into its low half.
-__device__ __forceinline__ int carry(int y, int b_hi, bool lane0)
+// into its low half.  m0 is all ones in lane 0 (a bit operation: a
+// v_cndmask on a mask in VCC takes five times as long).
+__device__ __forceinline__ uint32_t carry(uint32_t y, uint32_t b_hi, uint32_t m0)
 {
-    const int rot = __builtin_amdgcn_update_dpp(0, y, kDppWaveRor1, 0xF, 0xF, false);
-    const int fix = (int)__builtin_amdgcn_alignbit((unsigned)rot, (unsigned)b_hi, 16);
-    return lane0 ? fix : rot;
+    const uint32_t rot = dpp_ror1(y);
+    return bfi(m0, __builtin_amdgcn_alignbit(rot, b_hi, 16), rot);
 }
 
-// Tags: state k = 0 (diagonal s), 1 (a), 2 (b), 3 (a2), 4 (b2).  Under
-// v_min the smallest tag wins a tie, so left alignment (first strict maximum)
-// tags k, right alignment (last maximum, '>=' chain) tags 7-k.
-template <bool RIGHT> struct Tags {
-    static constexpr int S = RIGHT ? 7 : 0, A = RIGHT ? 6 : 1, B = RIGHT ? 5 : 2;
-    static constexpr int A2 = RIGHT ? 4 : 3, B2 = RIGHT ? 3 : 4;
-};
-
-// Constants of the scaled representation (both halves):
-//   stored  U = -8u, V = -8v, X = -8(x+G1) - BIAS, X2 = -8(x2+G2) - BIAS,
-//           Y, Y2 likewise; BIAS = 0 (left) or 8 (right)
-//   cands   A = (X+V) + CA = -8a + tagA, ..., S = -8s + tagS
-//   update  T = (X+V) + 8e - (Z & ~7) = -8(a-z+q) - BIAS, X' = min(T, -BIAS)
-// A transposed pair (query in the stripes, target swept) has the cell above
-// and the cell to the left exchanged: its A and A2 candidates are the
-// reference's b and b2 (insertions), its B and B2 the reference's a and a2.
-// They take those candidates' tags and direction-byte flag bits, so the min
-// chain keeps the reference's tie order and the byte is the reference's byte.
-struct Consts {
-    v2s CA, CB, CA2, CB2, E1, E2, LIM, SM, SD;
-    v2u shA, shB, shA2, shB2;  // logical shift taking a T's sign (bit 15) to its flag bit
-    int mA, mB, mA2, mB2;      // that flag bit in both halves
-};
-
-template <bool RIGHT>
-__device__ __forceinline__ Consts make_consts(const KswScore &sc, bool transposed)
+// Element i (the same in every lane) of a lane's array.
+template <int R> __device__ __forceinline__ uint32_t row_of(const uint32_t (&v)[R], int i)
 {
-    using T = Tags<RIGHT>;
-    const int bias = RIGHT ? 8 : 0;
-    const int tA = transposed ? T::B : T::A, tB = transposed ? T::A : T::B;
-    const int tA2 = transposed ? T::B2 : T::A2, tB2 = transposed ? T::A2 : T::B2;
-    // flag bits of the reference's byte: a 3, b 4, a2 5, b2 6
-    const int fA = transposed ? 4 : 3, fB = transposed ? 3 : 4, fA2 = transposed ? 6 : 5, fB2 = transposed ? 5 : 6;
-    Consts k;
-    k.CA = splat(8 * sc.G1 + tA + bias);
-    k.CB = splat(8 * sc.G1 + tB + bias);
-    k.CA2 = splat(8 * sc.G2 + tA2 + bias);
-    k.CB2 = splat(8 * sc.G2 + tB2 + bias);
-    k.E1 = splat(8 * sc.e);
-    k.E2 = splat(8 * sc.e2);
-    k.LIM = splat(-bias);
-    k.SM = splat(-8 * sc.mch + T::S);
-    k.SD = splat(-8 * (sc.mis - sc.mch));
-    k.shA = (v2u){(unsigned short)(15 - fA), (unsigned short)(15 - fA)};
-    k.shB = (v2u){(unsigned short)(15 - fB), (unsigned short)(15 - fB)};
-    k.shA2 = (v2u){(unsigned short)(15 - fA2), (unsigned short)(15 - fA2)};
-    k.shB2 = (v2u){(unsigned short)(15 - fB2), (unsigned short)(15 - fB2)};
-    k.mA = 0x10001 << fA, k.mB = 0x10001 << fB, k.mA2 = 0x10001 << fA2, k.mB2 = 0x10001 << fB2;
-    return k;
-}
-
-// Two cells (low and high half).  In: X/X2/V from the cells above (replaced
-// by these cells' outputs for the cells below), U/Y/Y2 from the cells to the
-// left (replaced for the cells to the right), tb/qb the target and query
-// codes.  Returns the two direction bytes in the low byte of each half (0
-// when SCORE_ONLY).
-template <bool RIGHT, bool SCORE_ONLY>
-__device__ __forceinline__ int cell2(const Consts &k, v2s S, v2s &X, v2s &X2, v2s &V, v2s &U, v2s &Y, v2s &Y2)
-{
-    const v2s XV = X + V, X2V = X2 + V, YU = Y + U, Y2U = Y2 + U;
-    const v2s A = XV + k.CA, B = YU + k.CB, A2 = X2V + k.CA2, B2 = Y2U + k.CB2;
-    const v2s Z = vmin(vmin(vmin(vmin(S, A), B), A2), B2);
-    const v2s Z8 = vec(bits(Z) & (int)0xFFF8FFF8u);
-    const v2s M1 = k.E1 - Z8, M2 = k.E2 - Z8;
-    const v2s Ta = XV + M1, Tb = YU + M1, Ta2 = X2V + M2, Tb2 = Y2U + M2;
-    const v2s Un = Z8 - V, Vn = Z8 - U;
-    X = vmin(Ta, k.LIM), Y = vmin(Tb, k.LIM), X2 = vmin(Ta2, k.LIM), Y2 = vmin(Tb2, k.LIM);
-    U = Un, V = Vn;
-    if (SCORE_ONLY) return 0;
-    // state index (tags) and the four continuation flags (sign bits of T,
-    // each shifted to its bit of the byte)
-    int d = RIGHT ? (~bits(Z) & 0x00070007) : (bits(Z) & 0x00070007);
-    d = and_or(bits(__builtin_bit_cast(v2s, __builtin_bit_cast(v2u, Ta) >> k.shA)), k.mA, d);
-    d = and_or(bits(__builtin_bit_cast(v2s, __builtin_bit_cast(v2u, Tb) >> k.shB)), k.mB, d);
-    d = and_or(bits(__builtin_bit_cast(v2s, __builtin_bit_cast(v2u, Ta2) >> k.shA2)), k.mA2, d);
-    d = and_or(bits(__builtin_bit_cast(v2s, __builtin_bit_cast(v2u, Tb2) >> k.shB2)), k.mB2, d);
-    return d;
-}
-
-// Score candidate S of two cells (match/mismatch) from their codes: with
-// ONE = (1, 1) opaque to the optimiser, min(tb ^ qb, ONE) stays one
-// v_pk_min_u16 (0 match, 1 mismatch) and the score one v_pk_mad_u16.
-__device__ __forceinline__ v2s score_mm(const Consts &k, v2u tb, v2u qb, int one)
-{
-    const v2u mm = __builtin_elementwise_min(tb ^ qb, __builtin_bit_cast(v2u, one));
-    return k.SM + __builtin_bit_cast(v2s, mm) * k.SD;
-}
-
-// Sets one half of a packed register.
-__device__ __forceinline__ v2s set_half(v2s v, int value, bool hi)
-{
-    const int b = bits(v);
-    return vec(hi ? (b & 0xffff) | (value << 16) : (int)((unsigned)b & 0xffff0000u) | (value & 0xffff));
+    uint32_t x = v[0];
+#pragma unroll
+    for (int r = 1; r < R; ++r) x = bfi(i == r ? ~0u : 0u, v[r], x);
+    return x;
 }
 
 // Team progress: wave w publishes, for its k-th pass, k*(qlen+1) + the
@@ -271,37 +194,38 @@ __device__ __forceinline__ int wait_count_wide(const int32_t *slot, int need, in
 // Two column-buffer dwords (one entry): plain accesses within a workgroup,
 // device-scope ones across CUs.
 template <bool WIDE>
-__device__ __forceinline__ void load_entry(const int32_t *src, int &a, int &b)
+__device__ __forceinline__ void load_entry(const int32_t *src, uint32_t &a, uint32_t &b)
 {
     if (WIDE) {
         const uint64_t v = __hip_atomic_load((const uint64_t *)src, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        a = (int)(uint32_t)v, b = (int)(uint32_t)(v >> 32);
+        a = (uint32_t)v, b = (uint32_t)(v >> 32);
     } else {
-        a = src[0], b = src[1];
+        a = (uint32_t)src[0], b = (uint32_t)src[1];
     }
 }
 
 template <bool WIDE>
-__device__ __forceinline__ void store_entry(int32_t *dst, int a, int b)
+__device__ __forceinline__ void store_entry(int32_t *dst, uint32_t a, uint32_t b)
 {
     if (WIDE) {
-        const uint64_t v = (uint64_t)(uint32_t)a | (uint64_t)(uint32_t)b << 32;
+        const uint64_t v = (uint64_t)a | (uint64_t)b << 32;
         __hip_atomic_store((uint64_t *)dst, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     } else {
-        dst[0] = a, dst[1] = b;
+        dst[0] = (int32_t)a, dst[1] = (int32_t)b;
     }
 }
 
 // mqe partial of one stripe from the snapshot of U at column qlen-1 (one
-// half of Us): H(i,qlen-1) = H(-1,qlen-1) + sum_{i'<=i} u(i'), kept in the
-// -8 domain; the smallest running sum (largest H) with ties to the larger
-// row, and the stripe total.
+// half of Us, biased by p): H(i,qlen-1) = H(-1,qlen-1) + sum_{i'<=i} u(i'),
+// kept negated and scaled as the state; the smallest running sum (largest H)
+// with ties to the larger row, and the stripe total.
 template <int R>
-__device__ __forceinline__ void stripe_rec(const v2s (&Us)[R], bool hi, int i0, int tlen, int lane, StripeRec *out)
+__device__ __forceinline__ void stripe_rec(const uint32_t (&Us)[R], bool hi, int p, int i0, int tlen, int lane,
+                                           StripeRec *out)
 {
     int u[R], lsum = 0;
 #pragma unroll
-    for (int r = 0; r < R; ++r) u[r] = hi ? hi16(bits(Us[r])) : lo16(bits(Us[r])), lsum += u[r];
+    for (int r = 0; r < R; ++r) u[r] = (hi ? hi16(Us[r]) : lo16(Us[r])) - p, lsum += u[r];
     int incl = lsum;
 #pragma unroll
     for (int off = 1; off < kWave; off <<= 1) {
@@ -330,25 +254,62 @@ __device__ __forceinline__ void stripe_rec(const v2s (&Us)[R], bool hi, int i0, 
     }
 }
 
+// What follows row tlen-1 over a pair's columns: the sum of v so far, its
+// smallest value and the last column that has it (negated and scaled).
+struct RowTrack {
+    int acc = 0, best = 0x7fffffff, col = -1;
+};
+
+// Takes 64 columns of row tlen-1: lane l's v of column col (valid when
+// 0 <= col < qlen, the columns ascending with the lane).
+__device__ __forceinline__ void track_row(RowTrack &t, int v, int col, int qlen, int lane)
+{
+    const bool in = col >= 0 && col < qlen;
+    int sum = in ? v : 0;
+#pragma unroll
+    for (int off = 1; off < kWave; off <<= 1) {
+        const int o = __shfl_up(sum, off, kWave);
+        if (lane >= off) sum += o;
+    }
+    sum += t.acc;
+    int best = in ? sum : 0x7fffffff, at = in ? col : -1;
+#pragma unroll
+    for (int off = 1; off < kWave; off <<= 1) {
+        const int ob = __shfl_xor(best, off, kWave), oa = __shfl_xor(at, off, kWave);
+        if (ob < best || (ob == best && oa > at)) best = ob, at = oa;
+    }
+    t.acc = __builtin_amdgcn_readlane(sum, kWave - 1);
+    if (best <= t.best && at >= 0) t.best = best, t.col = at;
+}
+
 // One pass (stripes 2p and 2p+1) of one pair, computed by the calling wave.
 // Roles (uniform): the first pass takes row -1 as the low stripe's upper
 // boundary instead of the column buffer; the last pass holds row tlen-1
 // (score / mte) and publishes nothing; every other pass publishes the high
 // stripe's bottom row.  Lanes compute every step; each half's left state is
 // (re)initialised at its first column and U is snapshot at its last one, so
-// the cells a half computes outside its columns never reach a result.
+// the cells a half computes outside its columns never reach a result (they
+// are cells of the same recurrence under a boundary of constant H, so they
+// stay in range).
+// Columns go in blocks of 64: the boundary entries and query codes of a block
+// are loaded one per lane, kAhead steps before it, and move to lane 0 one
+// step at a time.  A block clear of starts and ends runs several steps per
+// loop iteration, without their tests.  LAST: the pass that holds row tlen-1.
 // WIDE: the team spans several CUs (progress counts in device memory,
 // kWideCtlStride dwords apart; a wait that gives up sets `late`).
-template <bool RIGHT, int MODE, bool WIDE, bool LUT, int R>
-__device__ __forceinline__ void pass_body(const StripeArgs &a, const Consts &kc, int job_id, int p, const KswJob &jb,
-                                          int qlen, int tlen, int32_t *prog, int W, int &late, int &stop)
+template <bool RIGHT, int MODE, bool WIDE, bool LUT, int R, bool LAST>
+__device__ __forceinline__ void pass_run(const StripeArgs &a, const typename CellOf<RIGHT, MODE>::type &kc, int job_id,
+                                          int p, const KswJob &jb, int qlen, int tlen, int32_t *prog, int W, int &late,
+                                          int &stop)
 {
-    constexpr int SR = kWave * R;  // rows per stripe
+    constexpr int SR = kWave * R;           // rows per stripe
+    constexpr int kUnroll = R == 8 ? 2 : 4;  // steps per iteration of a plain block
     const KswScore &sc = a.sc;
-    const int nstripes = (tlen + SR - 1) / SR, npass = (nstripes + 1) / 2;
-    const bool first = p == 0, last = p == npass - 1, has_hi = 2 * p + 1 < nstripes;
+    const int nstripes = (tlen + SR - 1) / SR;
+    const bool first = p == 0, has_hi = 2 * p + 1 < nstripes;
     const int lane = threadIdx.x % kWave;
-    const bool lane0 = lane == 0;
+    uint32_t m0 = lane == 0 ? ~0u : 0u;
+    asm volatile("" : "+v"(m0));
     const uint8_t *qs = a.seq + jb.q_off;
     const uint8_t *ts = a.seq + jb.t_off;
     uint8_t *dir = a.dir + jb.dir_off;
@@ -356,7 +317,7 @@ __device__ __forceinline__ void pass_body(const StripeArgs &a, const Consts &kc,
     const int nsteps = qlen + kWave - 1 + kLag;
     // row tlen-1 (score, mte): stripe s_last, half h_last of the last pass
     const int h_last = ((tlen - 1) / SR) & 1;
-    const int rho_last = last ? (tlen - 1) % R : -1;
+    const int rho_last = (tlen - 1) % R;
     const int lane_last = ((tlen - 1) % SR) / R;
     // progress slots: pass p-1 is wave (p-1) % W's ((p-1)/W)-th pass
     constexpr int PS = WIDE ? kWideCtlStride : 1;
@@ -366,43 +327,160 @@ __device__ __forceinline__ void pass_body(const StripeArgs &a, const Consts &kc,
     const int base_mine = p / W * (qlen + 1);
 
     const int ilo = 2 * p * SR + lane * R, ihi = ilo + SR;  // this lane's first rows
-    v2u TB[R];
-    v2s U[R], Y[R], Y2[R], Us[R];
+    uint32_t TB[R], Us[R];
+    cell::Right st[R];
 #pragma unroll
     for (int r = 0; r < R; ++r) {
         const int tl = ilo + r < tlen ? (int)ts[ilo + r] : 0, th = ihi + r < tlen ? (int)ts[ihi + r] : 0;
         // LUT: the v_perm selector of row r's two score bytes (table byte
         // tl of the low half's table, byte th of the high half's, zero high
         // bytes); else the two target codes
-        TB[r] = LUT ? __builtin_bit_cast(v2u, (uint32_t)tl | 12u << 8 | (uint32_t)(th + 4) << 16 | 12u << 24)
-                    : (v2u){(unsigned short)tl, (unsigned short)th};
-        U[r] = (v2s){(short)(-8 * edge_diff(sc, ilo + r)), (short)(-8 * edge_diff(sc, ihi + r))};
-        Y[r] = kc.LIM, Y2[r] = kc.LIM, Us[r] = U[r];
+        TB[r] = LUT ? ((uint32_t)tl | 12u << 8 | (uint32_t)(th + 4) << 16 | 12u << 24)
+                    : ((uint32_t)tl | (uint32_t)th << 16);
+        Us[r] = (uint32_t)(kc.diff(edge_diff(sc, ilo + r)) & 0xffff) | (uint32_t)kc.diff(edge_diff(sc, ihi + r)) << 16;
+        st[r].u = Us[r], st[r].y = kc.y0(), st[r].y2 = kc.y20();
     }
-    int row_acc = 0, mte_best = 0x7fffffff, mte_j = -1;  // row tlen-1 in the -8 domain
-    int Xo = bits(kc.LIM), X2o = bits(kc.LIM), Vo = 0, Qo = 0;  // this lane's bottom-row outputs
-    int bin0 = 0, bin1 = 0, bnx0 = 0, bnx1 = 0;  // lane-0 boundary queue (rotating), next block
-    int out0 = 0, out1 = 0;                      // lane-63 output queue (rotating)
-    int known = 0;                               // columns of pass p-1 known published
-    auto wait_prev = [&](int need) {
-        if (WIDE) known = wait_count_wide(prog_prev, need, known, late);
-        else known = wait_count(prog_prev, need, known);
+    const uint32_t p2 = splat(kc.p);  // v of a boundary of constant H
+    cell::Down down;                  // this lane's bottom-row outputs
+    down.x = kc.x0(), down.x2 = kc.x20(), down.v = p2;
+    // The lane-0 queues: x (high half) and x2 of the boundary; its v (high
+    // half), with the query code in the low half when there is no table; the
+    // score table of the query code.
+    const uint32_t entry0 = (kc.x0() & 0xffff0000u) | (kc.x20() & 0xffffu);
+    // LUT: byte k of a half's table is the score candidate of target code k
+    // against that half's query code (sm when equal, sx otherwise)
+    const uint32_t sx_rep = (uint32_t)(kc.sx & 0xff) * 0x01010101u;
+    const uint32_t s_flip = (uint32_t)((kc.sm ^ kc.sx) & 0xff);
+    int known = 0;  // columns of pass p-1 known published
+    auto load_block = [&](int nb, uint32_t &e0, uint32_t &e1, uint32_t &eq) {
+        const int col = nb + lane;
+        e0 = entry0, e1 = p2 & 0xffff0000u;
+        if (first) {
+            e1 = (uint32_t)kc.diff(edge_diff(sc, col)) << 16;
+        } else {
+            const int need = base_prev + min(nb + kWave, qlen);
+            if (WIDE) known = wait_count_wide(prog_prev, need, known, late);
+            else known = wait_count(prog_prev, need, known);
+            if (col < qlen) load_entry<WIDE>(bnd + 2 * col, e0, e1);
+        }
+        eq = col < qlen ? (uint32_t)qs[col] : 0u;
+        if (!LUT) e1 = (e1 & 0xffff0000u) | eq;
     };
-    if (!first) {
-        wait_prev(base_prev + min(kWave, qlen));
-        if (lane < qlen) load_entry<WIDE>(bnd + 2 * lane, bin0, bin1);
-    }
-    const int lim_hi = bits(kc.LIM) << 16;
-    // LUT: per step, byte k of a half's table is the score candidate of
-    // target code k against that half's query code (SM when equal, SX
-    // otherwise); the query codes travel as 8 * code
-    const uint32_t sx_rep = (uint32_t)(lo16(bits(kc.SM + kc.SD)) & 0xff) * 0x01010101u;
-    const uint32_t s_flip = (uint32_t)((lo16(bits(kc.SM)) ^ lo16(bits(kc.SM + kc.SD))) & 0xff);
-    int one = 0x00010001;
+    uint32_t bin0, bin1, binq, nx0 = 0, nx1 = 0, nxq = 0;
+    load_block(0, bin0, bin1, binq);
+    if (LUT) binq = sx_rep ^ (s_flip << (8 * binq));
+    uint32_t tab_lo = sx_rep, tab_hi = sx_rep, code = 0;
+    uint32_t out0 = 0, out1 = 0;  // lane-63 output queue; in the last pass out1 holds row tlen-1's v
+    RowTrack row;
+    uint32_t one = 0x00010001u;
     asm volatile("" : "+s"(one));
-    uint32_t qword = 0;
-    for (int c = 0; c < nsteps; ++c) {
-        if (a.stop && (c & 255) == 0) {
+    const uint32_t sm2 = splat(kc.sm), sd2 = splat(kc.sx - kc.sm);
+    uint8_t *dst = dir + ((uint64_t)p * nsteps * kWave + lane) * (MODE == kTracks ? 4 * R : 2 * R);
+
+    auto step = [&](int c, auto edge) {
+        constexpr bool EDGE = decltype(edge)::value;
+        // this step's inputs from above, the queues one step on
+        cell::Down d;
+        d.x = carry(down.x, bin0, m0), d.x2 = carry(down.x2, bin0 << 16, m0), d.v = carry(down.v, bin1, m0);
+        if (LUT) {
+            tab_hi = dpp_shr1(dpp_ror1(tab_lo), tab_hi);
+            const uint32_t q0 = binq;
+            binq = dpp_shl1(0, binq);
+            tab_lo = dpp_shr1(q0, tab_lo);
+        } else {
+            code = carry(code, bin1 << 16, m0);
+        }
+        bin0 = dpp_shl1(0, bin0), bin1 = dpp_shl1(0, bin1);
+        const int jl = c - lane;
+        if (EDGE) {
+            // a half starts at its first column: the lanes there take the
+            // half's initial left state (U from Us, which holds it until the
+            // half's last column)
+            const uint32_t m = jl == 0 ? 0x0000ffffu : jl == kLag ? 0xffff0000u : 0u;
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                st[r].u = bfi(m, Us[r], st[r].u);
+                st[r].y = bfi(m, kc.y0(), st[r].y), st[r].y2 = bfi(m, kc.y20(), st[r].y2);
+            }
+        }
+        cell::DirWord w[R];
+        uint32_t vr[R];
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            uint32_t s;
+            if (LUT) {
+                s = perm(tab_hi, tab_lo, TB[r]);
+            } else {
+                // min(t ^ q, ONE) with an opaque ONE stays one v_pk_min_u16 (0
+                // match, 1 mismatch), the score one v_pk_mad_u16
+                const cell::v2u mm = __builtin_elementwise_min(__builtin_bit_cast(cell::v2u, TB[r] ^ code),
+                                                               __builtin_bit_cast(cell::v2u, one));
+                s = __builtin_bit_cast(uint32_t, __builtin_bit_cast(cell::v2u, sm2) +
+                                                     mm * __builtin_bit_cast(cell::v2u, sd2));
+            }
+            w[r] = kc.step(s, d, st[r]);
+            vr[r] = d.v;
+        }
+        down = d;
+        if (EDGE) {
+            // a half ends at column qlen-1: keep U for the mqe partials
+            const int je = jl - (qlen - 1);
+            const uint32_t m = je == 0 ? 0x0000ffffu : je == kLag ? 0xffff0000u : 0u;
+#pragma unroll
+            for (int r = 0; r < R; ++r) Us[r] = bfi(m, st[r].u, Us[r]);
+        }
+        if (MODE == kDirs) {
+            // 2R bytes per lane: byte 4g + 2h + (rho & 1) is row 2g + (rho & 1)
+            // of half h
+            if (R == 8) {
+                uint4 o;
+                o.x = kc.pack(w[0], w[1]), o.y = kc.pack(w[2], w[3]);
+                o.z = kc.pack(w[4 % R], w[5 % R]), o.w = kc.pack(w[6 % R], w[7 % R]);
+                *(uint4 *)dst = o;
+            } else {
+                uint2 o;
+                o.x = kc.pack(w[0], w[1]), o.y = kc.pack(w[2], w[3]);
+                *(uint2 *)dst = o;
+            }
+            dst += kWave * 2 * R;
+        } else if (MODE == kTracks) {
+            // 4R bytes per lane: the p track (new V) then the p2 track (new
+            // U), each in the byte order of the direction bytes
+            uint32_t tv[R / 2], tu[R / 2];
+#pragma unroll
+            for (int g = 0; g < R / 2; ++g) {
+                tv[g] = perm(vr[2 * g + 1], vr[2 * g], 0x06020400u);
+                tu[g] = perm(st[2 * g + 1].u, st[2 * g].u, 0x06020400u);
+            }
+            if (R == 8) {
+                uint4 o;
+                o.x = tv[0], o.y = tv[1], o.z = tv[2 % (R / 2)], o.w = tv[3 % (R / 2)];
+                ((uint4 *)dst)[0] = o;
+                o.x = tu[0], o.y = tu[1], o.z = tu[2 % (R / 2)], o.w = tu[3 % (R / 2)];
+                ((uint4 *)dst)[1] = o;
+            } else {
+                uint2 o;
+                o.x = tv[0], o.y = tv[1];
+                ((uint2 *)dst)[0] = o;
+                o.x = tu[0], o.y = tu[1];
+                ((uint2 *)dst)[1] = o;
+            }
+            dst += kWave * 4 * R;
+        }
+        if (!LAST) {
+            // lane 63 appends the high stripe's bottom-row output (column
+            // c-127: x in the high half, x2 in the low half; v in the high
+            // half) to the queue
+            out0 = dpp_shl1(perm(down.x, down.x2, 0x07060302u), out0), out1 = dpp_shl1(down.v, out1);
+        } else {
+            // row tlen-1's v joins the queue
+            out1 = dpp_shl1((uint32_t)__builtin_amdgcn_readlane((int)row_of<R>(vr, rho_last), lane_last), out1);
+        }
+    };
+
+#pragma unroll 1
+    for (int c0 = 0; c0 < nsteps; c0 += kWave) {
+        if (a.stop && (c0 & 255) == 0) {
             // the host's stop flag: publish a count past every wait of the
             // team and end (nothing of this pair is delivered)
             stop = __builtin_amdgcn_readfirstlane(__hip_atomic_load(a.stop, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM));
@@ -412,171 +490,65 @@ __device__ __forceinline__ void pass_body(const StripeArgs &a, const Consts &kc,
                 return;
             }
         }
-        // lane 0's low-stripe inputs for column c, each in a high half
-        int bxh, bx2h, bvh;
-        if (first) {
-            bxh = lim_hi, bx2h = lim_hi, bvh = (-8 * edge_diff(sc, c)) << 16;
+        const int c1 = min(c0 + kWave, nsteps), nb = c0 + kWave;
+        const bool plain = c0 >= kWave + kLag && nb < qlen;
+        // the next block's entries are waited for and loaded kAhead steps
+        // before it starts (late enough that the producer need only be that
+        // far ahead, early enough to hide the load)
+        for (int c = c0, end = min(nb - kAhead, c1);; end = c1) {
+            if (plain) {
+#pragma unroll 1
+                for (; c < end; c += kUnroll) {
+#pragma unroll
+                    for (int k = 0; k < kUnroll; ++k) step(c + k, std::integral_constant<bool, false>());
+                }
+            } else {
+#pragma unroll 1
+                for (; c < end; ++c) step(c, std::integral_constant<bool, true>());
+            }
+            if (c >= c1) break;
+            load_block(nb, nx0, nx1, nxq);
+        }
+        bin0 = nx0, bin1 = nx1;
+        if (LUT) binq = sx_rep ^ (s_flip << (8 * nxq));
+        if (!LAST) {
+            // the queue's columns go out, the newest in lane 63
+            const int col = c1 - kWave - kLag - (kWave - 1) + lane;
+            if (col >= 0 && col < qlen) store_entry<WIDE>(bnd + 2 * col, out0, out1);
+            const int count = base_mine + max(0, min(c1 - (kWave - 1) - kLag, qlen));
+            if (WIDE) publish_wide(prog_mine, count);
+            else publish(prog_mine, count);
         } else {
-            bxh = bin0, bx2h = bin0 << 16, bvh = bin1;
-        }
-        if ((c & 3) == 0) qword = c < qlen ? *(const uint32_t *)(qs + c) : 0u;
-        const int qh = (int)((qword >> (8 * (c & 3))) & 0xffu) << (LUT ? 19 : 16);
-        v2s X = vec(carry(Xo, bxh, lane0)), X2 = vec(carry(X2o, bx2h, lane0)), V = vec(carry(Vo, bvh, lane0));
-        const int Qw = carry(Qo, qh, lane0);
-        if (!first) {
-            // rotate the queue so lane 0 sees column c+1 next step; the
-            // next block's entries are waited for and loaded kAhead steps
-            // before the block starts (late enough that the producer need
-            // only be that far ahead, early enough to hide the load)
-            if ((c & (kWave - 1)) == kWave - 1 - kAhead) {
-                const int nb = c + 1 + kAhead;  // the next block's first column
-                wait_prev(base_prev + min(nb + kWave, qlen));
-                bnx0 = 0, bnx1 = 0;
-                if (nb + lane < qlen) load_entry<WIDE>(bnd + 2 * (nb + lane), bnx0, bnx1);
-            }
-            if ((c & (kWave - 1)) == kWave - 1) {
-                bin0 = bnx0, bin1 = bnx1;
-            } else {
-                bin0 = dpp_shl1(0, bin0), bin1 = dpp_shl1(0, bin1);
-            }
-        }
-        // a half starts at its first column: the lanes there take the
-        // half's initial left state (U from Us, which holds it until the
-        // half's last column; only the first 128 steps can hold a start, the
-        // guard is wave-uniform)
-        const int jl = c - lane;
-        if (c < kWave + kLag) {
-            const int m = jl == 0 ? 0x0000ffff : jl == kLag ? (int)0xffff0000u : 0;
-#pragma unroll
-            for (int r = 0; r < R; ++r) {
-                U[r] = vec(bfi(m, bits(Us[r]), bits(U[r])));
-                Y[r] = vec(bfi(m, bits(kc.LIM), bits(Y[r]))), Y2[r] = vec(bfi(m, bits(kc.LIM), bits(Y2[r])));
-            }
-        }
-        const v2u qb = __builtin_bit_cast(v2u, Qw);
-        uint32_t tab_lo = 0, tab_hi = 0;
-        if (LUT) {
-            tab_lo = sx_rep ^ (s_flip << (Qw & 31));
-            tab_hi = sx_rep ^ (s_flip << ((Qw >> 16) & 31));
-        }
-        auto score = [&](int r) -> v2s {
-            return LUT ? vec((int)__builtin_amdgcn_perm(tab_hi, tab_lo, bits(__builtin_bit_cast(v2s, TB[r]))))
-                       : score_mm(kc, TB[r], qb, one);
-        };
-        int d[R];
-        if (!last) {
-#pragma unroll
-            for (int r = 0; r < R; ++r) {
-                d[r] = cell2<RIGHT, MODE != kDirs>(kc, score(r), X, X2, V, U[r], Y[r], Y2[r]);
-                if (MODE == kTracks) d[r] = bits(V);
-            }
-        } else {
-            // the last pass also follows V along row tlen-1
-            v2s vl = V;
-#pragma unroll
-            for (int r = 0; r < R; ++r) {
-                d[r] = cell2<RIGHT, MODE != kDirs>(kc, score(r), X, X2, V, U[r], Y[r], Y2[r]);
-                if (MODE == kTracks) d[r] = bits(V);
-                if (r == rho_last) vl = V;
-            }
-            const int jh = jl - kLag * h_last;
-            const int v = h_last ? hi16(bits(vl)) : lo16(bits(vl));
-            if (lane == lane_last && jh >= 0 && jh < qlen) {
-                row_acc += v;
-                if (row_acc <= mte_best) mte_best = row_acc, mte_j = jh;
-            }
-        }
-        // a half ends at column qlen-1: keep U for the mqe partials
-        if (c >= qlen - 1 && c < qlen - 1 + kWave + kLag) {
-            const int je = jl - (qlen - 1);
-            const int m = je == 0 ? 0x0000ffff : je == kLag ? (int)0xffff0000u : 0;
-#pragma unroll
-            for (int r = 0; r < R; ++r) Us[r] = vec(bfi(m, bits(U[r]), bits(Us[r])));
-        }
-        Xo = bits(X), X2o = bits(X2), Vo = bits(V), Qo = Qw;
-        if (MODE == kDirs) {
-            // 2R bytes per lane: byte 4g + 2h + (rho & 1) is row 2g + (rho & 1)
-            // of half h
-            uint8_t *dst = dir + (((uint64_t)p * nsteps + c) * kWave + lane) * (2 * R);
-            if (R == 8) {
-                uint4 w;
-                w.x = __builtin_amdgcn_perm((unsigned)d[1], (unsigned)d[0], 0x06020400u);
-                w.y = __builtin_amdgcn_perm((unsigned)d[3], (unsigned)d[2], 0x06020400u);
-                w.z = __builtin_amdgcn_perm((unsigned)d[5 % R], (unsigned)d[4 % R], 0x06020400u);
-                w.w = __builtin_amdgcn_perm((unsigned)d[7 % R], (unsigned)d[6 % R], 0x06020400u);
-                *(uint4 *)dst = w;
-            } else {
-                uint2 w;
-                w.x = __builtin_amdgcn_perm((unsigned)d[1], (unsigned)d[0], 0x06020400u);
-                w.y = __builtin_amdgcn_perm((unsigned)d[3], (unsigned)d[2], 0x06020400u);
-                *(uint2 *)dst = w;
-            }
-        } else if (MODE == kTracks) {
-            // 4R bytes per lane: the p track (new V) then the p2 track (new
-            // U), each in the byte order of the direction bytes; a value is
-            // stored as -8w >> 3 = -w (exact: both are multiples of 8)
-            int vt[R], ut[R];
-#pragma unroll
-            for (int r = 0; r < R; ++r) {
-                vt[r] = bits(vec(d[r]) >> (v2s){3, 3});
-                ut[r] = bits(U[r] >> (v2s){3, 3});
-            }
-            uint8_t *dst = dir + (((uint64_t)p * nsteps + c) * kWave + lane) * (4 * R);
-            if (R == 8) {
-                uint4 wv, wu;
-                wv.x = __builtin_amdgcn_perm((unsigned)vt[1], (unsigned)vt[0], 0x06020400u);
-                wv.y = __builtin_amdgcn_perm((unsigned)vt[3], (unsigned)vt[2], 0x06020400u);
-                wv.z = __builtin_amdgcn_perm((unsigned)vt[5 % R], (unsigned)vt[4 % R], 0x06020400u);
-                wv.w = __builtin_amdgcn_perm((unsigned)vt[7 % R], (unsigned)vt[6 % R], 0x06020400u);
-                wu.x = __builtin_amdgcn_perm((unsigned)ut[1], (unsigned)ut[0], 0x06020400u);
-                wu.y = __builtin_amdgcn_perm((unsigned)ut[3], (unsigned)ut[2], 0x06020400u);
-                wu.z = __builtin_amdgcn_perm((unsigned)ut[5 % R], (unsigned)ut[4 % R], 0x06020400u);
-                wu.w = __builtin_amdgcn_perm((unsigned)ut[7 % R], (unsigned)ut[6 % R], 0x06020400u);
-                ((uint4 *)dst)[0] = wv, ((uint4 *)dst)[1] = wu;
-            } else {
-                uint2 wv, wu;
-                wv.x = __builtin_amdgcn_perm((unsigned)vt[1], (unsigned)vt[0], 0x06020400u);
-                wv.y = __builtin_amdgcn_perm((unsigned)vt[3], (unsigned)vt[2], 0x06020400u);
-                wu.x = __builtin_amdgcn_perm((unsigned)ut[1], (unsigned)ut[0], 0x06020400u);
-                wu.y = __builtin_amdgcn_perm((unsigned)ut[3], (unsigned)ut[2], 0x06020400u);
-                ((uint2 *)dst)[0] = wv, ((uint2 *)dst)[1] = wu;
-            }
-        }
-        if (!last) {
-            // lane 63 appends the high stripe's bottom-row output (column
-            // c-127: x in the high half, x2 in the low half; v in the high
-            // half) to the queue; every 64 steps the queue is written out
-            const int w0 = (int)__builtin_amdgcn_perm((unsigned)Xo, (unsigned)X2o, 0x07060302u);
-            out0 = dpp_shl1(w0, out0), out1 = dpp_shl1(Vo, out1);
-            if ((c & (kWave - 1)) == kWave - 1 || c == nsteps - 1) {
-                const int col = c - (kWave - 1) - kLag - (kWave - 1) + lane;
-                if (col >= 0 && col < qlen) store_entry<WIDE>(bnd + 2 * col, out0, out1);
-                const int count = base_mine + max(0, min(c - (kWave - 1) - kLag + 1, qlen));
-                if (WIDE) publish_wide(prog_mine, count);
-                else publish(prog_mine, count);
-            }
+            const int v = (h_last ? hi16(out1) : lo16(out1)) - kc.p, c = c1 - kWave + lane;
+            track_row(row, v, c >= c0 ? c - lane_last - kLag * h_last : -1, qlen, lane);
         }
     }
-    stripe_rec<R>(Us, false, ilo, tlen, lane, a.recs + jb.stripe_off + 2 * p);
-    if (has_hi) stripe_rec<R>(Us, true, ihi, tlen, lane, a.recs + jb.stripe_off + 2 * p + 1);
-    if (last) {
-        // score / mte from the lane that owns row tlen-1
-        const int sc_row = __builtin_amdgcn_readlane(row_acc, lane_last);
-        const int mte_b = __builtin_amdgcn_readlane(mte_best, lane_last);
-        const int mte_jj = __builtin_amdgcn_readlane(mte_j, lane_last);
-        if (lane == 0) {
-            const int64_t h_anchor = (int64_t)sc.G1 - sc.qe_orig;
-            const int h_left_last_row = (int)(h_anchor + edge_prefix(sc, tlen - 1));  // H(tlen-1, -1)
-            KswOut o;
-            o.score = h_left_last_row - (sc_row >> 3);
-            o.mte = h_left_last_row - (mte_b >> 3);
-            o.mte_q = mte_jj;
-            o.mqe = KSW_NEG_INF_I, o.mqe_t = -1;  // finalised by the backtrack kernel
-            o.max = 0, o.max_t = -1, o.max_q = -1;
-            o.zdropped = 0, o.stopped = 0, o.reach_end = 0, o.n_cigar = 0;
-            a.out[job_id] = o;
-        }
+    stripe_rec<R>(Us, false, kc.p, ilo, tlen, lane, a.recs + jb.stripe_off + 2 * p);
+    if (has_hi) stripe_rec<R>(Us, true, kc.p, ihi, tlen, lane, a.recs + jb.stripe_off + 2 * p + 1);
+    if (LAST && lane == 0) {
+        constexpr int SH = CellOf<RIGHT, MODE>::shift;
+        const int64_t h_anchor = (int64_t)sc.G1 - sc.qe_orig;
+        const int h_left_last_row = (int)(h_anchor + edge_prefix(sc, tlen - 1));  // H(tlen-1, -1)
+        KswOut o;
+        o.score = h_left_last_row - (row.acc >> SH);
+        o.mte = h_left_last_row - (row.best >> SH);
+        o.mte_q = row.col;
+        o.mqe = KSW_NEG_INF_I, o.mqe_t = -1;  // finalised by the backtrack kernel
+        o.max = 0, o.max_t = -1, o.max_q = -1;
+        o.zdropped = 0, o.stopped = 0, o.reach_end = 0, o.n_cigar = 0;
+        a.out[job_id] = o;
     }
+}
+
+template <bool RIGHT, int MODE, bool WIDE, bool LUT, int R>
+__device__ __forceinline__ void pass_body(const StripeArgs &a, const typename CellOf<RIGHT, MODE>::type &kc, int job_id,
+                                          int p, const KswJob &jb, int qlen, int tlen, int32_t *prog, int W, int &late,
+                                          int &stop)
+{
+    if (p == pass_count(tlen, R) - 1)
+        pass_run<RIGHT, MODE, WIDE, LUT, R, true>(a, kc, job_id, p, jb, qlen, tlen, prog, W, late, stop);
+    else
+        pass_run<RIGHT, MODE, WIDE, LUT, R, false>(a, kc, job_id, p, jb, qlen, tlen, prog, W, late, stop);
 }
 
 }  // namespace
@@ -632,10 +604,11 @@ struct StripeTracks {
     __device__ int32_t cost(int i, int j) const { return ts[i] == qs[j] ? mch : mis; }
 };
 
-template <int R>
+template <int R, int MODE>
 __device__ __forceinline__ void pair_epilogue(const StripeArgs &a, int job_id, const KswJob &jb,
-                                              uint64_t (*tile)[64], bool tracks, int *shared_n, int nthr)
+                                              uint64_t (*tile)[64], int *shared_n, int nthr)
 {
+    constexpr bool tracks = MODE == kTracks;
     constexpr int SR = kWave * R;  // rows per stripe
     const int tid = threadIdx.x;
     // the host's stop flag, read once for the whole workgroup: a stopped
@@ -665,7 +638,7 @@ __device__ __forceinline__ void pair_epilogue(const StripeArgs &a, int job_id, c
         }
         const int64_t h_anchor = (int64_t)a.sc.G1 - a.sc.qe_orig;
         const int h_top_last_col = (int)(h_anchor + edge_prefix(a.sc, kq - 1));  // H(-1, kq-1)
-        const int col_max = h_top_last_col - (best >> 3);
+        const int col_max = h_top_last_col - (best >> CellOf<false, MODE>::shift);
         if (!tr) {
             o.mqe = col_max, o.mqe_t = best_i;
         } else {
@@ -841,7 +814,7 @@ __device__ __forceinline__ void pair_epilogue(const StripeArgs &a, int job_id, c
 // once (s_barrier then waits on the surviving waves only), so pairs of
 // different team sizes share one launch.  Wave w computes passes w, w+W,
 // ...; then the team runs the pair's epilogue (mqe, start cell, backtrack).
-template <bool RIGHT, int MODE, int R>
+template <bool RIGHT, int MODE, int R, bool LUT>
 __global__ void __launch_bounds__(kWave * kMaxTeam) ksw_stripe_kernel(StripeArgs a)
 {
     constexpr int SR = kWave * R;
@@ -855,18 +828,14 @@ __global__ void __launch_bounds__(kWave * kMaxTeam) ksw_stripe_kernel(StripeArgs
     if (w >= W) return;
     prog[w] = 0;  // every lane of wave w writes the same zero
     __syncthreads();
-    const Consts kc = make_consts<RIGHT>(a.sc, jb.transposed != 0);
+    const typename CellOf<RIGHT, MODE>::type kc(a.sc, jb.transposed != 0);
     const int qlen = __builtin_amdgcn_readfirstlane(jb.qlen), tlen = __builtin_amdgcn_readfirstlane(jb.tlen);
     const int npass = ((tlen + SR - 1) / SR + 1) / 2;
     int late = 0, stop = 0;  // (no bounded waits within a workgroup)
-    if (jb.lut)
-        for (int p = w; p < npass && !stop; p += W)
-            pass_body<RIGHT, MODE, false, true, R>(a, kc, job, p, jb, qlen, tlen, prog, W, late, stop);
-    else
-        for (int p = w; p < npass && !stop; p += W)
-            pass_body<RIGHT, MODE, false, false, R>(a, kc, job, p, jb, qlen, tlen, prog, W, late, stop);
+    for (int p = w; p < npass && !stop; p += W)
+        pass_body<RIGHT, MODE, false, LUT, R>(a, kc, job, p, jb, qlen, tlen, prog, W, late, stop);
     __syncthreads();  // every pass written: stripe partials, score / mte, direction bytes
-    pair_epilogue<R>(a, job, jb, tile, MODE == kTracks, &shared_n, W * kWave);
+    pair_epilogue<R, MODE>(a, job, jb, tile, &shared_n, W * kWave);
 }
 
 // Persistent one-wave workers over a device work queue.  The launch's job
@@ -878,7 +847,7 @@ __global__ void __launch_bounds__(kWave * kMaxTeam) ksw_stripe_kernel(StripeArgs
 // each pass to the next through the wave's own LDS count.  qhead is zero at
 // launch (ksw_stripe_qhead_kernel, a fill kernel rather than a memset so a
 // captured graph replays it).
-template <bool RIGHT, int MODE, int R>
+template <bool RIGHT, int MODE, int R, bool LUT>
 __global__ void __launch_bounds__(kWave) __attribute__((amdgpu_waves_per_eu(4)))
 ksw_stripe_queue_kernel(StripeArgs a, int32_t *qhead)
 {
@@ -895,18 +864,14 @@ ksw_stripe_queue_kernel(StripeArgs a, int32_t *qhead)
         const KswJob jb = a.jobs[job];
         prog[0] = 0;
         __syncthreads();
-        const Consts kc = make_consts<RIGHT>(a.sc, jb.transposed != 0);
+        const typename CellOf<RIGHT, MODE>::type kc(a.sc, jb.transposed != 0);
         const int qlen = __builtin_amdgcn_readfirstlane(jb.qlen), tlen = __builtin_amdgcn_readfirstlane(jb.tlen);
         const int npass = ((tlen + SR - 1) / SR + 1) / 2;
         int late = 0, stop = 0;
-        if (jb.lut)
-            for (int p = 0; p < npass && !stop; ++p)
-                pass_body<RIGHT, MODE, false, true, R>(a, kc, job, p, jb, qlen, tlen, prog, 1, late, stop);
-        else
-            for (int p = 0; p < npass && !stop; ++p)
-                pass_body<RIGHT, MODE, false, false, R>(a, kc, job, p, jb, qlen, tlen, prog, 1, late, stop);
+        for (int p = 0; p < npass && !stop; ++p)
+            pass_body<RIGHT, MODE, false, LUT, R>(a, kc, job, p, jb, qlen, tlen, prog, 1, late, stop);
         __syncthreads();
-        pair_epilogue<R>(a, job, jb, tile, MODE == kTracks, &shared_n, kWave);
+        pair_epilogue<R, MODE>(a, job, jb, tile, &shared_n, kWave);
         __syncthreads();  // tile and prog are the next pair's
     }
 }
@@ -921,7 +886,7 @@ __global__ void __launch_bounds__(64) ksw_stripe_qhead_kernel(int32_t *qhead, in
 // which the dispatcher spreads over the XCDs' CUs; wave v of a team of W
 // waves computes passes v, v+W, ...  A pair's control block holds one
 // progress count per wave; a wave whose wait gave up raises its late word.
-template <bool RIGHT, int MODE, int R>
+template <bool RIGHT, int MODE, int R, bool LUT>
 __global__ void __launch_bounds__(kWave * kMaxTeam) ksw_stripe_wide_kernel(StripeArgs a)
 {
     constexpr int SR = kWave * R;
@@ -940,16 +905,12 @@ __global__ void __launch_bounds__(kWave * kMaxTeam) ksw_stripe_wide_kernel(Strip
     const int job = __builtin_amdgcn_readfirstlane(a.order[slot]);
     int32_t *ctl = a.wctl + (int64_t)slot * kWideCtl;
     const KswJob jb = a.jobs[job];
-    const Consts kc = make_consts<RIGHT>(a.sc, jb.transposed != 0);
+    const typename CellOf<RIGHT, MODE>::type kc(a.sc, jb.transposed != 0);
     const int qlen = __builtin_amdgcn_readfirstlane(jb.qlen), tlen = __builtin_amdgcn_readfirstlane(jb.tlen);
     const int npass = ((tlen + SR - 1) / SR + 1) / 2;
     int late = 0, stop = 0;
-    if (jb.lut)
-        for (int p = v; p < npass && !stop; p += W)
-            pass_body<RIGHT, MODE, true, true, R>(a, kc, job, p, jb, qlen, tlen, ctl, W, late, stop);
-    else
-        for (int p = v; p < npass && !stop; p += W)
-            pass_body<RIGHT, MODE, true, false, R>(a, kc, job, p, jb, qlen, tlen, ctl, W, late, stop);
+    for (int p = v; p < npass && !stop; p += W)
+        pass_body<RIGHT, MODE, true, LUT, R>(a, kc, job, p, jb, qlen, tlen, ctl, W, late, stop);
     if ((late || a.force_late) && threadIdx.x % kWave == 0)
         __hip_atomic_store(ctl + kWideCtlLate, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
@@ -968,7 +929,7 @@ __global__ void __launch_bounds__(256) ksw_stripe_wctl_kernel(int32_t *wctl)
 // team of kWideGroup waves (LDS progress counts, no cross-workgroup waits),
 // into the same direction bytes, column buffer and stripe partials; the
 // plan's redo word counts such pairs.
-template <bool RIGHT, int MODE, int R>
+template <bool RIGHT, int MODE, int R, bool LUT>
 __global__ void __launch_bounds__(kWave * kWideGroup) ksw_stripe_wide_epilogue_kernel(StripeArgs a)
 {
     constexpr int SR = kWave * R;
@@ -984,64 +945,64 @@ __global__ void __launch_bounds__(kWave * kWideGroup) ksw_stripe_wide_epilogue_k
         const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kWave);
         prog[w] = 0;
         __syncthreads();
-        const Consts kc = make_consts<RIGHT>(a.sc, jb.transposed != 0);
+        const typename CellOf<RIGHT, MODE>::type kc(a.sc, jb.transposed != 0);
         const int qlen = __builtin_amdgcn_readfirstlane(jb.qlen), tlen = __builtin_amdgcn_readfirstlane(jb.tlen);
         const int npass = ((tlen + SR - 1) / SR + 1) / 2;
         int late2 = 0, stop = 0;
-        for (int p = w; p < npass && !stop; p += kWideGroup) {
-            if (jb.lut) pass_body<RIGHT, MODE, false, true, R>(a, kc, job, p, jb, qlen, tlen, prog, kWideGroup, late2, stop);
-            else pass_body<RIGHT, MODE, false, false, R>(a, kc, job, p, jb, qlen, tlen, prog, kWideGroup, late2, stop);
-        }
+        for (int p = w; p < npass && !stop; p += kWideGroup)
+            pass_body<RIGHT, MODE, false, LUT, R>(a, kc, job, p, jb, qlen, tlen, prog, kWideGroup, late2, stop);
         __syncthreads();
         if (threadIdx.x == 0) atomicAdd(a.werr, 1);
     }
-    pair_epilogue<R>(a, job, jb, tile, MODE == kTracks, &shared_n, (int)blockDim.x);
+    pair_epilogue<R, MODE>(a, job, jb, tile, &shared_n, (int)blockDim.x);
 }
 
 // Dispatch over the kernel variants: group (left, right, score-only,
-// tracks) and rows per lane (8 or 4).
-template <template <bool, int, int> class F, typename... Args>
-static auto by_variant(int group, int R, Args &&...args)
+// tracks), rows per lane (8 or 4) and score form (byte table or not).
+template <template <bool, int, int, bool> class F, int R, bool LUT, typename... Args>
+static auto by_group(int group, Args &&...args)
 {
-    const bool r8 = R != 4;
     switch (group) {
-    case kGroupRight:
-        return r8 ? F<true, kDirs, 8>::run(args...) : F<true, kDirs, 4>::run(args...);
-    case kGroupScoreOnly:
-        return r8 ? F<false, kScoreOnly, 8>::run(args...) : F<false, kScoreOnly, 4>::run(args...);
-    case kGroupTracks:
-        return r8 ? F<false, kTracks, 8>::run(args...) : F<false, kTracks, 4>::run(args...);
-    default:
-        return r8 ? F<false, kDirs, 8>::run(args...) : F<false, kDirs, 4>::run(args...);
+    case kGroupRight: return F<true, kDirs, R, LUT>::run(args...);
+    case kGroupScoreOnly: return F<false, kScoreOnly, R, LUT>::run(args...);
+    case kGroupTracks: return F<false, kTracks, R, LUT>::run(args...);
+    default: return F<false, kDirs, R, LUT>::run(args...);
     }
 }
 
-template <bool RIGHT, int MODE, int R>
+template <template <bool, int, int, bool> class F, typename... Args>
+static auto by_variant(int group, int R, bool lut, Args &&...args)
+{
+    if (R != 4) return lut ? by_group<F, 8, true>(group, args...) : by_group<F, 8, false>(group, args...);
+    return lut ? by_group<F, 4, true>(group, args...) : by_group<F, 4, false>(group, args...);
+}
+
+template <bool RIGHT, int MODE, int R, bool LUT>
 struct LaunchStripe {
     static hipError_t run(const StripeArgs &a, int team, hipStream_t st)
     {
-        hipLaunchKernelGGL((ksw_stripe_kernel<RIGHT, MODE, R>), dim3(a.njobs), dim3(kWave * team), 0, st, a);
+        hipLaunchKernelGGL((ksw_stripe_kernel<RIGHT, MODE, R, LUT>), dim3(a.njobs), dim3(kWave * team), 0, st, a);
         return hipGetLastError();
     }
 };
 
-template <bool RIGHT, int MODE, int R>
+template <bool RIGHT, int MODE, int R, bool LUT>
 struct LaunchQueue {
     static hipError_t run(const StripeArgs &a, int32_t *qhead, int workers, hipStream_t st)
     {
-        hipLaunchKernelGGL((ksw_stripe_queue_kernel<RIGHT, MODE, R>), dim3(workers), dim3(kWave), 0, st, a, qhead);
+        hipLaunchKernelGGL((ksw_stripe_queue_kernel<RIGHT, MODE, R, LUT>), dim3(workers), dim3(kWave), 0, st, a, qhead);
         return hipGetLastError();
     }
 };
 
-template <bool RIGHT, int MODE, int R>
+template <bool RIGHT, int MODE, int R, bool LUT>
 struct QueueWorkers {
     static int run()
     {
         int per_cu = 0, dev = 0;
         hipDeviceProp_t prop;
         if (hipGetDevice(&dev) != hipSuccess || hipGetDeviceProperties(&prop, dev) != hipSuccess) return 1024;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, ksw_stripe_queue_kernel<RIGHT, MODE, R>, kWave, 0) !=
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, ksw_stripe_queue_kernel<RIGHT, MODE, R, LUT>, kWave, 0) !=
                 hipSuccess ||
             per_cu <= 0)
             return prop.multiProcessorCount * 4;
@@ -1049,11 +1010,11 @@ struct QueueWorkers {
     }
 };
 
-hipError_t launch_stripe_queue(const StripeArgs &a, int group, int R, int32_t *qhead, hipStream_t st)
+hipError_t launch_stripe_queue(const StripeArgs &a, int group, int R, bool lut, int32_t *qhead, hipStream_t st)
 {
     if (a.njobs <= 0) return hipSuccess;
     if (!qhead || (R != 4 && R != 8) || group < 0 || group >= kGroups) return hipErrorInvalidValue;
-    return by_variant<LaunchQueue>(group, R, a, qhead, std::min(a.njobs, stripe_queue_workers(group, R)), st);
+    return by_variant<LaunchQueue>(group, R, lut, a, qhead, std::min(a.njobs, stripe_queue_workers(group, R)), st);
 }
 
 hipError_t clear_queue_heads(int32_t *qhead, int n, hipStream_t st)
@@ -1070,25 +1031,25 @@ int stripe_queue_workers(int group, int R)
     if (group < 0 || group >= kGroups) group = kGroupLeft;
     const int ri = R == 4 ? 1 : 0;
     if (cache[group][ri] > 0) return cache[group][ri];
-    const int n = by_variant<QueueWorkers>(group, R);
+    const int n = by_variant<QueueWorkers>(group, R, true);
     __atomic_store_n(&cache[group][ri], n, __ATOMIC_RELAXED);
     return n;
 }
 
-hipError_t launch_stripe(const StripeArgs &a, int group, int team, int R, hipStream_t st)
+hipError_t launch_stripe(const StripeArgs &a, int group, int team, int R, bool lut, hipStream_t st)
 {
     if (a.njobs <= 0) return hipSuccess;
     if (team < 1 || team > kMaxTeam || (R != 4 && R != 8) || group < 0 || group >= kGroups) return hipErrorInvalidValue;
-    return by_variant<LaunchStripe>(group, R, a, team, st);
+    return by_variant<LaunchStripe>(group, R, lut, a, team, st);
 }
 
 namespace {
 
-template <bool RIGHT, int MODE, int R>
+template <bool RIGHT, int MODE, int R, bool LUT>
 struct LaunchWide {
     static hipError_t run(const StripeArgs &a0, const int32_t *h_wfirst, int max_wgs, hipStream_t st)
     {
-        void (*fn)(StripeArgs) = ksw_stripe_wide_kernel<RIGHT, MODE, R>;
+        void (*fn)(StripeArgs) = ksw_stripe_wide_kernel<RIGHT, MODE, R, LUT>;
         StripeArgs a = a0;
         int off = 0;
         while (off < a0.njobs) {
@@ -1111,38 +1072,38 @@ struct LaunchWide {
     }
 };
 
-template <bool RIGHT, int MODE, int R>
+template <bool RIGHT, int MODE, int R, bool LUT>
 struct WideCapacity {
     static int run()
     {
         int dev = 0, cus = 0, per_cu = 0;
         if (hipGetDevice(&dev) != hipSuccess ||
             hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-            hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void *)ksw_stripe_wide_kernel<RIGHT, MODE, R>,
+            hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void *)ksw_stripe_wide_kernel<RIGHT, MODE, R, LUT>,
                                                          kWave * kWideGroup, 0) != hipSuccess)
             return 0;
         return cus * per_cu;
     }
 };
 
-template <bool RIGHT, int MODE, int R>
+template <bool RIGHT, int MODE, int R, bool LUT>
 struct LaunchWideEpilogue {
     static hipError_t run(const StripeArgs &a, hipStream_t st)
     {
-        hipLaunchKernelGGL((ksw_stripe_wide_epilogue_kernel<RIGHT, MODE, R>), dim3(a.njobs), dim3(kWave * kWideGroup),
+        hipLaunchKernelGGL((ksw_stripe_wide_epilogue_kernel<RIGHT, MODE, R, LUT>), dim3(a.njobs), dim3(kWave * kWideGroup),
                            0, st, a);
         return hipGetLastError();
     }
 };
 
-template <bool RIGHT, int MODE, int R>
+template <bool RIGHT, int MODE, int R, bool LUT>
 struct Resident {
     static int run()
     {
         int per_cu = 0, dev = 0;
         hipDeviceProp_t prop;
         if (hipGetDevice(&dev) != hipSuccess || hipGetDeviceProperties(&prop, dev) != hipSuccess) return 1024;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, ksw_stripe_kernel<RIGHT, MODE, R>, kWave, 0) !=
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, ksw_stripe_kernel<RIGHT, MODE, R, LUT>, kWave, 0) !=
                 hipSuccess ||
             per_cu <= 0)
             return prop.multiProcessorCount * 4;
@@ -1152,7 +1113,7 @@ struct Resident {
 
 }  // namespace
 
-hipError_t launch_stripe_wide(const StripeArgs &a, int group, int R, const int32_t *h_wfirst, int max_wgs,
+hipError_t launch_stripe_wide(const StripeArgs &a, int group, int R, bool lut, const int32_t *h_wfirst, int max_wgs,
                               hipStream_t st)
 {
     if (a.njobs <= 0) return hipSuccess;
@@ -1162,18 +1123,18 @@ hipError_t launch_stripe_wide(const StripeArgs &a, int group, int R, const int32
         const int n = h_wfirst[k + 1] - h_wfirst[k];
         if (n < 1 || n * kWideGroup > kMaxWide) return hipErrorInvalidValue;
     }
-    return by_variant<LaunchWide>(group, R, a, h_wfirst, max_wgs, st);
+    return by_variant<LaunchWide>(group, R, lut, a, h_wfirst, max_wgs, st);
 }
 
 // Cached per variant: the occupancy query reads the device properties.
-int stripe_wide_capacity(int group, int R)
+int stripe_wide_capacity(int group, int R, bool lut)
 {
-    static int cache[kGroups][2] = {};
+    static int cache[kGroups][2][2] = {};
     if (group < 0 || group >= kGroups) group = kGroupLeft;
-    const int ri = R == 4 ? 1 : 0;
-    if (cache[group][ri] > 0) return cache[group][ri];
-    const int n = by_variant<WideCapacity>(group, R);
-    __atomic_store_n(&cache[group][ri], n, __ATOMIC_RELAXED);
+    int &c = cache[group][R == 4 ? 1 : 0][lut ? 1 : 0];
+    if (c > 0) return c;
+    const int n = by_variant<WideCapacity>(group, R, lut);
+    __atomic_store_n(&c, n, __ATOMIC_RELAXED);
     return n;
 }
 
@@ -1183,12 +1144,12 @@ hipError_t clear_wide_err(int32_t *werr, hipStream_t st)
     return hipGetLastError();
 }
 
-hipError_t launch_stripe_wide_epilogue(const StripeArgs &a, int group, int R, hipStream_t st)
+hipError_t launch_stripe_wide_epilogue(const StripeArgs &a, int group, int R, bool lut, hipStream_t st)
 {
     if (a.njobs <= 0) return hipSuccess;
     if (!a.wctl || !a.werr) return hipErrorInvalidValue;
     if ((R != 4 && R != 8) || group < 0 || group >= kGroups) return hipErrorInvalidValue;
-    return by_variant<LaunchWideEpilogue>(group, R, a, st);
+    return by_variant<LaunchWideEpilogue>(group, R, lut, a, st);
 }
 
 // Cached per variant: the occupancy query reads the device properties.
@@ -1198,7 +1159,7 @@ int stripe_resident_waves(int group, int R)
     if (group < 0 || group >= kGroups) group = kGroupLeft;
     const int ri = R == 4 ? 1 : 0;
     if (cache[group][ri] > 0) return cache[group][ri];
-    const int n = by_variant<Resident>(group, R);
+    const int n = by_variant<Resident>(group, R, true);
     __atomic_store_n(&cache[group][ri], n, __ATOMIC_RELAXED);
     return n;
 }
