@@ -702,7 +702,7 @@ int plan_create(Plan **out, const ksw2_pair_t *pairs, const int *idx, int nidx, 
                 if (mine(k) && !wide(k)) members.push_back(k), tmax = std::max(tmax, team[k]);
             if (!members.empty()) {
                 longest_first(members);
-                p->launches.push_back({grp, tmax, (int)order.size(), (int)members.size(), grp % Plan::kLanes, 0, 0, 0, lut});
+                p->launches.push_back({grp, tmax, (int)order.size(), (int)members.size(), grp % Plan::kWideLane, 0, 0, 0, lut});
                 order.insert(order.end(), members.begin(), members.end());
             }
         }
@@ -1111,8 +1111,11 @@ int plan_launch(Plan *p, const Progress *prog)
     stripe_args(p, poll, sa);
     if (p->n_wide > 0) {
         // wide launches (the longest pairs) first, within two quarters of
-        // the device, then their epilogues, which do not wait
-        hipStream_t st = lane(0);
+        // the device, then their epilogues, which do not wait.  On a lane of
+        // their own: on the left-aligned group's lane, the one-workgroup
+        // teams of the other pairs waited for them (2,000 uneven pairs
+        // through one plan: 233 ms a call, 195 ms with both at once)
+        hipStream_t st = lane(Plan::kWideLane);
         if (!st) return KSW2_HIP_EDEVICE;
         KSW_HIP_TRY(clear_wide_err(p->d_werr, st));
         bool wide_now = true;

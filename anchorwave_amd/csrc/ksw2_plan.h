@@ -230,7 +230,7 @@ struct Plan {
     hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};
     bool own_events = true;          // false: ev[] belong to the caller (PlanEnv::events)
     // launches of different kernel groups overlap on their own streams
-    static constexpr int kLanes = 4;
+    static constexpr int kLanes = 4, kWideLane = kLanes - 1;
     hipStream_t lane_stream[kLanes] = {nullptr, nullptr, nullptr, nullptr};
     hipEvent_t lane_done[kLanes] = {nullptr, nullptr, nullptr, nullptr};
     float last_dp_ms = 0.f, last_bt_ms = 0.f;
