@@ -315,13 +315,33 @@ int ksw2_hip_plan_dirs(const ksw2_hip_plan *plan, int index, uint8_t *out, size_
         if (p->order[x] == index) k = x;
     if (k < 0 || k >= p->n_fast) return set_err(KSW2_HIP_EINVAL);  // general-kernel pair: other layout
     const kswhip::KswJob &j = p->jobs[k];
-    if (R) *R = j.R;
+    // a thin-kernel pair is reported, and its bytes are given, in the
+    // stripe layout of four rows per lane
+    const bool thin = j.R == kThinR, tracks = track_pair(j.flag);
+    const int rows = thin ? 4 : j.R;
+    if (R) *R = rows;
     if (transposed) *transposed = j.transposed;
     if (!out) return set_err(KSW2_HIP_OK);  // the geometry only
-    const uint64_t need = (track_pair(j.flag) ? 2 : 1) * kswhip::dir_bytes(j.qlen, j.tlen, j.R);
+    const uint64_t need = (tracks ? 2 : 1) * dir_bytes(j.qlen, j.tlen, rows);
     if (bytes < need || (j.flag & KSW_EZ_SCORE_ONLY)) return set_err(KSW2_HIP_EINVAL);
-    if (hipMemcpy(out, p->d_dir + j.dir_off, need, hipMemcpyDeviceToHost) != hipSuccess)
+    if (!thin) {
+        if (hipMemcpy(out, p->d_dir + j.dir_off, need, hipMemcpyDeviceToHost) != hipSuccess)
+            return set_err(KSW2_HIP_EDEVICE);
+        return set_err(KSW2_HIP_OK);
+    }
+    std::vector<uint8_t> raw(job_dir_bytes(j));
+    if (hipMemcpy(raw.data(), p->d_dir + j.dir_off, raw.size(), hipMemcpyDeviceToHost) != hipSuccess)
         return set_err(KSW2_HIP_EDEVICE);
+    memset(out, 0, need);
+    const int chunks = thin_chunks(j.qlen);
+    for (int i = 0; i < j.tlen; ++i)
+        for (int c = 0; c < j.qlen; ++c) {
+            if (!tracks) {
+                out[dir_index(i, c, j.qlen, rows)] = raw[thin_dir_index(i, c, chunks)];
+                continue;
+            }
+            for (int t = 0; t < 2; ++t) out[track_index(t, i, c, j.qlen, rows)] = raw[thin_track_index(t, i, c, chunks)];
+        }
     return set_err(KSW2_HIP_OK);
 }
 

@@ -380,6 +380,42 @@ static int choose_rows(const ksw2_pair_t *pairs, const std::vector<int> &fast, c
     return 8 * waves <= stripe_resident_waves(kGroupLeft, 4) ? 4 : 8;
 }
 
+// Whether a plan's stripe-kernel pairs run on the thin kernel: a plan whose
+// time is its pairs' chains (latency_plan, no measured layout for its largest
+// pair), of at most 384 workgroups of four passes (one and a half per CU, one
+// launch's share of the device).  One pair of 300 bp, 1, 2 and 5 kbp took
+// 0.185, 0.41, 1.00 and 2.57 ms (walk included) on four rows per lane spread
+// over CUs and 0.17, 0.36, 0.78 and 1.87 ms on the thin kernel.  At the limit:
+// 384 pairs of 300 bp 0.30 against 0.26 ms, 192 of 1 kbp 0.60 against 0.61, 80
+// and 96 of 2 kbp 1.56 and 1.65 against 1.00 and 1.64, 38 of 5 kbp 2.74
+// against 2.45.  Beyond it the thin passes' instructions per cell (half as many
+// again) no longer fit beside each other: 512 pairs of 300 bp 0.30 against
+// 0.38 ms, 50 of 5 kbp 2.78 against 4.07.  KSW2_HIP_THIN=0 turns it off (tests).
+constexpr int kThinGroups = 384;
+static bool thin_plan(const ksw2_pair_t *pairs, const std::vector<int> &fast, const PlanEnv *env)
+{
+    const char *ev = getenv("KSW2_HIP_THIN");
+    if ((ev && atoi(ev) == 0) || !latency_plan(pairs, fast, env)) return false;
+    int64_t groups = 0;
+    int big = fast[0];
+    for (int id : fast) {
+        groups += (thin_passes(stripe_geom(pairs[id]).kt) + kWideGroup - 1) / kWideGroup;
+        if ((double)pairs[id].qlen * pairs[id].tlen > (double)pairs[big].qlen * pairs[big].tlen) big = id;
+    }
+    const StripeGeom g = stripe_geom(pairs[big]);
+    return groups <= kThinGroups && !tune_lookup(g.kq, g.kt);
+}
+
+uint64_t job_dir_bytes(const KswJob &j)
+{
+    if (j.flag & KSW_EZ_SCORE_ONLY) return 0;
+    return (track_pair(j.flag) ? 2 : 1) *
+           (j.R == kThinR ? thin_dir_bytes(j.qlen, j.tlen) : dir_bytes(j.qlen, j.tlen, j.R));
+}
+
+// (the thin layout takes no more than the stripe layouts this bounds: its
+// rows are padded to 128, its passes hold at most qlen + 127 columns and its
+// partials half a stripe's)
 uint64_t pair_footprint(const ksw2_pair_t &p, bool general)
 {
     // CIGAR slot, twice: the arena and the dense region plan_fetch copies from
@@ -521,7 +557,8 @@ int plan_create(Plan **out, const ksw2_pair_t *pairs, const int *idx, int nidx, 
                                                        : kGroupLeft;
         g[grp].push_back(idx[k]);
     }
-    p->R = choose_rows(pairs, fast, env);
+    p->thin = thin_plan(pairs, fast, env);
+    p->R = p->thin ? kThinR : choose_rows(pairs, fast, env);
     const int R = p->R, SR = kWave * R;
     std::vector<int> grp_of;
     for (int grp = 0; grp < kGroups; ++grp)
@@ -547,6 +584,7 @@ int plan_create(Plan **out, const ksw2_pair_t *pairs, const int *idx, int nidx, 
         const StripeGeom g = stripe_geom(pp);
         j.transposed = g.tr ? 1 : 0;
         j.qlen = g.kq, j.tlen = g.kt, j.flag = pp.flag, j.end_bonus = pp.end_bonus;
+        p->max_swept = std::max(p->max_swept, g.kq);
         j.R = R;
         j.lut = lut_ok(pp, gsc.k) ? 1 : 0;
         if (resident) {
@@ -557,11 +595,10 @@ int plan_create(Plan **out, const ksw2_pair_t *pairs, const int *idx, int nidx, 
             j.t_off = so, so = round_up(so + g.kt, 16);
         }
         j.dir_off = dof;
-        if (!(pp.flag & KSW_EZ_SCORE_ONLY))
-            dof = round_up(dof + (track_pair(pp) ? 2 : 1) * dir_bytes(g.kq, g.kt, R), 256);
+        dof = round_up(dof + job_dir_bytes(j), 256);
         j.bnd_off = bo, bo += round_up(2ull * g.kq, 64);
         j.cig_off = co, co += round_up((uint64_t)pp.qlen + pp.tlen + 2, 16);
-        j.stripe_off = stripes, stripes += (g.kt + SR - 1) / SR;
+        j.stripe_off = stripes, stripes += p->thin ? (thin_passes(g.kt) + 1) / 2 : (g.kt + SR - 1) / SR;
         p->cig_off[k] = j.cig_off;
     }
     p->nstripes_total = stripes;
@@ -618,10 +655,11 @@ int plan_create(Plan **out, const ksw2_pair_t *pairs, const int *idx, int nidx, 
     std::vector<int32_t> order;
     if (p->n_fast > 0) {
         double total_steps = 0;
-        for (const KswJob &j : p->jobs) total_steps += pair_steps(j);
+        if (!p->thin)
+            for (const KswJob &j : p->jobs) total_steps += pair_steps(j);
         const double T = env && env->team_T > 0
                              ? env->team_T
-                             : std::max(1.0, total_steps / std::max(1, stripe_resident_waves(kGroupLeft, R)));
+                             : std::max(1.0, total_steps / std::max(1, p->thin ? 1 : stripe_resident_waves(kGroupLeft, R)));
         const uint64_t wave_bytes = env ? env->wave_bytes : 0;
         int forced = env ? env->team : 0;
         if (const char *ev = getenv("KSW2_HIP_TEAM")) forced = atoi(ev);
@@ -629,6 +667,13 @@ int plan_create(Plan **out, const ksw2_pair_t *pairs, const int *idx, int nidx, 
         if (const char *ev = getenv("KSW2_HIP_WIDE")) wide_forced = std::max(0, std::min(kMaxWide / kWideGroup, atoi(ev)));
         std::vector<int> team(p->n_fast);
         for (int k = 0; k < p->n_fast; ++k) {
+            if (p->thin) {
+                // a wave per pass, spread over workgroups of four; as one
+                // workgroup when no waiting-launch slots are free
+                team[k] = std::min(thin_passes(p->jobs[k].tlen), kThinMaxTeam);
+                p->jobs[k].team = std::min(team[k], kThinTeam);
+                continue;
+            }
             // KSW2_HIP_TEAM=-1 (tests): team sizes 1..16 in turn, one launch
             const int f = forced < 0 ? 1 + k % kMaxTeam : forced;
             team[k] = wide_forced ? kWideGroup * wide_forced : choose_team(p->jobs[k], T, f, wave_bytes);
@@ -641,9 +686,9 @@ int plan_create(Plan **out, const ksw2_pair_t *pairs, const int *idx, int nidx, 
         // team size in its KswJob: when no waiting-launch slots are free at
         // launch (other threads' calls hold them), it runs as a one-workgroup
         // team instead of waiting.
-        std::vector<char> spread(p->n_fast, 0);
+        std::vector<char> spread(p->n_fast, p->thin ? 1 : 0);
         std::vector<char> tuned(p->n_fast, 0);
-        if (!wide_forced && forced == 0 && latency_plan(pairs, fast, env)) {
+        if (!p->thin && !wide_forced && forced == 0 && latency_plan(pairs, fast, env)) {
             // measured lone-pair layouts (a pair of another bin than the one
             // that set the plan's rows keeps its team size, within its passes)
             for (int k = 0; k < p->n_fast; ++k) {
@@ -656,7 +701,7 @@ int plan_create(Plan **out, const ksw2_pair_t *pairs, const int *idx, int nidx, 
                 spread[k] = e->spread && t > kWideGroup && t <= kMaxTeam;
             }
         }
-        if (!wide_forced && ((!env && forced == 0) || (env && env->spread && forced >= 0))) {
+        if (!p->thin && !wide_forced && ((!env && forced == 0) || (env && env->spread && forced >= 0))) {
             int64_t waves = 0;
             for (int k = 0; k < p->n_fast; ++k) waves += team[k];
             if (4 * waves <= stripe_resident_waves(kGroupLeft, R))
@@ -668,7 +713,11 @@ int plan_create(Plan **out, const ksw2_pair_t *pairs, const int *idx, int nidx, 
         for (int k = 0; k < p->n_fast; ++k)
             if (wide(k) && !spread[k]) p->optional_wide = false;
         auto longest_first = [&](std::vector<int> &m) {
-            std::stable_sort(m.begin(), m.end(), [&](int x, int y) { return pair_steps(p->jobs[x]) > pair_steps(p->jobs[y]); });
+            auto steps = [&](int k) {
+                const KswJob &j = p->jobs[k];
+                return p->thin ? (double)thin_passes(j.tlen) * j.qlen : pair_steps(j);
+            };
+            std::stable_sort(m.begin(), m.end(), [&](int x, int y) { return steps(x) > steps(y); });
         };
         for (int part = 0; part < 2 * kGroups; ++part) {
             const int grp = part / 2;
@@ -686,7 +735,7 @@ int plan_create(Plan **out, const ksw2_pair_t *pairs, const int *idx, int nidx, 
                 for (int k : members) {
                     p->h_wfirst.push_back(blocks);
                     blocks += (team[k] + kWideGroup - 1) / kWideGroup;
-                    tmax = std::max(tmax, team[k]);
+                    tmax = std::max(tmax, p->thin ? p->jobs[k].team : team[k]);
                 }
                 p->h_wfirst.push_back(blocks);
                 // team: the largest, for a one-workgroup launch of spread pairs
@@ -1117,7 +1166,7 @@ int plan_launch(Plan *p, const Progress *prog)
         // through one plan: 233 ms a call, 195 ms with both at once)
         hipStream_t st = lane(Plan::kWideLane);
         if (!st) return KSW2_HIP_EDEVICE;
-        KSW_HIP_TRY(clear_wide_err(p->d_werr, st));
+        if (!p->thin) KSW_HIP_TRY(clear_wide_err(p->d_werr, st));  // (the thin launches clear their own)
         bool wide_now = true;
         {
             std::lock_guard<std::mutex> lk(g_wait_mu);
@@ -1131,8 +1180,14 @@ int plan_launch(Plan *p, const Progress *prog)
                     if (!l.wide) continue;
                     sa.order = p->d_order + l.off, sa.njobs = l.count;
                     sa.wctl = p->d_wctl + (int64_t)l.woff * kWideCtl, sa.wfirst = p->d_wfirst + l.wf;
-                    const int half = std::max(1, stripe_wide_capacity(l.grp, p->R, l.lut) / 2);
-                    KSW_HIP_TRY(launch_stripe_wide(sa, l.grp, p->R, l.lut, p->h_wfirst.data() + l.wf, half, st));
+                    const int32_t *wfirst = p->h_wfirst.data() + l.wf;
+                    if (p->thin) {
+                        const int half = std::max(1, thin_capacity(l.grp, l.lut) / 2);
+                        KSW_HIP_TRY(launch_thin(sa, l.grp, l.lut, wfirst, half, 0, p->max_swept, st));
+                    } else {
+                        const int half = std::max(1, stripe_wide_capacity(l.grp, p->R, l.lut) / 2);
+                        KSW_HIP_TRY(launch_stripe_wide(sa, l.grp, p->R, l.lut, wfirst, half, st));
+                    }
                 }
                 if (!wait_slots_release(st, q)) return KSW2_HIP_EDEVICE;
             }
@@ -1140,7 +1195,10 @@ int plan_launch(Plan *p, const Progress *prog)
         for (const Plan::Launch &l : p->launches) {
             if (!l.wide) continue;
             sa.order = p->d_order + l.off, sa.njobs = l.count, sa.wctl = p->d_wctl + (int64_t)l.woff * kWideCtl;
-            if (wide_now) KSW_HIP_TRY(launch_stripe_wide_epilogue(sa, l.grp, p->R, l.lut, st));
+            if (p->thin) {
+                if (!wide_now) KSW_HIP_TRY(launch_thin(sa, l.grp, l.lut, nullptr, 0, l.team, p->max_swept, st));
+                KSW_HIP_TRY(launch_thin_epilogue(sa, l.grp, l.lut, st));
+            } else if (wide_now) KSW_HIP_TRY(launch_stripe_wide_epilogue(sa, l.grp, p->R, l.lut, st));
             else KSW_HIP_TRY(launch_stripe(sa, l.grp, l.team, p->R, l.lut, st));  // one-workgroup teams
         }
     }
@@ -1230,7 +1288,7 @@ bool plan_dir_span(const Plan *p, int k, uint64_t *off, uint64_t *len)
     const KswJob &j = p->jobs[k];
     if (j.flag & KSW_EZ_SCORE_ONLY) return false;
     *off = (uint64_t)(p->d_dir - p->pool->base) + j.dir_off;
-    *len = (track_pair(j.flag) ? 2 : 1) * dir_bytes(j.qlen, j.tlen, j.R);
+    *len = job_dir_bytes(j);
     return true;
 }
 

@@ -73,6 +73,21 @@ __device__ __forceinline__ uint32_t perm(uint32_t hi, uint32_t lo, uint32_t sel)
     return __builtin_amdgcn_perm(hi, lo, sel);
 }
 
+// Lane k takes lane k+1's value (lane 63 `old`), lane k takes lane k-1's
+// (lane 0 `old`), lane k takes lane k-1's (lane 0 lane 63's).
+__device__ __forceinline__ uint32_t dpp_shl1(uint32_t old, uint32_t src)
+{
+    return (uint32_t)__builtin_amdgcn_update_dpp((int)old, (int)src, 0x130, 0xF, 0xF, false);
+}
+__device__ __forceinline__ uint32_t dpp_shr1(uint32_t old, uint32_t src)
+{
+    return (uint32_t)__builtin_amdgcn_update_dpp((int)old, (int)src, 0x138, 0xF, 0xF, false);
+}
+__device__ __forceinline__ uint32_t dpp_ror1(uint32_t src)
+{
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)src, 0x13C, 0xF, 0xF, false);
+}
+
 // State of two cells: x, x2, v go down (from the cells above to those
 // below), u, y, y2 go right.
 struct Down {
@@ -191,4 +206,17 @@ struct RawCell {
 };
 
 }  // namespace cell
+
+// What a pass stores per cell.
+enum Mode { kDirs = 0, kScoreOnly = 1, kTracks = 2 };
+
+// The cell of a mode and how far its sums are scaled (as a shift).
+template <bool RIGHT, int MODE> struct CellOf {
+    typedef cell::RawCell type;
+    static constexpr int shift = 0;
+};
+template <bool RIGHT> struct CellOf<RIGHT, kDirs> {
+    typedef cell::DirCell<RIGHT> type;
+    static constexpr int shift = 3;
+};
 }  // namespace kswhip

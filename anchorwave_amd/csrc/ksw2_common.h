@@ -195,4 +195,46 @@ KSW_HD inline uint64_t track_index(int track, int i, int j, int qlen, int R = kR
     return (d / (2 * R)) * (4 * R) + (uint64_t)track * (2 * R) + (d % (2 * R));
 }
 
+// Thin layout (ksw2_thin.hip): passes of 128 rows, two per lane; a lane
+// stores four steps as kThinLane direction bytes (twice that of tracks).
+// `chunks` is thin_chunks() of the swept length; the chunk numbered `chunks`
+// shares chunk 0's place (other lanes use it).
+constexpr int kThinR = 1;  // KswJob::R of a pair in this layout
+constexpr int kThinRows = 2 * kWave;
+constexpr int kThinLane = 8;
+KSW_HD inline int thin_passes(int tlen) { return (tlen + kThinRows - 1) / kThinRows; }
+KSW_HD inline int thin_chunks(int qlen) { return (qlen + kThinRows - 1) / 4; }
+KSW_HD inline uint64_t thin_dir_bytes(int qlen, int tlen)
+{
+    return (uint64_t)thin_passes(tlen) * (uint64_t)thin_chunks(qlen) * kWave * kThinLane;
+}
+// Byte of cell (i = striped, j = swept) within a track (or the direction
+// bytes), and the lane group (of kThinLane bytes per track) it belongs to.
+KSW_HD inline uint64_t thin_group(int i, int j, int chunks, int *byte)
+{
+    const int p = i / kThinRows, k = i % kThinRows / 2, h = i & 1, c = j + 2 * k + h;
+    const int ch = c / 4 == chunks ? 0 : c / 4;
+    *byte = 4 * (c / 2 % 2) + 2 * h + c % 2;
+    return ((uint64_t)p * chunks + ch) * kWave + k;
+}
+KSW_HD inline uint64_t thin_dir_index(int i, int j, int chunks)
+{
+    int b;
+    const uint64_t g = thin_group(i, j, chunks, &b);
+    return g * kThinLane + b;
+}
+KSW_HD inline uint64_t thin_track_index(int track, int i, int j, int chunks)
+{
+    int b;
+    const uint64_t g = thin_group(i, j, chunks, &b);
+    return g * (2 * kThinLane) + track * kThinLane + b;
+}
+
+// Per-pass partial of the mqe bookkeeping (as StripeRec, in half its space):
+// the sum over the pass's rows, and its smallest running sum << 7 | the row
+// within the pass that has it.
+struct ThinRec {
+    int32_t total, best_row;
+};
+
 }  // namespace kswhip

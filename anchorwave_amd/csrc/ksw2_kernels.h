@@ -167,6 +167,21 @@ hipError_t clear_wide_err(int32_t *werr, hipStream_t st);
 // Waves of the stripe kernel that fit on the device at once.
 int stripe_resident_waves(int group, int R = kRowsPerLane);
 
+// Thin kernel (ksw2_thin.hip): the stripe kernel's results for a few pairs
+// in a fraction of the time, one wave per 128 rows.  h_wfirst (the host copy
+// of a.wfirst): each job's passes spread over its own number of workgroups
+// of kWideGroup waves (at most kThinMaxTeam waves), launched in chunks of at
+// most max_wgs workgroups, as launch_stripe_wide; null: one workgroup of
+// `team` waves per job, which waits on nothing outside itself.  kq: the
+// longest swept length.  launch_thin_epilogue then runs each job's epilogue.
+constexpr int kThinMaxTeam = 1024;
+constexpr int kThinTeam = 8;  // waves of a job that has one workgroup, at most
+hipError_t launch_thin(const StripeArgs &a, int group, bool lut, const int32_t *h_wfirst, int max_wgs, int team, int kq,
+                       hipStream_t st);
+hipError_t launch_thin_epilogue(const StripeArgs &a, int group, bool lut, hipStream_t st);
+// Workgroups of kWideGroup waves of the thin kernel the device holds at once.
+int thin_capacity(int group, bool lut);
+
 // Zero-fills `bytes` bytes at `p` (16-byte aligned) with a kernel on `st`
 // (a fill kernel, not a memset, so that a captured graph replays it).
 hipError_t launch_fill_zero(void *p, uint64_t bytes, hipStream_t st);

@@ -66,6 +66,8 @@ struct StripeGeom {
     int kq, kt;
 };
 StripeGeom stripe_geom(const ksw2_pair_t &p);
+// Bytes a stripe-kernel job stores: direction bytes or tracks.
+uint64_t job_dir_bytes(const KswJob &j);
 // Device bytes a pair needs while its plan is alive.
 uint64_t pair_footprint(const ksw2_pair_t &p, bool general);
 // Threads of the general kernel's workgroup for one pair (64..1024).
@@ -165,7 +167,9 @@ struct Plan {
     int n = 0;                       // pairs in the plan
     int n_tracks_gen = 0;            // general pairs with the Singletrack walk
     int n_fast = 0, n_gen = 0;       // slots [0, n_fast) stripe kernel, then general kernel
-    int R = kRowsPerLane;            // rows per lane of the stripe kernel
+    int R = kRowsPerLane;            // rows per lane of the stripe kernel (kThinR: the thin kernel)
+    bool thin = false;               // the stripe-kernel pairs run on the thin kernel
+    int max_swept = 0;               // their longest swept sequence
     std::vector<KswJob> jobs;        // host copy, stripe-kernel slots
     std::vector<GenJob> gjobs;       // host copy, general-kernel slots
     std::vector<int> order;          // plan slot -> caller index

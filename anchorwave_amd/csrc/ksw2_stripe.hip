@@ -61,51 +61,24 @@
 
 #include "ksw2_cell.h"
 #include "ksw2_common.h"
+#include "ksw2_epilogue.h"
 #include "ksw2_kernels.h"
-#include "ksw2_walk.h"
 
 namespace kswhip {
 
 namespace {
 
-constexpr int kDppWaveShl1 = 0x130, kDppWaveShr1 = 0x138;
-constexpr int kDppWaveRor1 = 0x13C;
 constexpr int kLag = kWave;      // steps the high stripe trails the low one
 constexpr int kAhead = 16;       // steps before a block its boundary entries are loaded
 
-// What a pass stores per cell.
-enum Mode { kDirs = 0, kScoreOnly = 1, kTracks = 2 };
-
 using cell::bfi;
+using cell::dpp_ror1;
+using cell::dpp_shl1;
+using cell::dpp_shr1;
 using cell::hi16;
 using cell::lo16;
 using cell::perm;
 using cell::splat;
-
-// The cell of a mode and how far its sums are scaled (as a shift).
-template <bool RIGHT, int MODE> struct CellOf {
-    typedef cell::RawCell type;
-    static constexpr int shift = 0;
-};
-template <bool RIGHT> struct CellOf<RIGHT, kDirs> {
-    typedef cell::DirCell<RIGHT> type;
-    static constexpr int shift = 3;
-};
-
-// Lane k takes lane k+1's value (lane 63 `old`), lane k takes lane k-1's
-// (lane 0 `old`), lane k takes lane k-1's (lane 0 lane 63's).
-__device__ __forceinline__ uint32_t dpp_shl1(uint32_t old, uint32_t src)
-{
-    return (uint32_t)__builtin_amdgcn_update_dpp((int)old, (int)src, kDppWaveShl1, 0xF, 0xF, false);
-}
-__device__ __forceinline__ uint32_t dpp_shr1(uint32_t old, uint32_t src)
-{
-    return (uint32_t)__builtin_amdgcn_update_dpp((int)old, (int)src, kDppWaveShr1, 0xF, 0xF, false);
-}
-__device__ __forceinline__ uint32_t dpp_ror1(uint32_t src)
-{
-    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)src, kDppWaveRor1, 0xF, 0xF, false);
-}
 
 // The value from the cell above for every lane: lane k takes lane k-1's
 // (both halves); lane 0 takes lane 63's low half of the previous step into
@@ -385,12 +358,12 @@ __device__ __forceinline__ void pass_run(const StripeArgs &a, const typename Cel
         if (LUT) {
             tab_hi = dpp_shr1(dpp_ror1(tab_lo), tab_hi);
             const uint32_t q0 = binq;
-            binq = dpp_shl1(0, binq);
+            binq = dpp_shl1(binq, binq);
             tab_lo = dpp_shr1(q0, tab_lo);
         } else {
             code = carry(code, bin1 << 16, m0);
         }
-        bin0 = dpp_shl1(0, bin0), bin1 = dpp_shl1(0, bin1);
+        bin0 = dpp_shl1(bin0, bin0), bin1 = dpp_shl1(bin1, bin1);
         const int jl = c - lane;
         if (EDGE) {
             // a half starts at its first column: the lanes there take the
@@ -553,262 +526,6 @@ __device__ __forceinline__ void pass_body(const StripeArgs &a, const typename Ce
 
 }  // namespace
 
-// Epilogue of one pair, run by the whole workgroup once every pass is done:
-// folds the per-stripe mqe partials in row order (ties to the later row, the
-// '>=' of minimap2/ksw2_extd2_sse.c:371), picks the start cell as in
-// minimap2/ksw2_extd2_sse.c:398-418 and walks the direction bytes with the
-// state machine of ksw_backtrack (minimap2/ksw2.h:160-192) for an unbanded
-// matrix (no cell of the path can leave the band there, so the off/off_end
-// forcing never triggers).  The walk reads a tile of 8 lanes x 64 columns (up
-// to 64 rows x 64 columns of one stripe) staged in LDS by the workgroup; when
-// the path leaves the tile the next one is staged, so HBM latency is paid
-// once per tile rather than once per step.  Every thread runs the same walk
-// (uniform control flow, LDS broadcast reads) while other workgroups keep the
-// SIMDs busy; thread 0 writes the run-length encoded CIGAR, which is reversed
-// at the end unless KSW_EZ_REV_CIGAR.  With a host mirror, the result and the
-// CIGAR are then copied to pinned host memory and the pair's completion flag
-// is raised (system-scope release), so a caller can take this pair's result
-// while the launch still runs.
-//
-// With the two Singletrack tracks instead of direction bytes, the first wave
-// runs the Singletrack walk (track_walk) for a global alignment; with
-// KSW_EZ_EXTZ_ONLY or KSW_EZ_SEMIGLOBAL_END the result is zdropped with no
-// path (minimap2/ksw2_extd2_avx.c:752-760), and a failed walk reports
-// n_cigar = -1 (no CIGAR, zdropped).
-
-// Singletrack tracks of one stripe-kernel pair (layout of the tracks mode),
-// read in the reference's coordinates (i target, j query).  A transposed
-// pair stores cell (i, j) at (j, i) and its horizontal and vertical
-// differences exchanged.
-template <int R>
-struct StripeTracks {
-    static constexpr int SR = kWave * R;
-    const uint8_t *dir;
-    const uint8_t *qs, *ts;   // the reference's query and target
-    uint64_t nsteps;
-    int32_t mch, mis;
-    bool tr;
-    __device__ int32_t get(int track, int i, int j) const
-    {
-        if (tr) {
-            const int t = i;
-            i = j, j = t, track = 1 - track;
-        }
-        const int s = i / SR, pp = s >> 1, h = s & 1, k = (i % SR) / R, rho = i % R;
-        const uint64_t c = (uint64_t)(j + k + kLag * h);
-        const uint8_t b =
-            dir[((pp * nsteps + c) * kWave + k) * (4 * R) + track * (2 * R) + 4 * (rho >> 1) + 2 * h + (rho & 1)];
-        return -(int32_t)(int8_t)b;
-    }
-    __device__ int forced(int, int) const { return 0; }
-    __device__ int32_t cost(int i, int j) const { return ts[i] == qs[j] ? mch : mis; }
-};
-
-template <int R, int MODE>
-__device__ __forceinline__ void pair_epilogue(const StripeArgs &a, int job_id, const KswJob &jb,
-                                              uint64_t (*tile)[64], int *shared_n, int nthr)
-{
-    constexpr bool tracks = MODE == kTracks;
-    constexpr int SR = kWave * R;  // rows per stripe
-    const int tid = threadIdx.x;
-    // the host's stop flag, read once for the whole workgroup: a stopped
-    // pair's passes may have ended early, so it takes no walk
-    int stopped = 0;
-    if (a.stop) {
-        if (tid == 0) *shared_n = __hip_atomic_load(a.stop, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-        __syncthreads();
-        stopped = *shared_n;
-        __syncthreads();
-    }
-    KswOut o = a.out[job_id];
-    if (stopped) o.stopped = 1;
-    const int flag = jb.flag;
-    // kq, kt: the swept and striped lengths; qlen, tlen: the reference's
-    const bool tr = jb.transposed != 0;
-    const int kq = jb.qlen, kt = jb.tlen;
-    const int qlen = tr ? kt : kq, tlen = tr ? kq : kt;
-    {
-        // the stripes' partials at the last swept column, in row order
-        const int nstripes = (kt + SR - 1) / SR;
-        int carry_ = 0, best = 0x7fffffff, best_i = -1;
-        for (int s = 0; s < nstripes; ++s) {
-            const StripeRec rec = a.recs[jb.stripe_off + s];
-            if (rec.best_i >= 0 && carry_ + rec.best <= best) best = carry_ + rec.best, best_i = rec.best_i;
-            carry_ += rec.total;
-        }
-        const int64_t h_anchor = (int64_t)a.sc.G1 - a.sc.qe_orig;
-        const int h_top_last_col = (int)(h_anchor + edge_prefix(a.sc, kq - 1));  // H(-1, kq-1)
-        const int col_max = h_top_last_col - (best >> CellOf<false, MODE>::shift);
-        if (!tr) {
-            o.mqe = col_max, o.mqe_t = best_i;
-        } else {
-            // the last swept column is the reference's last row (mte) and the
-            // last striped row, tracked by the last pass, its last column (mqe)
-            o.mqe = o.mte, o.mqe_t = o.mte_q;
-            o.mte = col_max, o.mte_q = best_i;
-        }
-    }
-    int i0 = -1, j0 = -1;
-    int n = 0;
-    uint32_t *cig = a.cig + jb.cig_off;
-    if (stopped) {
-        // no walk: the passes, the stripe partials and this pair's result
-        // slot may be incomplete
-    } else if (tracks) {
-        if (!o.stopped && !o.zdropped && !(flag & (0x40 | 0x800))) {
-            if (tid < kWave) {
-                StripeTracks<R> A;
-                A.dir = a.dir + jb.dir_off;
-                A.qs = a.seq + (tr ? jb.t_off : jb.q_off), A.ts = a.seq + (tr ? jb.q_off : jb.t_off);
-                A.nsteps = (uint64_t)kq + kWave - 1 + kLag;
-                A.mch = a.sc.mch, A.mis = a.sc.mis;
-                A.tr = tr;
-                const WalkGaps g = {-a.sc.q, -a.sc.e, -a.sc.q2, -a.sc.e2};
-                const int nn = track_walk(A, qlen, tlen, g, cig);
-                if (tid == 0) *shared_n = nn;
-            }
-            __syncthreads();
-            n = *shared_n;
-            if (n < 0) o.zdropped = 1;
-        } else if (!o.stopped && !o.zdropped) {
-            o.zdropped = 1;
-        }
-    } else if (!(flag & 0x01)) {  // KSW_EZ_SCORE_ONLY: no path
-        if (!o.stopped && !o.zdropped && (flag & 0x800)) {          // SEMIGLOBAL_END
-            if (o.mqe > o.mte) o.score = o.mqe, i0 = o.mqe_t, j0 = qlen - 1;
-            else o.score = o.mte, i0 = tlen - 1, j0 = o.mte_q;
-        } else if (!o.stopped && !o.zdropped && !(flag & 0x40)) {   // global
-            i0 = tlen - 1, j0 = qlen - 1;
-        } else if (!o.zdropped && (flag & 0x40) && o.mqe + jb.end_bonus > o.max) {  // EXTZ_ONLY
-            o.reach_end = 1, i0 = o.mqe_t, j0 = qlen - 1;
-        } else if (o.max_t >= 0 && o.max_q >= 0) {
-            i0 = o.max_t, j0 = o.max_q;
-        }
-    }
-    if (i0 >= 0 || j0 >= 0) {
-        const uint8_t *dir = a.dir + jb.dir_off;
-        const uint64_t nsteps = (uint64_t)kq + kWave - 1 + kLag;
-        int i = i0, j = j0, state = 0;
-        // the staged tile, in stored coordinates (striped row, swept column)
-        int t_r_lo = 1, t_r_hi = 0, t_c_lo = 1, t_c_hi = 0;
-        int run_op = -1, run_len = 0;
-        auto push = [&](int op, int len) {
-            if (op == run_op) {
-                run_len += len;
-            } else {
-                if (run_len > 0 && tid == 0) cig[n] = (uint32_t)run_len << 4 | (uint32_t)run_op;
-                if (run_len > 0) ++n;
-                run_op = op, run_len = len;
-            }
-        };
-        while (i >= 0 && j >= 0) {
-            const int r = tr ? j : i, c = tr ? i : j;  // stored coordinates of cell (i, j)
-            if (r < t_r_lo || r > t_r_hi || c < t_c_lo || c > t_c_hi) {
-                // stage lanes kb..k of stripe s (rows up to r) x columns c-63..c
-                const int s = r / SR, k = (r - s * SR) / R, kb = k >= 7 ? k - 7 : 0;
-                const int pp = s >> 1, h = s & 1;
-                t_r_lo = s * SR + kb * R, t_r_hi = s * SR + k * R + R - 1;
-                t_c_hi = c, t_c_lo = c >= 63 ? c - 63 : 0;
-                const int c_lo = t_c_lo + kb + kLag * h, c_hi = t_c_hi + k + kLag * h;
-                __syncthreads();  // the previous tile is no longer read
-                for (int cc = c_lo + tid; cc <= c_hi; cc += nthr) {
-                    const uint8_t *src = dir + (((uint64_t)pp * nsteps + (uint64_t)cc) * kWave + kb) * (2 * R);
-                    for (int kr = 0; kr <= k - kb; ++kr) {
-                        const int jj = cc - kLag * h - (kb + kr);
-                        if (jj >= t_c_lo && jj <= t_c_hi) {
-                            // the R row bytes of half h: bytes 2h, 2h+1 of each dword
-                            const unsigned sel = h ? 0x07060302u : 0x05040100u;
-                            if (R == 8) {
-                                const uint4 w = ((const uint4 *)src)[kr];
-                                const uint32_t lo = __builtin_amdgcn_perm(w.y, w.x, sel);
-                                const uint32_t hi = __builtin_amdgcn_perm(w.w, w.z, sel);
-                                tile[kr][jj - t_c_lo] = (uint64_t)hi << 32 | lo;
-                            } else {
-                                const uint2 w = ((const uint2 *)src)[kr];
-                                tile[kr][jj - t_c_lo] = __builtin_amdgcn_perm(w.y, w.x, sel);
-                            }
-                        }
-                    }
-                }
-                __syncthreads();
-            }
-            const int rel = r - t_r_lo;
-            if (state == 0) {
-                // A run of diagonal moves at once: from state 0 the walk
-                // stays in state 0 and moves diagonally while each cell's
-                // argmax (its low three bits) is 0.  Lane k tests cell
-                // (r - k, c - k) of the staged tile (within the tile and the
-                // matrix); the run is the lanes before the first that fails.
-                const int lim = min(min(rel, c - t_c_lo), min(i, j));
-                const int lk = tid & (kWave - 1);
-                int fail = 1;
-                if (lk <= lim) {
-                    const int rr = rel - lk;
-                    fail = ((int)(tile[rr / R][c - lk - t_c_lo] >> (8 * (rr % R))) & 7) != 0;
-                }
-                const uint64_t fb = __ballot(fail);
-                const int run = fb ? (int)__builtin_ctzll(fb) : kWave;
-                if (run > 0) {
-                    push(0, run);
-                    i -= run, j -= run;
-                    continue;
-                }
-            } else {
-                // A run of gap moves at once: state s (1-4) stays while each
-                // cell's continuation bit (s + 2) is set, moving i (s = 1, 3)
-                // or j (s = 2, 4) back by one, which is one stored row or one
-                // column.  Lane k tests the k-th cell of the run.
-                const int s = state;
-                const bool di = s == 1 || s == 3, rows = di != tr;
-                const int lim = min(rows ? rel : c - t_c_lo, di ? i : j);
-                const int lk = tid & (kWave - 1);
-                int fail = 1;
-                if (lk <= lim) {
-                    const int rr = rows ? rel - lk : rel, cc = rows ? c : c - lk;
-                    fail = !((int)(tile[rr / R][cc - t_c_lo] >> (8 * (rr % R) + s + 2)) & 1);
-                }
-                const uint64_t fb = __ballot(fail);
-                const int run = fb ? (int)__builtin_ctzll(fb) : kWave;
-                if (run > 0) {
-                    push(di ? 2 : 1, run);
-                    if (di) i -= run;
-                    else j -= run;
-                    continue;
-                }
-            }
-            const int tmp = (int)(tile[rel / R][c - t_c_lo] >> (8 * (rel % R))) & 0xff;
-            if (state == 0) state = tmp & 7;
-            else if (!(tmp >> (state + 2) & 1)) state = 0;
-            if (state == 0) state = tmp & 7;
-            if (state == 0) push(0, 1), --i, --j;
-            else if (state == 1 || state == 3) push(2, 1), --i;
-            else push(1, 1), --j;
-        }
-        if (i >= 0) push(2, i + 1);
-        if (j >= 0) push(1, j + 1);
-        push(-2, 0);  // flush the last run
-        __syncthreads();
-        if (!(flag & 0x80))
-            for (int x = tid; x < (n >> 1); x += nthr) {
-                const uint32_t t = cig[x];
-                cig[x] = cig[n - 1 - x];
-                cig[n - 1 - x] = t;
-            }
-    }
-    o.n_cigar = n;
-    if (tid == 0) a.out[job_id] = o;
-    if (a.host_flag) {
-        __syncthreads();
-        uint32_t *hc = a.host_cig + jb.cig_off;
-        if (n < 0) n = 0;
-        for (int x = tid; x < n; x += nthr) hc[x] = cig[x];
-        if (tid == 0) a.host_out[job_id] = o;
-        __threadfence_system();
-        __syncthreads();
-        if (tid == 0) __hip_atomic_store(a.host_flag + job_id, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
-    }
-}
-
 // One workgroup per pair of this launch's job list.  A pair's team is its
 // own W waves (jb.team, at most blockDim.x / 64): the waves beyond it end at
 // once (s_barrier then waits on the surviving waves only), so pairs of
@@ -835,7 +552,8 @@ __global__ void __launch_bounds__(kWave * kMaxTeam) ksw_stripe_kernel(StripeArgs
     for (int p = w; p < npass && !stop; p += W)
         pass_body<RIGHT, MODE, false, LUT, R>(a, kc, job, p, jb, qlen, tlen, prog, W, late, stop);
     __syncthreads();  // every pass written: stripe partials, score / mte, direction bytes
-    pair_epilogue<R, MODE>(a, job, jb, tile, &shared_n, W * kWave);
+    StripeLayout<R, MODE> lay(tile);
+    pair_epilogue(a, job, jb, lay, &shared_n, W * kWave);
 }
 
 // Persistent one-wave workers over a device work queue.  The launch's job
@@ -871,7 +589,8 @@ ksw_stripe_queue_kernel(StripeArgs a, int32_t *qhead)
         for (int p = 0; p < npass && !stop; ++p)
             pass_body<RIGHT, MODE, false, LUT, R>(a, kc, job, p, jb, qlen, tlen, prog, 1, late, stop);
         __syncthreads();
-        pair_epilogue<R, MODE>(a, job, jb, tile, &shared_n, kWave);
+        StripeLayout<R, MODE> lay(tile);
+        pair_epilogue(a, job, jb, lay, &shared_n, kWave);
         __syncthreads();  // tile and prog are the next pair's
     }
 }
@@ -954,7 +673,8 @@ __global__ void __launch_bounds__(kWave * kWideGroup) ksw_stripe_wide_epilogue_k
         __syncthreads();
         if (threadIdx.x == 0) atomicAdd(a.werr, 1);
     }
-    pair_epilogue<R, MODE>(a, job, jb, tile, &shared_n, (int)blockDim.x);
+    StripeLayout<R, MODE> lay(tile);
+    pair_epilogue(a, job, jb, lay, &shared_n, (int)blockDim.x);
 }
 
 // Dispatch over the kernel variants: group (left, right, score-only,
