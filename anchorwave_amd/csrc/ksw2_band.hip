@@ -1,7 +1,7 @@
 // ksw2_band.hip -- gfx950 kernel for banded ksw_extd2 calls inside the
 // stripe kernel's exactness domain (match 0, mismatch <= 0, the scoring
 // bounds that keep every int8 intermediate in range, no z-drop, no
-// wildcard), typically long pairs under a wide band (w = 4096).
+// wildcard), from the narrow bands of certification to w = 4096 and beyond.
 //
 // The reference sweeps anti-diagonals r; on each it updates the positions
 // t of the 16/64-rounded range [stB, en16] in place
@@ -12,41 +12,48 @@
 // wrap at a non-64-aligned start, row r re-initialised at column 0).  This
 // kernel evaluates the same cells in (t, r) coordinates:
 //
-//  * Stripes.  The positions are cut into stripes of 256; lane k of a wave
-//    holds positions t0 + 4k .. t0 + 4k + 3 of its stripe in registers (the
-//    in-place state u, v, x, y, x2, y2, s and H of each) and steps through
-//    the anti-diagonals that reach the stripe.  Within a lane the positions
-//    are updated from the highest down, so each still reads its upper
-//    neighbour's value from the previous anti-diagonal; the lane's top
-//    position takes the lane above's bottom values through a DPP shift, and
-//    lane 0 takes the previous stripe's bottom position from a per-pair
-//    buffer indexed by r.  A position outside [stB, en16] is not updated:
-//    its stale value is simply the register it keeps.
-//  * Because stB is a multiple of 64 and en16 + 1 of 16, a lane's four
-//    positions are all inside [stB, en16] or all outside: the commit and the
-//    direction-byte store are per lane (four bytes, aligned).
-//  * Teams.  W waves per pair (W = 16 for w = 4096: a stripe's
-//    anti-diagonals start 2 SR after its predecessor's, so about 2w / 2 SR
-//    stripes are in flight); wave w takes stripes w, w + W, ...  The waves
-//    sit in workgroups of four (one wave per SIMD) that the dispatcher
-//    spreads over the CUs, so a pair's waves do not share SIMDs.  Stripe s
-//    trails stripe s-1 by at least 64 anti-diagonals through progress
-//    counts in device memory; counts and hand-off entries use device-scope
-//    (sc1) accesses, coherent across the XCDs' L2s, and a count is stored
-//    only after the entries it covers are complete.  Three buffers by
-//    stripe mod 3: a producer three stripes ahead reuses a buffer, and the
-//    leads between the stripes in between keep it from overwriting an entry
-//    before it is read.
-//  * A wait that outlasts kWaitTicks (a workgroup the dispatcher could not
-//    place) gives up: the pair is flagged for the general kernel, which
-//    recomputes it, and every wave still runs to its end.
+//  * Stripes.  The positions are cut into stripes of 128; lane k of a wave
+//    holds positions t0 + 2k and t0 + 2k + 1 in the halves of its registers
+//    (the in-place state u, v, x, y, x2, y2, the score s, and H in 32 bits)
+//    and steps through the anti-diagonals that reach the stripe.  A position
+//    takes the one above it through a DPP shift, the stripe's first from the
+//    stripe above through a hand-off.  Every lane computes every step: a
+//    position above en16 is set to the initial state when it enters the band,
+//    and below stB nothing reads it.
+//  * Why 128 positions.  A banded pair's time is its chain of anti-diagonals,
+//    so what counts is the length of a step: one packed cell here (two, and
+//    H of four positions, at 256 positions a stripe).  A stripe starts 256
+//    anti-diagonals after the one above it, plus what the hand-off costs.
+//  * Waves.  Wave w of a pair's W takes stripes w, w + W, ...; about
+//    (2w + 420) / 256 are in flight.  They sit in workgroups of four, one wave
+//    per SIMD.  A stripe's last position (x, x2, v, H, one entry per
+//    anti-diagonal) goes to the next wave of a workgroup through a ring in
+//    LDS, four anti-diagonals at a time, and from the last wave of a workgroup
+//    to the first of the next through the pair's buffer in device memory, 16
+//    at a time: two device-scope 8-byte stores per entry that carry the
+//    reading stripe's number, which the reader looks for, so no count is
+//    published and nothing waits for a store to complete.  One buffer
+//    serves all stripes: an entry is overwritten three stripes and at least
+//    three anti-diagonals after the block that holds it has been read.
+//  * A wait on device memory that outlasts 10 s (a workgroup the dispatcher
+//    could not place) gives up: the pair is flagged for the general kernel,
+//    which recomputes it, and every wave still runs to its end.  Waits in LDS
+//    are on waves of the same workgroup.
+//  * Steps go in blocks of 16, aligned so that the band's end moves on even
+//    steps and its start on odd ones.  A block in which neither end is near
+//    the stripe, or only one of them, or clear of the rare rules (column 0,
+//    t == r, the last position, row and anti-diagonal) runs unrolled without
+//    the tests it does not need; the others go step by step with every rule.
 //  * H bookkeeping (minimap2/ksw2_extd2_sse.c:332-375): H[en0] from the
 //    position above plus u, H[t] += v on [st0, en0), mte on position tlen-1,
 //    mqe where column qlen-1 is the band's start, the score at the last
-//    anti-diagonal.  The maximum is not tracked: in this domain H never
-//    exceeds ez->max's initial 0 (match score 0), so ksw_apply_zdrop never
-//    changes it; every position checks that and a pair that ever sees H > 0
-//    is flagged for the general kernel (redo), which tracks the maximum.
+//    anti-diagonal.  Held as -8 H + p r (p the bias of v and u), so one
+//    v_dot2 adds a half of v.  The maximum is not tracked: H never exceeds
+//    ez->max's initial 0.  (Every z is <= 0, capped at the match score.  Let
+//    K(t, r) = H(t, r) - u(t, r).  A position enters the band with K = H of
+//    the position above, and on the next anti-diagonal H = K + z and K grows
+//    by the v it takes from above, as H of the position above does; where it
+//    takes the initial v instead, at st16, K falls.  So K <= 0 and H <= 0.)
 //  * Band exit (st > en) is pure geometry: the host passes the number of
 //    anti-diagonals the reference completes.
 //
@@ -55,6 +62,11 @@
 // general backtrack kernel walks them; the KswOut fields; the redo flag.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+
+#include <algorithm>
+#include <type_traits>
+
+#include "ksw2_cell.h"
 #include "ksw2_common.h"
 #include "ksw2_kernels.h"
 
@@ -62,19 +74,19 @@ namespace kswhip {
 
 namespace {
 
-constexpr int R = kBandRowsPerLane;  // positions per lane (4: one step of a stripe is short)
-constexpr int SR = kWave * R;        // positions per stripe
-static_assert(R == 4, "a lane's direction bytes and query window are one dword");
-// Hand-off granularity, measured on the banded long pairs (64 x 100-300
-// kbp, w = 4096): blocks, lead and publications of 64/64/32 anti-diagonals
-// 0.625 s per call, 32/32/16 0.596 s, 16/16/8 0.594 s, 16/16/16 0.582 s,
-// 8/8/8 0.620 s.
-constexpr int kBlock = 16;       // anti-diagonals per block of hand-off loads
-constexpr int kPublish = 16;     // anti-diagonals between progress publications
-constexpr int kLead = 16;        // lead a stripe waits for on its predecessor
-constexpr int kBufs = 3;         // hand-off buffers, by stripe mod 3
-static_assert(kBlock % kPublish == 0, "publications fall on block offsets");
-constexpr int kDppWaveShr1 = 0x138, kDppWaveShl1 = 0x130;
+using cell::add_hi;
+using cell::add_lo;
+using cell::bfi;
+using cell::dpp_shr1;
+using cell::hi16;
+using cell::lo16;
+using cell::perm;
+using cell::sign2;
+using cell::splat;
+using cell::sub2;
+
+constexpr int SR = kBandStripe;                 // positions per stripe
+constexpr int kBlock = 16;                      // anti-diagonals per block
 constexpr uint64_t kWaitTicks = 1000000000ull;  // 10 s of the 100 MHz real-time clock
 
 struct Band {
@@ -100,625 +112,504 @@ __device__ __forceinline__ Band band_of(int r, int qlen, int tlen, int w, int tl
     return b;
 }
 
-// Anti-diagonals that can touch positions [t0, t0 + SR): a position t is
-// computed only when stB <= t <= en16 and scored only when st0 <= t <=
-// sc_end, which bound r to [2(t-15) - w - 1, 2(t+63) + w].
-__device__ __forceinline__ void stripe_range(int t0, int w, int r_end, int &lo, int &hi)
+// A wave's hand-off ring: the entries of the position above its stripe (x, x2
+// and v in the high halves, H) and the query codes of its first position, one
+// per anti-diagonal: entry c is the state as anti-diagonal c - 1 left it.  The
+// wave above writes the entries (the first wave of a workgroup its own, from
+// the pair's buffer; the last writes the ring past its own and copies it there).
+constexpr int kRing = 256;
+struct BandRing {
+    uint32_t e[5][kRing];
+    int32_t filled, taken;  // anti-diagonals written and read, counted from stripe kk of the wave at kk * span
+    int32_t pad[14];
+};
+// The lanes that hold no stripe's last position write to the space after a
+// workgroup's rings.
+constexpr int ring_bytes(int waves)
 {
-    lo = max(0, 2 * t0 - w - 40);
-    hi = min(r_end - 1, 2 * (t0 + SR - 1) + w + 130);
+    return (waves + 1) * (int)sizeof(BandRing) + (int)sizeof(uint32_t) * (3 * kRing + kWave + kBlock);
 }
 
-// lane k takes lane k-1's v, lane 0 keeps `old`
-__device__ __forceinline__ int dpp_shr1(int old, int v)
+__device__ __forceinline__ int32_t ring_load(const int32_t *x)
 {
-    return __builtin_amdgcn_update_dpp(old, v, kDppWaveShr1, 0xF, 0xF, false);
+    return __builtin_amdgcn_readfirstlane(__hip_atomic_load(x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP));
 }
-// lane k takes lane k+1's v (lane 63 keeps its own)
-__device__ __forceinline__ int dpp_shl1(int v) { return __builtin_amdgcn_update_dpp(v, v, kDppWaveShl1, 0xF, 0xF, false); }
-
-// Progress count: stored after the wave's earlier hand-off stores are
-// complete (s_waitcnt vmcnt(0)); both are device-scope stores that bypass
-// the XCD-private caches.
-__device__ __forceinline__ void publish(int32_t *slot, int value)
+// (a wave's LDS operations complete in order, so a count stored after an
+// entry is seen after it; the empty asm keeps the compiler to that order)
+__device__ __forceinline__ void ring_store(int32_t *x, int32_t v)
 {
     asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_waitcnt(0xF70);  // vmcnt(0)
-    asm volatile("" ::: "memory");
-    if (__lane_id() == 0) __hip_atomic_store(slot, value, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(x, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
-__device__ __forceinline__ int load_count(const int32_t *slot)
+// Entry of the pair's buffer: two dwords with the reader's number in the low
+// half of the second, and H with that number.
+__device__ __forceinline__ uint64_t load_half(const int32_t *buf, int r, int k)
 {
-    return __builtin_amdgcn_readfirstlane(__hip_atomic_load(slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+    return __hip_atomic_load((const uint64_t *)buf + 2 * r + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
+__device__ __forceinline__ void store_half(int32_t *buf, int r, int k, uint32_t a, uint32_t b)
+{
+    __hip_atomic_store((uint64_t *)buf + 2 * r + k, (uint64_t)a | (uint64_t)b << 32, __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ uint32_t reader_tag(int s) { return (uint32_t)(s % 65535 + 1); }  // never 0
 
-// Spins until the producer's published count reaches `need` (uniform exit
-// test on lane 0's value).  A producer always ends a stripe by publishing a
-// count past every need of its consumer, so the wait ends once the
-// producer runs; past kWaitTicks it gives up, sets `late` and returns a
-// count that satisfies every later wait of the wave.
-__device__ __forceinline__ int wait_count(const int32_t *slot, int need, int known, int &late)
-{
-    if (known >= need) return known;
-    int seen = load_count(slot);
-    if (seen < need) {
-        const uint64_t t_start = wall_clock64();
-        while (seen < need) {
-            __builtin_amdgcn_s_sleep(2);
-            seen = load_count(slot);
-            if (seen < need && wall_clock64() - t_start > kWaitTicks) {
-                late = 1;
-                seen = INT32_MAX;
-            }
-        }
-    }
-    asm volatile("" ::: "memory");  // the entry loads stay behind the wait
-    return seen;
-}
-
-__device__ __forceinline__ int pack3(int x, int v, int x2)
-{
-    return (x & 0xff) | (v & 0xff) << 8 | (x2 & 0xff) << 16;
-}
-__device__ __forceinline__ int byte_s(int w, int k) { return (int)(int8_t)(uint8_t)((unsigned)w >> (8 * k)); }
-
-// A lane's R direction bytes (one aligned store).
-__device__ __forceinline__ void store_dirs(uint8_t *dst, const uint32_t (&dw)[2])
-{
-    if (R == 8) {
-        uint2 w8;
-        w8.x = dw[0], w8.y = dw[1];
-        *(uint2 *)dst = w8;
-    } else {
-        *(uint32_t *)dst = dw[0];
-    }
-}
+__device__ __forceinline__ uint32_t part(const uint4 &x, int k) { return k == 0 ? x.x : k == 1 ? x.y : k == 2 ? x.z : x.w; }
 
 }  // namespace
 
-// Scaled, tagged state (the stripe kernel's representation): every
-// difference w is kept as -8w (u, v) or -8(w + G) - BIAS (x, y with G1; x2,
-// y2 with G2), BIAS = 0 for left and 8 for right alignment, so that one
-// chain of mins over s, a, b, a2, b2 (each -8*value + a 3-bit tag) gives
-// both the reference's maximum and the index its strict '>' (left) or '>='
-// (right) chain picks; T = (x + v) + 8e - 8z is -8a' - BIAS, whose sign is
-// the continuation flag and min(T, -BIAS) the new x.
-struct BandConsts {
-    int CA, CB, CA2, CB2, E1, E2, LIM, SM, SMM, CAP;
-};
-
-template <bool RIGHT>
-__device__ __forceinline__ BandConsts band_consts(const KswScore &sc)
-{
-    const int bias = RIGHT ? 8 : 0;
-    const int tS = RIGHT ? 7 : 0, tA = RIGHT ? 6 : 1, tB = RIGHT ? 5 : 2, tA2 = RIGHT ? 4 : 3, tB2 = RIGHT ? 3 : 4;
-    BandConsts k;
-    k.CA = 8 * sc.G1 + tA + bias, k.CB = 8 * sc.G1 + tB + bias;
-    k.CA2 = 8 * sc.G2 + tA2 + bias, k.CB2 = 8 * sc.G2 + tB2 + bias;
-    k.E1 = 8 * sc.e, k.E2 = 8 * sc.e2, k.LIM = -bias;
-    k.SM = -8 * sc.mch + tS, k.SMM = -8 * sc.mis + tS;
-    k.CAP = -8 * sc.mch;  // z = min(z, mat[0]) in the -8 domain
-    return k;
-}
-
-// One cell in the scaled form.  In: x, v, x2 of the position above, u, y,
-// y2 of this position (scaled), mm = mismatch.  Out: the new state; returns
-// the direction byte (0 when SCORE_ONLY).
+// The band's blocks are placed so that (r + w) % 16 == 0 at their first
+// anti-diagonal; `c` below is r + (w % 16).  What bounds it: the chain of a
+// pair's anti-diagonals, a step of 54 (neither end of the band in the stripe)
+// to 67 instructions (its start), and some 20 a step around them, of a wave
+// alone on its SIMD.  Measured, against stripes of 256 positions handed on
+// through progress counts in device memory: a pair of 20 kbp, w = 256, 1.1 and
+// 0.24 us per anti-diagonal; 16 pairs of 60-120 kbp, w = 4096, 213 and 64 ms;
+// 2,048 pairs of 2 kbp, w = 256, 26 ms on the general kernel and 4.5 ms here.
 template <bool RIGHT, bool SCORE_ONLY>
-__device__ __forceinline__ int band_cell(const BandConsts &k, int X, int V, int X2, int U, int Y, int Y2, bool mm,
-                                         int &Un, int &Vn, int &Xn, int &Yn, int &X2n, int &Y2n)
+__global__ void __launch_bounds__(kWave * kBandGroup) __attribute__((amdgpu_waves_per_eu(3))) ksw_band_kernel(BandArgs a)
 {
-    const int S = mm ? k.SMM : k.SM;
-    const int A = X + V + k.CA, B = Y + U + k.CB, A2 = X2 + V + k.CA2, B2 = Y2 + U + k.CB2;
-    const int Z = min(min(min(min(S, A), B), A2), B2);
-    const int Z8 = max(Z & ~7, k.CAP);
-    const int M1 = k.E1 - Z8, M2 = k.E2 - Z8;
-    const int Ta = X + V + M1, Tb = Y + U + M1, Ta2 = X2 + V + M2, Tb2 = Y2 + U + M2;
-    Un = Z8 - V, Vn = Z8 - U;
-    Xn = min(Ta, k.LIM), Yn = min(Tb, k.LIM), X2n = min(Ta2, k.LIM), Y2n = min(Tb2, k.LIM);
-    if (SCORE_ONLY) return 0;
-    int d = RIGHT ? (~Z & 7) : (Z & 7);
-    d |= (int)(((uint32_t)Ta >> 31) << 3) | (int)(((uint32_t)Tb >> 31) << 4);
-    d |= (int)(((uint32_t)Ta2 >> 31) << 5) | (int)(((uint32_t)Tb2 >> 31) << 6);
-    return d;
-}
-
-// Two positions per register: position 2m of a lane in the low half of
-// register m, 2m+1 in the high half.  The scaled values and every sum the
-// cell forms fit in 16 bits in this domain (the stripe kernel's argument:
-// int8 differences times 8 plus constants below 2^11), so the packed cell
-// gives the 32-bit cell's values.
-typedef short v2s __attribute__((ext_vector_type(2)));
-typedef unsigned short v2u __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ int bits(v2s v) { return __builtin_bit_cast(int, v); }
-__device__ __forceinline__ int bits(v2u v) { return __builtin_bit_cast(int, v); }
-__device__ __forceinline__ v2s vec(int x) { return __builtin_bit_cast(v2s, x); }
-__device__ __forceinline__ v2u uvec(int x) { return __builtin_bit_cast(v2u, x); }
-__device__ __forceinline__ v2s splat(int x) { return (v2s){(short)x, (short)x}; }
-__device__ __forceinline__ v2s vmin(v2s a, v2s b) { return __builtin_elementwise_min(a, b); }
-__device__ __forceinline__ v2s vmax(v2s a, v2s b) { return __builtin_elementwise_max(a, b); }
-__device__ __forceinline__ int lo16(int x) { return (int)(int16_t)(x & 0xffff); }
-__device__ __forceinline__ int hi16(int x) { return x >> 16; }
-// (x >> 3) of each half, sign-extended to 32 bits
-__device__ __forceinline__ int lo16_div8(int x) { return __builtin_amdgcn_sbfe(x, 3, 13); }
-__device__ __forceinline__ int hi16_div8(int x) { return x >> 19; }
-// the high half of `hi` and the low half of `lo`: positions (2m-1, 2m)
-__device__ __forceinline__ int above_pair(int lo_reg, int hi_reg)
-{
-    return (int)__builtin_amdgcn_alignbit((unsigned)hi_reg, (unsigned)lo_reg, 16);
-}
-
-struct BandConsts2 {
-    v2s CA, CB, CA2, CB2, E1, E2, LIM, SM, SD, CAP;
-};
-
-__device__ __forceinline__ BandConsts2 pack_consts(const BandConsts &k)
-{
-    BandConsts2 p;
-    p.CA = splat(k.CA), p.CB = splat(k.CB), p.CA2 = splat(k.CA2), p.CB2 = splat(k.CB2);
-    p.E1 = splat(k.E1), p.E2 = splat(k.E2), p.LIM = splat(k.LIM);
-    p.SM = splat(k.SM), p.SD = splat(k.SMM - k.SM), p.CAP = splat(k.CAP);
-    return p;
-}
-
-// band_cell on two positions.  X/V/X2: the positions above; U/Y/Y2 this
-// pair's, replaced with the new values, as are X/V/X2 (the new values of
-// this pair); mm 0/1 per half.  Returns the two direction bytes in the low
-// byte of each half.
-template <bool RIGHT, bool SCORE_ONLY>
-__device__ __forceinline__ int band_cell2(const BandConsts2 &k, v2u mm, v2s &X, v2s &V, v2s &X2, v2s &U, v2s &Y,
-                                          v2s &Y2)
-{
-    v2u m = mm;
-    asm volatile("" : "+v"(m));  // keep the multiply-add form
-    const v2s S = k.SM + __builtin_bit_cast(v2s, m) * k.SD;
-    const v2s XV = X + V, X2V = X2 + V, YU = Y + U, Y2U = Y2 + U;
-    const v2s A = XV + k.CA, B = YU + k.CB, A2 = X2V + k.CA2, B2 = Y2U + k.CB2;
-    const v2s Z = vmin(vmin(vmin(vmin(S, A), B), A2), B2);
-    const v2s Z8 = vmax(vec(bits(Z) & (int)0xFFF8FFF8u), k.CAP);
-    const v2s M1 = k.E1 - Z8, M2 = k.E2 - Z8;
-    const v2s Ta = XV + M1, Tb = YU + M1, Ta2 = X2V + M2, Tb2 = Y2U + M2;
-    const v2s Un = Z8 - V, Vn = Z8 - U;
-    X = vmin(Ta, k.LIM), Y = vmin(Tb, k.LIM), X2 = vmin(Ta2, k.LIM), Y2 = vmin(Tb2, k.LIM);
-    U = Un, V = Vn;
-    if (SCORE_ONLY) return 0;
-    int d = RIGHT ? (~bits(Z) & 0x00070007) : (bits(Z) & 0x00070007);
-    d |= bits(__builtin_bit_cast(v2u, Ta) >> (v2u){12, 12}) & 0x00080008;
-    d |= bits(__builtin_bit_cast(v2u, Tb) >> (v2u){11, 11}) & 0x00100010;
-    d |= bits(__builtin_bit_cast(v2u, Ta2) >> (v2u){10, 10}) & 0x00200020;
-    d |= bits(__builtin_bit_cast(v2u, Tb2) >> (v2u){9, 9}) & 0x00400040;
-    return d;
-}
-
-// Per-stripe state of a lane: four positions in two packed registers per
-// quantity, the score bit of each position as 0/1 halves, H in 32 bits.
-struct Lane4 {
-    v2s U[2], V[2], X[2], Y[2], X2[2], Y2[2];
-    v2u MM[2];
-    int H[4];
-};
-
-// The inputs from the positions above for the lane's two pairs: (p-1, p0)
-// and (p1, p2), with position -1 from `top` (high half).
-struct Above {
-    v2s X[2], V[2], X2[2];
-};
-
-__device__ __forceinline__ Above above_of(const Lane4 &st, int tx, int tv, int tx2)
-{
-    Above a;
-    a.X[0] = vec(above_pair(tx, bits(st.X[0]))), a.X[1] = vec(above_pair(bits(st.X[0]), bits(st.X[1])));
-    a.V[0] = vec(above_pair(tv, bits(st.V[0]))), a.V[1] = vec(above_pair(bits(st.V[0]), bits(st.V[1])));
-    a.X2[0] = vec(above_pair(tx2, bits(st.X2[0]))), a.X2[1] = vec(above_pair(bits(st.X2[0]), bits(st.X2[1])));
-    return a;
-}
-
-// The four direction bytes of a lane, positions in order.
-__device__ __forceinline__ uint32_t pack_dirs(int d0, int d1)
-{
-    return __builtin_amdgcn_perm((unsigned)d1, (unsigned)d0, 0x06040200u);
-}
-
-// Query codes of the lane's pairs from its window: (q0, q1), (q2, q3).
-__device__ __forceinline__ void query_pairs(uint32_t qwin, v2u &q0, v2u &q1)
-{
-    q0 = uvec((int)__builtin_amdgcn_perm(0u, qwin, 0x0c010c00u));
-    q1 = uvec((int)__builtin_amdgcn_perm(0u, qwin, 0x0c030c02u));
-}
-
-__device__ __forceinline__ v2u mismatch(v2u tb, v2u qb) { return __builtin_elementwise_min(tb ^ qb, (v2u){1, 1}); }
-
-// A band-edge step in a block clear of the rare boundary rules: the
-// interior form plus what the band's edges change.  LEAD: the band starts
-// above the stripe (st0 < t0), so no start rule applies; TRAIL: it ends
-// below the stripe (en0 > t0 + SR - 1), so no end rule applies.
-//  * Inputs of the start (minimap2/ksw2_extd2_sse.c:158-172): position stB
-//    reads position stB+15 of anti-diagonal r-1 when st16 != stB (the
-//    AVX-512 lane wrap), position st16 the initial x, v, x2 unless position
-//    st16-1 was computed on r-1.  Both become the inputs of that position
-//    (the above-values of a position are read by the one below only).
-//  * Score bits: positions [st0, sc_end] take this anti-diagonal's mismatch.
-//  * H: set at en0 from the position above, += v on [st0, en0); kept below
-//    st0 (a band one position wide reads it), free to drift above en0 (a
-//    position enters at en0 from the position above).
-//  * Commit: a lane above en16 keeps its state (it enters the band later
-//    with it); below stB a lane's positions are never read again.
-template <bool RIGHT, bool SCORE_ONLY, bool LEAD, bool TRAIL>
-__device__ __forceinline__ void edge_step(const BandConsts2 &kc, const Band &b, int t0, int tl, int lane, Lane4 &st,
-                                          const v2u (&TB)[2], uint32_t qwin, int tx, int tv, int tx2, int ch,
-                                          bool keep_prev, int U0, int L0, int &hmax, uint8_t *prow)
-{
-    Above a = above_of(st, tx, tv, tx2);
-    if (!LEAD) {
-        if (b.st16 != b.stB && b.stB >= t0 && b.stB < t0 + SR) {
-            // position stB (low half of pair 0 of its lane) takes position
-            // stB+15 (high half of pair 1 of lane (stB+15-t0)/R)
-            const int src = (b.stB + 15 - t0) / R;
-            const int wx = __builtin_amdgcn_readlane(bits(st.X[1]), src);
-            const int wv = __builtin_amdgcn_readlane(bits(st.V[1]), src);
-            const int wx2 = __builtin_amdgcn_readlane(bits(st.X2[1]), src);
-            if (lane == (b.stB - t0) / R) {
-                a.X[0] = vec((bits(a.X[0]) & (int)0xffff0000u) | ((unsigned)wx >> 16));
-                a.V[0] = vec((bits(a.V[0]) & (int)0xffff0000u) | ((unsigned)wv >> 16));
-                a.X2[0] = vec((bits(a.X2[0]) & (int)0xffff0000u) | ((unsigned)wx2 >> 16));
-            }
-        }
-        if (!keep_prev && b.st16 >= t0 && b.st16 < t0 + SR) {
-            const int k16 = (b.st16 - t0) % R, m = k16 >> 1;
-            const int hm = (k16 & 1) ? (int)0xffff0000u : 0xffff;
-            if (lane == (b.st16 - t0) / R) {
-                const int l0 = bits(splat(L0)) & hm, u0 = bits(splat(U0)) & hm;
-                if (m == 0) {
-                    a.X[0] = vec((bits(a.X[0]) & ~hm) | l0), a.V[0] = vec((bits(a.V[0]) & ~hm) | u0);
-                    a.X2[0] = vec((bits(a.X2[0]) & ~hm) | l0);
-                } else {
-                    a.X[1] = vec((bits(a.X[1]) & ~hm) | l0), a.V[1] = vec((bits(a.V[1]) & ~hm) | u0);
-                    a.X2[1] = vec((bits(a.X2[1]) & ~hm) | l0);
-                }
-            }
-        }
-    }
-    const bool la = (LEAD || tl >= b.stB) && (TRAIL || tl + R - 1 <= b.en16);
-    const int lam = la ? -1 : 0;
-    // score bits: positions [st0, sc_end] take this anti-diagonal's mismatch
-    {
-        v2u q0, q1;
-        query_pairs(qwin, q0, q1);
-        const int lo = LEAD ? 0 : min(max(b.st0 - tl, 0), R);
-        const int hi = TRAIL ? R : min(max(b.sc_end - tl + 1, 0), R);
-        const uint32_t upd = ((1u << hi) - 1u) & ~((1u << lo) - 1u);
-        const int um0 = (int)((upd & 1u) * 0xffffu | (upd & 2u) * 0x7fff8000u);
-        const int um1 = (int)((upd >> 2 & 1u) * 0xffffu | (upd >> 2 & 2u) * 0x7fff8000u);
-        st.MM[0] = uvec((bits(mismatch(TB[0], q0)) & um0) | (bits(st.MM[0]) & ~um0));
-        st.MM[1] = uvec((bits(mismatch(TB[1], q1)) & um1) | (bits(st.MM[1]) & ~um1));
-    }
-    Lane4 nw;
-#pragma unroll
-    for (int m = 0; m < 2; ++m) {
-        nw.X[m] = a.X[m], nw.V[m] = a.V[m], nw.X2[m] = a.X2[m];
-        nw.U[m] = st.U[m], nw.Y[m] = st.Y[m], nw.Y2[m] = st.Y2[m];
-    }
-    const int d0 = band_cell2<RIGHT, SCORE_ONLY>(kc, st.MM[0], nw.X[0], nw.V[0], nw.X2[0], nw.U[0], nw.Y[0], nw.Y2[0]);
-    const int d1 = band_cell2<RIGHT, SCORE_ONLY>(kc, st.MM[1], nw.X[1], nw.V[1], nw.X2[1], nw.U[1], nw.Y[1], nw.Y2[1]);
-    // H: set at en0 from the position above, += v on [st0, en0); kept below
-    // st0, free to drift above en0
-    const int un3[4] = {lo16_div8(bits(nw.U[0])), hi16_div8(bits(nw.U[0])), lo16_div8(bits(nw.U[1])),
-                        hi16_div8(bits(nw.U[1]))};
-    const int vn3[4] = {lo16_div8(bits(nw.V[0])), hi16_div8(bits(nw.V[0])), lo16_div8(bits(nw.V[1])),
-                        hi16_div8(bits(nw.V[1]))};
-#pragma unroll
-    for (int k = R - 1; k >= 0; --k) {
-        const int t = tl + k;
-        const int hab = k > 0 ? st.H[k - 1] : ch;
-        const int vdec = (LEAD || t >= b.st0) ? vn3[k] : 0;
-        const int hn = !TRAIL && t == b.en0 ? hab - un3[k] : st.H[k] - vdec;
-        st.H[k] = hn;
-        const bool inb = (LEAD || t >= b.st0) && (TRAIL || t <= b.en0);
-        hmax = max(hmax, inb ? hn : KSW_NEG_INF_I);
-    }
-    // commit: a lane above en16 keeps its state (it enters the band later
-    // with it); below stB a lane's positions are never read again
-#pragma unroll
-    for (int m = 0; m < 2; ++m) {
-        if (TRAIL) {
-            st.U[m] = nw.U[m], st.V[m] = nw.V[m], st.X[m] = nw.X[m];
-            st.Y[m] = nw.Y[m], st.X2[m] = nw.X2[m], st.Y2[m] = nw.Y2[m];
-        } else {
-            st.U[m] = vec((bits(nw.U[m]) & lam) | (bits(st.U[m]) & ~lam));
-            st.V[m] = vec((bits(nw.V[m]) & lam) | (bits(st.V[m]) & ~lam));
-            st.X[m] = vec((bits(nw.X[m]) & lam) | (bits(st.X[m]) & ~lam));
-            st.Y[m] = vec((bits(nw.Y[m]) & lam) | (bits(st.Y[m]) & ~lam));
-            st.X2[m] = vec((bits(nw.X2[m]) & lam) | (bits(st.X2[m]) & ~lam));
-            st.Y2[m] = vec((bits(nw.Y2[m]) & lam) | (bits(st.Y2[m]) & ~lam));
-        }
-    }
-    if (!SCORE_ONLY && la) *(uint32_t *)(prow + (tl - b.stB)) = pack_dirs(d0, d1);
-}
-
-// Up to kBandTeam waves per pair in workgroups of up to kBandGroup.  A
-// pair needs about (2w + 2 SR + 300) / (2 SR + 190) stripes in flight (a
-// stripe's anti-diagonals start 2 SR after its predecessor's, plus the
-// lead), 13 for w = 4096 at SR = 256.
-template <bool RIGHT, bool SCORE_ONLY>
-__global__ void __launch_bounds__(kWave * kBandGroup) ksw_band_kernel(BandArgs a)
-{
-    const int nthr = blockDim.x, tid = threadIdx.x, lane = tid % kWave;
+    extern __shared__ __align__(16) uint8_t band_lds[];
+    BandRing *rings = (BandRing *)band_lds;
+    const int group = blockDim.x / kWave, lane = threadIdx.x % kWave;
     const int wgs = a.wgs, g = blockIdx.x % wgs;
-    const int W = __builtin_amdgcn_readfirstlane(wgs * (nthr / kWave));
-    const int wv = __builtin_amdgcn_readfirstlane(g * (nthr / kWave) + tid / kWave);
+    const int W = __builtin_amdgcn_readfirstlane(wgs * group);
+    const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kWave);
+    const int wv = __builtin_amdgcn_readfirstlane(g * group + w);
+    if ((int)threadIdx.x <= group) rings[threadIdx.x].filled = rings[threadIdx.x].taken = 0;
+    __syncthreads();
     const int job = __builtin_amdgcn_readfirstlane(a.order[blockIdx.x / wgs]);
     const GenJob jb = a.jobs[job];
     const int qlen = __builtin_amdgcn_readfirstlane(jb.qlen), tlen = __builtin_amdgcn_readfirstlane(jb.tlen);
     const int bw = __builtin_amdgcn_readfirstlane(jb.w), flag = __builtin_amdgcn_readfirstlane(jb.flag);
     const int tlenB = __builtin_amdgcn_readfirstlane(jb.tlenB), r_end = __builtin_amdgcn_readfirstlane(jb.r_end);
-    const int ncolB = jb.ncolB;
+    const int ncolB = __builtin_amdgcn_readfirstlane(jb.ncolB);
     const bool generic = flag & 0x04;
     const int nr = qlen + tlen - 1;
     const KswScore &sc = a.sc.k;
-    const BandConsts kc = band_consts<RIGHT>(sc);
-    const BandConsts2 kc2 = pack_consts(kc);
-    const int G1 = sc.G1, G2 = sc.G2, bias = RIGHT ? 8 : 0;
-    // scaled constants: u, v = -G1 -> 8 G1; x, y, x2, y2 at their initial
-    // values (-G1, -G2) -> -BIAS
-    const int U0 = 8 * G1, L0 = -bias;
+    cell::DirCell<RIGHT> kc(sc, false);
     const uint8_t *qs = a.seq + jb.q_off, *ts = a.seq + jb.t_off;
     uint8_t *p = a.dir + jb.dir_off;
     int32_t *off = a.offs + jb.off_off, *off_end = off + nr;
-    int32_t *ctl = a.bnd + jb.bnd_off;      // control block (zeroed before the launch)
-    int32_t *buf = ctl + kBandCtl;          // kBufs buffers of 2 * nr dwords
-    int32_t *prog = ctl;                    // count of wave w at prog[w * kBandCtlStride]
+    int32_t *ctl = a.bnd + jb.bnd_off;  // control block and buffer (cleared before the launch)
+    int32_t *buf = ctl + kBandCtl;
 
     if (!SCORE_ONLY)
-        for (int r = g * nthr + tid; r < r_end; r += wgs * nthr) {
+        for (int r = g * (int)blockDim.x + (int)threadIdx.x; r < r_end; r += wgs * (int)blockDim.x) {
             const Band b = band_of(r, qlen, tlen, bw, tlenB, generic);
             off[r] = b.stB, off_end[r] = b.en16;
         }
 
-    // per-lane results over this wave's stripes
-    int mqe_h = KSW_NEG_INF_I, mqe_t = -1, mte_h = KSW_NEG_INF_I, mte_q = -1, score = KSW_NEG_INF_I, pos = 0;
+    uint32_t v_init = splat(kc.diff(-sc.G1)), sm2 = splat(kc.sm), sd2 = splat(kc.sx - kc.sm);
+    // (in vector registers: the scalar ones run out, and are then kept in lanes)
+    asm volatile("" : "+v"(v_init), "+v"(sm2), "+v"(sd2), "+v"(kc.cA2), "+v"(kc.cB2), "+v"(kc.zc), "+v"(kc.e1), "+v"(kc.e2));
+    asm volatile("" : "+v"(kc.lA), "+v"(kc.lB), "+v"(kc.lA2), "+v"(kc.lB2), "+v"(kc.mA), "+v"(kc.mB), "+v"(kc.mA2));
+    uint32_t one = 0x00010001u;
+    asm volatile("" : "+s"(one));
+    const int wofs = bw & 15, span = nr + 64;
     const int nstripes = (tlenB + SR - 1) / SR;
-    int known = 0, late = 0, stop = 0;
-    for (int s = wv, kk = 0; s < nstripes && !stop; s += W, ++kk) {
-        const int t0 = s * SR, tl = t0 + lane * R;
-        int r_lo, r_hi, p_lo = 0, p_hi = -1;
-        stripe_range(t0, bw, r_end, r_lo, r_hi);
-        if (s > 0) stripe_range(t0 - SR, bw, r_end, p_lo, p_hi);
-        const int pw = (s + W - 1) % W, pbase = (s - 1) / W * (nr + 2);  // producer wave, its count base
-        int32_t *out_buf = buf + (uint64_t)(s % kBufs) * 2 * nr;
-        const int32_t *in_buf = buf + (uint64_t)((s + kBufs - 1) % kBufs) * 2 * nr;
-        // per position: the in-place state (scaled, two positions per
-        // register) and H; the score s as a 0/1 half (1: mismatch; s is mch
-        // or mis in this domain, mch = 0 at first); the target codes as
-        // 16-bit halves (zero past tlen, as the reference's zero-padded
-        // target copy)
-        Lane4 st;
-        v2u TB[2];
-#pragma unroll
-        for (int m = 0; m < 2; ++m) {
-            st.U[m] = st.V[m] = splat(U0);
-            st.X[m] = st.Y[m] = st.X2[m] = st.Y2[m] = splat(L0);
-            st.MM[m] = (v2u){0, 0};
-            const int ta = tl + 2 * m, tb = ta + 1;
-            TB[m] = (v2u){(unsigned short)(ta < tlen ? ts[ta] : 0), (unsigned short)(tb < tlen ? ts[tb] : 0)};
-        }
-#pragma unroll
-        for (int k = 0; k < R; ++k) st.H[k] = KSW_NEG_INF_I;
-        // query window: byte k of qwin[0] is the query code of position
-        // tl + k's column r - (tl + k) (0 outside the query, as the
-        // reference's zero-tailed reversed query).  Each step lane k's new
-        // byte is the one lane k-1 drops (its byte 3); lane 0 takes Q(r - t0)
-        // from the block registers.
-        uint32_t qwin[1] = {0u};
-#pragma unroll
-        for (int k = 0; k < R; ++k) {
-            const int j = r_lo - 1 - tl - k;
-            const uint32_t c = j >= 0 && j < qlen ? (uint32_t)qs[j] : 0u;
-            qwin[k >> 2] |= c << (8 * (k & 3));
-        }
-        // per block of kBlock steps starting at rb, lane k < kBlock holds in
-        // registers what lane 0 needs at step rb + k: the query code
-        // Q(rb + k - t0) and the predecessor's entry rb + k - 1 (x, v, x2
-        // scaled, and H; initial values before its first anti-diagonal, its
-        // last entry after its last).  Loaded once per block, after the wait
-        // that guarantees the entries are written, so no step waits on
-        // memory; every step moves them down one lane, so lane 0 holds the
-        // current step's.
-        int bq = 0, bx = 0, bv = 0, bx2 = 0, bh = KSW_NEG_INF_I;
-        int lst16 = -1, len16 = -1;  // st16, en16 of anti-diagonal r-1
-        if (r_lo > 0) {
-            const Band bp = band_of(r_lo - 1, qlen, tlen, bw, tlenB, generic);
-            lst16 = bp.st16, len16 = bp.en16;
-        }
-        int hmax = KSW_NEG_INF_I;  // largest in-band H (checked against 0 at the end)
-        uint8_t *prow = p + (uint64_t)r_lo * ncolB;  // direction row of anti-diagonal r
-        for (int rb = r_lo; rb <= r_hi; rb += kBlock) {
-            if (a.stop && ((rb - r_lo) & 255) < kBlock) {
-                // the host's stop flag, every 256 anti-diagonals: end the
-                // wave (nothing of this pair is delivered)
-                stop = __builtin_amdgcn_readfirstlane(
-                    __hip_atomic_load(a.stop, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM));
-                if (stop) break;
+    // anti-diagonals that touch positions [t0, t0 + SR): computed when
+    // stB <= t <= en16, scored when st0 <= t <= sc_end <= en0 + 15
+    auto lo_of = [&](int t0) { return max(0, max(t0 - 16, 2 * t0 - 32 - bw)); };
+    auto hi_of = [&](int t0) { return min(r_end - 1, min(qlen + t0 + SR - 2, 2 * (t0 + SR - 1) + bw)); };
+    auto start_of = [&](int t0) { return lo_of(t0) + wofs & ~(kBlock - 1); };
+    // (and two on, whose entries say what the last one left: the position after
+    // the stripe can be the band's only one on both)
+    auto end_of = [&](int t0) { return (hi_of(t0) + 2 + wofs | (kBlock - 1)) + 1; };
+
+    // per-lane results over this wave's stripes
+    int mqe_h = KSW_NEG_INF_I, mqe_t = -1, mte_h = KSW_NEG_INF_I, mte_q = -1, score = KSW_NEG_INF_I;
+    int late = 0, stop = 0;
+    auto stopped = [&]() {
+        if (a.stop)
+            stop = __builtin_amdgcn_readfirstlane(__hip_atomic_load(a.stop, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM));
+        return stop != 0;
+    };
+    // one workgroup of as many waves as stripes in flight: the last hands on to
+    // the first through the first's ring (with fewer, each would wait for room
+    // in the next one's ring, the last for a stripe that the first has yet to
+    // begin)
+    const bool circle = wgs == 1 && group > 1 && 2 * bw + 420 <= 256 * W;
+    BandRing &in = rings[w], &out = rings[circle && w + 1 == group ? 0 : w + 1];
+    uint32_t *const spill = (uint32_t *)(rings + group + 1);
+    auto has_stripe = [&](int s) { return s < nstripes && lo_of(s * SR) <= hi_of(s * SR); };
+    // stripe s, the kk-th of this wave.  FED: its entries come from another
+    // wave of the workgroup; LEAVES: its own go to the pair's buffer
+    auto stripe = [&](int s, int kk, auto fed_by_wave, auto to_buffer) {
+        constexpr bool FED = decltype(fed_by_wave)::value, LEAVES = decltype(to_buffer)::value;
+        const int t0 = s * SR, tl = t0 + 2 * lane;
+        const int r_hi = hi_of(t0), c_lo = start_of(t0), c_end = end_of(t0);
+        const int base = kk * span, in_base = w > 0 ? base : base - span;  // of this stripe's counts and the one's above
+        const int p_lo = s > 0 ? start_of(t0 - SR) : 0, p_end = s > 0 ? end_of(t0 - SR) : 0;
+        const int p_hi = s > 0 ? hi_of(t0 - SR) : -2;
+        const bool has_next = LEAVES || has_stripe(s + 1);
+        const int n_lo = has_next ? start_of(t0 + SR) : 0;
+        const bool feeds = !LEAVES && has_next, enters = !FED && s > 0;
+        const uint32_t tag = reader_tag(s), next_tag = reader_tag(s + 1);
+
+        cell::Right st;
+        cell::Down dn;
+        st.u = dn.v = v_init, st.y = kc.y0(), st.y2 = kc.y20(), dn.x = kc.x0(), dn.x2 = kc.x20();
+        uint32_t sco = sm2;  // the score candidates (the match score until first written)
+        int h0 = 0, h1 = 0;
+        auto qcode = [&](int j) { return j >= 0 && j < qlen ? (uint32_t)qs[j] : 0u; };
+        const uint32_t tb = (tl < tlen ? (uint32_t)ts[tl] : 0u) | (tl + 1 < tlen ? (uint32_t)ts[tl + 1] << 16 : 0u);
+        uint32_t qb = qcode(c_lo - wofs - 1 - tl) | qcode(c_lo - wofs - 2 - tl) << 16;
+        const uint32_t pos = ((uint32_t)tl & 0xffffu) | (uint32_t)(tl + 1) << 16;
+
+        // ---- a block's query codes and (the first wave of a workgroup) its
+        // entries from the pair's buffer: asked for a block ahead, put into
+        // the ring 12 steps later
+        uint64_t na = 0, nh = 0;
+        uint32_t nq = 0;
+        auto entry_valid = [&](int c) { return lane < kBlock && c >= p_lo && c - wofs >= 0 && c - wofs <= min(p_hi + 2, nr); };
+        auto fetch = [&](int cb) {
+            const int c = cb + lane, j = c - wofs - t0;
+            nq = qs[min(max(j, 0), qlen - 1)];
+            if (enters) {
+                const int r = min(max(c - wofs, 0), nr);
+                na = load_half(buf, r, 0), nh = load_half(buf, r, 1);
             }
-            if (s > 0) known = wait_count(prog + pw * kBandCtlStride, pbase + min(rb + kLead, p_hi) + 1, known, late);
-            {
-                const int j = rb + lane - t0;
-                bq = j >= 0 && j < qlen ? (int)qs[j] : 0;
-                const int e = min(rb + lane - 1, p_hi);
-                int pk = pack3(-G1, -G1, -G2), h = KSW_NEG_INF_I;
-                if (lane < kBlock && s > 0 && p_hi >= p_lo && e >= p_lo) {
-                    const uint64_t en = __hip_atomic_load((const uint64_t *)(in_buf + 2 * e), __ATOMIC_RELAXED,
-                                                          __HIP_MEMORY_SCOPE_AGENT);
-                    pk = (int)(uint32_t)en, h = (int)(uint32_t)(en >> 32);
-                }
-                // take the loads here: the steps of the block then read the
-                // registers without waiting on memory (the step's own stores
-                // would otherwise be waited for on every step)
-                asm volatile("" : "+v"(bq), "+v"(pk), "+v"(h));
-                // scaled, in the high half (the position above pair 0)
-                bx = (-8 * (byte_s(pk, 0) + G1) - bias) << 16, bv = (-8 * byte_s(pk, 1)) << 16;
-                bx2 = (-8 * (byte_s(pk, 2) + G2) - bias) << 16, bh = h;
-            }
-            const int rbe = min(rb + kBlock - 1, r_hi);
-            // whether the block is clear of the rare boundary rules (the
-            // injection at t == r, a start below 16, the last position or
-            // anti-diagonal, the mqe column): r - en0, st0, en0 and r - st0
-            // never decrease with r, so the block's ends decide
-            bool plain;
-            {
-                const Band b0 = band_of(rb, qlen, tlen, bw, tlenB, generic);
-                const Band b1 = band_of(rbe, qlen, tlen, bw, tlenB, generic);
-                plain = rb - b0.en0 > 15 && b0.st0 >= 16 && b0.en0 > 0 && b1.en0 < tlen - 1 && rbe < nr - 1 &&
-                        rbe - b1.st0 < qlen - 1;
-            }
-            for (int r = rb; r <= rbe; ++r, prow += ncolB) {
-                const Band b = band_of(r, qlen, tlen, bw, tlenB, generic);
-                // query window: each lane's new byte is the one the lane
-                // above drops, lane 0's the block's current query code
-                qwin[0] = qwin[0] << 8 | ((uint32_t)dpp_shr1(bq << 24, (int)qwin[0]) >> 24);
-                // position t0-1 as anti-diagonal r-1 left it (high halves): the
-                // lane above's bottom position, lane 0's from the block
-                // registers
-                const int tx = dpp_shr1(bx, bits(st.X[1])), tv = dpp_shr1(bv, bits(st.V[1]));
-                const int tx2 = dpp_shr1(bx2, bits(st.X2[1])), ch = dpp_shr1(bh, st.H[R - 1]);
-                bq = dpp_shl1(bq), bx = dpp_shl1(bx), bv = dpp_shl1(bv), bx2 = dpp_shl1(bx2), bh = dpp_shl1(bh);
-                // interior step: every position of the stripe strictly inside
-                // (st0, en0) -- all computed and scored, no boundary rule, no H
-                // entry, no mqe/mte/score position -- the lean form
-                if (b.st0 < t0 && t0 + SR - 1 < b.en0) {
-                    Above ab = above_of(st, tx, tv, tx2);
-                    v2u q0, q1;
-                    query_pairs(qwin[0], q0, q1);
-                    st.MM[0] = mismatch(TB[0], q0), st.MM[1] = mismatch(TB[1], q1);
-                    st.X[0] = ab.X[0], st.V[0] = ab.V[0], st.X2[0] = ab.X2[0];
-                    st.X[1] = ab.X[1], st.V[1] = ab.V[1], st.X2[1] = ab.X2[1];
-                    const int d0 = band_cell2<RIGHT, SCORE_ONLY>(kc2, st.MM[0], st.X[0], st.V[0], st.X2[0], st.U[0],
-                                                                 st.Y[0], st.Y2[0]);
-                    const int d1 = band_cell2<RIGHT, SCORE_ONLY>(kc2, st.MM[1], st.X[1], st.V[1], st.X2[1], st.U[1],
-                                                                 st.Y[1], st.Y2[1]);
-                    // v = -(V / 8)
-                    st.H[0] -= lo16_div8(bits(st.V[0])), st.H[1] -= hi16_div8(bits(st.V[0]));
-                    st.H[2] -= lo16_div8(bits(st.V[1])), st.H[3] -= hi16_div8(bits(st.V[1]));
-                    hmax = max(hmax, max(max(st.H[0], st.H[1]), max(st.H[2], st.H[3])));
-                    if (!SCORE_ONLY) *(uint32_t *)(prow + (tl - b.stB)) = pack_dirs(d0, d1);
-                } else if (plain) {
-                    const bool keep_prev = b.st16 - 1 >= lst16 && b.st16 - 1 <= len16;
-                    if (b.st0 < t0)
-                        edge_step<RIGHT, SCORE_ONLY, true, false>(kc2, b, t0, tl, lane, st, TB, qwin[0], tx, tv, tx2,
-                                                                  ch, keep_prev, U0, L0, hmax, prow);
-                    else if (t0 + SR - 1 < b.en0)
-                        edge_step<RIGHT, SCORE_ONLY, false, true>(kc2, b, t0, tl, lane, st, TB, qwin[0], tx, tv, tx2,
-                                                                  ch, keep_prev, U0, L0, hmax, prow);
-                    else
-                        edge_step<RIGHT, SCORE_ONLY, false, false>(kc2, b, t0, tl, lane, st, TB, qwin[0], tx, tv, tx2,
-                                                                   ch, keep_prev, U0, L0, hmax, prow);
-                } else {
-                    // every rule, on the 32-bit form of the lane's state
-                    int U[R], Y[R], Y2[R], X[R], V[R], X2[R];
-                    int *H = st.H;
-#pragma unroll
-                    for (int m = 0; m < 2; ++m) {
-                        U[2 * m] = lo16(bits(st.U[m])), U[2 * m + 1] = hi16(bits(st.U[m]));
-                        V[2 * m] = lo16(bits(st.V[m])), V[2 * m + 1] = hi16(bits(st.V[m]));
-                        X[2 * m] = lo16(bits(st.X[m])), X[2 * m + 1] = hi16(bits(st.X[m]));
-                        Y[2 * m] = lo16(bits(st.Y[m])), Y[2 * m + 1] = hi16(bits(st.Y[m]));
-                        X2[2 * m] = lo16(bits(st.X2[m])), X2[2 * m + 1] = hi16(bits(st.X2[m]));
-                        Y2[2 * m] = lo16(bits(st.Y2[m])), Y2[2 * m + 1] = hi16(bits(st.Y2[m]));
-                    }
-                    uint32_t smask = (bits(st.MM[0]) & 1) | (bits(st.MM[0]) >> 15 & 2) |
-                                     (bits(st.MM[1]) & 1) << 2 | (bits(st.MM[1]) >> 13 & 8);
-                    const uint32_t tcw[1] = {((uint32_t)bits(TB[0]) & 0xffu) | ((uint32_t)bits(TB[0]) >> 8 & 0xff00u) |
-                                             ((uint32_t)bits(TB[1]) & 0xffu) << 16 | ((uint32_t)bits(TB[1]) & 0xff0000u) << 8};
-                    const int cx = hi16(tx), cv = hi16(tv), cx2 = hi16(tx2);
-                    // the AVX-512 lane wrap: position stB reads position stB+15
-                    // (row 7 of the next lane) from anti-diagonal r-1
-                    const bool wrap = b.st16 != b.stB;
-                    int wx = 0, wvv = 0, wx2 = 0;
-                    if (wrap && b.stB >= t0 && b.stB < t0 + SR) {
-                        const int src = (b.stB + 15 - t0) / R;  // position stB+15 is row R-1 of this lane
-                        wx = __builtin_amdgcn_readlane(X[R - 1], src);
-                        wvv = __builtin_amdgcn_readlane(V[R - 1], src);
-                        wx2 = __builtin_amdgcn_readlane(X2[R - 1], src);
-                    }
-                    const bool keep_prev = b.st16 > 0 && b.st16 - 1 >= lst16 && b.st16 - 1 <= len16;
-                    const int edgeV = -8 * edge_diff(sc, r);
-                    const bool inject = b.en16 >= r;
-                    const bool la = tl >= b.stB && tl + R - 1 <= b.en16;
-                    uint32_t dw[2] = {0u, 0u};
-#pragma unroll
-                    for (int k = R - 1; k >= 0; --k) {
-                        const int t = tl + k;
-                        int xin = k > 0 ? X[k - 1] : cx, vin = k > 0 ? V[k - 1] : cv, x2in = k > 0 ? X2[k - 1] : cx2;
-                        if (t == b.st16) {
-                            if (b.st16 == 0) xin = L0, vin = edgeV, x2in = L0;
-                            else if (!keep_prev) xin = L0, vin = U0, x2in = L0;
-                        } else if (wrap && t == b.stB) {
-                            xin = wx, vin = wvv, x2in = wx2;
+        };
+        auto fill = [&](int cb) {
+            const int c = cb + lane, j = c - wofs - t0, k = c & (kRing - 1);
+            if (lane < kBlock) in.e[4][k] = j >= 0 && j < qlen ? nq << 16 : 0u;
+            if (enters) {
+                const bool have = entry_valid(c);
+                auto missing = [&]() {
+                    return __ballot(have && ((uint32_t)(na >> 32 & 0xffffu) != tag || (uint32_t)(nh >> 32) != tag)) != 0;
+                };
+                if (__builtin_expect(missing() && !late && !stop, 0)) {
+                    // not all written yet: load again until they are
+                    const uint64_t t_start = wall_clock64();
+                    for (;;) {
+                        if (have) na = load_half(buf, c - wofs, 0), nh = load_half(buf, c - wofs, 1);
+                        if (!missing() || stopped()) break;
+                        if (wall_clock64() - t_start > kWaitTicks) {
+                            late = 1;
+                            break;
                         }
-                        int uin = U[k], yin = Y[k], y2in = Y2[k];
-                        if (inject && t == r) uin = edgeV, yin = L0, y2in = L0;
-                        if (t >= b.st0 && t <= b.sc_end) {
-                            const uint32_t qc = (qwin[k >> 2] >> (8 * (k & 3))) & 0xffu;
-                            const uint32_t tc = (tcw[k >> 2] >> (8 * (k & 3))) & 0xffu;
-                            smask = (smask & ~(1u << k)) | (tc != qc ? 1u << k : 0u);
-                        }
-                        int un, vn, xn, yn, x2n, y2n;
-                        const int d = band_cell<RIGHT, SCORE_ONLY>(kc, xin, vin, x2in, uin, yin, y2in,
-                                                                   (smask >> k) & 1u, un, vn, xn, yn, x2n, y2n);
-                        if (!SCORE_ONLY) {
-                            dw[k >> 2] |= (uint32_t)d << (8 * (k & 3));
-                            asm volatile("" : "+v"(dw[k >> 2]));
-                        }
-                        if (la) {
-                            // H bookkeeping on [st0, en0]; the position above still
-                            // holds its H of anti-diagonal r-1
-                            const int ut = -(un >> 3), vt = -(vn >> 3);
-                            if (t == b.en0) {
-                                const int hab = k > 0 ? H[k - 1] : ch;
-                                const int h = r == 0 ? vt - sc.qe_orig : b.en0 > 0 ? hab + ut : H[k] + vt;
-                                H[k] = h;
-                                if (b.en0 == tlen - 1 && h >= mte_h) mte_h = h, mte_q = r - b.en0;
-                                if (r == nr - 1 && b.en0 == tlen - 1) score = h;
-                            } else if (t >= b.st0 && t < b.en0) {
-                                H[k] += vt;
-                            }
-                            if (t >= b.st0 && t <= b.en0) {
-                                if (H[k] > 0) pos = 1;
-                                if (t == b.st0 && r - b.st0 == qlen - 1 && H[k] >= mqe_h) mqe_h = H[k], mqe_t = t;
-                            }
-                            U[k] = un, V[k] = vn, X[k] = xn, Y[k] = yn, X2[k] = x2n, Y2[k] = y2n;
-                        }
-                    }
-                    if (!SCORE_ONLY && la) store_dirs(prow + (tl - b.stB), dw);
-                    // back to the packed form
-#pragma unroll
-                    for (int m = 0; m < 2; ++m) {
-                        st.U[m] = vec((int)__builtin_amdgcn_perm((unsigned)U[2 * m + 1], (unsigned)U[2 * m], 0x05040100u));
-                        st.V[m] = vec((int)__builtin_amdgcn_perm((unsigned)V[2 * m + 1], (unsigned)V[2 * m], 0x05040100u));
-                        st.X[m] = vec((int)__builtin_amdgcn_perm((unsigned)X[2 * m + 1], (unsigned)X[2 * m], 0x05040100u));
-                        st.Y[m] = vec((int)__builtin_amdgcn_perm((unsigned)Y[2 * m + 1], (unsigned)Y[2 * m], 0x05040100u));
-                        st.X2[m] =
-                            vec((int)__builtin_amdgcn_perm((unsigned)X2[2 * m + 1], (unsigned)X2[2 * m], 0x05040100u));
-                        st.Y2[m] =
-                            vec((int)__builtin_amdgcn_perm((unsigned)Y2[2 * m + 1], (unsigned)Y2[2 * m], 0x05040100u));
-                        st.MM[m] = uvec((int)((smask >> (2 * m) & 1u) | (smask >> (2 * m + 1) & 1u) << 16));
                     }
                 }
-                lst16 = b.st16, len16 = b.en16;
-                // this stripe's bottom position for the next stripe, unscaled
-                if (lane == kWave - 1) {
-                    const int x = -((hi16(bits(st.X[1])) + bias) >> 3) - G1, v = -(hi16(bits(st.V[1])) >> 3);
-                    const int x2 = -((hi16(bits(st.X2[1])) + bias) >> 3) - G2;
-                    const uint64_t en = (uint64_t)(uint32_t)pack3(x, v, x2) | (uint64_t)(uint32_t)st.H[R - 1] << 32;
-                    __hip_atomic_store((uint64_t *)(out_buf + 2 * r), en, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                }
-                if (((r - rb) & (kPublish - 1)) == kPublish - 1)
-                    publish(prog + wv * kBandCtlStride, kk * (nr + 2) + r + 1);
+                if (lane < kBlock)
+                    in.e[0][k] = (uint32_t)na, in.e[1][k] = (uint32_t)na << 16, in.e[2][k] = (uint32_t)(na >> 32),
+                    in.e[3][k] = (uint32_t)nh;
             }
+        };
+        // ---- four anti-diagonals' entries
+        int known = FED ? 0 : 0x7fffffff;
+        // (what: the arrays that the steps after these can need)
+        auto read4 = [&](int c, uint4 (&e)[5], auto what) {
+            constexpr int WHAT = decltype(what)::value;
+            if (FED && (WHAT & 7) && __builtin_expect(known < in_base + min(c + 4, p_end), 0)) {
+                while ((known = ring_load(&in.filled)) < in_base + min(c + 4, p_end)) {
+                    if (stopped()) break;
+                    __builtin_amdgcn_s_sleep(1);
+                }
+            }
+            asm volatile("" ::: "memory");  // the entries are read after their count
+#pragma unroll
+            for (int k = 0; k < 5; ++k)
+                if (WHAT >> k & 1) e[k] = *(const uint4 *)&in.e[k][c & (kRing - 1)];
+        };
+        // ---- a block's entries from the ring to the pair's buffer
+        uint32_t b0 = 0, b1 = 0, b2 = 0, b3 = 0;
+        auto take = [&](int cb) {
+            asm volatile("" ::: "memory");
+            const uint32_t *o = out.e[0] + (cb & (kRing - 1)) + min(lane, kBlock - 1);
+            b0 = o[0], b1 = o[kRing], b2 = o[2 * kRing], b3 = o[3 * kRing];
+        };
+        auto hand_on = [&](int cb) {
+            const int r = cb + lane - wofs;
+            if (lane < kBlock && r >= 0 && r <= min(r_hi + 2, nr)) {
+                store_half(buf, r, 0, perm(b0, b1, 0x07060302u), bfi(0xffff0000u, b2, next_tag));
+                store_half(buf, r, 1, b3, next_tag);
+            }
+        };
+
+        fetch(c_lo);
+        fill(c_lo);
+        uint4 e[5], f[5];
+        read4(c_lo, e, std::integral_constant<int, 31>());
+        int room = feeds ? ring_load(&out.taken) : 0;
+        int slot[4];  // where this lane writes the block's first entry, as offsets in LDS
+        // the state handed on, and the inputs from the position above
+        uint32_t tx, tx2, tv;
+        int th;
+        auto begin = [&](int i, int k, const uint4 (&e)[5]) {
+            auto o = [&](int x) -> uint32_t & { return *(uint32_t *)(band_lds + slot[x] + 4 * i); };
+            o(0) = dn.x, o(1) = dn.x2, o(2) = dn.v, o(3) = (uint32_t)h1;
+            qb = __builtin_amdgcn_alignbit(qb, dpp_shr1(part(e[4], k), qb), 16);
+        };
+        // the position above's x, x2 and v: the stripe's first position takes
+        // the entry's
+        auto from_above = [&](int k, const uint4 (&e)[5]) {
+            tx = dpp_shr1(part(e[0], k), dn.x), tx2 = dpp_shr1(part(e[1], k), dn.x2), tv = dpp_shr1(part(e[2], k), dn.v);
+        };
+        auto score_of = [&]() {
+            const cell::v2u mm = __builtin_elementwise_min(__builtin_bit_cast(cell::v2u, tb ^ qb),
+                                                           __builtin_bit_cast(cell::v2u, one));
+            return __builtin_bit_cast(uint32_t, __builtin_bit_cast(cell::v2u, sm2) + mm * __builtin_bit_cast(cell::v2u, sd2));
+        };
+        auto shift = [&]() {
+            dn.x = __builtin_amdgcn_alignbit(dn.x, tx, 16), dn.x2 = __builtin_amdgcn_alignbit(dn.x2, tx2, 16);
+            dn.v = __builtin_amdgcn_alignbit(dn.v, tv, 16);
+        };
+        // lanes whose positions enter the band: the initial state
+        auto enter = [&](bool mine) {
+            const uint32_t m = mine ? ~0u : 0u;
+            st.u = bfi(m, v_init, st.u), st.y = bfi(m, kc.y0(), st.y), st.y2 = bfi(m, kc.y20(), st.y2);
+            dn.v = bfi(m, v_init, dn.v), dn.x = bfi(m, kc.x0(), dn.x), dn.x2 = bfi(m, kc.x20(), dn.x2);
+        };
+
+#pragma unroll 1
+        for (int cb = c_lo; cb < c_end; cb += kBlock) {
+            // the host's stop flag, every 256 anti-diagonals: end (nothing of
+            // this pair is delivered; the waves that wait read the flag too)
+            if (__builtin_expect((cb & 255) == 0 && stopped(), 0)) break;
+            const int r0 = cb - wofs, r15 = r0 + kBlock - 1, nb = cb + kBlock;
+            if (feeds) {
+                // the entries it overwrites have been read (by the stripe
+                // after this one, or that wave's stripe before)
+                const int need = nb - kRing > n_lo ? base + nb - kRing : base;
+                while (__builtin_expect(room < need, 0)) {
+                    if (stopped()) break;
+                    __builtin_amdgcn_s_sleep(1);
+                    room = ring_load(&out.taken);
+                }
+            }
+            slot[0] = (int)((uint8_t *)(lane == kWave - 1 && has_next ? out.e[0] + (cb & (kRing - 1)) : spill + lane) - band_lds);
+#pragma unroll
+            for (int k = 1; k < 4; ++k) {
+                // (a register each: one base took an addition for each store)
+                slot[k] = slot[k - 1] + 4 * kRing;
+                asm volatile("" : "+v"(slot[k]));
+            }
+            // around each four steps
+            int pr = 0;
+            auto before4 = [&](int i, uint4 (&next)[5], auto what) {
+                if (FED && (decltype(what)::value & 7)) pr = __hip_atomic_load(&in.filled, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                if (i == 0) {
+                    if (LEAVES) take(cb - kBlock);
+                    fetch(nb);
+                }
+                if (i == kBlock - 4) fill(nb);
+                read4(cb + i + 4, next, what);
+            };
+            auto after4 = [&](int i, auto what) {
+                if (feeds) ring_store(&out.filled, base + cb + i + 4);
+                if (FED && (decltype(what)::value & 7)) known = __builtin_amdgcn_readfirstlane(pr);
+                if (i == 0 && LEAVES && cb > c_lo) hand_on(cb - kBlock);
+            };
+            // the band's ends move as 2r -+ w, nothing rare in the block
+            const int S0 = (r0 - bw) >> 1, E0 = (r0 + bw) >> 1;
+            const bool plain = r0 >= 16 && E0 + 7 + 15 < tlenB && S0 >= 16 && bw < 30000 && r0 - E0 > 15 && E0 + 7 < tlen - 1 && r15 <= r_hi && r15 < nr - 1 &&
+                               r15 - (S0 + 8) < qlen - 1;
+            auto block = [&](auto edges) {
+                constexpr bool START = decltype(edges)::value & 1, END = decltype(edges)::value & 2;
+                const __amdgpu_buffer_rsrc_t rows =
+                    __builtin_amdgcn_make_buffer_rsrc(p + (uint64_t)r0 * ncolB, 0, 0x7fffffff, 0x00027000);
+                int soff = 0;               // of the anti-diagonal's row, less what stB moved by
+                uint32_t m16 = 0, mB = 0;   // lanes of st16 (when it takes the initial values) and of a wrapped stB
+                const int B0 = S0 & ~63;
+                int voff = tl - B0;         // of this lane's bytes in the row (out of range: none stored)
+                auto set_start = [&](int b_st, bool kept) {
+                    const int stB = b_st & ~63, st16 = b_st & ~15;
+                    m16 = !kept && tl == st16 ? ~0u : 0u;
+                    mB = st16 != stB && tl == stB ? ~0u : 0u;
+                    voff = tl < stB ? -1 : tl - B0;
+                };
+                auto move_start = [&](int b_st, bool kept) {
+                    asm volatile("");  // (a branch, not selects)
+                    const int cut = voff;
+                    set_start(b_st, kept);
+                    if (END) voff = cut < 0 ? cut : voff;
+                };
+                uint32_t below = 0;         // START: pos - st0
+                uint32_t e0 = 0, e1 = 0;    // END: masks of the low and high position at en0
+                if (START) set_start(S0, false), below = sub2(pos, splat(S0));
+                if (END) {
+                    if (__builtin_expect((E0 & 15) == 0, 0)) enter((unsigned)(tl - E0) < 16u);
+                    voff = tl < (E0 | 15) ? voff : -1;
+                    e0 = tl == E0 ? ~0u : 0u, e1 = tl + 1 == E0 ? ~0u : 0u;
+                }
+                // END: the last scored position - pos, on even and odd steps
+                // (it is at most en0 + 15, short of tlenB in a plain block)
+                uint32_t above0 = 0, above1 = 0;
+                if (END) {
+                    above0 = sub2(splat(S0 + (generic ? bw : ((bw + 16) & ~15) - 1)), pos);
+                    above1 = sub2(splat(S0 + 1 + (generic ? bw - 1 : ((bw + 15) & ~15) - 1)), pos);
+                }
+                // four steps from i4; MOVES: st16 moves on in them
+                auto steps4 = [&](int i4, auto moves, const uint4 (&e)[5]) {
+                    constexpr bool MOVES = decltype(moves)::value;
+                    const int s4 = S0 + (i4 >> 1);
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        const int b_st = s4 + ((k + 1) >> 1);
+                        begin(i4 + k, k, e);
+                        if (k % 2 == 1) {
+                            // (stB moves on only where st16 does)
+                            if (MOVES || !START) soff -= (b_st & 63) == 0 ? 64 : 0;
+                            if (START) below = sub2(below, one);
+                        }
+                        if (MOVES && k > 0 && __builtin_expect((b_st & 15) == 0, 0)) {
+                            // (st16 - 1 was computed on the anti-diagonal before)
+                            move_start(b_st, k % 2 == 1);
+                        }
+                        if (END && k % 2 == 0) th = (int)dpp_shr1(part(e[3], k), (uint32_t)h1);
+                        // (START alone: the stripe's first position is below the
+                        // start or takes its values)
+                        if (START && !END)
+                            tx = cell::dpp_shr1_0(dn.x), tx2 = cell::dpp_shr1_0(dn.x2), tv = cell::dpp_shr1_0(dn.v);
+                        else
+                            from_above(k, e);
+                        if (START) {
+                            // (position stB + 15 is seven lanes after stB's, lane 0 or 32)
+                            tx = bfi(m16, kc.x0(), bfi(mB, cell::dpp_row_shl7(dn.x), tx));
+                            tx2 = bfi(m16, kc.x20(), bfi(mB, cell::dpp_row_shl7(dn.x2), tx2));
+                            tv = bfi(m16, v_init, bfi(mB, cell::dpp_row_shl7(dn.v), tv));
+                        }
+                        shift();
+                        const uint32_t sn = score_of();
+                        uint32_t keep = 0;  // halves that keep their score
+                        if (START) keep = below;
+                        if (END) {
+                            uint32_t &above = k % 2 ? above1 : above0;
+                            keep = START ? keep | above : above;
+                            above = cell::add2(above, one);
+                        }
+                        sco = START || END ? bfi(sign2(keep), sco, sn) : sn;
+                        const cell::DirWord o = kc.template step<true>(sco, dn, st);
+                        if (END && k % 2 == 0) {
+                            // en0 is one on from the step before: H from the
+                            // position above (on odd steps H + v is the same)
+                            const int c0 = add_lo(st.u, th), c1 = add_hi(st.u, h0);
+                            h0 = (int)bfi(e0, (uint32_t)c0, (uint32_t)add_lo(dn.v, h0));
+                            h1 = (int)bfi(e1, (uint32_t)c1, (uint32_t)add_hi(dn.v, h1));
+                            const uint32_t t = e0;  // where it moves to
+                            e0 = cell::dpp_shr1_0(e1), e1 = t;
+                        } else {
+                            h0 = add_lo(dn.v, h0), h1 = add_hi(dn.v, h1);
+                        }
+                        if (!SCORE_ONLY)
+                            __builtin_amdgcn_raw_buffer_store_b16((short)cell::DirCell<RIGHT>::pack1(o), rows, voff, soff, 0);
+                        soff += ncolB;
+                    }
+                };
+#pragma unroll
+                for (int i4 = 0; i4 < kBlock; i4 += 4) {
+                    // (a group's entries are loaded during the one before it,
+                    // into the arrays in turn)
+                    const int s4 = S0 + (i4 >> 1);
+                    const uint4 (&now)[5] = i4 & 4 ? f : e;
+                    const auto what = std::integral_constant<int, END ? 31 : START ? 16 : 23>();
+                    before4(i4, i4 & 4 ? e : f, what);
+                    if (START && i4 > 0 && __builtin_expect((s4 & 15) == 0, 0)) move_start(s4, false);
+                    if (START && END) steps4(i4, std::true_type(), now);
+                    else if (START && __builtin_expect((s4 + 2 & 15) < 2, 0)) steps4(i4, std::true_type(), now);
+                    else steps4(i4, std::false_type(), now);
+                    after4(i4, what);
+                }
+            };
+            if (__builtin_expect(plain, 1)) {
+                const bool starts = S0 + 8 >= t0, ends = t0 + SR - 1 >= E0;
+                if (!starts && !ends) block(std::integral_constant<int, 0>());
+                else if (!ends && S0 > t0) block(std::integral_constant<int, 1>());
+                else if (!starts) block(std::integral_constant<int, 2>());
+                else block(std::integral_constant<int, 3>());
+            } else {
+                // every rule
+                int lst16 = -1, len16 = -1;  // st16, en16 of anti-diagonal r-1
+                if (r0 > 0 && r0 <= r_hi) {
+                    const Band bp = band_of(r0 - 1, qlen, tlen, bw, tlenB, generic);
+                    lst16 = bp.st16, len16 = bp.en16;
+                }
+#pragma unroll 1
+                for (int i4 = 0; i4 < kBlock; i4 += 4) {
+                    before4(i4, f, std::integral_constant<int, 31>());
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        const int r = r0 + i4 + k;
+                        begin(i4 + k, k, e);
+                        if (r < 0 || r > r_hi) {
+                            h0 += kc.p, h1 += kc.p;  // H stays
+                            continue;
+                        }
+                        from_above(k, e);
+                        const Band b = band_of(r, qlen, tlen, bw, tlenB, generic);
+                        th = (int)dpp_shr1(part(e[3], k), (uint32_t)h1);
+                        if (b.en16 != len16) {
+                            // (what lane 0 takes from the stripe above is that
+                            // position's, whatever enters)
+                            enter(tl > len16 && tl <= b.en16);
+                            from_above(k, e);
+                        }
+                        const bool keep_prev = b.st16 > 0 && b.st16 - 1 >= lst16 && b.st16 - 1 <= len16;
+                        const uint32_t edge = splat(kc.diff(edge_diff(sc, r)));
+                        if (b.st16 != b.stB) {
+                            const int wl = (b.stB + 15 - t0) / 2 & (kWave - 1);
+                            const uint32_t wx = (uint32_t)__builtin_amdgcn_readlane((int)dn.x, wl);
+                            const uint32_t wx2 = (uint32_t)__builtin_amdgcn_readlane((int)dn.x2, wl);
+                            const uint32_t wvv = (uint32_t)__builtin_amdgcn_readlane((int)dn.v, wl);
+                            if (tl == b.stB) tx = wx, tx2 = wx2, tv = wvv;
+                        }
+                        if (tl == b.st16 && !keep_prev) tx = kc.x0(), tx2 = kc.x20(), tv = b.st16 == 0 ? edge : v_init;
+                        if (b.en16 >= r) {
+                            const uint32_t m = tl == r ? 0x0000ffffu : tl + 1 == r ? 0xffff0000u : 0u;
+                            st.u = bfi(m, edge, st.u), st.y = bfi(m, kc.y0(), st.y), st.y2 = bfi(m, kc.y20(), st.y2);
+                        }
+                        shift();
+                        const uint32_t scored = (tl >= b.st0 && tl <= b.sc_end ? 0x0000ffffu : 0u) |
+                                                (tl + 1 >= b.st0 && tl + 1 <= b.sc_end ? 0xffff0000u : 0u);
+                        sco = bfi(scored, score_of(), sco);
+                        const cell::DirWord o = kc.template step<true>(sco, dn, st);
+                        // H on [st0, en0]; elsewhere it stays
+                        int n0 = h0 + (tl >= b.st0 && tl < b.en0 ? lo16(dn.v) : kc.p);
+                        int n1 = h1 + (tl + 1 >= b.st0 && tl + 1 < b.en0 ? hi16(dn.v) : kc.p);
+                        if (r == 0) {
+                            if (tl == 0) n0 = lo16(dn.v) - kc.p + 8 * sc.qe_orig;
+                        } else if (b.en0 == 0) {
+                            if (tl == 0) n0 = h0 + lo16(dn.v);
+                        } else {
+                            if (tl == b.en0) n0 = th + lo16(st.u);
+                            if (tl + 1 == b.en0) n1 = h0 + hi16(st.u);
+                        }
+                        h0 = n0, h1 = n1;
+                        const int q0 = (kc.p * r - h0) >> 3, q1 = (kc.p * r - h1) >> 3;  // H
+                        if (b.en0 == tlen - 1 && (tl | 1) == (b.en0 | 1)) {
+                            const int h = b.en0 & 1 ? q1 : q0;
+                            if (h >= mte_h) mte_h = h, mte_q = r - b.en0;
+                            if (r == nr - 1) score = h;
+                        }
+                        if (r - b.st0 == qlen - 1 && (tl | 1) == (b.st0 | 1)) {
+                            const int h = b.st0 & 1 ? q1 : q0;
+                            if (h >= mqe_h) mqe_h = h, mqe_t = b.st0;
+                        }
+                        if (!SCORE_ONLY && tl >= b.stB && tl < b.en16)
+                            *(uint16_t *)(p + (uint64_t)r * ncolB + (tl - b.stB)) =
+                                (uint16_t)cell::DirCell<RIGHT>::pack1(o);
+                        lst16 = b.st16, len16 = b.en16;
+                    }
+                    after4(i4, std::integral_constant<int, 31>());
+#pragma unroll
+                    for (int k = 0; k < 5; ++k) e[k] = f[k];
+                }
+            }
+            if (FED) ring_store(&in.taken, in_base + (nb >= p_end ? span : nb));
+            if (feeds) room = ring_load(&out.taken);
         }
-        // past every need of the next stripe (of every later one when stopped)
-        publish(prog + wv * kBandCtlStride, stop ? 0x3fffffff : kk * (nr + 2) + nr + 1);
-        if (hmax > 0) pos = 1;
+        if (LEAVES) take(c_end - kBlock), hand_on(c_end - kBlock);
+        if (FED) ring_store(&in.taken, in_base + span);
+    };
+#pragma unroll 1
+    for (int s = wv, kk = 0; has_stripe(s) && !stop; s += W, ++kk) {
+        const bool fed = s > 0 && (w > 0 || circle), leaves = w + 1 == group && !circle && has_stripe(s + 1);
+        if (fed && !leaves) stripe(s, kk, std::true_type(), std::false_type());
+        else if (fed) stripe(s, kk, std::true_type(), std::true_type());
+        else if (!leaves) stripe(s, kk, std::false_type(), std::false_type());
+        else stripe(s, kk, std::false_type(), std::true_type());
     }
 
     // ---- results: mte and the score come from one position; mqe keeps the
@@ -730,52 +621,52 @@ __global__ void __launch_bounds__(kWave * kBandGroup) ksw_band_kernel(BandArgs a
         const int th = __shfl_xor(mte_h, o, kWave), tq = __shfl_xor(mte_q, o, kWave);
         if (tq >= 0 && (mte_q < 0 || th > mte_h)) mte_h = th, mte_q = tq;
         score = max(score, __shfl_xor(score, o, kWave));
-        pos |= __shfl_xor(pos, o, kWave);
     }
     // each wave leaves its record; the last to take a ticket combines them
     // in wave order and writes the pair's results
     int32_t *rec = ctl + kBandCtlRec;
-    pos |= late;
     int last = 0;
     if (lane == 0) {
         int32_t *m = rec + 8 * wv;
-        m[0] = mqe_h, m[1] = mqe_t, m[2] = mte_h, m[3] = mte_q, m[4] = score, m[5] = pos;
+        m[0] = mqe_h, m[1] = mqe_t, m[2] = mte_h, m[3] = mte_q, m[4] = score, m[5] = late;
         last = __hip_atomic_fetch_add(ctl + kBandCtlTicket, 1, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) == W - 1;
     }
     if (lane == 0 && last) {
-        mqe_h = KSW_NEG_INF_I, mqe_t = -1, mte_h = KSW_NEG_INF_I, mte_q = -1, score = KSW_NEG_INF_I, pos = 0;
+        mqe_h = KSW_NEG_INF_I, mqe_t = -1, mte_h = KSW_NEG_INF_I, mte_q = -1, score = KSW_NEG_INF_I;
         for (int k = 0; k < W; ++k) {
             const int32_t *m = rec + 8 * k;
             if (m[0] > mqe_h || (m[0] == mqe_h && m[1] > mqe_t)) mqe_h = m[0], mqe_t = m[1];
             if (m[3] >= 0 && (mte_q < 0 || m[2] > mte_h)) mte_h = m[2], mte_q = m[3];
             score = max(score, m[4]);
-            pos |= m[5];
+            late |= m[5];
         }
         KswOut o;
         o.score = score, o.mqe = mqe_h, o.mqe_t = mqe_t, o.mte = mte_h, o.mte_q = mte_q;
         o.max = 0, o.max_t = -1, o.max_q = -1;
         o.zdropped = r_end < nr ? 1 : 0, o.stopped = 0, o.reach_end = 0, o.n_cigar = 0;
         a.out[jb.out] = o;
-        a.redo[job] = (pos ? 1 : 0) | a.force_redo;
+        a.redo[job] = late | a.force_redo;
     }
 }
 
-// Zeroes the control blocks of a launch's jobs.
+// Clears the control blocks and buffers of a launch's jobs (blockIdx.y).
 __global__ void __launch_bounds__(256) ksw_band_ctl_kernel(int32_t *bnd, const GenJob *jobs, const int32_t *order)
 {
-    int32_t *ctl = bnd + jobs[order[blockIdx.x]].bnd_off;
-    for (int k = threadIdx.x; k < kBandCtl; k += blockDim.x) ctl[k] = 0;
+    const GenJob &jb = jobs[order[blockIdx.y]];
+    int32_t *ctl = bnd + jb.bnd_off;
+    const int n = kBandCtl + 4 * (jb.qlen + jb.tlen);
+    for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += gridDim.x * blockDim.x) ctl[k] = 0;
 }
 
 namespace {
 
 // Workgroups of one band-kernel variant that the device holds at once.
-int band_capacity(const void *fn, int threads)
+int band_capacity(const void *fn, int threads, int lds)
 {
     int dev = 0, cus = 0, per_cu = 0;
     if (hipGetDevice(&dev) != hipSuccess) return 0;
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, threads, 0) != hipSuccess) return 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, threads, lds) != hipSuccess) return 0;
     return cus * per_cu;
 }
 
@@ -788,22 +679,28 @@ hipError_t launch_band(const BandArgs &a0, int team, bool right, bool score_only
     BandArgs a = a0;
     const int wpg = team < kBandGroup ? team : kBandGroup;
     a.wgs = (team + wpg - 1) / wpg;
-    const int threads = kWave * wpg;
+    const int threads = kWave * wpg, lds = ring_bytes(wpg);
     void (*fn)(BandArgs) = score_only ? ksw_band_kernel<false, true>
                            : right    ? ksw_band_kernel<true, false>
                                       : ksw_band_kernel<false, false>;
-    // half the device's capacity per launch: the workgroups of a launch
-    // wait on one another, so all of them must be resident together, beside
-    // the kernels of other streams (which finish on their own) and one other
-    // waiting launch of at most half the device (the caller's admission)
-    const int cap = band_capacity((const void *)fn, threads);
-    if (cap < 2 * a.wgs) return hipErrorInvalidConfiguration;
-    const int chunk = cap / 2 / a.wgs;
+    // half the device's capacity per launch: the workgroups of a pair wait on
+    // one another, so all of them must be resident together, beside the
+    // kernels of other streams (which finish on their own) and one other
+    // waiting launch of at most half the device (the caller's admission).
+    // One workgroup per pair waits for no other: all pairs in one launch
+    int chunk = a0.njobs;
+    if (a.wgs > 1) {
+        const int cap = band_capacity((const void *)fn, threads, lds);
+        if (cap < 2 * a.wgs) return hipErrorInvalidConfiguration;
+        chunk = cap / 2 / a.wgs;
+    }
+    chunk = std::min(chunk, 65535);
     for (int off = 0; off < a0.njobs; off += chunk) {
         a.order = a0.order + off;
         a.njobs = a0.njobs - off < chunk ? a0.njobs - off : chunk;
-        hipLaunchKernelGGL(ksw_band_ctl_kernel, dim3(a.njobs), dim3(256), 0, st, a.bnd, a.jobs, a.order);
-        hipLaunchKernelGGL(fn, dim3(a.njobs * a.wgs), dim3(threads), 0, st, a);
+        hipLaunchKernelGGL(ksw_band_ctl_kernel, dim3(std::max(1, std::min(64, 1024 / a.njobs)), a.njobs), dim3(256), 0, st,
+                           a.bnd, a.jobs, a.order);
+        hipLaunchKernelGGL(fn, dim3(a.njobs * a.wgs), dim3(threads), lds, st, a);
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
     }

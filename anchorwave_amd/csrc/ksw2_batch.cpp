@@ -8,6 +8,7 @@
 #include <string.h>
 
 #include <algorithm>
+#include <map>
 #include <memory>
 #include <chrono>
 #include <mutex>
@@ -348,6 +349,8 @@ StripeGeom stripe_geom(const ksw2_pair_t &p)
     return StripeGeom{tr, tr ? p.tlen : p.qlen, tr ? p.qlen : p.tlen};
 }
 
+constexpr int kDeviceSimds = 4 * 256;
+
 static int norm_w(const ksw2_pair_t &p) { return p.w < 0 ? std::max(p.qlen, p.tlen) : p.w; }
 
 // Rows per lane of a plan's stripe kernel.  Eight rows per lane take the
@@ -432,7 +435,7 @@ uint64_t pair_footprint(const ksw2_pair_t &p, bool general)
     const int tlenB = (p.tlen + 63) / 64 * 64, qlenB = (p.qlen + 63) / 64 * 64;
     const uint64_t diags = (uint64_t)p.qlen + p.tlen - 1;
     const uint64_t rows = cigar ? tracks * diags * (uint64_t)gen_ncolB(p.qlen, p.tlen, norm_w(p)) + 256 : 0;
-    // (+ the band kernel's control block, three stripe buffers and redo flag, whichever kernel runs it)
+    // (+ the band kernel's control block, hand-off buffer and redo flag, whichever kernel runs it)
     return gen_layout(tlenB, qlenB).bytes + rows + (cigar ? 8 * diags : 0) + cig + seq + 24 * diags + 4 * kBandCtl + 516;
 }
 
@@ -455,56 +458,28 @@ bool band_domain(const ksw2_pair_t &p, int8_t m, const ScoreClass &cls)
     const char *fg = getenv("KSW2_HIP_FORCE_GENERAL");
     if (fg && atoi(fg) > 0) return false;
     if (p.flag & KSW_EZ_SINGLETRACK) return false;
-    // progress counts stripe * (qlen + tlen + 1) + anti-diagonal must fit int32
-    const int64_t nstripes = ((int64_t)p.tlen + 63) / 64 * 64 / (kWave * kBandRowsPerLane) + 1;
-    if ((nstripes + 1) * ((int64_t)p.qlen + p.tlen + 1) >= INT32_MAX) return false;
+    // the hand-off counts, a wave's stripes times (qlen + tlen + 63), and H,
+    // held as -8 H + p r with p <= 8 * 128 + 8, must fit int32
+    const int64_t nstripes = ((int64_t)p.tlen + 63) / 64 * 64 / 256 + 1;
+    if ((nstripes + 1) * ((int64_t)p.qlen + p.tlen + 63) >= INT32_MAX) return false;
+    if (2080ll * band_r_end(p.qlen, p.tlen, norm_w(p)) >= INT32_MAX) return false;
     return fast_path_reject(p, m, cls) == kRejBand;
 }
 
 bool takes_band(const ksw2_pair_t &p, int8_t m, const ScoreClass &cls)
 {
     const char *mn = getenv("KSW2_HIP_BAND_MIN");
-    const int min_width = mn ? atoi(mn) : kBandWide;
-    return band_domain(p, m, cls) && norm_w(p) + 1 >= min_width;
-}
-
-// Narrow bands (w + 1 < kBandWide) of one plan: the band kernel computes
-// whole 256-position stripes over 2w + 512 anti-diagonals each, the general
-// kernel only the band's cells, one workgroup per pair with a barrier per
-// anti-diagonal.  Measured on MI355X (2 kbp pairs, w = 256, and single
-// pairs of 2-50 kbp): the band kernel takes about 1.1 us per anti-diagonal
-// of a pair's chain and sustains 6.4e10 stripe positions per second, the
-// general kernel about 5.8 us per anti-diagonal and 4.4e10 in-band cells per
-// second.  So a few pairs finish several times sooner on the band kernel and
-// thousands sooner on the general kernel; the plan's narrow pairs take the
-// kernel whose predicted time is the shorter.
-static bool narrow_bands_to_band(const std::vector<const ksw2_pair_t *> &narrow)
-{
-    if (narrow.empty()) return false;
-    double nr_max = 0, stripe_work = 0, cells = 0;
-    for (const ksw2_pair_t *p : narrow) {
-        const double nr = (double)p->qlen + p->tlen - 1, w = norm_w(*p);
-        nr_max = std::max(nr_max, nr);
-        stripe_work += (double)((p->tlen + 255) / 256 * 256) * (2 * w + 512);
-        cells += std::min(2 * w + 1, (double)std::min(p->qlen, p->tlen)) * nr / 2;
-    }
-    const double t_band = std::max(1.1e-6 * nr_max, stripe_work / 6.4e10);
-    const double t_gen = std::max(5.8e-6 * nr_max, cells / 4.4e10);
-    return t_band < t_gen;
+    return (!mn || norm_w(p) + 1 >= atoi(mn)) && band_domain(p, m, cls);
 }
 
 int band_r_end(int qlen, int tlen, int w)
 {
-    const int nr = qlen + tlen - 1;
-    for (int r = 0; r < nr; ++r) {
-        int st = 0, en = tlen - 1;
-        if (st < r - qlen + 1) st = r - qlen + 1;
-        if (en > r) en = r;
-        if (st < (r - w + 1) >> 1) st = (r - w + 1) >> 1;
-        if (en > (r + w) >> 1) en = (r + w) >> 1;
-        if (st > en) return r;  // minimap2/ksw2_extd2_sse.c:152-155
-    }
-    return nr;
+    // the first anti-diagonal with st > en (minimap2/ksw2_extd2_sse.c:147-155):
+    // its start is past the last position, or its end before the first one
+    // that reaches column qlen-1, or (w = 0) no cell is on an odd one
+    const int64_t nr = (int64_t)qlen + tlen - 1;
+    if (w == 0) return (int)std::min<int64_t>(nr, 1);
+    return (int)std::min(nr, 2 * (int64_t)std::min(qlen, tlen) + w - 1);
 }
 
 // LDS ring slots of the general kernel for one pair (0: state in HBM).
@@ -603,21 +578,7 @@ int plan_create(Plan **out, const ksw2_pair_t *pairs, const int *idx, int nidx, 
     }
     p->nstripes_total = stripes;
     std::vector<char> band(p->n_gen, 0);
-    {
-        // bands at least kBandWide wide always take the band kernel; the
-        // narrower ones together, when it is predicted to finish them sooner
-        // (KSW2_HIP_BAND_MIN: a fixed width rule instead)
-        const bool fixed_rule = getenv("KSW2_HIP_BAND_MIN") != nullptr;
-        std::vector<const ksw2_pair_t *> narrow;
-        for (int gk = 0; gk < p->n_gen; ++gk) {
-            const ksw2_pair_t &pp = pairs[p->order[p->n_fast + gk]];
-            band[gk] = takes_band(pp, m, cls);
-            if (!band[gk] && !fixed_rule && band_domain(pp, m, cls)) band[gk] = 2, narrow.push_back(&pp);
-        }
-        const bool to_band = narrow_bands_to_band(narrow);
-        for (char &b : band)
-            if (b == 2) b = to_band;
-    }
+    for (int gk = 0; gk < p->n_gen; ++gk) band[gk] = takes_band(pairs[p->order[p->n_fast + gk]], m, cls);
     for (int gk = 0; gk < p->n_gen; ++gk) {
         const int slot = p->n_fast + gk;
         const ksw2_pair_t &pp = pairs[p->order[slot]];
@@ -780,30 +741,48 @@ int plan_create(Plan **out, const ksw2_pair_t *pairs, const int *idx, int nidx, 
                                         t >= 512 ? 0 : t >= 256 ? 1 : 2});
                 gorder.insert(gorder.end(), members.begin(), members.end());
             }
-        // band-kernel launches: per group and team (one wave per 512-position
-        // stripe, at most kMaxTeam), longest first
+        // band-kernel launches: per group and team, longest first.  A team has
+        // as many waves as the pair has stripes in flight: a stripe's
+        // anti-diagonals (2w + 2 * 128, and the starts and ends of blocks) over
+        // the 256 that its start trails the one above it by, with a margin for
+        // what the hand-offs add.
         p->band_off = (int)gorder.size();
         const char *bt = getenv("KSW2_HIP_BAND_TEAM");  // forces a team size (tests)
         const int band_team = bt ? std::max(1, std::min(kBandTeam, atoi(bt))) : 0;
-        for (int grp = 0; grp < 3; ++grp)
-            for (int team = kBandTeam; team >= 1; --team) {
-                std::vector<int> members;
-                for (int gk = 0; gk < p->n_gen; ++gk) {
-                    if (!band[gk]) continue;
-                    const GenJob &j = p->gjobs[gk];
-                    const int g = (j.flag & KSW_EZ_SCORE_ONLY) ? 2 : (j.flag & KSW_EZ_RIGHT) ? 1 : 0;
-                    const int brows = kWave * kBandRowsPerLane;
-                    const int tm = band_team ? band_team : std::min(kBandTeam, (j.tlenB + brows - 1) / brows);
-                    if (g == grp && tm == team) members.push_back(gk);
-                }
-                if (members.empty()) continue;
-                std::stable_sort(members.begin(), members.end(), [&](int x, int y) {
-                    const GenJob &a = p->gjobs[x], &b = p->gjobs[y];
-                    return (double)(a.qlen + a.tlen) * a.ncolB > (double)(b.qlen + b.tlen) * b.ncolB;
-                });
-                p->blaunches.push_back({grp, team, (int)gorder.size(), (int)members.size(), 0});
-                gorder.insert(gorder.end(), members.begin(), members.end());
+        // A group whose pairs would all find a SIMD per wave at its largest team
+        // takes that one, in one launch: launches follow one another.
+        std::map<std::pair<int, int>, std::vector<int>> teams;  // by group and (negated) team
+        int team_max[3] = {0, 0, 0}, members_of[3] = {0, 0, 0};
+        for (int gk = 0; gk < p->n_gen; ++gk) {
+            if (!band[gk]) continue;
+            const GenJob &j = p->gjobs[gk];
+            const int g = (j.flag & KSW_EZ_SCORE_ONLY) ? 2 : (j.flag & KSW_EZ_RIGHT) ? 1 : 0;
+            int tm = band_team;
+            if (!tm) {
+                const int64_t flight = (2 * (int64_t)j.w + 420) / 256 + 1;
+                tm = (int)std::min<int64_t>({flight, (j.tlenB + kBandStripe - 1) / kBandStripe, kBandTeam});
+                if (tm > kBandGroup) tm = (tm + kBandGroup - 1) / kBandGroup * kBandGroup;
             }
+            teams[{g, -tm}].push_back(gk);
+            team_max[g] = std::max(team_max[g], tm), ++members_of[g];
+        }
+        for (int g = 0; g < 3; ++g) {
+            if ((int64_t)members_of[g] * team_max[g] > kDeviceSimds) continue;
+            std::vector<int> &all = teams[{g, -team_max[g]}];
+            for (auto &t : teams)
+                if (t.first.first == g && &t.second != &all) all.insert(all.end(), t.second.begin(), t.second.end());
+            for (auto t = teams.begin(); t != teams.end();)
+                t = t->second.empty() || (t->first.first == g && &t->second != &all) ? teams.erase(t) : std::next(t);
+        }
+        for (auto &t : teams) {
+            std::vector<int> &members = t.second;
+            std::stable_sort(members.begin(), members.end(), [&](int x, int y) {
+                const GenJob &a = p->gjobs[x], &b = p->gjobs[y];
+                return (double)(a.qlen + a.tlen) * a.ncolB > (double)(b.qlen + b.tlen) * b.ncolB;
+            });
+            p->blaunches.push_back({t.first.first, -t.first.second, (int)gorder.size(), (int)members.size(), 0});
+            gorder.insert(gorder.end(), members.begin(), members.end());
+        }
         p->n_band = (int)gorder.size() - p->band_off;
     }
     p->seq_bytes = std::max<uint64_t>(so, 16), p->dir_bytes = std::max<uint64_t>(dof, 256);
@@ -1148,8 +1127,8 @@ int plan_launch(Plan *p, const Progress *prog)
             }
             if (!wait_slots_release(st, q)) return KSW2_HIP_EDEVICE;
         }
-        // pairs whose H went above 0 (the band kernel does not track the
-        // maximum) run again on the general kernel, on the same stream
+        // pairs whose waves gave up a wait run on the general kernel, on the
+        // same stream
         ga.order = p->d_gorder + p->band_off, ga.njobs = p->n_band, ga.ring = 0, ga.only_if = p->d_redo;
         KSW_HIP_TRY(launch_general(ga, 1024, st));
     }

@@ -59,6 +59,19 @@ __device__ __forceinline__ uint32_t min2(uint32_t a, uint32_t b)
     return __builtin_bit_cast(uint32_t,
                               __builtin_elementwise_min(__builtin_bit_cast(v2s, a), __builtin_bit_cast(v2s, b)));
 }
+__device__ __forceinline__ uint32_t max2(uint32_t a, uint32_t b)
+{
+    return __builtin_bit_cast(uint32_t,
+                              __builtin_elementwise_max(__builtin_bit_cast(v2s, a), __builtin_bit_cast(v2s, b)));
+}
+// All ones in the halves that are negative.
+__device__ __forceinline__ uint32_t sign2(uint32_t a)
+{
+    return __builtin_bit_cast(uint32_t, __builtin_bit_cast(v2s, a) >> (v2s){15, 15});
+}
+// The low (high) half of a, signed, plus b.
+__device__ __forceinline__ int add_lo(uint32_t a, int b) { return __builtin_amdgcn_sdot2(__builtin_bit_cast(v2s, a), (v2s){1, 0}, b, false); }
+__device__ __forceinline__ int add_hi(uint32_t a, int b) { return __builtin_amdgcn_sdot2(__builtin_bit_cast(v2s, a), (v2s){0, 1}, b, false); }
 // Smallest of three, per half; halves in [0, 0x7bff].
 __device__ __forceinline__ uint32_t min3(uint32_t a, uint32_t b, uint32_t c)
 {
@@ -82,6 +95,16 @@ __device__ __forceinline__ uint32_t dpp_shl1(uint32_t old, uint32_t src)
 __device__ __forceinline__ uint32_t dpp_shr1(uint32_t old, uint32_t src)
 {
     return (uint32_t)__builtin_amdgcn_update_dpp((int)old, (int)src, 0x138, 0xF, 0xF, false);
+}
+// Lane k takes lane k-1's value (lane 0 zero).
+__device__ __forceinline__ uint32_t dpp_shr1_0(uint32_t src)
+{
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)src, 0x138, 0xF, 0xF, true);
+}
+// Lane k takes lane k+7's value where both are in a row of 16 lanes.
+__device__ __forceinline__ uint32_t dpp_row_shl7(uint32_t src)
+{
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)src, 0x107, 0xF, 0xF, true);
 }
 __device__ __forceinline__ uint32_t dpp_ror1(uint32_t src)
 {
@@ -146,12 +169,16 @@ struct DirCell {
     // one half of v or u for the difference w
     __device__ __forceinline__ int diff(int w) const { return p - 8 * w; }
 
-    __device__ __forceinline__ DirWord step(uint32_t s, Down &d, Right &r) const
+    // STALE: some inputs were left by earlier anti-diagonals, outside a band;
+    // their candidates may be positive (a negative half), and the score is
+    // capped at the match score.
+    template <bool STALE = false> __device__ __forceinline__ DirWord step(uint32_t s, Down &d, Right &r) const
     {
         const uint32_t a = add2(d.x, d.v), b = add2(r.y, r.u);
         const uint32_t xv2 = add2(d.x2, d.v), yu2 = add2(r.y2, r.u);
-        const uint32_t z = min3(min3(s, a, b), add2(xv2, cA2), add2(yu2, cB2));
-        const uint32_t z8 = z & 0xfff8fff8u;
+        const uint32_t a2 = add2(xv2, cA2), b2 = add2(yu2, cB2);
+        const uint32_t z = STALE ? min2(min2(min2(b, b2), s), min2(a, a2)) : min3(min3(s, a, b), a2, b2);
+        const uint32_t z8 = STALE ? max2(z & 0xfff8fff8u, 0u) : z & 0xfff8fff8u;
         const uint32_t w = add2(z8, zc), m1 = sub2(e1, z8), m2 = sub2(e2, z8);
         const uint32_t ta = add2(a, m1), tb = add2(b, m1), ta2 = add2(xv2, m2), tb2 = add2(yu2, m2);
         const uint32_t un = sub2(w, d.v);
@@ -160,6 +187,12 @@ struct DirCell {
         DirWord o;
         o.z = z, o.f = bfi(mA, ta, bfi(mB, tb, bfi(mA2, ta2, tb2)));
         return o;
+    }
+    // Two direction bytes of one word (low half, high half).
+    __device__ __forceinline__ static uint32_t pack1(const DirWord &w)
+    {
+        const uint32_t b = __builtin_amdgcn_bitop3_b32(0x00070007u, w.z, w.f >> 8, RIGHT ? 0x3a : 0xca);
+        return perm(b, b, 0x0c0c0200u);
     }
     // Four direction bytes of two words: (first.lo, second.lo, first.hi,
     // second.hi).

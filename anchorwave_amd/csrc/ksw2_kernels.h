@@ -62,41 +62,39 @@ struct GenBacktrackArgs {
     int tiled_min;             // pairs with qlen + tlen >= this walk one per wave (staged rows)
 };
 
-// Band kernel (ksw2_band.hip): one workgroup of `team` waves per job.
+// Band kernel (ksw2_band.hip): `team` waves per job.
 struct BandArgs {
     const uint8_t *seq;
     uint8_t *dir;              // direction rows (reference layout)
     int32_t *offs;             // off[] / off_end[] per pair
-    int32_t *bnd;              // per pair: kBandCtl control dwords, then three stripe hand-off
-                               // buffers of 2 * (qlen+tlen-1) dwords
+    int32_t *bnd;              // per pair: kBandCtl control dwords, then a hand-off buffer of
+                               // 4 * (qlen+tlen) dwords
     const GenJob *jobs;
     const int32_t *order;      // this launch's jobs, `wgs` workgroups each
     int njobs;
     int wgs;                   // workgroups per job (set by launch_band)
     KswOut *out;
-    int32_t *redo;             // per job: 1 when H > 0 was seen (the general kernel must run it)
+    int32_t *redo;             // per job: 1 when a wait gave up (the general kernel must run it)
     GenScore sc;
     int force_redo;            // tests: flag every job for the general kernel
     // host-raised stop flag (pinned, mapped) sampled every 256 anti-diagonals
-    // of a stripe, or null: a stopped wave publishes a count past every wait
-    // and ends (the host reports such pairs stopped)
+    // of a stripe, or null: the waves end (the host reports such pairs stopped)
     const int32_t *stop;
 };
-constexpr int kBandTeam = 16;       // waves per pair, at most
+constexpr int kBandTeam = 60;       // waves per pair, at most
 constexpr int kBandGroup = 4;       // waves per workgroup: one per SIMD of a CU
-constexpr int kBandRowsPerLane = 4; // positions per lane; a stripe is 64 lanes of them
-// Control block of a band job: progress counts (one per team wave, 16
-// dwords apart), the finish ticket, per-wave result records.
-constexpr int kBandCtlStride = 16;
-constexpr int kBandCtlTicket = kBandTeam * kBandCtlStride;
-constexpr int kBandCtlRec = kBandCtlTicket + 16;
+constexpr int kBandStripe = 128;    // positions per stripe, two per lane
+// Control block of a band job: the finish ticket, per-wave result records.
+constexpr int kBandCtlTicket = 0;
+constexpr int kBandCtlRec = 16;
 constexpr int kBandCtl = 512;
 static_assert(kBandCtlRec + 8 * kBandTeam <= kBandCtl, "band control block");
-// Band kernel for a team of `team` waves per job: kBandGroup-wave
-// workgroups on different CUs that hand stripes on through device-scope
-// counters.  Launches go in chunks of at most half the device's workgroups;
-// with at most two such waiting launches at once (the caller's admission),
-// no spinning workgroup waits on one that cannot be placed.
+// Band kernel for a team of `team` waves per job, in workgroups of
+// kBandGroup (a larger team is rounded up to whole ones) on different CUs
+// that hand stripes on through device memory.  Such launches go in chunks of
+// at most half the device's workgroups; with at most two waiting launches at
+// once (the caller's admission), no spinning workgroup waits on one that
+// cannot be placed.
 hipError_t launch_band(const BandArgs &a, int team, bool right, bool score_only, hipStream_t st);
 
 // Singletrack walk of general pairs: one wavefront per job (all general

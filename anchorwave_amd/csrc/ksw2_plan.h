@@ -78,12 +78,8 @@ int gen_ring(const ksw2_pair_t &p);
 // departure from the stripe kernel's domain is a band narrower than the
 // matrix, and no Singletrack.
 bool band_domain(const ksw2_pair_t &p, int8_t m, const ScoreClass &cls);
-// Bands at least this wide in the band kernel's domain always take it;
-// narrower ones take it when a plan's narrow pairs are predicted to finish
-// sooner there than on the general kernel.
-constexpr int kBandWide = 512;
-// True when a pair in the band kernel's domain has a band at least
-// KSW2_HIP_BAND_MIN (default kBandWide) wide.
+// True when a pair is in the band kernel's domain (and its band, if
+// KSW2_HIP_BAND_MIN is set, at least that wide).
 bool takes_band(const ksw2_pair_t &p, int8_t m, const ScoreClass &cls);
 // Anti-diagonals the reference completes before the band leaves the
 // matrix (qlen + tlen - 1 when it never does).
@@ -196,7 +192,7 @@ struct Plan {
     };
     std::vector<BLaunch> blaunches;
     int n_band = 0, band_off = 0;    // band jobs: d_gorder[band_off .. band_off + n_band)
-    int32_t *d_redo = nullptr;       // per general job: the band kernel asks the general kernel to rerun it
+    int32_t *d_redo = nullptr;       // per general job: the band kernel asks the general kernel to run it
     int nstripes_total = 0;
     uint64_t seq_bytes = 0, dir_bytes = 0, bnd_dwords = 0, cig_words = 0;
     uint8_t *block = nullptr;        // own device block (no pool)

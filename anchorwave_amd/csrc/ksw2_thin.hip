@@ -204,7 +204,7 @@ __device__ __forceinline__ void thin_run(const StripeArgs &a, const typename Cel
         if (p == 0) {
             x = kc.x0(), x2 = kc.x20(), v = (uint32_t)kc.diff(edge_diff(sc, col)) << 16;
         } else {
-            if (__ballot(have && (uint32_t)(ne >> 32 & 0xffffu) != tag) != 0 && !late && !stop) {
+            if (__builtin_expect(__ballot(have && (uint32_t)(ne >> 32 & 0xffffu) != tag) != 0 && !late && !stop, 0)) {
                 // not all written yet: load again until they are
                 const uint64_t t_start = wall_clock64();
                 for (;;) {
@@ -227,7 +227,7 @@ __device__ __forceinline__ void thin_run(const StripeArgs &a, const typename Cel
     // ---- this pass's boundary entries, four columns at a time
     int known = FED ? 0 : 0x7fffffff;
     auto read4 = [&](int c, uint4 (&e)[4]) {
-        if (known < base + min(c + 4, qlen)) {
+        if (__builtin_expect(known < base + min(c + 4, qlen), 0)) {
             while ((known = __builtin_amdgcn_readfirstlane(ring_load(&in.filled))) < base + min(c + 4, qlen)) {
                 if (stopped()) break;
             }
@@ -339,7 +339,7 @@ __device__ __forceinline__ void thin_run(const StripeArgs &a, const typename Cel
     for (int c0 = 0; c0 < nsteps; c0 += kBlock) {
         // the host's stop flag, every 256 columns: end (nothing of this pair is
         // delivered; the waves that wait for this one read the flag too)
-        if ((c0 & 255) == 0 && stopped()) return;
+        if (__builtin_expect((c0 & 255) == 0 && stopped(), 0)) return;
         const int nb = c0 + kBlock;
         const bool writes = nb > col_off;  // the block has columns to hand on
         if (w + 1 < group && writes) {
@@ -347,7 +347,7 @@ __device__ __forceinline__ void thin_run(const StripeArgs &a, const typename Cel
             // feeds no wave, too writes where the wave after it may still be
             // reading its pass before)
             const int need = max(FEEDS ? base + nb - kSkew - kRing : base, base);
-            while (room < need) {
+            while (__builtin_expect(room < need, 0)) {
                 if (stopped()) return;
                 room = __builtin_amdgcn_readfirstlane(ring_load(&out.taken));
             }
@@ -370,7 +370,7 @@ __device__ __forceinline__ void thin_run(const StripeArgs &a, const typename Cel
 #pragma unroll
             for (int x = 0; x < 4; ++x) e[x] = f[x];
         };
-        if (c0 >= 2 * kWave && nb + 4 <= qlen) {
+        if (__builtin_expect(c0 >= 2 * kWave && nb + 4 <= qlen, 1)) {
 #pragma unroll
             for (int k = 0; k < kBlock; k += 4) group4(k, std::integral_constant<int, 0>());
         } else {
