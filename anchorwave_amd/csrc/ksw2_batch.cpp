@@ -793,7 +793,11 @@ int plan_create(Plan **out, const ksw2_pair_t *pairs, const int *idx, int nidx, 
         return code;
     };
     if (env && env->stream) {
-        p->stream = env->stream;  // caller's stream: every launch goes there
+        p->stream = env->stream;  // caller's stream: every launch goes there, or to its lanes
+        p->lanes = env->lanes, p->pinned = env->pinned;
+        if (p->lanes)
+            for (int l = 0; l < Plan::kLanes; ++l)
+                p->lane_stream[l] = p->lanes->stream[l], p->lane_done[l] = p->lanes->done[l];
     } else {
         p->own_streams = true;  // lane streams are created on first use (plan_launch)
         if (hipStreamCreateWithFlags(&p->stream, hipStreamNonBlocking) != hipSuccess) return fail(KSW2_HIP_EDEVICE);
@@ -812,19 +816,19 @@ int plan_create(Plan **out, const ksw2_pair_t *pairs, const int *idx, int nidx, 
         at = round_up(at + std::max<uint64_t>(bytes, 1), 256);
         return o;
     };
-    const uint64_t o_seq = take(p->seq_bytes), o_dir = take(p->dir_bytes), o_bnd = take(p->bnd_dwords * 4);
-    const uint64_t o_cig = take(p->cig_words * 8), o_jobs = take(sizeof(KswJob) * std::max(p->n_fast, 1));
-    const uint64_t o_out = take(sizeof(KswOut) * std::max(p->n, 1));
+    // (what is uploaded is at its head, one copy from pinned memory)
+    const uint64_t o_seq = take(p->seq_bytes), o_jobs = take(sizeof(KswJob) * std::max(p->n_fast, 1));
     const uint64_t o_order = take(sizeof(int32_t) * std::max<size_t>(order.size(), 1));
-    const uint64_t o_recs = take(sizeof(StripeRec) * std::max(stripes, 1));
     uint64_t o_state = 0, o_offs = 0, o_gjobs = 0, o_gorder = 0;
-    if (p->n_gen > 0) {
-        o_state = take(p->state_bytes), o_offs = take(p->offs_ints * 4);
-        o_gjobs = take(sizeof(GenJob) * p->n_gen), o_gorder = take(sizeof(int32_t) * gorder.size());
-    }
+    if (p->n_gen > 0) o_gjobs = take(sizeof(GenJob) * p->n_gen), o_gorder = take(sizeof(int32_t) * gorder.size());
+    const uint64_t o_wfirst = p->n_wide > 0 ? take(4ull * p->h_wfirst.size()) : 0;
+    p->upload_bytes = at;
+    const uint64_t o_dir = take(p->dir_bytes), o_bnd = take(p->bnd_dwords * 4);
+    const uint64_t o_cig = take(p->cig_words * 8), o_out = take(sizeof(KswOut) * std::max(p->n, 1));
+    const uint64_t o_recs = take(sizeof(StripeRec) * std::max(stripes, 1));
+    if (p->n_gen > 0) o_state = take(p->state_bytes), o_offs = take(p->offs_ints * 4);
     const uint64_t o_redo = p->n_band > 0 ? take(sizeof(int32_t) * p->n_gen) : 0;
     const uint64_t o_wctl = p->n_wide > 0 ? take(4ull * kWideCtl * (p->n_wide + 1)) : 0;  // failure word, blocks
-    const uint64_t o_wfirst = p->n_wide > 0 ? take(4ull * p->h_wfirst.size()) : 0;
     const uint64_t o_qhead = take(4ull * kMaxQueueHeads);
     p->block_bytes = at;
     uint8_t *base = nullptr;
@@ -868,6 +872,7 @@ int plan_create(Plan **out, const ksw2_pair_t *pairs, const int *idx, int nidx, 
         p->d_mout = env->mirror_out_dev, p->d_mcig = env->mirror_cig_dev, p->d_mflag = env->mirror_flag_dev;
         memset(p->h_mflag, 0, sizeof(int32_t) * p->n_fast);
     }
+    bool whole = false;  // the staged copy holds everything that is uploaded
     hipError_t e[6] = {hipSuccess, hipSuccess, hipSuccess, hipSuccess, hipSuccess, hipSuccess};
     if (resident) {
         p->own_seq = false;  // nothing to upload
@@ -899,8 +904,12 @@ int plan_create(Plan **out, const ksw2_pair_t *pairs, const int *idx, int nidx, 
         uint8_t *h_seq = nullptr;
         if (env && env->staging && env->staging_bytes >= p->seq_bytes) {
             h_seq = env->staging, p->own_seq = false;
-        } else if (hipHostMalloc((void **)&h_seq, p->seq_bytes, hipHostMallocDefault) != hipSuccess) {
+        } else if (p->pinned && p->pinned->grow(p->upload_bytes)) {
+            h_seq = p->pinned->base, p->own_seq = false, whole = true;
+        } else if (hipHostMalloc((void **)&h_seq, p->upload_bytes, hipHostMallocDefault) != hipSuccess) {
             return fail(KSW2_HIP_ENOMEM);
+        } else {
+            whole = true;
         }
         p->h_seq = h_seq;
         memset(h_seq, 0, p->seq_bytes);
@@ -915,20 +924,29 @@ int plan_create(Plan **out, const ksw2_pair_t *pairs, const int *idx, int nidx, 
             memcpy(h_seq + p->gjobs[gk].q_off, pp.query, (size_t)pp.qlen);
             memcpy(h_seq + p->gjobs[gk].t_off, pp.target, (size_t)pp.tlen);
         }
-        e[0] = hipMemcpyAsync(p->d_seq, h_seq, p->seq_bytes, hipMemcpyHostToDevice, p->stream);
+        if (whole) {
+            if (p->n_fast > 0) memcpy(h_seq + o_jobs, p->jobs.data(), sizeof(KswJob) * p->n_fast);
+            if (!order.empty()) memcpy(h_seq + o_order, order.data(), sizeof(int32_t) * order.size());
+            if (p->n_gen > 0) {
+                memcpy(h_seq + o_gjobs, p->gjobs.data(), sizeof(GenJob) * p->n_gen);
+                memcpy(h_seq + o_gorder, gorder.data(), sizeof(int32_t) * gorder.size());
+            }
+            if (p->n_wide > 0) memcpy(h_seq + o_wfirst, p->h_wfirst.data(), sizeof(int32_t) * p->h_wfirst.size());
+        }
+        e[0] = hipMemcpyAsync(p->d_seq, h_seq, whole ? p->upload_bytes : p->seq_bytes, hipMemcpyHostToDevice, p->stream);
     }
-    if (p->n_fast > 0)
+    if (p->n_fast > 0 && !whole)
         e[1] = hipMemcpyAsync(p->d_jobs, p->jobs.data(), sizeof(KswJob) * p->n_fast, hipMemcpyHostToDevice, p->stream);
-    if (!order.empty())
+    if (!order.empty() && !whole)
         e[2] = hipMemcpyAsync(p->d_order, order.data(), sizeof(int32_t) * order.size(), hipMemcpyHostToDevice,
                               p->stream);
-    if (p->n_gen > 0) {
+    if (p->n_gen > 0 && !whole) {
         e[3] = hipMemcpyAsync(p->d_gjobs, p->gjobs.data(), sizeof(GenJob) * p->n_gen, hipMemcpyHostToDevice,
                               p->stream);
         e[4] = hipMemcpyAsync(p->d_gorder, gorder.data(), sizeof(int32_t) * gorder.size(), hipMemcpyHostToDevice,
                               p->stream);
     }
-    if (p->n_wide > 0 && e[2] == hipSuccess)
+    if (p->n_wide > 0 && !whole && e[2] == hipSuccess)
         e[2] = hipMemcpyAsync(p->d_wfirst, p->h_wfirst.data(), sizeof(int32_t) * p->h_wfirst.size(),
                               hipMemcpyHostToDevice, p->stream);
     if (p->own_streams) {
@@ -1060,7 +1078,7 @@ int plan_launch(Plan *p, const Progress *prog)
         return KSW2_HIP_OK;
     }
     if (p->h_stop && p->own_stop) *(volatile int32_t *)p->h_stop = 0;
-    p->started = true;
+    p->started = true, p->fetched = false;
     const bool graphed = graph_eligible(p, prog);
     if (graphed && !p->graph && !p->graph_failed && p->runs >= 1) plan_capture(p);
     ++p->runs;
@@ -1080,7 +1098,7 @@ int plan_launch(Plan *p, const Progress *prog)
     }
     bool used[Plan::kLanes] = {false, false, false, false};
     auto lane = [&](int l) -> hipStream_t {
-        if (!p->own_streams) return p->stream;
+        if (!p->own_streams && !p->lanes) return p->stream;
         if (!p->lane_stream[l]) {
             // a lane is its stream and its completion event, created together
             hipStream_t s = nullptr;
@@ -1253,10 +1271,53 @@ int plan_wait(Plan *p, const Progress *prog)
     return KSW2_HIP_OK;
 }
 
+// A fetch whose arena range is larger than this copies only the CIGAR runs
+// (a compaction kernel, one more round trip); a smaller range, a single
+// call's for instance, is copied as it is.
+constexpr uint64_t kDenseFetchMin = 1ull << 20;
+
+// Words of slot k's place in the CIGAR arena.
+static uint64_t slot_words(const Plan *p, int k)
+{
+    return (uint64_t)(k < p->n_fast ? p->jobs[k].qlen + p->jobs[k].tlen
+                                    : p->gjobs[k - p->n_fast].qlen + p->gjobs[k - p->n_fast].tlen) + 2;
+}
+
+// The arena's words of the slots to deliver.
+static void arena_range(const Plan *p, const std::vector<char> *skip, uint64_t *lo, uint64_t *hi)
+{
+    *lo = p->cig_words, *hi = 0;
+    for (int k = 0; k < p->n; ++k)
+        if (!skip || !(*skip)[k])
+            *lo = std::min(*lo, p->cig_off[k]),
+            *hi = std::max(*hi, std::min<uint64_t>(p->cig_off[k] + slot_words(p, k), p->cig_words));
+}
+
+static uint64_t dense_fetch_min() { return getenv("KSW2_HIP_DENSE_FETCH") ? 0 : kDenseFetchMin; }  // tests: always dense
+
 int plan_run(Plan *p, const Progress *prog)
 {
     const int st = plan_launch(p, prog);
     if (st != KSW2_HIP_OK) return st;
+    // with pinned memory at hand the results follow the kernels, and a small
+    // arena range with them: a call then waits for the device once
+    if (p->pinned && p->started && p->n > 0 && !(prog && prog->cb)) {
+        uint64_t lo, hi;
+        arena_range(p, nullptr, &lo, &hi);
+        const uint64_t outs = round_up(sizeof(KswOut) * (uint64_t)p->n, 256);
+        const bool range = hi > lo && (hi - lo) * 4 <= dense_fetch_min();
+        // (the upload in it is over once ev[0] is: the block grows only then)
+        const uint64_t want = outs + (range ? (hi - lo) * 4 : 0);
+        if (want > p->pinned->bytes) KSW_HIP_TRY(hipEventSynchronize(p->ev[0]));
+        if (p->pinned->grow(want)) {
+            KSW_HIP_TRY(hipMemcpyAsync(p->pinned->base, p->d_out, sizeof(KswOut) * p->n, hipMemcpyDeviceToHost, p->stream));
+            if (range)
+                KSW_HIP_TRY(hipMemcpyAsync(p->pinned->base + outs, p->d_cig + lo, (hi - lo) * 4, hipMemcpyDeviceToHost,
+                                           p->stream));
+            KSW_HIP_TRY(hipStreamSynchronize(p->stream));
+            p->fetched = true;
+        }
+    }
     return plan_wait(p, prog);
 }
 
@@ -1270,11 +1331,6 @@ bool plan_dir_span(const Plan *p, int k, uint64_t *off, uint64_t *len)
     *len = job_dir_bytes(j);
     return true;
 }
-
-// A fetch whose arena range is larger than this copies only the CIGAR runs
-// (a compaction kernel, one more round trip); a smaller range, a single
-// call's for instance, is copied as it is.
-constexpr uint64_t kDenseFetchMin = 1ull << 20;
 
 // Delivers slot k's result with its CIGAR runs at `runs`.
 static int deliver_runs(const Plan *p, int k, const KswOut &o, const uint32_t *runs, ksw_extz_t *z, void *km)
@@ -1312,27 +1368,21 @@ int plan_fetch(Plan *p, ksw_extz_t *ez, void *km, const std::vector<char> *skip)
     int todo = 0;
     for (int k = 0; k < p->n; ++k) todo += !skip || !(*skip)[k];
     if (todo == 0) return KSW2_HIP_OK;  // every pair taken from the host mirror
-    auto slot_words = [&](int k) -> uint64_t {
-        return (uint64_t)(k < p->n_fast ? p->jobs[k].qlen + p->jobs[k].tlen
-                                        : p->gjobs[k - p->n_fast].qlen + p->gjobs[k - p->n_fast].tlen) + 2;
-    };
-    // the arena's words of the slots still to deliver (pairs already taken
-    // from the host mirror are skipped)
-    uint64_t lo = p->cig_words, hi = 0;
-    for (int k = 0; k < p->n; ++k)
-        if (!skip || !(*skip)[k])
-            lo = std::min(lo, p->cig_off[k]),
-            hi = std::max(hi, std::min<uint64_t>(p->cig_off[k] + slot_words(k), p->cig_words));
+    // (pairs already taken from the host mirror are skipped)
+    uint64_t lo, hi;
+    arena_range(p, skip, &lo, &hi);
     std::vector<KswOut> outs(p->n);
-    KSW_HIP_TRY(hipMemcpyAsync(outs.data(), p->d_out, sizeof(KswOut) * p->n, hipMemcpyDeviceToHost, p->stream));
-    const uint64_t dense_min = getenv("KSW2_HIP_DENSE_FETCH") ? 0 : kDenseFetchMin;  // tests: always dense
-    if (hi > lo && (hi - lo) * 4 > dense_min) {
+    if (p->fetched)
+        memcpy(outs.data(), p->pinned->base, sizeof(KswOut) * p->n);
+    else
+        KSW_HIP_TRY(hipMemcpyAsync(outs.data(), p->d_out, sizeof(KswOut) * p->n, hipMemcpyDeviceToHost, p->stream));
+    if (hi > lo && (hi - lo) * 4 > dense_fetch_min()) {
         // A large range: the runs of the slots to deliver are moved on the
         // device into the dense region behind the arena (the move list at
         // its head), so the host copies only the runs, a few hundred KB for
         // a batch whose arena holds tens of MB.  When the runs and the list
         // would not fit the region, the range is copied as it is.
-        KSW_HIP_TRY(hipStreamSynchronize(p->stream));
+        if (!p->fetched) KSW_HIP_TRY(hipStreamSynchronize(p->stream));
         std::vector<CigarMove> moves;
         std::vector<uint64_t> at(p->n, 0);
         uint64_t total = 0;
@@ -1340,14 +1390,18 @@ int plan_fetch(Plan *p, ksw_extz_t *ez, void *km, const std::vector<char> *skip)
         for (int k = 0; k < p->n; ++k) {
             if ((skip && (*skip)[k]) || outs[k].n_cigar <= 0) continue;
             const uint64_t n = (uint64_t)outs[k].n_cigar;
-            if (n > slot_words(k) || p->cig_off[k] + n > p->cig_words) in_slots = false;
+            if (n > slot_words(p, k) || p->cig_off[k] + n > p->cig_words) in_slots = false;
             at[k] = total;
             moves.push_back({p->cig_off[k], (uint32_t)total, (uint32_t)n});
             total += n;
         }
         const uint64_t list_words = 4 * (uint64_t)moves.size();
         if (in_slots && total < (1ull << 32) && list_words + total <= p->cig_words) {
-            std::unique_ptr<uint32_t[]> dense(new uint32_t[std::max<uint64_t>(total, 1)]);
+            // (into pinned memory where there is some: the outs were copied)
+            const bool pin = p->pinned && p->pinned->grow(total * 4);
+            std::unique_ptr<uint32_t[]> own(pin ? nullptr : new uint32_t[std::max<uint64_t>(total, 1)]);
+            uint32_t *dense = pin ? (uint32_t *)p->pinned->base : own.get();
+            p->fetched = false;
             if (total > 0) {
                 uint32_t *region = p->d_cig + p->cig_words;
                 CigarMove *d_moves = (CigarMove *)region;
@@ -1355,16 +1409,25 @@ int plan_fetch(Plan *p, ksw_extz_t *ez, void *km, const std::vector<char> *skip)
                 KSW_HIP_TRY(hipMemcpyAsync(d_moves, moves.data(), sizeof(CigarMove) * moves.size(),
                                            hipMemcpyHostToDevice, p->stream));
                 KSW_HIP_TRY(launch_cigar_compact(p->d_cig, d_dense, d_moves, (int)moves.size(), p->stream));
-                KSW_HIP_TRY(hipMemcpyAsync(dense.get(), d_dense, total * 4, hipMemcpyDeviceToHost, p->stream));
+                KSW_HIP_TRY(hipMemcpyAsync(dense, d_dense, total * 4, hipMemcpyDeviceToHost, p->stream));
                 KSW_HIP_TRY(hipStreamSynchronize(p->stream));
             }
             for (int k = 0; k < p->n; ++k) {
                 if (skip && (*skip)[k]) continue;
-                const int st = deliver_runs(p, k, outs[k], dense.get() + at[k], ez + p->order[k], km);
+                const int st = deliver_runs(p, k, outs[k], dense + at[k], ez + p->order[k], km);
                 if (st != KSW2_HIP_OK) return st;
             }
             return KSW2_HIP_OK;
         }
+    }
+    if (p->fetched && hi > lo && (hi - lo) * 4 <= dense_fetch_min()) {
+        // (the whole plan's range: nothing is skipped where it was fetched)
+        const uint32_t *range = (const uint32_t *)(p->pinned->base + round_up(sizeof(KswOut) * (uint64_t)p->n, 256));
+        for (int k = 0; k < p->n; ++k) {
+            const int st = deliver_runs(p, k, outs[k], range + (p->cig_off[k] - lo), ez + p->order[k], km);
+            if (st != KSW2_HIP_OK) return st;
+        }
+        return KSW2_HIP_OK;
     }
     std::unique_ptr<uint32_t[]> cig(new uint32_t[p->cig_words]);  // only [lo, hi) is filled and read
     if (hi > lo)
@@ -1396,6 +1459,9 @@ void plan_destroy(Plan *p)
     if (p->own_events)
         for (auto &e : p->ev)
             if (e) (void)hipEventDestroy(e);
+    if (p->lanes)  // back to the caller, with those created meanwhile
+        for (int l = 0; l < Plan::kLanes; ++l)
+            p->lanes->stream[l] = p->lane_stream[l], p->lanes->done[l] = p->lane_done[l];
     if (p->own_streams) {
         for (int l = 0; l < Plan::kLanes; ++l) {
             if (p->lane_done[l]) (void)hipEventDestroy(p->lane_done[l]);
@@ -1408,14 +1474,16 @@ void plan_destroy(Plan *p)
 
 namespace {
 
-// What a host thread's single calls reuse from one call to the next: a
-// stream, the plan's timing events, pinned staging for the sequences, a
-// pinned stop flag and a device block grown to the largest call so far (up
-// to kCallBlockMax).  A call then allocates and frees nothing, which matters
-// most when many executor threads call at once: hipFree and hipHostFree
-// wait for the device.  Freed when the thread ends, or by
+// What a host thread's calls reuse from one call to the next: a stream and
+// lanes, the plan's timing events, pinned memory for what goes up and what
+// comes back (up to kPinnedKeep), a pinned stop flag and a device block grown
+// to the largest call so far (up to kCallBlockMax).  A call then allocates and
+// frees nothing, which matters most when many executor threads call at once:
+// hipFree and hipHostFree wait for the device.  (A batch of 64 pairs of 1 kbp,
+// one round of the sliding window: 1.0 ms a call with its own block, streams,
+// events and six copies, 0.5 so.)  Given back when the thread ends, or by
 // ksw2_hip_release_cached_memory on the thread.
-constexpr uint64_t kCallBlockMax = 1ull << 30;
+constexpr uint64_t kCallBlockMax = 1ull << 30, kPinnedKeep = 256ull << 20;
 
 struct GrowPool : DevicePool {
     // one plan at a time; a larger one replaces the block (the previous
@@ -1446,30 +1514,21 @@ struct CallContext {
     bool ready = false;
     hipStream_t stream = nullptr;
     hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};
-    uint8_t *staging = nullptr;
-    uint64_t staging_bytes = 0;
+    PinnedBuffer pinned;
+    PlanLanes lanes;
     int32_t *h_stop = nullptr, *d_stop = nullptr;
     GrowPool pool;
+    bool busy = false;  // a call on this thread has it (a progress callback may call again)
 
-    bool prepare(uint64_t seq_bytes)
+    bool prepare()
     {
         if (!ready) {
-            if (hipStreamCreateWithFlags(&stream, hipStreamNonBlocking) != hipSuccess) return false;
+            if (!stream && hipStreamCreateWithFlags(&stream, hipStreamNonBlocking) != hipSuccess) return false;
             for (auto &e : ev)
-                if (hipEventCreate(&e) != hipSuccess) return false;
-            if (hipHostMalloc((void **)&h_stop, sizeof(int32_t), hipHostMallocMapped) != hipSuccess) return false;
+                if (!e && hipEventCreate(&e) != hipSuccess) return false;
+            if (!h_stop && hipHostMalloc((void **)&h_stop, sizeof(int32_t), hipHostMallocMapped) != hipSuccess) return false;
             if (hipHostGetDevicePointer((void **)&d_stop, h_stop, 0) != hipSuccess) return false;
             ready = true;
-        }
-        if (seq_bytes > staging_bytes) {
-            if (staging) (void)hipHostFree(staging);
-            staging = nullptr, staging_bytes = 0;
-            const uint64_t want = std::max<uint64_t>(seq_bytes + seq_bytes / 4, 1u << 16);
-            if (hipHostMalloc((void **)&staging, want, hipHostMallocDefault) != hipSuccess) {
-                staging = nullptr;
-                return false;
-            }
-            staging_bytes = want;
         }
         *(volatile int32_t *)h_stop = 0;
         return true;
@@ -1477,7 +1536,11 @@ struct CallContext {
     ~CallContext()
     {
         pool.drop();
-        if (staging) (void)hipHostFree(staging);
+        pinned.drop();
+        for (int l = 0; l < Plan::kLanes; ++l) {
+            if (lanes.done[l]) (void)hipEventDestroy(lanes.done[l]);
+            if (lanes.stream[l]) wait_slots_forget(lanes.stream[l]), (void)hipStreamDestroy(lanes.stream[l]);
+        }
         if (h_stop) (void)hipHostFree(h_stop);
         for (auto &e : ev)
             if (e) (void)hipEventDestroy(e);
@@ -1487,9 +1550,43 @@ struct CallContext {
 
 thread_local CallContext t_call;
 
+// A call's use of its thread's context.
+struct ContextUse {
+    const bool held;
+    ContextUse() : held(!t_call.busy && t_call.prepare()) { t_call.busy |= held; }
+    ~ContextUse()
+    {
+        if (!held) return;
+        t_call.busy = false;
+        if (t_call.pinned.bytes > kPinnedKeep) t_call.pinned.drop();
+    }
+};
+
 }  // namespace
 
-void release_call_context() { t_call.pool.drop(); }
+bool PinnedBuffer::grow(uint64_t want)
+{
+    if (want <= bytes) return true;
+    drop();
+    const uint64_t n = std::max<uint64_t>(want < kPinnedKeep / 2 ? want + want / 4 : want, 1u << 16);
+    if (hipHostMalloc((void **)&base, n, hipHostMallocDefault) != hipSuccess) {
+        base = nullptr;
+        return false;
+    }
+    bytes = n;
+    return true;
+}
+
+void PinnedBuffer::drop()
+{
+    if (base) (void)hipHostFree(base);
+    base = nullptr, bytes = 0;
+}
+
+void release_call_context()
+{
+    if (!t_call.busy) t_call.pool.drop(), t_call.pinned.drop();
+}
 
 int run_batch_host(int n, const ksw2_pair_t *pairs, int8_t m, const int8_t *mat, int8_t q, int8_t e, int8_t q2,
                    int8_t e2, ksw_extz_t *ez, void *km, const Progress *prog)
@@ -1545,17 +1642,18 @@ int run_batch_host(int n, const ksw2_pair_t *pairs, int8_t m, const int8_t *mat,
             env.spread = true;  // a plan of its own
             use = &env;
         }
-        if (todo.size() == 1 && total <= kCallBlockMax) {
-            const ksw2_pair_t &pp = pairs[todo[0]];
-            if (t_call.prepare((uint64_t)pp.qlen + pp.tlen + 64)) {
-                env.pool = &t_call.pool;
-                env.stream = t_call.stream;
-                env.events = t_call.ev;
-                env.staging = t_call.staging, env.staging_bytes = t_call.staging_bytes;
-                env.h_stop = t_call.h_stop, env.d_stop = t_call.d_stop;
-                env.spread = true;  // a plan of its own: 5-16 wave teams may spread over CUs
-                use = &env;
-            }
+        const ContextUse context;
+        if (context.held) {
+            if (total <= kCallBlockMax) env.pool = &t_call.pool;
+            env.stream = t_call.stream;
+            // (a lone pair has one launch at a time: its lanes would only add
+            // events)
+            if (todo.size() > 1) env.lanes = &t_call.lanes;
+            env.events = t_call.ev;
+            env.pinned = &t_call.pinned;
+            env.h_stop = t_call.h_stop, env.d_stop = t_call.d_stop;
+            env.spread = true;  // a plan of its own: 5-16 wave teams may spread over CUs
+            use = &env;
         }
         int st = plan_create(&plan, pairs, todo.data(), (int)todo.size(), m, cls, gsc, use);
         if (st == KSW2_HIP_OK) st = plan_run(plan, prog);

@@ -21,7 +21,6 @@
 
 namespace {
 
-using kswhip::code_of;
 using kswhip::Progress;
 
 constexpr int32_t kNegInf = -0x40000000;  // KSW_NEG_INF (minimap2/ksw2.h:18)
@@ -168,10 +167,8 @@ extern "C" int ksw2_hip_certify_batch(int n, const ksw2_certify_task_t *tasks, i
             continue;
         }
         w.q.resize((size_t)ql), w.d.resize((size_t)tl);
-        for (int64_t i = 0; i < ql; ++i)
-            if ((w.q[(size_t)i] = code_of(t.query[i])) == 4) w.flags |= KSW_EZ_GENERIC_SC;
-        for (int64_t i = 0; i < tl; ++i)
-            if ((w.d[(size_t)i] = code_of(t.target[i])) == 4) w.flags |= KSW_EZ_GENERIC_SC;
+        const bool wild_q = kswhip::codes_of(t.query, ql, w.q.data()), wild_d = kswhip::codes_of(t.target, tl, w.d.data());
+        if (wild_q || wild_d) w.flags |= KSW_EZ_GENERIC_SC;
         if (t.precomputed_optimal_score) r.optimal_score = *t.precomputed_optimal_score;
         else need_score.push_back((int)work.size());
         work.push_back(std::move(w));

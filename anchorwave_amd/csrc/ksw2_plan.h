@@ -109,6 +109,17 @@ struct DevicePool {
 
 // Where a plan gets its memory and stream: defaults are its own hipMalloc'd
 // block and its own streams (one per kernel-group lane).
+// What a plan borrows from its caller besides the device pool: lane streams
+// with their completion events (created by the plan on first use, kept by the
+// caller) and pinned memory that grows to what a plan asks for.
+struct PlanLanes;
+struct PinnedBuffer {
+    uint8_t *base = nullptr;
+    uint64_t bytes = 0;
+    bool grow(uint64_t want);  // at least `want` bytes (nothing uses the old ones)
+    void drop();
+};
+
 struct PlanEnv {
     DevicePool *pool = nullptr;
     hipStream_t stream = nullptr;
@@ -122,6 +133,11 @@ struct PlanEnv {
     KswOut *mirror_out = nullptr, *mirror_out_dev = nullptr;
     uint32_t *mirror_cig = nullptr, *mirror_cig_dev = nullptr;
     int32_t *mirror_flag = nullptr, *mirror_flag_dev = nullptr;
+    // Lanes and pinned memory of a caller that waits for the plan and fetches
+    // its results before it uses them again (null: the plan's own lanes, no
+    // lanes on a caller's stream).
+    PlanLanes *lanes = nullptr;
+    PinnedBuffer *pinned = nullptr;
     int team = 0;                    // > 0: every stripe-kernel pair gets this team size
     int rows = 0;                    // 4 or 8: the stripe kernel's rows per lane (0: the plan picks)
     bool spread = false;             // 5-16 wave teams may run spread (as in a plan of its own)
@@ -233,6 +249,10 @@ struct Plan {
     static constexpr int kLanes = 4, kWideLane = kLanes - 1;
     hipStream_t lane_stream[kLanes] = {nullptr, nullptr, nullptr, nullptr};
     hipEvent_t lane_done[kLanes] = {nullptr, nullptr, nullptr, nullptr};
+    PlanLanes *lanes = nullptr;      // where the lanes were borrowed from (PlanEnv::lanes)
+    PinnedBuffer *pinned = nullptr;  // PlanEnv::pinned
+    uint64_t upload_bytes = 0;       // head of the device block: sequences, jobs and orders
+    bool fetched = false;            // the last run's results and arena range are in `pinned`
     float last_dp_ms = 0.f, last_bt_ms = 0.f;
     // the plan's launches captured as one graph (plan_launch, from the
     // second run of an eligible plan), the capture's fork event, and counts
@@ -243,6 +263,11 @@ struct Plan {
     bool stop_requested = false;     // the progress callback stopped the last run
     bool started = false;            // the last run launched (not stopped at r = 0)
     int max_diags = 0;               // largest qlen + tlen - 1 in the plan
+};
+
+struct PlanLanes {
+    hipStream_t stream[Plan::kLanes] = {};
+    hipEvent_t done[Plan::kLanes] = {};
 };
 
 int plan_create(Plan **out, const ksw2_pair_t *pairs, const int *idx, int nidx, int8_t m, const ScoreClass &cls,

@@ -52,8 +52,7 @@ void push_op(std::vector<uint32_t> &ops, uint32_t op, int64_t len)
 void encode(const char *s, int64_t from, int64_t len, std::vector<uint8_t> &out, int &flags)
 {
     out.resize((size_t)len);
-    for (int64_t i = 0; i < len; ++i)
-        if ((out[(size_t)i] = kswhip::code_of(s[from + i])) == 4) flags |= KSW_EZ_GENERIC_SC;
+    if (len > 0 && kswhip::codes_of(s + from, len, out.data())) flags |= KSW_EZ_GENERIC_SC;
 }
 
 }  // namespace
