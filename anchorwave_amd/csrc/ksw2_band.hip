@@ -226,6 +226,9 @@ __global__ void __launch_bounds__(kWave * kBandGroup) __attribute__((amdgpu_wave
             stop = __builtin_amdgcn_readfirstlane(__hip_atomic_load(a.stop, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM));
         return stop != 0;
     };
+    // (while waiting it is looked at now and then: the load goes over the bus)
+    int spins = 0;
+    auto stopped_waiting = [&]() { return (++spins & 1023) == 0 ? stopped() : stop != 0; };
     // one workgroup of as many waves as stripes in flight: the last hands on to
     // the first through the first's ring (with fewer, each would wait for room
     // in the next one's ring, the last for a stripe that the first has yet to
@@ -285,7 +288,7 @@ __global__ void __launch_bounds__(kWave * kBandGroup) __attribute__((amdgpu_wave
                     const uint64_t t_start = wall_clock64();
                     for (;;) {
                         if (have) na = load_half(buf, c - wofs, 0), nh = load_half(buf, c - wofs, 1);
-                        if (!missing() || stopped()) break;
+                        if (!missing() || stopped_waiting()) break;
                         if (wall_clock64() - t_start > kWaitTicks) {
                             late = 1;
                             break;
@@ -304,7 +307,7 @@ __global__ void __launch_bounds__(kWave * kBandGroup) __attribute__((amdgpu_wave
             constexpr int WHAT = decltype(what)::value;
             if (FED && (WHAT & 7) && __builtin_expect(known < in_base + min(c + 4, p_end), 0)) {
                 while ((known = ring_load(&in.filled)) < in_base + min(c + 4, p_end)) {
-                    if (stopped()) break;
+                    if (stopped_waiting()) break;
                     __builtin_amdgcn_s_sleep(1);
                 }
             }
@@ -374,7 +377,7 @@ __global__ void __launch_bounds__(kWave * kBandGroup) __attribute__((amdgpu_wave
                 // after this one, or that wave's stripe before)
                 const int need = nb - kRing > n_lo ? base + nb - kRing : base;
                 while (__builtin_expect(room < need, 0)) {
-                    if (stopped()) break;
+                    if (stopped_waiting()) break;
                     __builtin_amdgcn_s_sleep(1);
                     room = ring_load(&out.taken);
                 }

@@ -164,6 +164,12 @@ void wait_slots_forget(hipStream_t st)
         }
 }
 
+bool wait_slots_idle()
+{
+    std::lock_guard<std::mutex> lk(g_wait_mu);
+    return wait_slots_free() >= 2;
+}
+
 bool wait_slots_prepare()
 {
     std::lock_guard<std::mutex> lk(g_wait_mu);
@@ -394,15 +400,23 @@ static int choose_rows(const ksw2_pair_t *pairs, const std::vector<int> &fast, c
 // against 2.45.  Beyond it the thin passes' instructions per cell (half as many
 // again) no longer fit beside each other: 512 pairs of 300 bp 0.30 against
 // 0.38 ms, 50 of 5 kbp 2.78 against 4.07.  KSW2_HIP_THIN=0 turns it off (tests).
-constexpr int kThinGroups = 384;
-static bool thin_plan(const ksw2_pair_t *pairs, const std::vector<int> &fast, const PlanEnv *env)
+bool thin_enabled()
 {
     const char *ev = getenv("KSW2_HIP_THIN");
-    if ((ev && atoi(ev) == 0) || !latency_plan(pairs, fast, env)) return false;
+    return (!ev || atoi(ev) != 0) && !getenv("KSW2_HIP_ROWS") && !getenv("KSW2_HIP_TEAM") && !getenv("KSW2_HIP_WIDE");
+}
+
+int thin_groups(const ksw2_pair_t &p) { return (thin_passes(stripe_geom(p).kt) + kWideGroup - 1) / kWideGroup; }
+
+static bool thin_plan(const ksw2_pair_t *pairs, const std::vector<int> &fast, const PlanEnv *env)
+{
+    if (!thin_enabled()) return false;
+    if (env && env->thin) return !fast.empty();
+    if (!latency_plan(pairs, fast, env)) return false;
     int64_t groups = 0;
     int big = fast[0];
     for (int id : fast) {
-        groups += (thin_passes(stripe_geom(pairs[id]).kt) + kWideGroup - 1) / kWideGroup;
+        groups += thin_groups(pairs[id]);
         if ((double)pairs[id].qlen * pairs[id].tlen > (double)pairs[big].qlen * pairs[big].tlen) big = id;
     }
     const StripeGeom g = stripe_geom(pairs[big]);
@@ -670,7 +684,7 @@ int plan_create(Plan **out, const ksw2_pair_t *pairs, const int *idx, int nidx, 
                     if (!tuned[k] && team[k] > kWideGroup && team[k] <= kMaxTeam) spread[k] = 1;
         }
         auto wide = [&](int k) { return wide_forced > 0 || team[k] > kMaxTeam || spread[k]; };
-        p->optional_wide = true;
+        p->optional_wide = !(env && env->thin);
         for (int k = 0; k < p->n_fast; ++k)
             if (wide(k) && !spread[k]) p->optional_wide = false;
         auto longest_first = [&](std::vector<int> &m) {

@@ -179,6 +179,7 @@ struct Engine::Flight {
     std::vector<char> delivered;
     int undelivered_fast = 0;
     int stream = 0;
+    bool thin = false;              // on the thin kernel
     double cells = 0, t_start = 0;  // for the statistics
     uint64_t bytes = 0;             // footprints admitted, less direction bytes given back at delivery
 };
@@ -191,6 +192,7 @@ Engine::Engine(int8_t m, const int8_t *mat, const KswScore &sc, const ScoreClass
     stats_ = ev ? atoi(ev) : 0;
     if (const char *mt = getenv("KSW2_HIP_MAX_TEAM")) max_team_ = std::max(1, std::min(kMaxWide, atoi(mt)));
     if (const char *bf = getenv("KSW2_HIP_BACKFILL")) backfill_ = std::max(0, atoi(bf));
+    thin_ = thin_enabled();
     if (const char *sp = getenv("KSW2_HIP_SERVE_SPREAD")) serve_spread_ = atoi(sp);
     if (const char *bs = getenv("KSW2_HIP_BATCH_SPREAD")) batch_spread_ = atoi(bs) != 0;
     if (const char *ff = getenv("KSW2_HIP_FAIL_FLIGHTS")) fail_flights_ = std::max(0, atoi(ff));
@@ -757,6 +759,32 @@ bool Engine::admit_locked(std::unique_lock<std::mutex> &lk)
         const Task *head = q.front();
         const int key = batch_ ? (head->general ? 0 : -1) : team_for(head->passes, head->steps, head->general, T, cap);
         const double span = key > 0 ? head->steps / key : 0;  // the head's steps per wave
+        // Serving flights whose teams are capped by the pairs' pass count (the
+        // device has waves to spare) run on the thin kernel, where a pair's
+        // time is its columns and a lag per 128 rows: at most two such flights
+        // at once, each at most kThinGroups workgroups, half the device.  A
+        // burst of 256 tasks (half of them 5 kbp, the longest some 20 kbp) took
+        // 50-54 ms with one workgroup of eight-row passes per pair, whose
+        // longest pairs ran 22 ms on 16 waves, 19-23 ms so (25 with every capped
+        // flight here, and two of 384 workgroups at once then took up to 25 ms
+        // each; 23-26 with one flight at a time).  Tasks of up to eight passes
+        // take a workgroup each, four rows per lane, unless all that waits fits
+        // one flight: their flights need no waiting launch.
+        auto chain = [](const Task *t) { return (double)t->pair.qlen + t->pair.tlen; };
+        auto capped = [&](const Task *t) {
+            return !t->general && team_for(t->passes, t->steps, t->general, T, max_team_) >= t->passes;
+        };
+        size_t waiting = 0;
+        for (const auto &w : queue_) waiting += w.size();
+        bool thin = !batch_ && thin_ && capped(head) && thin_groups(head->pair) <= kThinGroups &&
+                    (2 * head->passes > kMaxTeam || (int64_t)waiting * thin_groups(head->pair) <= kThinGroups);
+        if (thin) {
+            int running = 0;
+            for (const auto &f : flights_) running += f->thin;
+            if (running >= 2) continue;
+            thin = wait_slots_idle();
+        }
+        int64_t groups = 0;
         std::vector<Task *> pick;
         uint64_t bytes = kPlanSlack, seq = 0, cigw = 0;
         int64_t waves = 0;
@@ -767,6 +795,8 @@ bool Engine::admit_locked(std::unique_lock<std::mutex> &lk)
             // serving: one team size (one launch) and similar durations per
             // flight; batch: general and stripe pairs in flights of their own
             const bool same = batch_ ? (key == 0) == t->general
+                              : thin ? capped(t) && chain(t) <= 2 * chain(head) && 2 * chain(t) >= chain(head) &&
+                                           groups + thin_groups(t->pair) <= kThinGroups
                                      : team_for(t->passes, t->steps, t->general, T, cap) == key &&
                                            (key == 0 || (t->steps / key <= 2 * span && 2 * t->steps / key >= span));
             if (!same) {
@@ -774,7 +804,9 @@ bool Engine::admit_locked(std::unique_lock<std::mutex> &lk)
                 ++it;
                 continue;
             }
-            const int w = key > 0 ? key : key < 0 ? (t->cls == 2 ? std::min(kMaxWide, t->passes) : 1) : t->waves;
+            const int w = thin      ? std::max(1, (int)((int64_t)thin_groups(t->pair) * resident_waves_ / (2 * kThinGroups)))
+                          : key > 0 ? key
+                          : key < 0 ? (t->cls == 2 ? std::min(kMaxWide, t->passes) : 1) : t->waves;
             if (!pick.empty() && waves + w > free_waves) break;
             // a flight holds at most its class's share of the pool, except that
             // its first task may use any free block (a task larger than the share)
@@ -785,6 +817,7 @@ bool Engine::admit_locked(std::unique_lock<std::mutex> &lk)
             }
             pick.push_back(t);
             t->held = w;
+            if (thin) groups += thin_groups(t->pair);
             bytes += t->footprint, waves += w, steps += t->steps, seq += (uint64_t)t->pair.qlen + t->pair.tlen + 32;
             cigw += ((uint64_t)t->pair.qlen + t->pair.tlen + 2 + 15) / 16 * 16;
             it = q.erase(it);
@@ -803,7 +836,9 @@ bool Engine::admit_locked(std::unique_lock<std::mutex> &lk)
         // passes, so a flight with a forced team runs eight rows otherwise.
         const bool light = queues_empty() && 8 * (busy_waves_ + waves) <= resident_waves_;
         int rows = key > 0 ? 8 : 0, team = std::max(key, 0);
-        if (!batch_ && key > 0 && key == head->passes && 2 * key <= kMaxTeam && 4 * waves <= free_waves) {
+        if (thin) {
+            rows = 0, team = 0;
+        } else if (!batch_ && key > 0 && key == head->passes && 2 * key <= kMaxTeam && 4 * waves <= free_waves) {
             rows = 4, team = 2 * key, waves *= 2;
             for (Task *t : pick) t->held *= 2;
         }
@@ -834,7 +869,7 @@ bool Engine::admit_locked(std::unique_lock<std::mutex> &lk)
         }
         auto f = std::make_unique<Flight>();
         f->tasks = pick;
-        f->stream = s;
+        f->stream = s, f->thin = thin;
         for (const Task *tk : pick) f->cells += tk->cells;
         for (Task *t : pick) f->pairs.push_back(t->pair);
         busy_[s] = true;
@@ -847,7 +882,7 @@ bool Engine::admit_locked(std::unique_lock<std::mutex> &lk)
         env.staging = staging_[s], env.staging_bytes = staging_bytes_[s];
         env.h_stop = h_stop_, env.d_stop = d_stop_;
         env.poll_stop = true;  // stop_all_locked raises it
-        env.team = team, env.rows = rows;
+        env.team = team, env.rows = rows, env.thin = thin;
         if (batch_) {
             // teams by memory: each wave holds at most its share of the pool
             // (the step budget stays the flight's own unless asked otherwise)

@@ -110,6 +110,7 @@ private:
     uint64_t budget_;
     int device_ = 0;
     int resident_waves_ = 4096;
+    bool thin_ = true;  // serving flights may run on the thin kernel
     std::unique_ptr<DevicePool> pool_;
     hipStream_t streams_[kMaxStreams] = {};
     bool busy_[kMaxStreams] = {};

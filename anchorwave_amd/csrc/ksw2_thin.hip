@@ -183,6 +183,11 @@ __device__ __forceinline__ void thin_run(const StripeArgs &a, const typename Cel
             stop = __builtin_amdgcn_readfirstlane(__hip_atomic_load(a.stop, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM));
         return stop != 0;
     };
+    // while waiting it is looked at now and then: a load over the bus on every
+    // look at a count made each wait last one, and a thousand waves' loads
+    // filled the bus (38 pairs of 5 kbp in a server's flight: 50 ms, 2.5 so)
+    int spins = 0;
+    auto stopped_waiting = [&]() { return (++spins & 1023) == 0 ? stopped() : stop != 0; };
 
     // ---- wave 0: column-buffer entries of a block, asked for 16 steps before
     // they are put into the ring and 20 before the first is used.  One set of
@@ -209,7 +214,7 @@ __device__ __forceinline__ void thin_run(const StripeArgs &a, const typename Cel
                 const uint64_t t_start = wall_clock64();
                 for (;;) {
                     if (have) ne = load_entry(bnd, col);
-                    if (__ballot(have && (uint32_t)(ne >> 32 & 0xffffu) != tag) == 0 || stopped()) break;
+                    if (__ballot(have && (uint32_t)(ne >> 32 & 0xffffu) != tag) == 0 || stopped_waiting()) break;
                     if (wall_clock64() - t_start > kWaitTicks) {
                         late = 1;
                         break;
@@ -229,7 +234,8 @@ __device__ __forceinline__ void thin_run(const StripeArgs &a, const typename Cel
     auto read4 = [&](int c, uint4 (&e)[4]) {
         if (__builtin_expect(known < base + min(c + 4, qlen), 0)) {
             while ((known = __builtin_amdgcn_readfirstlane(ring_load(&in.filled))) < base + min(c + 4, qlen)) {
-                if (stopped()) break;
+                if (stopped_waiting()) break;
+                __builtin_amdgcn_s_sleep(1);
             }
         }
         asm volatile("" ::: "memory");  // the entries are read after their count
@@ -348,7 +354,8 @@ __device__ __forceinline__ void thin_run(const StripeArgs &a, const typename Cel
             // reading its pass before)
             const int need = max(FEEDS ? base + nb - kSkew - kRing : base, base);
             while (__builtin_expect(room < need, 0)) {
-                if (stopped()) return;
+                if (stopped_waiting()) return;
+                __builtin_amdgcn_s_sleep(1);
                 room = __builtin_amdgcn_readfirstlane(ring_load(&out.taken));
             }
         }

@@ -85,3 +85,26 @@ def test_thin_more_passes_than_waves():
     q = np.concatenate([t[5000:5300], W.random_seq(rng, 40)])
     _check([(q, t)], ksw2.KSW_EZ_SCORE_ONLY)
     _check([(q, t)], 0)
+
+
+def test_thin_in_server_flights():
+    """A burst of long and short tasks to a server: flights on the thin kernel
+    beside flights of one-workgroup teams, all as the oracle has them."""
+    rng = np.random.default_rng(95)
+    tasks = []
+    for k, tl in enumerate([9000, 8300, 8192, 8193, 12000] + [300, 1500, 2000, 4100] * 5):
+        t = W.random_seq(rng, tl)
+        q = W.mutate(rng, t, 0.08, 0.02)
+        tasks.append((q, t) if k % 3 else (t, q))
+    flags = [FLAGS[k % len(FLAGS)] for k in range(len(tasks))]
+    for count in (1, len(tasks)):  # alone, and all at once
+        server = ksw2.Server()
+        tickets = {server.submit(q, t, flag=f): k for k, ((q, t), f) in enumerate(zip(tasks[:count], flags))}
+        seen = 0
+        while seen < count:
+            for ticket, got, _ in server.poll(count, -1):
+                q, t = tasks[tickets[ticket]]
+                ref = O.run_oracle(q, t, flag=flags[tickets[ticket]])
+                assert same(got, ref), diff(got, ref)
+                seen += 1
+        server.close()
