@@ -741,6 +741,31 @@ int plan_create(Plan **out, const ksw2_pair_t *pairs, const int *idx, int nidx, 
             thr[gk] = gen_threads(pp);
             ring[gk] = gen_ring(pp);
         }
+        // A plan of its own that leaves SIMDs with few waves: more threads per
+        // pair, up to one per position of its widest anti-diagonal, while the
+        // pairs' waves are at most four per SIMD (two beyond 256 threads,
+        // whose barrier costs more).  Extensions of 1 kbp under w = 500, from
+        // 128 threads: one pair 9.0 -> 6.8 ms (512 threads), 64 pairs 10.1 ->
+        // 7.6 (512), 512 pairs 10.8 -> 8.5 (256; 8.7 with 512), 1,024 pairs
+        // 11.3 -> 10.2 (256; 15.7 with 512); 2,048 pairs 14.0 and 18.9 (256).
+        if (!getenv("KSW2_HIP_GEN_THREADS") && (!env || env->spread)) {
+            int64_t waves = 0;
+            for (int gk = 0; gk < p->n_gen; ++gk) waves += band[gk] ? 0 : thr[gk] / kWave;
+            // (all that can take twice as many, or none: launches of mixed
+            // sizes wait for their largest)
+            for (int t = 128; t <= 1024; t <<= 1) {
+                std::vector<int> grow;
+                int64_t more = 0;
+                for (int gk = 0; gk < p->n_gen; ++gk) {
+                    const ksw2_pair_t &pp = pairs[p->order[p->n_fast + gk]];
+                    const int window = std::min(std::min(pp.qlen, pp.tlen), norm_w(pp) + 1) + 128;
+                    if (!band[gk] && 2 * thr[gk] == t && t <= window + 64) grow.push_back(gk), more += t / 2 / kWave;
+                }
+                if (waves + more > (t <= 256 ? 4 : 2) * (int64_t)kDeviceSimds) continue;
+                for (int gk : grow) thr[gk] = t;
+                waves += more;
+            }
+        }
         for (int t = 1024; t >= 64; t >>= 1)
             for (int rs = kGenRingMax; rs >= 0; rs = rs > 256 ? rs >> 1 : rs - 256) {
                 std::vector<int> members;

@@ -70,6 +70,31 @@ __device__ __forceinline__ bool apply_zdrop(Track &z, int H, int r, int t, int z
 
 __device__ __forceinline__ int edge_i8(const KswScore &sc, int r) { return edge_diff(sc, r); }
 
+// A wave's largest value and smallest unsigned one, in every lane: within
+// rows of 16 lanes, then from row to row, the last lane has it.  (Six steps
+// of a shuffle through LDS took some 130 cycles each, twice an anti-diagonal:
+// 512 extensions of 1 kbp under w = 500 at 256 threads 9.7 ms, 8.5 so.)
+template <int CTRL, int ROWS> __device__ __forceinline__ int dpp_or(int other, int v)
+{
+    return __builtin_amdgcn_update_dpp(other, v, CTRL, ROWS, 0xF, false);
+}
+__device__ __forceinline__ int wave_max(int v)
+{
+    v = max(v, dpp_or<0x111, 0xF>(INT32_MIN, v)), v = max(v, dpp_or<0x112, 0xF>(INT32_MIN, v));
+    v = max(v, dpp_or<0x114, 0xF>(INT32_MIN, v)), v = max(v, dpp_or<0x118, 0xF>(INT32_MIN, v));
+    v = max(v, dpp_or<0x142, 0xA>(INT32_MIN, v)), v = max(v, dpp_or<0x143, 0xC>(INT32_MIN, v));
+    return __builtin_amdgcn_readlane(v, kWave - 1);
+}
+__device__ __forceinline__ uint32_t wave_min(uint32_t x)
+{
+    auto low = [](int a, int b) { return (int)min((uint32_t)a, (uint32_t)b); };
+    int v = (int)x;
+    v = low(v, dpp_or<0x111, 0xF>(-1, v)), v = low(v, dpp_or<0x112, 0xF>(-1, v));
+    v = low(v, dpp_or<0x114, 0xF>(-1, v)), v = low(v, dpp_or<0x118, 0xF>(-1, v));
+    v = low(v, dpp_or<0x142, 0xA>(-1, v)), v = low(v, dpp_or<0x143, 0xC>(-1, v));
+    return (uint32_t)__builtin_amdgcn_readlane(v, kWave - 1);
+}
+
 }  // namespace
 
 // RING: the per-position state lives in LDS, in rings of a.ring slots
@@ -91,6 +116,9 @@ __global__ void __launch_bounds__(kWave * kMaxWaves) ksw_general_kernel(GenArgs 
     const KswScore &sc = gs.k;
     const int nthr = blockDim.x, tid = threadIdx.x, lane = tid % kWave, wv = tid / kWave;
     const int nw = nthr / kWave;
+    // t mod nthr (a mask: nthr is a power of two unless a size is forced)
+    const bool pow2 = (nthr & (nthr - 1)) == 0;
+    auto thread_of = [&](int t) { return pow2 ? t & (nthr - 1) : t % nthr; };
     const int qlen = __builtin_amdgcn_readfirstlane(jb.qlen), tlen = __builtin_amdgcn_readfirstlane(jb.tlen);
     const int w = __builtin_amdgcn_readfirstlane(jb.w), flag = __builtin_amdgcn_readfirstlane(jb.flag);
     const int tlenB = jb.tlenB, qlenB = jb.qlenB;
@@ -179,7 +207,7 @@ __global__ void __launch_bounds__(kWave * kMaxWaves) ksw_general_kernel(GenArgs 
                 const int h_st0 = st0 == en0 ? h_en0 : F.h_st0;
                 if (en0 == tlen - 1 && h_en0 >= z.mte) z.mte = h_en0, z.mte_q = rr - en0;
                 if (rr - st0 == qlen - 1 && h_st0 >= z.mqe) z.mqe = h_st0, z.mqe_t = st0;
-                if (en0 % nthr == tid) H[en0 & mk] = h_en0;  // owner keeps H[en0]
+                if (thread_of(en0) == tid) H[en0 & mk] = h_en0;  // owner keeps H[en0]
                 if (apply_zdrop(z, max_H, rr, max_t, jb.zdrop, e2)) stop = true;
                 else if (rr == qlen + tlen - 2 && en0 == tlen - 1) z.score = h_en0;
             } else {
@@ -256,7 +284,7 @@ __global__ void __launch_bounds__(kWave * kMaxWaves) ksw_general_kernel(GenArgs 
         Fin &F = fin[cr];
         if (a.stop && (r & 255) == 0 && tid == 0)
             F.stop = __hip_atomic_load(a.stop, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-        int t = stB + ((tid - stB) % nthr + nthr) % nthr;
+        int t = stB + (pow2 ? tid - stB & (nthr - 1) : ((tid - stB) % nthr + nthr) % nthr);
         for (; t <= t_end; t += nthr) {
             int sct = 0;
             const bool in_sc = t >= st0 && t <= sc_end;
@@ -343,20 +371,16 @@ __global__ void __launch_bounds__(kWave * kMaxWaves) ksw_general_kernel(GenArgs 
             }
         }
         // values the bookkeeping needs at positions outside [stB, en16]
-        if (!approx && r > 0 && en0 >= 1 && en0 - 1 < stB && (en0 - 1) % nthr == tid)
+        if (!approx && r > 0 && en0 >= 1 && en0 - 1 < stB && thread_of(en0 - 1) == tid)
             F.h_old_en0m1 = H[(en0 - 1) & mk];
         if (approx && r > 0) {
             const int t1 = last_H0_t + 1;
-            if ((t1 < stB || t1 > en16) && t1 < tlenB && t1 % nthr == tid) F.u_h0 = u[t1 & mk];
+            if ((t1 < stB || t1 > en16) && t1 < tlenB && thread_of(t1) == tid) F.u_h0 = u[t1 & mk];
         }
         if (!approx) {
             // wave reduction of (H, rank): larger H, then smaller rank
-#pragma unroll
-            for (int o = 1; o < kWave; o <<= 1) {
-                const int oh = __shfl_xor(bh, o, kWave);
-                const uint32_t orank = (uint32_t)__shfl_xor((int)br, o, kWave);
-                if (oh > bh || (oh == bh && orank < br)) bh = oh, br = orank;
-            }
+            const int wh = wave_max(bh);
+            br = wave_min(bh == wh ? br : 0xffffffffu), bh = wh;
             if (lane == 0) F.best_h[wv] = bh, F.best_rank[wv] = br;
         }
         p_st0 = st0, p_en0 = en0, p_en1 = en1;
