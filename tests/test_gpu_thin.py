@@ -83,8 +83,16 @@ def test_thin_more_passes_than_waves():
     rng = np.random.default_rng(33)
     t = W.random_seq(rng, 1024 * 128 + 700)
     q = np.concatenate([t[5000:5300], W.random_seq(rng, 40)])
-    _check([(q, t)], ksw2.KSW_EZ_SCORE_ONLY)
-    _check([(q, t)], 0)
+    for flag in (ksw2.KSW_EZ_SCORE_ONLY, 0):
+        _check([(q, t)], flag)
+        # (a call may take a layout of the measured table; a server's flight
+        # of a lone long task does not)
+        server = ksw2.Server()
+        server.submit(q, t, flag=flag)
+        (_, got, _), = server.poll(1, -1)
+        server.close()
+        ref = O.run_oracle(q, t, flag=flag)
+        assert same(got, ref), diff(got, ref)
 
 
 def test_thin_in_server_flights():
