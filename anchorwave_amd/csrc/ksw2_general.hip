@@ -497,24 +497,56 @@ __global__ void __launch_bounds__(64) ksw_general_backtrack_kernel(GenBacktrackA
     a.out[jb.out] = o;
 }
 
-// The same walk for long pairs, one wave per pair.  A step moves to
-// anti-diagonal r-1 or r-2 and to target position i or i-1, so the next 128
-// anti-diagonals stay within positions [i-127, i] of the current (r, i):
-// the wave stages those 128 rows (132 bytes each, from the 4-byte boundary
-// at or below i-127, zero outside the row; lane L stages rows r-L and
-// r-64-L) and their off/off_end in LDS, and the walk reads LDS until it
-// leaves the tile.  The walk is uniform (scalar) but for runs of diagonal
-// moves and runs of gap moves, each taken at once by a ballot over the
-// lanes; the CIGAR runs go out one store per run, and the wave reverses
-// them at the end.
-constexpr int kTileRows = 128, kTileDw = 33;
+// The same walk for long pairs, by the first wave of a workgroup.  A step
+// moves to anti-diagonal r-1 or r-2 and to target position i or i-1, so the
+// next 128 anti-diagonals stay within positions [i-127, i] of the current
+// (r, i): a tile of those 128 rows (132 bytes each, from the 4-byte boundary
+// at or below i-127, zero outside the row) and their off/off_end are staged
+// in LDS, and the walk reads LDS until it leaves the tile.  Meanwhile the
+// other waves stage the tile below, where a diagonal path enters it, with 16
+// positions to spare on its right: a path of 20 kbp took 1.15 ms when the
+// walking wave staged its own, half of it waiting for the tile's bytes, 0.80 ms
+// so.  The walk is uniform (scalar) but for runs of diagonal moves and runs
+// of gap moves, each taken at once by a ballot over the lanes; the CIGAR runs
+// go out one store per run, and the wave reverses them at the end.
+constexpr int kTileRows = 128, kTileDw = 33, kTileSpare = 16, kTileWaves = 4;
+static_assert(kTileRows <= (kTileWaves - 1) * kWave, "a thread of the other waves per row");
 
-__global__ void __launch_bounds__(64) ksw_general_backtrack_tiled_kernel(GenBacktrackArgs a)
-{
-    __shared__ uint32_t tile[kTileRows * kTileDw];
+struct RowTile {
+    uint32_t byte[kTileRows * kTileDw];
     // per staged row: off[], off_end[] and the position of its first byte
-    __shared__ int t_ro[kTileRows], t_re[kTileRows], t_base[kTileRows];
-    const int lane = threadIdx.x;
+    int ro[kTileRows], re[kTileRows], base[kTileRows];
+};
+
+// Row L of the tile of anti-diagonals (r0 - 128, r0] from position ws.
+__device__ __forceinline__ void stage_row(RowTile &t, int L, int r0, int ws, const uint32_t *p32, const int32_t *off,
+                                          const int32_t *off_end, int nd)
+{
+    const int row = r0 - L;
+    if (row < 0) {
+        t.ro[L] = 0, t.re[L] = -1, t.base[L] = 0;
+        return;
+    }
+    // all loads in flight at once (clamped in-row addresses), then the bytes
+    // outside the row zeroed
+    const int ro = off[row], d0 = (ws - ro) >> 2;  // floor
+    const uint32_t *src = p32 + (uint64_t)row * (uint32_t)nd;
+    uint32_t v[kTileDw];
+#pragma unroll
+    for (int q = 0; q < kTileDw; ++q) v[q] = src[min(max(d0 + q, 0), nd - 1)];
+    t.ro[L] = ro, t.re[L] = off_end[row], t.base[L] = ro + 4 * d0;
+#pragma unroll
+    for (int q = 0; q < kTileDw; ++q) {
+        const int d = d0 + q;
+        t.byte[L * kTileDw + q] = d >= 0 && d < nd ? v[q] : 0u;
+    }
+}
+
+__global__ void __launch_bounds__(kWave * kTileWaves) ksw_general_backtrack_tiled_kernel(GenBacktrackArgs a)
+{
+    __shared__ RowTile tiles[2];
+    __shared__ int at[2][2];  // where the walk is after a tile, in turn
+    const int lane = threadIdx.x % kWave, wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kWave);
     const GenJob jb = a.jobs[blockIdx.x];
     const int flag = __builtin_amdgcn_readfirstlane(jb.flag);
     const int qlen = __builtin_amdgcn_readfirstlane(jb.qlen), tlen = __builtin_amdgcn_readfirstlane(jb.tlen);
@@ -529,133 +561,128 @@ __global__ void __launch_bounds__(64) ksw_general_backtrack_tiled_kernel(GenBack
         const uint32_t *p32 = (const uint32_t *)(a.dir + jb.dir_off);
         const int32_t *off = a.offs + jb.off_off, *off_end = off + (qlen + tlen - 1);
         uint32_t *cig = a.cig + jb.cig_off;
-        const uint8_t *tb = (const uint8_t *)tile;
         int i = __builtin_amdgcn_readfirstlane(i0), j = __builtin_amdgcn_readfirstlane(j0), state = 0;
         int run_op = -1, run_len = 0;
-        int r0 = -1, ws = 0;  // tile: anti-diagonals (r0 - 128, r0], positions from ws
-        // lane L: off[], off_end[] of rows r0 - L (ro[0] ...) and r0 - 64 - L
-        // (ro[1] ...) and the position of their first staged bytes
-        int ro[2] = {0, 0}, re[2] = {-1, -1}, base[2] = {0, 0};
+        int cur = 0, r0 = -1, ws = 0;  // the walk's tile: anti-diagonals (r0 - 128, r0], positions from ws
+        int next_r0 = -1, next_ws = 0; // the tile staged meanwhile (none: -1)
         const int nd = ncolB >> 2;
-        while (i >= 0 && j >= 0) {
-            const int r = i + j;
-            if (r0 < 0 || r <= r0 - kTileRows || i < ws) {
-                r0 = r, ws = i - 127;
-                __syncthreads();  // the walk's last reads of the old tile are done
-                // all loads of both rows in flight at once (clamped in-row
-                // addresses), then the bytes outside the row zeroed
-                uint32_t v[2][kTileDw];
-                int d0[2];
-#pragma unroll
-                for (int h = 0; h < 2; ++h) {
-                    const int row = r0 - kWave * h - lane;
-                    ro[h] = 0, re[h] = -1, base[h] = 0, d0[h] = 0;
-                    if (row >= 0) {
-                        ro[h] = off[row], re[h] = off_end[row];
-                        d0[h] = (ws - ro[h]) >> 2;  // floor
-                        base[h] = ro[h] + 4 * d0[h];
-                        const uint32_t *src = p32 + (uint64_t)row * (uint32_t)nd;
-#pragma unroll
-                        for (int q = 0; q < kTileDw; ++q) v[h][q] = src[min(max(d0[h] + q, 0), nd - 1)];
-                    }
+        for (int turn = 0; i >= 0 && j >= 0; turn ^= 1) {
+            {
+                const int r = i + j;
+                if (next_r0 >= 0 && r <= next_r0 && r > next_r0 - kTileRows && i >= next_ws && i <= next_ws + 127) {
+                    cur ^= 1, r0 = next_r0, ws = next_ws;
+                } else {
+                    r0 = r, ws = i - 127;
+                    if ((int)threadIdx.x < kTileRows) stage_row(tiles[cur], threadIdx.x, r0, ws, p32, off, off_end, nd);
+                    __syncthreads();
                 }
-#pragma unroll
-                for (int h = 0; h < 2; ++h) {
-                    const int Lr = kWave * h + lane;
-                    t_ro[Lr] = ro[h], t_re[Lr] = re[h], t_base[Lr] = base[h];
-                    if (r0 - Lr >= 0) {
-#pragma unroll
-                        for (int q = 0; q < kTileDw; ++q) {
-                            const int d = d0[h] + q;
-                            tile[Lr * kTileDw + q] = d >= 0 && d < nd ? v[h][q] : 0u;
-                        }
-                    }
-                }
+                next_r0 = r0 - kTileRows;
+                next_ws = i - (kTileRows - (r0 - r)) / 2 + kTileSpare - 127;
+            }
+            const RowTile &tile = tiles[cur];
+            if (wv > 0) {
+                const int L = (int)threadIdx.x - kWave;
+                if (next_r0 >= 0 && L < kTileRows) stage_row(tiles[cur ^ 1], L, next_r0, next_ws, p32, off, off_end, nd);
                 __syncthreads();
+                i = at[turn][0], j = at[turn][1];
+                continue;
             }
-            const int L = r0 - r;
-            if (state == 0) {
-                // A run of diagonal moves at once: from state 0 the walk
-                // stays in state 0 and moves to (i-1, j-1), anti-diagonal
-                // r-2, while a cell is not forced and its argmax (low three
-                // bits) is 0.  Lane k tests cell (i-k, j-k) of the tile (row
-                // L+2k); the run is the lanes before the first that fails.
-                const int Lk = L + 2 * lane, ik = i - lane;
-                const int Lc = min(Lk, kTileRows - 1);
-                const int o_k = t_ro[Lc], e_k = t_re[Lc], b_k = t_base[Lc];
-                int fail = 1;
-                if (Lk < kTileRows && ik >= 0 && lane <= j && ik >= ws && ik >= o_k && ik <= e_k) {
-                    const int byte = tb[Lk * kTileDw * 4 + (ik - b_k)];
-                    const int tmp = (uint32_t)(ik - o_k) < (uint32_t)ncolB ? byte : 0;
-                    fail = (tmp & 7) != 0;
-                }
-                const uint64_t fb = __ballot(fail);
-                const int run = fb ? (int)__builtin_ctzll(fb) : kWave;
-                if (run > 0) {
-                    i -= run, j -= run;
-                    if (run_op == 0) {
-                        run_len += run;
-                    } else {
-                        if (run_len > 0 && lane == 0) cig[n] = (uint32_t)run_len << 4 | (uint32_t)run_op;
-                        if (run_len > 0) ++n;
-                        run_op = 0, run_len = run;
+            const uint8_t *tb = (const uint8_t *)tile.byte;
+            const int *t_ro = tile.ro, *t_re = tile.re, *t_base = tile.base;
+            // lane L: off[], off_end[] of rows r0 - L (ro[0] ...) and r0 - 64 - L
+            // (ro[1] ...) and the position of their first staged bytes
+            const int ro[2] = {t_ro[lane], t_ro[kWave + lane]}, re[2] = {t_re[lane], t_re[kWave + lane]};
+            const int base[2] = {t_base[lane], t_base[kWave + lane]};
+            while (i >= 0 && j >= 0) {
+                const int r = i + j;
+                if (r <= r0 - kTileRows || i < ws) break;
+                const int L = r0 - r;
+                if (state == 0) {
+                    // A run of diagonal moves at once: from state 0 the walk
+                    // stays in state 0 and moves to (i-1, j-1), anti-diagonal
+                    // r-2, while a cell is not forced and its argmax (low three
+                    // bits) is 0.  Lane k tests cell (i-k, j-k) of the tile (row
+                    // L+2k); the run is the lanes before the first that fails.
+                    const int Lk = L + 2 * lane, ik = i - lane;
+                    const int Lc = min(Lk, kTileRows - 1);
+                    const int o_k = t_ro[Lc], e_k = t_re[Lc], b_k = t_base[Lc];
+                    int fail = 1;
+                    if (Lk < kTileRows && ik >= 0 && lane <= j && ik >= ws && ik >= o_k && ik <= e_k) {
+                        const int byte = tb[Lk * kTileDw * 4 + (ik - b_k)];
+                        const int tmp = (uint32_t)(ik - o_k) < (uint32_t)ncolB ? byte : 0;
+                        fail = (tmp & 7) != 0;
                     }
-                    continue;
-                }
-            } else {
-                // A run of gap moves at once: in state s (1-4) the walk
-                // keeps s while a cell's continuation bit (s + 2) is set, or
-                // while the cell is forced into s itself, and moves to
-                // (i-1, j) for s = 1, 3 or (i, j-1) for s = 2, 4, anti-
-                // diagonal r-1.  Lane k tests the k-th cell of the run (row
-                // L+k).
-                const int s = state;
-                const bool di = s == 1 || s == 3;
-                const int Lk = L + lane, ik = di ? i - lane : i;
-                const int Lc = min(Lk, kTileRows - 1);
-                const int o_k = t_ro[Lc], e_k = t_re[Lc], b_k = t_base[Lc];
-                int fail = 1;
-                if (Lk < kTileRows && lane <= (di ? i : j)) {
-                    const int force = ik > e_k ? 1 : ik < o_k ? 2 : -1;
-                    const int byte = tb[Lk * kTileDw * 4 + (ik - b_k)];
-                    const int tmp = force < 0 && (uint32_t)(ik - o_k) < (uint32_t)ncolB ? byte : 0;
-                    fail = force >= 0 ? force != s : !(tmp >> (s + 2) & 1);
-                }
-                const uint64_t fb = __ballot(fail);
-                const int run = fb ? (int)__builtin_ctzll(fb) : kWave;
-                if (run > 0) {
-                    const int op = di ? 2 : 1;
-                    if (di) i -= run;
-                    else j -= run;
-                    if (run_op == op) {
-                        run_len += run;
-                    } else {
-                        if (run_len > 0 && lane == 0) cig[n] = (uint32_t)run_len << 4 | (uint32_t)run_op;
-                        if (run_len > 0) ++n;
-                        run_op = op, run_len = run;
+                    const uint64_t fb = __ballot(fail);
+                    const int run = fb ? (int)__builtin_ctzll(fb) : kWave;
+                    if (run > 0) {
+                        i -= run, j -= run;
+                        if (run_op == 0) {
+                            run_len += run;
+                        } else {
+                            if (run_len > 0 && lane == 0) cig[n] = (uint32_t)run_len << 4 | (uint32_t)run_op;
+                            if (run_len > 0) ++n;
+                            run_op = 0, run_len = run;
+                        }
+                        continue;
                     }
-                    continue;
+                } else {
+                    // A run of gap moves at once: in state s (1-4) the walk
+                    // keeps s while a cell's continuation bit (s + 2) is set, or
+                    // while the cell is forced into s itself, and moves to
+                    // (i-1, j) for s = 1, 3 or (i, j-1) for s = 2, 4, anti-
+                    // diagonal r-1.  Lane k tests the k-th cell of the run (row
+                    // L+k).
+                    const int s = state;
+                    const bool di = s == 1 || s == 3;
+                    const int Lk = L + lane, ik = di ? i - lane : i;
+                    const int Lc = min(Lk, kTileRows - 1);
+                    const int o_k = t_ro[Lc], e_k = t_re[Lc], b_k = t_base[Lc];
+                    int fail = 1;
+                    if (Lk < kTileRows && lane <= (di ? i : j) && ik >= ws) {
+                        const int force = ik > e_k ? 1 : ik < o_k ? 2 : -1;
+                        const int byte = tb[Lk * kTileDw * 4 + (ik - b_k)];
+                        const int tmp = force < 0 && (uint32_t)(ik - o_k) < (uint32_t)ncolB ? byte : 0;
+                        fail = force >= 0 ? force != s : !(tmp >> (s + 2) & 1);
+                    }
+                    const uint64_t fb = __ballot(fail);
+                    const int run = fb ? (int)__builtin_ctzll(fb) : kWave;
+                    if (run > 0) {
+                        const int op = di ? 2 : 1;
+                        if (di) i -= run;
+                        else j -= run;
+                        if (run_op == op) {
+                            run_len += run;
+                        } else {
+                            if (run_len > 0 && lane == 0) cig[n] = (uint32_t)run_len << 4 | (uint32_t)run_op;
+                            if (run_len > 0) ++n;
+                            run_op = op, run_len = run;
+                        }
+                        continue;
+                    }
+                }
+                const int h = L >> 6, Lh = L & (kWave - 1);
+                const int o_r = __builtin_amdgcn_readlane(h ? ro[1] : ro[0], Lh);
+                const int e_r = __builtin_amdgcn_readlane(h ? re[1] : re[0], Lh);
+                const int b_r = __builtin_amdgcn_readlane(h ? base[1] : base[0], Lh);
+                // (the row's byte is read whether or not it is used: the tile
+                // holds zeros outside the row, and i - b_r is within the tile)
+                const int byte = __builtin_amdgcn_readfirstlane((int)tb[L * kTileDw * 4 + (i - b_r)]);
+                const int force = i > e_r ? 1 : i < o_r ? 2 : -1;
+                const int tmp = force < 0 && (uint32_t)(i - o_r) < (uint32_t)ncolB ? byte : 0;
+                const int op = backtrack_op(tmp, force, state);
+                i -= op != 1, j -= op != 2;
+                if (op == run_op) {
+                    ++run_len;
+                } else {
+                    if (run_len > 0 && lane == 0) cig[n] = (uint32_t)run_len << 4 | (uint32_t)run_op;
+                    if (run_len > 0) ++n;
+                    run_op = op, run_len = 1;
                 }
             }
-            const int h = L >> 6, Lh = L & (kWave - 1);
-            const int o_r = __builtin_amdgcn_readlane(h ? ro[1] : ro[0], Lh);
-            const int e_r = __builtin_amdgcn_readlane(h ? re[1] : re[0], Lh);
-            const int b_r = __builtin_amdgcn_readlane(h ? base[1] : base[0], Lh);
-            // (the row's byte is read whether or not it is used: the tile
-            // holds zeros outside the row, and i - b_r is within the tile)
-            const int byte = __builtin_amdgcn_readfirstlane((int)tb[L * kTileDw * 4 + (i - b_r)]);
-            const int force = i > e_r ? 1 : i < o_r ? 2 : -1;
-            const int tmp = force < 0 && (uint32_t)(i - o_r) < (uint32_t)ncolB ? byte : 0;
-            const int op = backtrack_op(tmp, force, state);
-            i -= op != 1, j -= op != 2;
-            if (op == run_op) {
-                ++run_len;
-            } else {
-                if (run_len > 0 && lane == 0) cig[n] = (uint32_t)run_len << 4 | (uint32_t)run_op;
-                if (run_len > 0) ++n;
-                run_op = op, run_len = 1;
-            }
+            if (lane == 0) at[turn][0] = i, at[turn][1] = j;
+            __syncthreads();
         }
+        if (wv > 0) return;
         // the tails merge with the last run (push of ksw_backtrack)
         if (i >= 0) {
             if (run_op == 2) run_len += i + 1;
@@ -679,7 +706,7 @@ __global__ void __launch_bounds__(64) ksw_general_backtrack_tiled_kernel(GenBack
             // lane 0's stores complete before the wave reads them back with
             // device-scope loads (past the CU's L1)
             __builtin_amdgcn_s_waitcnt(0xF70);  // vmcnt(0)
-            __syncthreads();
+            asm volatile("" ::: "memory");
             for (int x = lane; x < (n >> 1); x += kWave) {
                 const uint32_t lo = __hip_atomic_load(cig + x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 const uint32_t hi = __hip_atomic_load(cig + n - 1 - x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -688,7 +715,7 @@ __global__ void __launch_bounds__(64) ksw_general_backtrack_tiled_kernel(GenBack
             }
         }
     }
-    if (lane == 0) {
+    if (threadIdx.x == 0) {
         o.n_cigar = n;
         a.out[jb.out] = o;
     }
@@ -787,7 +814,7 @@ hipError_t launch_general_backtrack(const GenBacktrackArgs &a, hipStream_t st)
 {
     if (a.njobs <= 0) return hipSuccess;
     hipLaunchKernelGGL(ksw_general_backtrack_kernel, dim3((a.njobs + 63) / 64), dim3(64), 0, st, a);
-    hipLaunchKernelGGL(ksw_general_backtrack_tiled_kernel, dim3(a.njobs), dim3(64), 0, st, a);
+    hipLaunchKernelGGL(ksw_general_backtrack_tiled_kernel, dim3(a.njobs), dim3(kWave * kTileWaves), 0, st, a);
     return hipGetLastError();
 }
 

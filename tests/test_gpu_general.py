@@ -183,3 +183,23 @@ def test_wave_walk_on_every_pair(name, monkeypatch):
     test_scenarios_vs_oracle(name)
     if name == "band_narrow":
         test_golden_vectors_batched()
+
+
+@pytest.mark.parametrize("gap", [15, 17, 63, 64, 127, 128, 129, 260])
+def test_wave_walk_leaves_its_staged_tile(gap):
+    """Gaps around the size of a tile of rows, in both directions and back to
+    back: the path enters the next tile beside the one staged for it (which
+    holds 16 positions right of a diagonal path and 47 left of it), or beyond
+    it."""
+    rng = np.random.default_rng(510 + gap)
+    tuples = []
+    for k in range(8):
+        a, b, c = (W.random_seq(rng, int(rng.integers(100, 420))) for _ in range(3))
+        extra = W.random_seq(rng, gap)
+        q = np.concatenate([W.mutate(rng, a, 0.1, 0.02), extra, W.mutate(rng, b, 0.1, 0.02), c])
+        t = np.concatenate([a, b, W.random_seq(rng, gap) if k & 1 else extra[:0], c])
+        q, t = (q, t) if k & 2 else (t, q)
+        tuples.append((q, t, FLAGS[k // 4], 2 * gap + 40))
+    for (q, t, f, w), g in zip(tuples, ksw2.extd2_batch(tuples)):
+        r = O.run_oracle(q, t, flag=f, w=w)
+        assert same(g, r), f"qlen={len(q)} tlen={len(t)} w={w} flag={f:#x}: {diff(g, r)}"
