@@ -81,7 +81,7 @@ struct GenJob {
     int32_t tlenB, qlenB;      // lengths rounded up to 64
     int32_t out;               // slot in the output array
     int32_t r_end;             // band kernel: anti-diagonals the reference completes
-    uint64_t bnd_off;          // band kernel: dword offset of its two stripe buffers
+    uint64_t bnd_off;          // band kernel: dword offset of its control block and hand-off buffer
 };
 
 // State block of one general pair: ten int8 arrays of tlenB (u, y, y2, s and

@@ -232,11 +232,10 @@ def banded_leg(args) -> dict:
 
 
 def general_leg(args, pairs) -> dict:
-    """The general kernel's workload in AnchorWave: narrow bands, as the
-    score-certified path asks for (alignSlidingWindow.cpp:1297-1310 widens
-    the band from twice the length difference).  The fixed batch's pairs at
-    w = 256, below the band kernel's minimum width, through
-    ksw_extd2_hip_batch; GCUPS over in-band cells up to each band exit."""
+    """Narrow bands, as the score-certified path asks for
+    (alignSlidingWindow.cpp:1297-1310 widens the band from twice the length
+    difference; once the general kernel's workload, now the band kernel's).
+    The fixed batch's pairs at w = 256 through ksw_extd2_hip_batch; GCUPS over in-band cells up to each band exit."""
     w = args.general_w
     sub = pairs[: args.general]
     cells = sum(band_cells(len(q), len(t), w) for q, t in sub)
