@@ -306,6 +306,28 @@ int ksw2_hip_plan_graph(const ksw2_hip_plan *plan, int *runs, int *replays)
     return set_err(KSW2_HIP_OK);
 }
 
+int ksw2_hip_plan_facts(const ksw2_hip_plan *plan, ksw2_hip_plan_facts_t *facts)
+{
+    if (!plan || !facts) return set_err(KSW2_HIP_EINVAL);
+    const kswhip::Plan *p = plan->p;
+    *facts = {};
+    (p->thin ? facts->thin_pairs : facts->stripe_pairs) = p->n_fast;
+    facts->band_pairs = p->n_band, facts->general_pairs = p->n_gen - p->n_band;
+    facts->waiting = p->waiting, facts->one_workgroup = p->one_workgroup;
+    if (!p->started) return set_err(KSW2_HIP_OK);
+    if (p->n_wide > 0 && hipMemcpy(&facts->redone, p->d_werr, sizeof(int32_t), hipMemcpyDeviceToHost) != hipSuccess)
+        return set_err(KSW2_HIP_EDEVICE);
+    if (p->n_band > 0) {
+        std::vector<int32_t> redo(p->n_gen), order(p->n_band);
+        if (hipMemcpy(redo.data(), p->d_redo, sizeof(int32_t) * redo.size(), hipMemcpyDeviceToHost) != hipSuccess ||
+            hipMemcpy(order.data(), p->d_gorder + p->band_off, sizeof(int32_t) * order.size(), hipMemcpyDeviceToHost) !=
+                hipSuccess)
+            return set_err(KSW2_HIP_EDEVICE);
+        for (int32_t j : order) facts->redone += redo[j] != 0;
+    }
+    return set_err(KSW2_HIP_OK);
+}
+
 int ksw2_hip_plan_dirs(const ksw2_hip_plan *plan, int index, uint8_t *out, size_t bytes, int *R, int *transposed)
 {
     if (!plan || index < 0 || index >= plan->p->n) return set_err(KSW2_HIP_EINVAL);

@@ -1118,6 +1118,7 @@ int plan_launch(Plan *p, const Progress *prog)
     }
     if (p->h_stop && p->own_stop) *(volatile int32_t *)p->h_stop = 0;
     p->started = true, p->fetched = false;
+    p->waiting = p->one_workgroup = 0;
     const bool graphed = graph_eligible(p, prog);
     if (graphed && !p->graph && !p->graph_failed && p->runs >= 1) plan_capture(p);
     ++p->runs;
@@ -1178,6 +1179,7 @@ int plan_launch(Plan *p, const Progress *prog)
             std::lock_guard<std::mutex> lk(g_wait_mu);
             int q[2];
             if (!wait_slots_acquire(st, q)) return KSW2_HIP_EDEVICE;
+            p->waiting |= 2;
             for (const Plan::BLaunch &l : p->blaunches) {
                 ba.order = p->d_gorder + l.off, ba.njobs = l.count;
                 KSW_HIP_TRY(launch_band(ba, l.team, l.grp == 1, l.grp == 2, st));  // chunks of half the device
@@ -1202,13 +1204,15 @@ int plan_launch(Plan *p, const Progress *prog)
         // through one plan: 233 ms a call, 195 ms with both at once)
         hipStream_t st = lane(Plan::kWideLane);
         if (!st) return KSW2_HIP_EDEVICE;
-        if (!p->thin) KSW_HIP_TRY(clear_wide_err(p->d_werr, st));  // (the thin launches clear their own)
+        if (!p->thin) KSW_HIP_TRY(clear_wide_err(p->d_werr, st));  // (a run's first thin launch clears it)
+        bool clear_err = p->thin;
         bool wide_now = true;
         {
             std::lock_guard<std::mutex> lk(g_wait_mu);
             // spread pairs only: run wide only if two quarters are free now
             const bool no_spread = getenv("KSW2_HIP_SPREAD_FALLBACK") != nullptr;  // tests
             wide_now = !p->optional_wide || (!no_spread && wait_slots_free() >= 2);
+            p->waiting |= wide_now ? 1 : 0, p->one_workgroup = wide_now ? 0 : p->n_wide;
             if (wide_now) {
                 int q[2];
                 if (!wait_slots_acquire(st, q)) return KSW2_HIP_EDEVICE;
@@ -1219,7 +1223,8 @@ int plan_launch(Plan *p, const Progress *prog)
                     const int32_t *wfirst = p->h_wfirst.data() + l.wf;
                     if (p->thin) {
                         const int half = std::max(1, thin_capacity(l.grp, l.lut) / 2);
-                        KSW_HIP_TRY(launch_thin(sa, l.grp, l.lut, wfirst, half, 0, p->max_swept, st));
+                        KSW_HIP_TRY(launch_thin(sa, l.grp, l.lut, wfirst, half, 0, p->max_swept, clear_err, st));
+                        clear_err = false;
                     } else {
                         const int half = std::max(1, stripe_wide_capacity(l.grp, p->R, l.lut) / 2);
                         KSW_HIP_TRY(launch_stripe_wide(sa, l.grp, p->R, l.lut, wfirst, half, st));
@@ -1232,7 +1237,8 @@ int plan_launch(Plan *p, const Progress *prog)
             if (!l.wide) continue;
             sa.order = p->d_order + l.off, sa.njobs = l.count, sa.wctl = p->d_wctl + (int64_t)l.woff * kWideCtl;
             if (p->thin) {
-                if (!wide_now) KSW_HIP_TRY(launch_thin(sa, l.grp, l.lut, nullptr, 0, l.team, p->max_swept, st));
+                if (!wide_now) KSW_HIP_TRY(launch_thin(sa, l.grp, l.lut, nullptr, 0, l.team, p->max_swept, clear_err, st));
+                clear_err = false;
                 KSW_HIP_TRY(launch_thin_epilogue(sa, l.grp, l.lut, st));
             } else if (wide_now) KSW_HIP_TRY(launch_stripe_wide_epilogue(sa, l.grp, p->R, l.lut, st));
             else KSW_HIP_TRY(launch_stripe(sa, l.grp, l.team, p->R, l.lut, st));  // one-workgroup teams

@@ -171,11 +171,12 @@ int stripe_resident_waves(int group, int R = kRowsPerLane);
 // of kWideGroup waves (at most kThinMaxTeam waves), launched in chunks of at
 // most max_wgs workgroups, as launch_stripe_wide; null: one workgroup of
 // `team` waves per job, which waits on nothing outside itself.  kq: the
-// longest swept length.  launch_thin_epilogue then runs each job's epilogue.
+// longest swept length; clear_err: zero the plan's redo count first (a run's
+// first thin launch).  launch_thin_epilogue then runs each job's epilogue.
 constexpr int kThinMaxTeam = 1024;
 constexpr int kThinTeam = 8;  // waves of a job that has one workgroup, at most
 hipError_t launch_thin(const StripeArgs &a, int group, bool lut, const int32_t *h_wfirst, int max_wgs, int team, int kq,
-                       hipStream_t st);
+                       bool clear_err, hipStream_t st);
 hipError_t launch_thin_epilogue(const StripeArgs &a, int group, bool lut, hipStream_t st);
 // Workgroups of kWideGroup waves of the thin kernel the device holds at once.
 int thin_capacity(int group, bool lut);

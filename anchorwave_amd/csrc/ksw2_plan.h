@@ -266,6 +266,9 @@ struct Plan {
     bool stop_requested = false;     // the progress callback stopped the last run
     bool started = false;            // the last run launched (not stopped at r = 0)
     int max_diags = 0;               // largest qlen + tlen - 1 in the plan
+    // the last run: launches that took waiting-launch slots (1 stripe or
+    // thin, 2 band), wide pairs that ran on one workgroup for want of them
+    int waiting = 0, one_workgroup = 0;
 };
 
 struct PlanLanes {

@@ -690,14 +690,14 @@ ksw_thin_kernel(StripeArgs a)
 }
 
 // Clears the late words and column buffers of a launch's pairs (blockIdx.y
-// the pair) and the plan's redo count.
-__global__ void __launch_bounds__(256) ksw_thin_clear_kernel(StripeArgs a)
+// the pair) and, with clear_err, the plan's redo count.
+__global__ void __launch_bounds__(256) ksw_thin_clear_kernel(StripeArgs a, bool clear_err)
 {
     const KswJob &jb = a.jobs[a.order[blockIdx.y]];
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     clear_entries(a.bnd + jb.bnd_off, jb.qlen, t, gridDim.x * blockDim.x);
     if (t == 0) a.wctl[(int64_t)blockIdx.y * kWideCtl + kWideCtlLate] = 0;
-    if (t == 0 && blockIdx.y == 0) *a.werr = 0;
+    if (clear_err && t == 0 && blockIdx.y == 0) *a.werr = 0;
 }
 
 // The epilogue of a launch's pairs, one workgroup each, after all passes.  A
@@ -738,13 +738,14 @@ namespace {
 
 template <bool RIGHT, int MODE, bool LUT>
 struct Thin {
-    static hipError_t passes(const StripeArgs &a0, const int32_t *h_wfirst, int max_wgs, int team, int kq, hipStream_t st)
+    static hipError_t passes(const StripeArgs &a0, const int32_t *h_wfirst, int max_wgs, int team, int kq, bool clear_err,
+                             hipStream_t st)
     {
         StripeArgs a = a0;
         const dim3 clear((unsigned)std::min(std::max((kq + 1023) / 1024, 1), 64), 1);
         if (!h_wfirst) {
             a.wfirst = nullptr;
-            hipLaunchKernelGGL(ksw_thin_clear_kernel, dim3(clear.x, a.njobs), dim3(256), 0, st, a);
+            hipLaunchKernelGGL(ksw_thin_clear_kernel, dim3(clear.x, a.njobs), dim3(256), 0, st, a, clear_err);
             hipLaunchKernelGGL((ksw_thin_kernel<RIGHT, MODE, LUT>), dim3(a.njobs), dim3(kWave * team),
                                ring_bytes(team), st, a);
             return hipGetLastError();
@@ -758,7 +759,8 @@ struct Thin {
             a.order = a0.order + off, a.wfirst = a0.wfirst + off;
             a.wctl = a0.wctl + (int64_t)off * kWideCtl;
             a.njobs = end - off;
-            hipLaunchKernelGGL(ksw_thin_clear_kernel, dim3(clear.x, a.njobs), dim3(256), 0, st, a);
+            hipLaunchKernelGGL(ksw_thin_clear_kernel, dim3(clear.x, a.njobs), dim3(256), 0, st, a,
+                               clear_err && off == 0);
             hipLaunchKernelGGL((ksw_thin_kernel<RIGHT, MODE, LUT>), dim3(blocks), dim3(kWave * kWideGroup),
                                ring_bytes(kWideGroup), st, a);
             const hipError_t e = hipGetLastError();
@@ -800,7 +802,7 @@ template <class F> auto by_thin(int group, bool lut, F f)
 }  // namespace
 
 hipError_t launch_thin(const StripeArgs &a, int group, bool lut, const int32_t *h_wfirst, int max_wgs, int team, int kq,
-                       hipStream_t st)
+                       bool clear_err, hipStream_t st)
 {
     if (a.njobs <= 0) return hipSuccess;
     if (!a.wctl || !a.werr || group < 0 || group >= kGroups || a.njobs > 65535) return hipErrorInvalidValue;
@@ -813,7 +815,7 @@ hipError_t launch_thin(const StripeArgs &a, int group, bool lut, const int32_t *
     } else if (team < 1 || team > kThinTeam) {
         return hipErrorInvalidValue;
     }
-    return by_thin(group, lut, [&](auto v) { return v.passes(a, h_wfirst, max_wgs, team, kq, st); });
+    return by_thin(group, lut, [&](auto v) { return v.passes(a, h_wfirst, max_wgs, team, kq, clear_err, st); });
 }
 
 hipError_t launch_thin_epilogue(const StripeArgs &a, int group, bool lut, hipStream_t st)

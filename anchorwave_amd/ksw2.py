@@ -63,6 +63,7 @@ EXPORTS = (
     "ksw2_hip_plan_graph",
     "ksw2_hip_plan_destroy",
     "ksw2_hip_plan_dirs",
+    "ksw2_hip_plan_facts",
     "ksw2_hip_certify_batch",
     "ksw2_hip_certify_free",
     "ksw2_hip_window_batch",
@@ -187,6 +188,8 @@ def lib():
         L.ksw2_hip_plan_dirs.argtypes = [C.c_void_p, C.c_int, C.c_void_p, C.c_size_t, C.POINTER(C.c_int),
                                          C.POINTER(C.c_int)]
         L.ksw2_hip_plan_dirs.restype = C.c_int
+        L.ksw2_hip_plan_facts.argtypes = [C.c_void_p, C.POINTER(PlanFacts)]
+        L.ksw2_hip_plan_facts.restype = C.c_int
         L.ksw2_hip_certify_batch.argtypes = [C.c_int, C.POINTER(CertifyTask), C.c_int32, C.c_int32, C.c_int32,
                                              C.c_int32, C.c_int32, C.c_double, C.POINTER(CertifyResult)]
         L.ksw2_hip_certify_batch.restype = C.c_int
@@ -522,6 +525,11 @@ def _pair_array(pairs, w=-1, zdrop=-1, end_bonus=0, flag=0):
     return arr, keep
 
 
+class PlanFacts(C.Structure):
+    _fields_ = [(k, C.c_int32) for k in ("thin_pairs", "stripe_pairs", "band_pairs", "general_pairs", "waiting",
+                                         "one_workgroup", "redone")]
+
+
 class Plan:
     """A device-resident batch (``ksw2_hip_plan_*``): upload once, run many
     times, fetch results.  Used by the benchmark to time device work with the
@@ -556,6 +564,14 @@ class Plan:
         if st != 0:
             raise KswError(f"ksw2_hip_plan_graph: {STATUS.get(st, st)}")
         return runs.value, rep.value
+
+    def facts(self) -> dict:
+        """The kernels the pairs take, and how the last run went."""
+        f = PlanFacts()
+        st = lib().ksw2_hip_plan_facts(self.h, C.byref(f))
+        if st != 0:
+            raise KswError(f"ksw2_hip_plan_facts: {STATUS.get(st, st)}")
+        return {k: getattr(f, k) for k, _ in PlanFacts._fields_}
 
     def fetch(self, timing: dict = None) -> List[Result]:
         """``ksw2_hip_plan_fetch`` into ``ksw_extz_t`` structs, as Results.

@@ -402,6 +402,17 @@ void ksw2_hip_window_free(int n, ksw2_window_result_t *results);
 int ksw2_hip_plan_dirs(const ksw2_hip_plan *plan, int index, uint8_t *out, size_t bytes, int *R,
                        int *transposed);
 
+/* Diagnostics: the kernels a plan's pairs take, and how its last run (a
+ * graph replay too) went. */
+typedef struct {
+    int32_t thin_pairs, stripe_pairs, band_pairs, general_pairs;
+    int32_t waiting;        /* launches whose workgroups wait on one another took a share of the device:
+                             * 1 thin or stripe launches, 2 band launches, 3 both */
+    int32_t one_workgroup;  /* pairs laid out for several workgroups that ran on one, no share being free */
+    int32_t redone;         /* pairs computed again because a wait gave up */
+} ksw2_hip_plan_facts_t;
+int ksw2_hip_plan_facts(const ksw2_hip_plan *plan, ksw2_hip_plan_facts_t *facts);
+
 #ifdef __cplusplus
 }
 #endif

@@ -1,0 +1,72 @@
+"""What a plan's last run did (ksw2_hip_plan_facts), for the launches whose
+results are the same whichever way they go: the kernel, whether waiting
+workgroups took their share of the device or one workgroup ran each pair, and
+how many pairs were computed again."""
+import numpy as np
+import pytest
+
+import oracle_py as O
+from anchorwave_amd import ksw2, workloads as W
+from helpers import diff, random_pairs, same
+
+pytestmark = pytest.mark.gpu
+
+FLAGS = [0, ksw2.KSW_EZ_RIGHT, ksw2.KSW_EZ_SCORE_ONLY, ksw2.KSW_EZ_SINGLETRACK]
+
+
+def _mixed(seed, n=8, hi=2600):
+    """Pairs of every launch group in one plan."""
+    return [(q, t, FLAGS[k % 4]) for k, (q, t) in enumerate(random_pairs(seed, n, 200, hi))]
+
+
+def _run(tuples, runs=1):
+    plan = ksw2.Plan(tuples)
+    for _ in range(runs):
+        plan.run()
+    got, facts = plan.fetch(), plan.facts()
+    plan.close()
+    for k, (tup, g) in enumerate(zip(tuples, got)):
+        r = O.run_oracle(tup[0], tup[1], flag=tup[2], w=tup[3] if len(tup) > 3 else -1)
+        assert same(g, r), f"pair {k}: {diff(g, r)}"
+    return facts
+
+
+def test_thin_plan_takes_its_share():
+    f = _run(_mixed(700))
+    assert (f["thin_pairs"], f["stripe_pairs"], f["waiting"], f["one_workgroup"], f["redone"]) == (8, 0, 1, 0, 0)
+
+
+def test_thin_plan_on_one_workgroup(monkeypatch):
+    monkeypatch.setenv("KSW2_HIP_SPREAD_FALLBACK", "1")
+    f = _run(_mixed(701))
+    assert (f["thin_pairs"], f["waiting"], f["one_workgroup"], f["redone"]) == (8, 0, 8, 0)
+
+
+@pytest.mark.parametrize("runs", [1, 3])
+@pytest.mark.parametrize("fallback", [False, True])
+def test_every_redone_pair_is_counted(fallback, runs, monkeypatch):
+    """Over several thin launches of one run (a group each), and a run at a time."""
+    monkeypatch.setenv("KSW2_HIP_WIDE_REDO", "1")
+    if fallback:
+        monkeypatch.setenv("KSW2_HIP_SPREAD_FALLBACK", "1")
+    f = _run(_mixed(702), runs)
+    assert (f["thin_pairs"], f["redone"]) == (8, 8)
+
+
+def test_thin_limit():
+    """96 pairs of four workgroups each are the last plan on the thin kernel
+    (a query longer than 2,048 would make it five)."""
+    pairs = [(q[:2000], t, 0) for q, t in W.fixed(seed=8, n=97)]
+    assert _run(pairs[:96])["thin_pairs"] == 96
+    assert _run(pairs)["stripe_pairs"] == 97
+
+
+def test_band_redo_is_counted(monkeypatch):
+    monkeypatch.setenv("KSW2_HIP_BAND_REDO", "1")
+    rng = np.random.default_rng(703)
+    tuples = []
+    for k in range(4):
+        t = W.random_seq(rng, 1500)
+        tuples.append((W.mutate(rng, t, 0.1, 0.02), t, FLAGS[k % 3], 700))
+    f = _run(tuples)
+    assert (f["band_pairs"], f["general_pairs"], f["redone"]) == (4, 0, 4)
