@@ -104,7 +104,7 @@ bool normalise_scoring(int8_t m, const int8_t *mat, int8_t q, int8_t e, int8_t q
     bool ok = q >= 0 && e > e2 && q2 >= 0 && e2 >= 0 && mat[0] == 0 && mis <= 0;
     ok = ok && 2 * G1 <= 128 && G1 + G2 <= 128 && G1 + e2 <= 128 && q2 - mis <= 128 && 2 * G1 - q <= 128;
     ok = ok && G2 <= 127 && long_diff >= -128 && long_diff <= 127;
-    cls->fast_ok = ok;
+    cls->fast_ok = ok, cls->G1 = G1;
     return true;
 }
 

@@ -462,6 +462,19 @@ void make_gen_score(int8_t m, const int8_t *mat, const KswScore &sc, const Score
     for (int k = 0; k < m * m && k < kMaxM * kMaxM; ++k) g->mat[k] = mat[k];
 }
 
+// Waves of a banded pair: as many as it has stripes in flight, which is a
+// stripe's anti-diagonals (2w + 2 * 128, and the starts and ends of blocks)
+// over the 256 that its start trails the one above it by, with a margin for
+// what the hand-offs add.
+static int band_team(int w, int tlenB)
+{
+    const char *bt = getenv("KSW2_HIP_BAND_TEAM");  // forces a team size (tests)
+    if (bt) return std::max(1, std::min(kBandTeam, atoi(bt)));
+    const int64_t flight = (2 * (int64_t)w + 420) / 256 + 1;
+    const int team = (int)std::min<int64_t>({flight, (tlenB + kBandStripe - 1) / kBandStripe, kBandTeam});
+    return team > kBandGroup ? (team + kBandGroup - 1) / kBandGroup * kBandGroup : team;
+}
+
 // The band kernel's domain, whatever the band's width: the pair's only
 // departure from the stripe kernel's is a band narrower than the matrix, no
 // Singletrack (KSW2_HIP_BAND=0 or KSW2_HIP_FORCE_GENERAL: none).
@@ -472,11 +485,18 @@ bool band_domain(const ksw2_pair_t &p, int8_t m, const ScoreClass &cls)
     const char *fg = getenv("KSW2_HIP_FORCE_GENERAL");
     if (fg && atoi(fg) > 0) return false;
     if (p.flag & KSW_EZ_SINGLETRACK) return false;
-    // the hand-off counts, a wave's stripes times (qlen + tlen + 63), and H,
-    // held as -8 H + p r with p <= 8 * 128 + 8, must fit int32
-    const int64_t nstripes = ((int64_t)p.tlen + 63) / 64 * 64 / 256 + 1;
-    if ((nstripes + 1) * ((int64_t)p.qlen + p.tlen + 63) >= INT32_MAX) return false;
-    if (2080ll * band_r_end(p.qlen, p.tlen, norm_w(p)) >= INT32_MAX) return false;
+    // int32 holds the hand-off counts, a wave's stripes times (qlen + tlen +
+    // 63), and H, kept as -8 H + p r with p <= 8 G1 + 8: u and v are in
+    // [-G1, G1], stale or not (z >= y + u with y >= -G1, and z <= 0), so an
+    // anti-diagonal adds at most 16 G1 + 8: 12 M anti-diagonals with gap
+    // scores of 8/2 (G1 = 10), 2 M with the largest ones (G1 = 64).  The
+    // counts, of a team's two waves or more, end at 524 kbp of both.
+    const int64_t nr = (int64_t)p.qlen + p.tlen - 1;
+    if (nr + 64 >= INT32_MAX) return false;
+    const int tlenB = (p.tlen + 63) / 64 * 64, team = std::min(band_team(norm_w(p), tlenB), 2);
+    const int64_t stripes = (tlenB + kBandStripe - 1) / kBandStripe;
+    if ((stripes + team - 1) / team * (nr + 64) >= INT32_MAX) return false;
+    if (16ll * (cls.G1 + 1) * (band_r_end(p.qlen, p.tlen, norm_w(p)) + 128ll) >= INT32_MAX) return false;
     return fast_path_reject(p, m, cls) == kRejBand;
 }
 
@@ -780,14 +800,8 @@ int plan_create(Plan **out, const ksw2_pair_t *pairs, const int *idx, int nidx, 
                                         t >= 512 ? 0 : t >= 256 ? 1 : 2});
                 gorder.insert(gorder.end(), members.begin(), members.end());
             }
-        // band-kernel launches: per group and team, longest first.  A team has
-        // as many waves as the pair has stripes in flight: a stripe's
-        // anti-diagonals (2w + 2 * 128, and the starts and ends of blocks) over
-        // the 256 that its start trails the one above it by, with a margin for
-        // what the hand-offs add.
+        // band-kernel launches: per group and team (band_team), longest first.
         p->band_off = (int)gorder.size();
-        const char *bt = getenv("KSW2_HIP_BAND_TEAM");  // forces a team size (tests)
-        const int band_team = bt ? std::max(1, std::min(kBandTeam, atoi(bt))) : 0;
         // A group whose pairs would all find a SIMD per wave at its largest team
         // takes that one, in one launch: launches follow one another.
         std::map<std::pair<int, int>, std::vector<int>> teams;  // by group and (negated) team
@@ -796,12 +810,7 @@ int plan_create(Plan **out, const ksw2_pair_t *pairs, const int *idx, int nidx, 
             if (!band[gk]) continue;
             const GenJob &j = p->gjobs[gk];
             const int g = (j.flag & KSW_EZ_SCORE_ONLY) ? 2 : (j.flag & KSW_EZ_RIGHT) ? 1 : 0;
-            int tm = band_team;
-            if (!tm) {
-                const int64_t flight = (2 * (int64_t)j.w + 420) / 256 + 1;
-                tm = (int)std::min<int64_t>({flight, (j.tlenB + kBandStripe - 1) / kBandStripe, kBandTeam});
-                if (tm > kBandGroup) tm = (tm + kBandGroup - 1) / kBandGroup * kBandGroup;
-            }
+            const int tm = band_team(j.w, j.tlenB);
             teams[{g, -tm}].push_back(gk);
             team_max[g] = std::max(team_max[g], tm), ++members_of[g];
         }

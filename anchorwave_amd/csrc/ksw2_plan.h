@@ -16,6 +16,7 @@ struct ScoreClass {
     bool fast_ok;     // scoring for which the fast kernel is exact
     int m;
     int sc_N;         // wildcard score of the match/mismatch mode
+    int G1;           // KswScore::G1
 };
 
 bool normalise_scoring(int8_t m, const int8_t *mat, int8_t q, int8_t e, int8_t q2, int8_t e2, KswScore *sc,
