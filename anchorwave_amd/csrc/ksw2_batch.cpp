@@ -1184,17 +1184,23 @@ int plan_launch(Plan *p, const Progress *prog)
         ba.force_redo = fr && atoi(fr) > 0 ? 1 : 0;
         hipStream_t st = lane(0);
         if (!st) return KSW2_HIP_EDEVICE;
-        {
+        auto launch = [&](const Plan::BLaunch &l) {
+            ba.order = p->d_gorder + l.off, ba.njobs = l.count;
+            return launch_band(ba, l.team, l.grp == 1, l.grp == 2, st);
+        };
+        // (a pair of one workgroup waits for no other: it needs no share)
+        auto waits = [](const Plan::BLaunch &l) { return l.team > kBandGroup; };
+        if (std::any_of(p->blaunches.begin(), p->blaunches.end(), waits)) {
             std::lock_guard<std::mutex> lk(g_wait_mu);
             int q[2];
             if (!wait_slots_acquire(st, q)) return KSW2_HIP_EDEVICE;
             p->waiting |= 2;
-            for (const Plan::BLaunch &l : p->blaunches) {
-                ba.order = p->d_gorder + l.off, ba.njobs = l.count;
-                KSW_HIP_TRY(launch_band(ba, l.team, l.grp == 1, l.grp == 2, st));  // chunks of half the device
-            }
+            for (const Plan::BLaunch &l : p->blaunches)
+                if (waits(l)) KSW_HIP_TRY(launch(l));  // chunks of half the device
             if (!wait_slots_release(st, q)) return KSW2_HIP_EDEVICE;
         }
+        for (const Plan::BLaunch &l : p->blaunches)
+            if (!waits(l)) KSW_HIP_TRY(launch(l));
         // pairs whose waves gave up a wait run on the general kernel, on the
         // same stream
         ga.order = p->d_gorder + p->band_off, ga.njobs = p->n_band, ga.ring = 0, ga.only_if = p->d_redo;

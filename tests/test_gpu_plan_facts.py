@@ -70,3 +70,26 @@ def test_band_redo_is_counted(monkeypatch):
         tuples.append((W.mutate(rng, t, 0.1, 0.02), t, FLAGS[k % 3], 700))
     f = _run(tuples)
     assert (f["band_pairs"], f["general_pairs"], f["redone"]) == (4, 0, 4)
+
+
+@pytest.mark.parametrize("w,ql,share", [(100, 1500, 0), (301, 1500, 0), (302, 1500, 2), (700, 1500, 2), (700, 500, 0)])
+def test_bands_of_one_workgroup_take_no_share(w, ql, share):
+    """Bands whose stripes in flight (or whose stripes) fit four waves."""
+    rng = np.random.default_rng(704)
+    tuples = []
+    for k in range(6):
+        t = W.random_seq(rng, ql)
+        tuples.append((W.mutate(rng, t, 0.1, 0.02), t, FLAGS[k % 3], min(w, ql - 100)))
+    f = _run(tuples)
+    assert (f["band_pairs"], f["waiting"]) == (6, share)
+
+
+def test_bands_of_one_and_of_several_workgroups():
+    """One plan of both, in groups large enough to keep their teams apart."""
+    rng = np.random.default_rng(705)
+    tuples = []
+    for k in range(220):
+        t = W.random_seq(rng, 800)
+        tuples.append((W.mutate(rng, t, 0.1, 0.02), t, FLAGS[k % 2], 60 if k % 4 < 2 else 420))
+    f = _run(tuples)
+    assert (f["band_pairs"], f["waiting"]) == (220, 2)
