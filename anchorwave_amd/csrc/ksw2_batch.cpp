@@ -705,8 +705,12 @@ int plan_create(Plan **out, const ksw2_pair_t *pairs, const int *idx, int nidx, 
         }
         auto wide = [&](int k) { return wide_forced > 0 || team[k] > kMaxTeam || spread[k]; };
         p->optional_wide = !(env && env->thin);
+        // (a thin pair of more than 16 passes of four rows per lane, which the
+        // stripe kernel would lay out wide, waits its turn like a wide one: in
+        // one workgroup of eight waves calls of 40 kbp from four threads ran
+        // at 15 a second, in turn at 41, on wide stripe teams at 29)
         for (int k = 0; k < p->n_fast; ++k)
-            if (wide(k) && !spread[k]) p->optional_wide = false;
+            if (wide(k) && (!spread[k] || (p->thin && pass_count(p->jobs[k].tlen, 4) > kMaxTeam))) p->optional_wide = false;
         auto longest_first = [&](std::vector<int> &m) {
             auto steps = [&](int k) {
                 const KswJob &j = p->jobs[k];

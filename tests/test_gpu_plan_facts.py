@@ -93,3 +93,16 @@ def test_bands_of_one_and_of_several_workgroups():
         tuples.append((W.mutate(rng, t, 0.1, 0.02), t, FLAGS[k % 2], 60 if k % 4 < 2 else 420))
     f = _run(tuples)
     assert (f["band_pairs"], f["waiting"]) == (220, 2)
+
+
+@pytest.mark.parametrize("tlen,share", [(8100, 0), (8192, 0), (8193, 1), (9000, 1)])
+def test_long_thin_pairs_wait_for_a_share(tlen, share, monkeypatch):
+    """Pairs of up to 8,192 rows run on one workgroup when no share is free,
+    longer ones wait for one: on one workgroup they would take several times
+    as long."""
+    monkeypatch.setenv("KSW2_HIP_SPREAD_FALLBACK", "1")
+    rng = np.random.default_rng(tlen)
+    t = W.random_seq(rng, tlen)
+    q = np.resize(W.mutate(rng, t, 0.05, 0.01), 8000)
+    f = _run([(q, t, ksw2.KSW_EZ_SCORE_ONLY)])
+    assert (f["thin_pairs"], f["waiting"], f["one_workgroup"]) == (1, share, 1 - share)
