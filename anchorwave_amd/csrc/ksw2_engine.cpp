@@ -179,7 +179,7 @@ struct Engine::Flight {
     std::vector<char> delivered;
     int undelivered_fast = 0;
     int stream = 0;
-    bool thin = false;              // on the thin kernel
+    double thin_s = 0;              // > 0: on the thin kernel, its predicted seconds
     double cells = 0, t_start = 0;  // for the statistics
     uint64_t bytes = 0;             // footprints admitted, less direction bytes given back at delivery
 };
@@ -717,6 +717,25 @@ static int team_for(int passes, double steps, bool general, double T, int cap)
     return team > kMaxTeam ? (team + kWideGroup - 1) / kWideGroup * kWideGroup : team;
 }
 
+// A task's predicted seconds on the thin kernel: a column and the lag of each
+// 128 rows in 0.13 us steps, and the walk.
+double Engine::thin_seconds(const Task *t)
+{
+    const StripeGeom g = stripe_geom(t->pair);
+    return 1e-6 * (0.13 * (g.kq + 170.0 * thin_passes(g.kt)) + 0.03 * ((double)g.kq + g.kt));
+}
+
+// And on a team of one wave per pass at eight rows per lane: a step takes 0.51
+// us on a wave alone on its SIMD, 0.43 for each where they share one (a
+// workgroup of up to 16 waves has four SIMDs).
+double Engine::team_seconds(const Task *t)
+{
+    const StripeGeom g = stripe_geom(t->pair);
+    const int share = t->passes <= kMaxTeam ? (t->passes + 3) / 4 : 1;
+    return 1e-6 * (std::max(0.51, 0.43 * share) * (g.kq + 208.0 * std::min(t->passes, kMaxWide)) +
+                   0.03 * ((double)g.kq + g.kt));
+}
+
 // Forms and launches flights while streams, waves and memory allow: each free
 // stream takes the waiting tasks of its size class, in queue order, as far as
 // pool memory and the waves allow; tasks that do not fit are passed over for
@@ -741,24 +760,9 @@ bool Engine::admit_locked(std::unique_lock<std::mutex> &lk)
         // shorter tasks when no long ones wait, the others never take long ones
         static const int pref[kClasses][kClasses] = {{0, 1, -1}, {1, 0, -1}, {2, 1, 0}};
         const int own = batch_ ? kBatchStreamClass[s % 4] : stream_class_[s];
-        int cls = -1;
-        for (int k = 0; k < kClasses && pref[own][k] >= 0; ++k)
-            if (!queue_[pref[own][k]].empty()) {
-                cls = pref[own][k];
-                break;
-            }
-        if (cls < 0) continue;
-        std::deque<Task *> &q = queue_[cls];
-        auto *pool = static_cast<FirstFitPool *>(pool_.get());
-        const uint64_t share = (uint64_t)(kFlightShare[cls] * (double)budget_);
-        const uint64_t free_block = pool->largest_free();
-        const uint64_t avail = std::min(free_block, share);
         // per-wave step budget: work queued and in flight over the device's waves
         const double T = std::max(1.0, (queued_steps_ + inflight_steps_) / resident_waves_);
         const int cap = (int)std::min<int64_t>(free_waves, max_team_);
-        const Task *head = q.front();
-        const int key = batch_ ? (head->general ? 0 : -1) : team_for(head->passes, head->steps, head->general, T, cap);
-        const double span = key > 0 ? head->steps / key : 0;  // the head's steps per wave
         // Serving flights whose teams are capped by the pairs' pass count (the
         // device has waves to spare) run on the thin kernel, where a pair's
         // time is its columns and a lag per 128 rows: at most two such flights
@@ -776,15 +780,54 @@ bool Engine::admit_locked(std::unique_lock<std::mutex> &lk)
         };
         size_t waiting = 0;
         for (const auto &w : queue_) waiting += w.size();
-        bool thin = !batch_ && thin_ && capped(head) && thin_groups(head->pair) <= kThinGroups &&
-                    (2 * head->passes > kMaxTeam || (int64_t)waiting * thin_groups(head->pair) <= kThinGroups);
-        if (thin) {
-            int running = 0;
-            for (const auto &f : flights_) running += f->thin;
-            if (running >= 2) continue;
-            thin = wait_slots_idle();
+        auto wants_thin = [&](const Task *t) {
+            return !batch_ && thin_ && capped(t) && thin_groups(t->pair) <= kThinGroups &&
+                   (2 * t->passes > kMaxTeam || (int64_t)waiting * thin_groups(t->pair) <= kThinGroups);
+        };
+        // While two thin flights run, a task that wants a third is passed over
+        // if the first of them to end, and the task's own time on the thin
+        // kernel, come before its team would be done, or if that is wide and
+        // waits for a share of the device itself; otherwise it runs on its team
+        // now.  Either way the tasks behind it get their turn (the other
+        // classes have streams of their own).  The burst of 256 tasks takes 16-19
+        // ms on four hardware queues and 13-16 on sixteen, 17-24 and 16-21 when
+        // the stream's whole class waited for a third flight's turn.
+        const double now = now_s();
+        int thin_running = 0;
+        double thin_wait = 0;  // seconds until one of them ends, as predicted (one that is late: as late again)
+        for (const auto &f : flights_)
+            if (f->thin_s > 0) {
+                const double left = std::abs(f->thin_s - (now - f->t_start));
+                thin_wait = thin_running++ ? std::min(thin_wait, left) : left;
+            }
+        auto held_back = [&](const Task *t) {
+            return thin_running >= 2 && wants_thin(t) &&
+                   (t->passes > kMaxTeam || thin_wait + thin_seconds(t) <= team_seconds(t));
+        };
+        int cls = -1;
+        Task *head = nullptr;
+        for (int k = 0; k < kClasses && pref[own][k] >= 0; ++k)
+            if (!queue_[pref[own][k]].empty()) {
+                cls = pref[own][k];
+                break;
+            }
+        if (cls < 0) continue;
+        int passed = 0;
+        for (Task *t : queue_[cls]) {
+            if (!held_back(t)) head = t;
+            if (head || ++passed > backfill_) break;
         }
+        if (!head) continue;
+        std::deque<Task *> &q = queue_[cls];
+        auto *pool = static_cast<FirstFitPool *>(pool_.get());
+        const uint64_t share = (uint64_t)(kFlightShare[cls] * (double)budget_);
+        const uint64_t free_block = pool->largest_free();
+        const uint64_t avail = std::min(free_block, share);
+        const int key = batch_ ? (head->general ? 0 : -1) : team_for(head->passes, head->steps, head->general, T, cap);
+        const double span = key > 0 ? head->steps / key : 0;  // the head's steps per wave
+        const bool thin = thin_running < 2 && wants_thin(head) && wait_slots_idle();
         int64_t groups = 0;
+        double thin_s = 0;
         std::vector<Task *> pick;
         uint64_t bytes = kPlanSlack, seq = 0, cigw = 0;
         int64_t waves = 0;
@@ -795,6 +838,7 @@ bool Engine::admit_locked(std::unique_lock<std::mutex> &lk)
             // serving: one team size (one launch) and similar durations per
             // flight; batch: general and stripe pairs in flights of their own
             const bool same = batch_ ? (key == 0) == t->general
+                              : held_back(t) ? false
                               : thin ? capped(t) && chain(t) <= 2 * chain(head) && 2 * chain(t) >= chain(head) &&
                                            groups + thin_groups(t->pair) <= kThinGroups
                                      : team_for(t->passes, t->steps, t->general, T, cap) == key &&
@@ -817,7 +861,7 @@ bool Engine::admit_locked(std::unique_lock<std::mutex> &lk)
             }
             pick.push_back(t);
             t->held = w;
-            if (thin) groups += thin_groups(t->pair);
+            if (thin) groups += thin_groups(t->pair), thin_s = std::max(thin_s, thin_seconds(t));
             bytes += t->footprint, waves += w, steps += t->steps, seq += (uint64_t)t->pair.qlen + t->pair.tlen + 32;
             cigw += ((uint64_t)t->pair.qlen + t->pair.tlen + 2 + 15) / 16 * 16;
             it = q.erase(it);
@@ -869,7 +913,7 @@ bool Engine::admit_locked(std::unique_lock<std::mutex> &lk)
         }
         auto f = std::make_unique<Flight>();
         f->tasks = pick;
-        f->stream = s, f->thin = thin;
+        f->stream = s, f->thin_s = thin_s;
         for (const Task *tk : pick) f->cells += tk->cells;
         for (Task *t : pick) f->pairs.push_back(t->pair);
         busy_[s] = true;

@@ -102,6 +102,8 @@ private:
     bool reap_locked(std::unique_lock<std::mutex> &lk);
     bool admit_locked(std::unique_lock<std::mutex> &lk);
     bool queues_empty() const;
+    static double thin_seconds(const Task *t);
+    static double team_seconds(const Task *t);
     void stop_all_locked();
 
     int8_t m_;
