@@ -1632,8 +1632,11 @@ bool PinnedBuffer::grow(uint64_t want)
 {
     if (want <= bytes) return true;
     drop();
-    const uint64_t n = std::max<uint64_t>(want < kPinnedKeep / 2 ? want + want / 4 : want, 1u << 16);
+    uint64_t n = std::max<uint64_t>(want < kPinnedKeep / 2 ? want + want / 4 : want, 1u << 16);
+    if (getenv("KSW2_HIP_FAIL_PINNED")) n = 1ull << 60;  // tests: more than there is
     if (hipHostMalloc((void **)&base, n, hipHostMallocDefault) != hipSuccess) {
+        // (the callers do without: the launches that follow read this error)
+        (void)hipGetLastError();
         base = nullptr;
         return false;
     }
