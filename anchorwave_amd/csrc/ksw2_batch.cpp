@@ -8,6 +8,7 @@
 #include <string.h>
 
 #include <algorithm>
+#include <atomic>
 #include <map>
 #include <memory>
 #include <chrono>
@@ -1546,23 +1547,33 @@ namespace {
 // hipFree and hipHostFree wait for the device.  (A batch of 64 pairs of 1 kbp,
 // one round of the sliding window: 1.0 ms a call with its own block, streams,
 // events and six copies, 0.5 so.)  Given back when the thread ends, or by
-// ksw2_hip_release_cached_memory on the thread.
+// ksw2_hip_release_cached_memory on the thread.  Batches grow what a thread
+// keeps beyond its single calls only while all threads together keep no more
+// than kBlocksKeep and kPinnedAllKeep: past that a batch gives back at its end
+// what it took (executor threads of one program, a GiB each, would otherwise
+// hold it until they end).
 constexpr uint64_t kCallBlockMax = 1ull << 30, kPinnedKeep = 256ull << 20;
+constexpr uint64_t kBlocksKeep = 8ull << 30, kPinnedAllKeep = 2ull << 30;
+std::atomic<uint64_t> g_blocks{0}, g_pinned{0};  // bytes the threads' contexts hold
 
 struct GrowPool : DevicePool {
+    bool lone = false;    // the call in progress is a single one
+    uint64_t single = 0;  // the largest block a single call asked for
     // one plan at a time; a larger one replaces the block (the previous
     // call's work has finished: every call waits for its plan)
     bool alloc(uint64_t n, uint64_t *off) override
     {
         if (n > bytes) {
-            if (base) (void)hipFree(base);
-            base = nullptr, bytes = 0;
-            if (hipMalloc(&base, n) != hipSuccess) {
+            drop();
+            const char *fb = getenv("KSW2_HIP_FAIL_BLOCK");  // tests: blocks of this many bytes cannot be had
+            if (hipMalloc(&base, fb && n >= strtoull(fb, nullptr, 10) ? 1ull << 60 : n) != hipSuccess) {
+                (void)hipGetLastError();
                 base = nullptr;
                 return false;
             }
-            bytes = n;
+            bytes = n, g_blocks += n;
         }
+        if (lone) single = std::max(single, n);
         *off = 0;
         return true;
     }
@@ -1570,7 +1581,8 @@ struct GrowPool : DevicePool {
     void drop()
     {
         if (base) (void)hipFree(base);
-        base = nullptr, bytes = 0;
+        g_blocks -= bytes;
+        base = nullptr, bytes = 0, single = 0;
     }
 };
 
@@ -1617,12 +1629,18 @@ thread_local CallContext t_call;
 // A call's use of its thread's context.
 struct ContextUse {
     const bool held;
-    ContextUse() : held(!t_call.busy && t_call.prepare()) { t_call.busy |= held; }
+    explicit ContextUse(bool lone) : held(!t_call.busy && t_call.prepare())
+    {
+        if (held) t_call.busy = true, t_call.pool.lone = lone;
+        else if (!t_call.busy) (void)hipGetLastError();  // (the call does without)
+    }
     ~ContextUse()
     {
         if (!held) return;
         t_call.busy = false;
-        if (t_call.pinned.bytes > kPinnedKeep) t_call.pinned.drop();
+        const bool batch = !t_call.pool.lone;
+        if (t_call.pinned.bytes > kPinnedKeep || (batch && g_pinned > kPinnedAllKeep)) t_call.pinned.drop();
+        if (batch && t_call.pool.bytes > t_call.pool.single && g_blocks > kBlocksKeep) t_call.pool.drop();
     }
 };
 
@@ -1640,13 +1658,14 @@ bool PinnedBuffer::grow(uint64_t want)
         base = nullptr;
         return false;
     }
-    bytes = n;
+    bytes = n, g_pinned += n;
     return true;
 }
 
 void PinnedBuffer::drop()
 {
     if (base) (void)hipHostFree(base);
+    g_pinned -= bytes;
     base = nullptr, bytes = 0;
 }
 
@@ -1698,39 +1717,55 @@ int run_batch_host(int n, const ksw2_pair_t *pairs, int8_t m, const int8_t *mat,
     std::unique_ptr<DevicePool> big;
     if (!small && total > kCallBlockMax && total <= mem_budget(true)) big = cached_block_pool(mem_budget(true), total);
     if (small || big || total <= mem_budget(false)) {
-        // one plan holds the whole batch; a single pair up to kCallBlockMax
-        // runs in the thread's cached context
+        // one plan holds the whole batch, in the thread's context and, up to
+        // kCallBlockMax, its block
         if (todo.empty()) return status;
-        Plan *plan = nullptr;
-        PlanEnv env;
-        const PlanEnv *use = nullptr;
-        if (big) {
-            env.pool = big.get();
-            env.spread = true;  // a plan of its own
-            use = &env;
+        bool no_memory = false;  // for the plan itself
+        auto one_plan = [&]() -> int {
+            Plan *plan = nullptr;
+            PlanEnv env;
+            const PlanEnv *use = nullptr;
+            if (big) {
+                env.pool = big.get();
+                env.spread = true;  // a plan of its own
+                use = &env;
+            }
+            const ContextUse context(todo.size() == 1);
+            if (context.held) {
+                if (total <= kCallBlockMax) env.pool = &t_call.pool;
+                env.stream = t_call.stream;
+                // (a lone pair has one launch at a time: its lanes would only add
+                // events)
+                if (todo.size() > 1) env.lanes = &t_call.lanes;
+                env.events = t_call.ev;
+                env.pinned = &t_call.pinned;
+                env.h_stop = t_call.h_stop, env.d_stop = t_call.d_stop;
+                env.spread = true;  // a plan of its own: 5-16 wave teams may spread over CUs
+                use = &env;
+            }
+            int st = plan_create(&plan, pairs, todo.data(), (int)todo.size(), m, cls, gsc, use);
+            no_memory = st == KSW2_HIP_ENOMEM;
+            if (st == KSW2_HIP_OK) st = plan_run(plan, prog);
+            if (st == KSW2_HIP_OK) st = plan_fetch(plan, ez, km);
+            plan_destroy(plan);
+            return st;
+        };
+        int st = one_plan();
+        if (no_memory) {
+            // what the library keeps may be in the way
+            (void)hipGetLastError();
+            release_call_context();
+            Engine::release_cached_block();
+            st = one_plan();
+            if (no_memory) (void)hipGetLastError();
         }
-        const ContextUse context;
-        if (context.held) {
-            if (total <= kCallBlockMax) env.pool = &t_call.pool;
-            env.stream = t_call.stream;
-            // (a lone pair has one launch at a time: its lanes would only add
-            // events)
-            if (todo.size() > 1) env.lanes = &t_call.lanes;
-            env.events = t_call.ev;
-            env.pinned = &t_call.pinned;
-            env.h_stop = t_call.h_stop, env.d_stop = t_call.d_stop;
-            env.spread = true;  // a plan of its own: 5-16 wave teams may spread over CUs
-            use = &env;
-        }
-        int st = plan_create(&plan, pairs, todo.data(), (int)todo.size(), m, cls, gsc, use);
-        if (st == KSW2_HIP_OK) st = plan_run(plan, prog);
-        if (st == KSW2_HIP_OK) st = plan_fetch(plan, ez, km);
-        plan_destroy(plan);
-        if (st != KSW2_HIP_OK) {
+        if (st == KSW2_HIP_OK) return status;
+        // (a batch that still finds no memory is streamed through what there is)
+        if (!no_memory || todo.size() == 1) {
             for (int k : todo) ez[k].zdropped = 1;  // the device path did not run
             return st;
         }
-        return status;
+        big.reset();
     }
     // larger than the budget: stream it through the engine, longest first
     // (CIGARs grown with realloc, as with km == NULL)

@@ -182,11 +182,14 @@ int ksw_extd2_hip_batch(int n, const ksw2_pair_t *pairs,
                         ksw_extz_t *ez);
 /* A batch larger than the device memory budget streams through a device
  * block of the whole budget, which the library keeps for the next such call
- * (allocating and releasing hundreds of GB costs seconds per call).  Single
- * calls (ksw_extd2_hip) likewise keep, per host thread, a stream, pinned
- * staging and a device block of up to 1 GiB grown to the thread's largest
- * call, released when the thread ends.  This releases the batch block and
- * the calling thread's device block; the next such call allocates again.
+ * (allocating and releasing hundreds of GB costs seconds per call).  Calls of
+ * up to 1 GiB (ksw_extd2_hip, and batches through ksw_extd2_hip_batch, the
+ * certification and the window calls) likewise keep, per host thread, streams,
+ * pinned memory of up to 256 MiB and a device block grown to the thread's
+ * largest call, released when the thread ends; a batch keeps what it grew
+ * only while all threads together hold at most 8 GiB of blocks and 2 GiB of
+ * pinned memory.  This releases the batch block and the calling thread's
+ * device block and pinned memory; the next such call allocates again.
  * No reference counterpart.  Returns KSW2_HIP_OK (also when nothing is
  * held). */
 int ksw2_hip_release_cached_memory(void);

@@ -1,4 +1,7 @@
 """Calls that find no memory to keep, and what threads keep between calls."""
+import ctypes as C
+import threading
+
 import pytest
 
 import oracle_py as O
@@ -29,3 +32,56 @@ def test_no_pinned_memory_to_keep(n, monkeypatch):
         if dense:
             monkeypatch.setenv("KSW2_HIP_DENSE_FETCH", "1")
         _check(_tuples(750 + n, n, 900))
+
+
+@pytest.mark.parametrize("n", [12, 60])
+def test_no_device_block_for_a_batch(n, monkeypatch):
+    """A batch whose block cannot be allocated is streamed through the memory
+    there is; a single call reports it, and the thread's next calls run."""
+    tuples = _tuples(760 + n, n, 900)
+    ksw2.release_cached_memory()
+    monkeypatch.setenv("KSW2_HIP_MEM_BUDGET", str(96 << 20))
+    monkeypatch.setenv("KSW2_HIP_FAIL_BLOCK", str(1 << 20))
+    _check(tuples)
+    q, t, f, w = tuples[0]
+    big = ksw2.extd2(*random_pairs(761, 1, 3000, 3000, 1.0)[0], check=False)
+    assert big.zdropped == 1 and big.n_cigar == 0
+    assert ksw2.lib().ksw2_hip_last_error() == -3  # KSW2_HIP_ENOMEM
+    assert same(ksw2.extd2(q[:50], t[:50], flag=f), O.run_oracle(q[:50], t[:50], flag=f))
+    monkeypatch.delenv("KSW2_HIP_FAIL_BLOCK")
+    _check(tuples)
+
+
+def _free_bytes():
+    hip = C.CDLL("libamdhip64.so")
+    free, total = C.c_size_t(), C.c_size_t()
+    assert hip.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+    return free.value
+
+
+def test_threads_keep_a_bounded_sum():
+    """Fourteen threads that each run a batch of some 0.9 GiB and live on: at
+    most 8 GiB stays with them."""
+    pairs = random_pairs(762, 1, 2000, 2000, 1.0) * 190
+    ref = O.run_oracle(*pairs[0])
+    ksw2.extd2_batch(pairs)
+    ksw2.release_cached_memory()
+    before = _free_bytes()
+    ran, done = threading.Barrier(15), threading.Event()
+    bad = []
+
+    def work():
+        bad.extend(k for k, g in enumerate(ksw2.extd2_batch(pairs)) if not same(g, ref))
+        ran.wait()
+        done.wait()
+
+    threads = [threading.Thread(target=work) for _ in range(14)]
+    for t in threads:
+        t.start()
+    ran.wait()
+    kept = before - _free_bytes()
+    done.set()
+    for t in threads:
+        t.join()
+    assert not bad
+    assert 1 << 30 < kept < (8 << 30) + (1 << 28), kept / 2**30
