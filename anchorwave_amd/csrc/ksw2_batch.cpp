@@ -356,7 +356,20 @@ StripeGeom stripe_geom(const ksw2_pair_t &p)
     return StripeGeom{tr, tr ? p.tlen : p.qlen, tr ? p.qlen : p.tlen};
 }
 
-constexpr int kDeviceSimds = 4 * 256;
+int device_cus()
+{
+    static std::atomic<int> known{0};
+    int cus = known;
+    if (cus <= 0) {
+        int dev = 0;
+        if (hipGetDevice(&dev) != hipSuccess ||
+            hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
+            return 256;
+        known = cus;
+    }
+    const char *ev = getenv("KSW2_HIP_CUS");
+    return ev ? std::max(1, std::min(atoi(ev), cus)) : cus;
+}
 
 static int norm_w(const ksw2_pair_t &p) { return p.w < 0 ? std::max(p.qlen, p.tlen) : p.w; }
 
@@ -409,6 +422,8 @@ bool thin_enabled()
 
 int thin_groups(const ksw2_pair_t &p) { return (thin_passes(stripe_geom(p).kt) + kWideGroup - 1) / kWideGroup; }
 
+int thin_group_limit() { return std::max(1, 3 * device_cus() / 2); }
+
 static bool thin_plan(const ksw2_pair_t *pairs, const std::vector<int> &fast, const PlanEnv *env)
 {
     if (!thin_enabled()) return false;
@@ -421,7 +436,7 @@ static bool thin_plan(const ksw2_pair_t *pairs, const std::vector<int> &fast, co
         if ((double)pairs[id].qlen * pairs[id].tlen > (double)pairs[big].qlen * pairs[big].tlen) big = id;
     }
     const StripeGeom g = stripe_geom(pairs[big]);
-    return groups <= kThinGroups && !tune_lookup(g.kq, g.kt);
+    return groups <= thin_group_limit() && !tune_lookup(g.kq, g.kt);
 }
 
 uint64_t job_dir_bytes(const KswJob &j)
@@ -665,8 +680,11 @@ int plan_create(Plan **out, const ksw2_pair_t *pairs, const int *idx, int nidx, 
         for (int k = 0; k < p->n_fast; ++k) {
             if (p->thin) {
                 // a wave per pass, spread over workgroups of four; as one
-                // workgroup when no waiting-launch slots are free
-                team[k] = std::min(thin_passes(p->jobs[k].tlen), kThinMaxTeam);
+                // workgroup when no waiting-launch slots are free.  (No more
+                // workgroups than a launch's share of the device: 1,024 waves
+                // are that on 256 CUs, a partition holds fewer.)
+                const int share = std::max(1, thin_capacity(grp_of[k], p->jobs[k].lut != 0) / 2);
+                team[k] = std::min({thin_passes(p->jobs[k].tlen), kThinMaxTeam, kWideGroup * share});
                 p->jobs[k].team = std::min(team[k], kThinTeam);
                 continue;
             }
@@ -786,7 +804,7 @@ int plan_create(Plan **out, const ksw2_pair_t *pairs, const int *idx, int nidx, 
                     const int window = std::min(std::min(pp.qlen, pp.tlen), norm_w(pp) + 1) + 128;
                     if (!band[gk] && 2 * thr[gk] == t && t <= window + 64) grow.push_back(gk), more += t / 2 / kWave;
                 }
-                if (waves + more > (t <= 256 ? 4 : 2) * (int64_t)kDeviceSimds) continue;
+                if (waves + more > (t <= 256 ? 4 : 2) * 4 * (int64_t)device_cus()) continue;
                 for (int gk : grow) thr[gk] = t;
                 waves += more;
             }
@@ -820,7 +838,7 @@ int plan_create(Plan **out, const ksw2_pair_t *pairs, const int *idx, int nidx, 
             team_max[g] = std::max(team_max[g], tm), ++members_of[g];
         }
         for (int g = 0; g < 3; ++g) {
-            if ((int64_t)members_of[g] * team_max[g] > kDeviceSimds) continue;
+            if ((int64_t)members_of[g] * team_max[g] > 4 * device_cus()) continue;
             std::vector<int> &all = teams[{g, -team_max[g]}];
             for (auto &t : teams)
                 if (t.first.first == g && &t.second != &all) all.insert(all.end(), t.second.begin(), t.second.end());

@@ -766,7 +766,7 @@ bool Engine::admit_locked(std::unique_lock<std::mutex> &lk)
         // Serving flights whose teams are capped by the pairs' pass count (the
         // device has waves to spare) run on the thin kernel, where a pair's
         // time is its columns and a lag per 128 rows: at most two such flights
-        // at once, each at most kThinGroups workgroups, half the device.  A
+        // at once, each at most thin_group_limit() workgroups, half the device.  A
         // burst of 256 tasks (half of them 5 kbp, the longest some 20 kbp) took
         // 50-54 ms with one workgroup of eight-row passes per pair, whose
         // longest pairs ran 22 ms on 16 waves, 19-23 ms so (25 with every capped
@@ -780,9 +780,10 @@ bool Engine::admit_locked(std::unique_lock<std::mutex> &lk)
         };
         size_t waiting = 0;
         for (const auto &w : queue_) waiting += w.size();
+        const int limit = thin_group_limit();
         auto wants_thin = [&](const Task *t) {
-            return !batch_ && thin_ && capped(t) && thin_groups(t->pair) <= kThinGroups &&
-                   (2 * t->passes > kMaxTeam || (int64_t)waiting * thin_groups(t->pair) <= kThinGroups);
+            return !batch_ && thin_ && capped(t) && thin_groups(t->pair) <= limit &&
+                   (2 * t->passes > kMaxTeam || (int64_t)waiting * thin_groups(t->pair) <= limit);
         };
         // While two thin flights run, a task that wants a third is passed over
         // if the first of them to end, and the task's own time on the thin
@@ -840,7 +841,7 @@ bool Engine::admit_locked(std::unique_lock<std::mutex> &lk)
             const bool same = batch_ ? (key == 0) == t->general
                               : held_back(t) ? false
                               : thin ? capped(t) && chain(t) <= 2 * chain(head) && 2 * chain(t) >= chain(head) &&
-                                           groups + thin_groups(t->pair) <= kThinGroups
+                                           groups + thin_groups(t->pair) <= limit
                                      : team_for(t->passes, t->steps, t->general, T, cap) == key &&
                                            (key == 0 || (t->steps / key <= 2 * span && 2 * t->steps / key >= span));
             if (!same) {
@@ -848,7 +849,7 @@ bool Engine::admit_locked(std::unique_lock<std::mutex> &lk)
                 ++it;
                 continue;
             }
-            const int w = thin      ? std::max(1, (int)((int64_t)thin_groups(t->pair) * resident_waves_ / (2 * kThinGroups)))
+            const int w = thin      ? std::max(1, (int)((int64_t)thin_groups(t->pair) * resident_waves_ / (2 * limit)))
                           : key > 0 ? key
                           : key < 0 ? (t->cls == 2 ? std::min(kMaxWide, t->passes) : 1) : t->waves;
             if (!pick.empty() && waves + w > free_waves) break;

@@ -6,6 +6,9 @@
 
 namespace kswhip {
 
+// CUs of the device (of its partition; KSW2_HIP_CUS, tests: as if it had fewer).
+int device_cus();
+
 struct StripeArgs {
     const uint8_t *seq;
     uint8_t *dir;
@@ -179,6 +182,7 @@ hipError_t launch_thin(const StripeArgs &a, int group, bool lut, const int32_t *
                        bool clear_err, hipStream_t st);
 hipError_t launch_thin_epilogue(const StripeArgs &a, int group, bool lut, hipStream_t st);
 // Workgroups of kWideGroup waves of the thin kernel the device holds at once.
+// (A launch's share is half of them, so a pair may have no more than that.)
 int thin_capacity(int group, bool lut);
 
 // Zero-fills `bytes` bytes at `p` (16-byte aligned) with a kernel on `st`

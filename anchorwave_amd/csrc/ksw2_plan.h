@@ -140,7 +140,7 @@ struct PlanEnv {
     PlanLanes *lanes = nullptr;
     PinnedBuffer *pinned = nullptr;
     // The stripe-kernel pairs run on the thin kernel (their workgroups, in sum,
-    // at most kThinGroups), queued behind other waiting launches if need be.
+    // at most thin_group_limit()), queued behind other waiting launches if need be.
     bool thin = false;
     int team = 0;                    // > 0: every stripe-kernel pair gets this team size
     int rows = 0;                    // 4 or 8: the stripe kernel's rows per lane (0: the plan picks)
@@ -282,10 +282,11 @@ int plan_create(Plan **out, const ksw2_pair_t *pairs, const int *idx, int nidx, 
 // The device the library runs on (device_init), -1 before it.
 int library_device();
 // The thin kernel in an engine's flights: whether it may run at all, a pair's
-// workgroups, and whether a waiting launch would start at once.
-constexpr int kThinGroups = 384;
+// workgroups and the most a plan of them may have (one and a half per CU), and
+// whether a waiting launch would start at once.
 bool thin_enabled();
 int thin_groups(const ksw2_pair_t &p);
+int thin_group_limit();
 bool wait_slots_idle();
 // Creates the process-wide events of the waiting-launch slots now, so that
 // later launches create none.  Returns false when a HIP call fails.

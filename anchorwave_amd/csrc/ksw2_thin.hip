@@ -775,16 +775,14 @@ struct Thin {
                            a);
         return hipGetLastError();
     }
-    static int capacity()
+    static int per_cu()
     {
-        int dev = 0, cus = 0, per_cu = 0;
-        if (hipGetDevice(&dev) != hipSuccess ||
-            hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
-            hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void *)ksw_thin_kernel<RIGHT, MODE, LUT>,
+        int per_cu = 0;
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, (const void *)ksw_thin_kernel<RIGHT, MODE, LUT>,
                                                          kWave * kWideGroup, ring_bytes(kWideGroup)) !=
                 hipSuccess)
             return 0;
-        return cus * per_cu;
+        return per_cu;
     }
 };
 
@@ -831,10 +829,12 @@ int thin_capacity(int group, bool lut)
     static int cache[kGroups][2] = {};
     if (group < 0 || group >= kGroups) group = kGroupLeft;
     int &c = cache[group][lut ? 1 : 0];
-    if (c > 0) return c;
-    const int n = by_thin(group, lut, [](auto v) { return v.capacity(); });
-    __atomic_store_n(&c, n, __ATOMIC_RELAXED);
-    return n;
+    int n = __atomic_load_n(&c, __ATOMIC_RELAXED);
+    if (n <= 0) {
+        n = by_thin(group, lut, [](auto v) { return v.per_cu(); });
+        __atomic_store_n(&c, n, __ATOMIC_RELAXED);
+    }
+    return n * device_cus();
 }
 
 }  // namespace kswhip

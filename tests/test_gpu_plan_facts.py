@@ -106,3 +106,17 @@ def test_long_thin_pairs_wait_for_a_share(tlen, share, monkeypatch):
     q = np.resize(W.mutate(rng, t, 0.05, 0.01), 8000)
     f = _run([(q, t, ksw2.KSW_EZ_SCORE_ONLY)])
     assert (f["thin_pairs"], f["waiting"], f["one_workgroup"]) == (1, share, 1 - share)
+
+
+@pytest.mark.parametrize("cus,kernel", [(64, "thin_pairs"), (28, "thin_pairs"), (16, "thin_pairs"), (15, "stripe_pairs")])
+def test_thin_pairs_on_a_smaller_device(cus, kernel, monkeypatch):
+    """As on a partition of few CUs: a pair of 24 workgroups is thin while
+    they are one and a half per CU, on no more waves than a launch's share
+    holds, and the same results."""
+    monkeypatch.setenv("KSW2_HIP_CUS", str(cus))
+    rng = np.random.default_rng(706)
+    t = W.random_seq(rng, 12000)
+    q = W.mutate(rng, t, 0.05, 0.01)[:11900]
+    for flag in FLAGS:
+        f = _run([(q, t, flag)])
+        assert (f[kernel], f["redone"]) == (1, 0)
