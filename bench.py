@@ -10,9 +10,10 @@ device backtrack that leaves every score and CIGAR in HBM.
 
 Prints one JSON line (rank 0).  Extra legs:
   cpu_baseline  the reference ksw_extd2_avx512 (oracle/_ref, compiled from the
-                reference sources) over the same 4,096 pairs on all host cores
-                (or the C restatement when that build is absent);
-  exact         every GPU result compared field by field with those CPU results;
+                reference sources) over the same 4,096 pairs on all host cores,
+                or, when that build is absent, the C restatement (a scalar
+                program of about 2 GCUPS) over a sample of PORT_CELLS cells;
+  exact         every GPU result with a CPU result compared field by field;
   one_at_a_time the same kernels launched on single-pair batches.
 """
 from __future__ import annotations
@@ -39,16 +40,21 @@ import numpy as np  # noqa: E402
 from anchorwave_amd import ksw2, workloads as W  # noqa: E402
 
 METRIC = "GCUPS, batched ksw_extd2 score+CIGAR (bit-exact); p50/p99 task latency"
-# Algorithmic integer work per cell of the reference inner loop with
-# traceback (minimap2/ksw2_extd2_sse.c:237-283): 51 ops.
-OPS_PER_CELL = 51
+# 16-bit operations per cell that the stripe kernel's middle pass issues: 248
+# packed VALU instructions a step for 16 cells a lane (two operations each).
+OPS_PER_CELL = 31
 N_CU, LANES, CLK_GHZ = 256, 64, 2.4
 PEAK_PACKED16_TOPS = N_CU * LANES * CLK_GHZ * 2 / 1e3   # 78.6 T int16 lane-ops/s
 HBM_PEAK_GBS = 8000.0
 
 
+# Cells per leg that the C restatement computes (some 20 s on 16 threads).
+PORT_CELLS = 4e10
+T_START = time.perf_counter()
+
+
 def log(msg: str) -> None:
-    print(msg, file=sys.stderr, flush=True)
+    print(f"{time.perf_counter() - T_START:7.1f} s {msg}", file=sys.stderr, flush=True)
 
 
 def read_profile_value(name: str, key: str):
@@ -85,6 +91,9 @@ def host_cpu() -> dict:
 
 
 def cpu_baseline(pairs, threads: int, flag: int = 0, w: int = -1):
+    """(which program, its GCUPS, results): the compiled reference over every
+    pair, or the C restatement over a seeded sample (None elsewhere) whose
+    cells are at most PORT_CELLS."""
     sys.path.insert(0, os.path.join(ROOT, "oracle"))
     import oracle_py as O  # checker / baseline only
 
@@ -94,15 +103,29 @@ def cpu_baseline(pairs, threads: int, flag: int = 0, w: int = -1):
     else:
         kind = "port"
         fn = lambda p: O.run_oracle(p[0], p[1], mat=W_MAT, flag=flag, w=w, **SC)  # noqa: E731
+    cells = [len(q) * len(t) if w < 0 else band_cells(len(q), len(t), w) for q, t in pairs]
+    take = list(range(len(pairs)))
+    if kind == "port" and sum(cells) > PORT_CELLS:
+        take, left = [], PORT_CELLS
+        for k in np.random.default_rng(13).permutation(len(pairs)):
+            if cells[k] <= left:
+                take.append(int(k))
+                left -= cells[k]
     # largest-cells-first, one pair per task
-    order = sorted(range(len(pairs)), key=lambda k: -len(pairs[k][0]) * len(pairs[k][1]))
+    order = sorted(take, key=lambda k: -cells[k])
     res = [None] * len(pairs)
     t0 = time.perf_counter()
     with ThreadPoolExecutor(threads) as ex:
         for k, r in zip(order, ex.map(lambda k: fn(pairs[k]), order)):
             res[k] = r
     dt = time.perf_counter() - t0
-    return kind, dt, res
+    return kind, sum(cells[k] for k in take) / dt / 1e9, res
+
+
+def agreement(gpu_res, cpu_res) -> dict:
+    both = [(g, c) for g, c in zip(gpu_res, cpu_res) if c is not None]
+    exact = sum(1 for g, c in both if g.__dict__ == c.__dict__)
+    return {"agree": exact, "of": len(both), "frac": exact / max(len(both), 1), "pairs": len(cpu_res)}
 
 
 def singletrack_leg(args, pairs, cells) -> dict:
@@ -127,11 +150,10 @@ def singletrack_leg(args, pairs, cells) -> dict:
     log(f"[bench] singletrack: {gcups:.1f} GCUPS ({out['device_ms']:.2f} ms device)")
     if not args.no_cpu:
         threads = args.cpu_threads or min(os.cpu_count() or 1, 16)
-        kind, dt, cpu_res = cpu_baseline(pairs, threads, flag=ksw2.KSW_EZ_SINGLETRACK)
-        exact = sum(1 for g, c in zip(res, cpu_res) if g.__dict__ == c.__dict__)
-        out["exact"] = {"agree": exact, "of": len(pairs), "frac": exact / len(pairs)}
-        out["cpu"] = {"kind": kind, "gcups": round(cells / dt / 1e9, 3), "cores": threads}
-        log(f"[bench] singletrack CPU {cells / dt / 1e9:.2f} GCUPS; exact {exact}/{len(pairs)}")
+        kind, rate, cpu_res = cpu_baseline(pairs, threads, flag=ksw2.KSW_EZ_SINGLETRACK)
+        out["exact"] = agreement(res, cpu_res)
+        out["cpu"] = {"kind": kind, "gcups": round(rate, 3), "cores": threads}
+        log(f"[bench] singletrack CPU {rate:.2f} GCUPS; exact {out['exact']}")
     return out
 
 
@@ -161,8 +183,8 @@ def single_pair_leg(args) -> dict:
            "gpu_gcups": round(cells / float(np.median(ts)) / 1e9, 3),
            "timing": "wall clock of one ksw_extd2_hip call (upload, DP, backtrack, CIGAR), median of 9"}
     if not args.no_cpu:
-        kind, dt, res = cpu_baseline([(q, t)], 1)
-        out["cpu"] = {"kind": kind, "ms": round(dt * 1e3, 3), "gcups": round(cells / dt / 1e9, 3), "cores": 1}
+        kind, rate, res = cpu_baseline([(q, t)], 1)
+        out["cpu"] = {"kind": kind, "ms": round(cells / rate / 1e6, 3), "gcups": round(rate, 3), "cores": 1}
         out["exact"] = g.__dict__ == res[0].__dict__
     log(f"[bench] single 5 kbp pair: {out}")
     return out
@@ -192,10 +214,9 @@ def threads_leg(args, pairs) -> dict:
            "gcups": round(cells / dt / 1e9, 2), "calls_per_s": round(len(sub) / dt, 1),
            "timing": "wall clock of all calls, 16 host threads each calling ksw_extd2_hip one pair at a time"}
     if not args.no_cpu:
-        kind, cdt, cres = cpu_baseline(sub, threads)
-        out["cpu"] = {"kind": kind, "gcups": round(cells / cdt / 1e9, 3), "cores": threads}
-        exact = sum(1 for g, c in zip(res, cres) if g.__dict__ == c.__dict__)
-        out["exact"] = {"agree": exact, "of": len(sub), "frac": exact / len(sub)}
+        kind, rate, cres = cpu_baseline(sub, threads)
+        out["cpu"] = {"kind": kind, "gcups": round(rate, 3), "cores": threads}
+        out["exact"] = agreement(res, cres)
     log(f"[bench] {threads} threads calling ksw_extd2_hip: {out}")
     return out
 
@@ -223,19 +244,19 @@ def banded_leg(args) -> dict:
            "timing": "wall clock of a second ksw_extd2_hip_batch call: upload, DP, backtrack, CIGAR download"}
     if not args.no_cpu:
         threads = args.cpu_threads or min(os.cpu_count() or 1, 16)
-        kind, cdt, cres = cpu_baseline(pb, threads, w=w)
-        exact = sum(1 for g, c in zip(gres, cres) if g.__dict__ == c.__dict__)
-        res["exact"] = {"agree": exact, "of": len(pb), "frac": exact / len(pb)}
-        res["cpu"] = {"kind": kind, "gcups": round(cells / cdt / 1e9, 3), "cores": threads}
-        log(f"[bench] banded CPU {cells / cdt / 1e9:.2f} GCUPS; exact {exact}/{len(pb)}")
+        kind, rate, cres = cpu_baseline(pb, threads, w=w)
+        res["exact"] = agreement(gres, cres)
+        res["cpu"] = {"kind": kind, "gcups": round(rate, 3), "cores": threads}
+        log(f"[bench] banded CPU {rate:.2f} GCUPS; exact {res['exact']}")
     return res
 
 
 def general_leg(args, pairs) -> dict:
     """Narrow bands, as the score-certified path asks for
     (alignSlidingWindow.cpp:1297-1310 widens the band from twice the length
-    difference; once the general kernel's workload, now the band kernel's).
-    The fixed batch's pairs at w = 256 through ksw_extd2_hip_batch; GCUPS over in-band cells up to each band exit."""
+    difference): the fixed batch's pairs at w = 256 through
+    ksw_extd2_hip_batch, on the band kernel; GCUPS over in-band cells up to
+    each band exit."""
     w = args.general_w
     sub = pairs[: args.general]
     cells = sum(band_cells(len(q), len(t), w) for q, t in sub)
@@ -246,17 +267,16 @@ def general_leg(args, pairs) -> dict:
     dt = tm["seconds"]
     exits = sum(1 for g in gres if g.zdropped)
     res = {"pairs": len(sub), "w": w, "in_band_cells": cells, "seconds": round(dt, 4),
-           "gcups": round(cells / dt / 1e9, 2), "band_exits": exits, "kernel": "ksw_general_kernel",
+           "gcups": round(cells / dt / 1e9, 2), "band_exits": exits, "kernel": "ksw_band_kernel",
            "timing": "wall clock of a second ksw_extd2_hip_batch call: upload, DP, backtrack, CIGAR download"}
-    log(f"[bench] general kernel (w={w}): {cells:.3g} in-band cells in {dt * 1e3:.1f} ms = "
+    log(f"[bench] narrow bands (w={w}): {cells:.3g} in-band cells in {dt * 1e3:.1f} ms = "
         f"{cells / dt / 1e9:.1f} GCUPS ({exits} band exits)")
     if not args.no_cpu:
         threads = args.cpu_threads or min(os.cpu_count() or 1, 16)
-        kind, cdt, cres = cpu_baseline(sub, threads, w=w)
-        exact = sum(1 for g, c in zip(gres, cres) if g.__dict__ == c.__dict__)
-        res["exact"] = {"agree": exact, "of": len(sub), "frac": exact / len(sub)}
-        res["cpu"] = {"kind": kind, "gcups": round(cells / cdt / 1e9, 3), "cores": threads}
-        log(f"[bench] general-kernel CPU {cells / cdt / 1e9:.2f} GCUPS; exact {exact}/{len(sub)}")
+        kind, rate, cres = cpu_baseline(sub, threads, w=w)
+        res["exact"] = agreement(gres, cres)
+        res["cpu"] = {"kind": kind, "gcups": round(rate, 3), "cores": threads}
+        log(f"[bench] narrow-band CPU {rate:.2f} GCUPS; exact {res['exact']}")
     return res
 
 
@@ -264,7 +284,7 @@ def uneven_leg(args) -> dict:
     """The uneven inter-anchor batch through ksw_extd2_hip_batch (host
     buffers in and out, chunked by the device memory budget), against the
     same kind of call made one pair at a time on a seeded sample, and checked
-    bit-exact against the CPU reference on every pair."""
+    bit-exact against the CPU reference."""
     log(f"[bench] uneven batch: generating {args.uneven} pairs")
     pu = W.uneven(seed=3, n=args.uneven)
     cu = W.cells(pu)
@@ -291,11 +311,10 @@ def uneven_leg(args) -> dict:
     if not args.no_cpu:
         threads = args.cpu_threads or min(os.cpu_count() or 1, 16)
         log(f"[bench] uneven batch: CPU reference on {threads} threads (exactness check)")
-        kind, cdt, cres = cpu_baseline(pu, threads)
-        exact = sum(1 for g, c in zip(gres, cres) if g.__dict__ == c.__dict__)
-        res["exact"] = {"agree": exact, "of": len(pu), "frac": exact / len(pu)}
-        res["cpu"] = {"kind": kind, "gcups": round(cu / cdt / 1e9, 3), "cores": threads}
-        log(f"[bench] uneven CPU {cu / cdt / 1e9:.2f} GCUPS; exact {exact}/{len(pu)}")
+        kind, rate, cres = cpu_baseline(pu, threads)
+        res["exact"] = agreement(gres, cres)
+        res["cpu"] = {"kind": kind, "gcups": round(rate, 3), "cores": threads}
+        log(f"[bench] uneven CPU {rate:.2f} GCUPS; exact {res['exact']}")
     return res
 
 
@@ -450,8 +469,11 @@ def main() -> int:
     ap.add_argument("--threads-leg", type=int, default=1024,
                     help="pairs of the 16-thread ksw_extd2_hip leg (0: skip it)")
     ap.add_argument("--general", type=int, default=4096,
-                    help="fixed-batch pairs of the narrow-band (general kernel) leg (0: skip it)")
-    ap.add_argument("--general-w", type=int, default=256, help="band of the general-kernel leg")
+                    help="fixed-batch pairs of the narrow-band leg (0: skip it)")
+    ap.add_argument("--general-w", type=int, default=256, help="band of the narrow-band leg")
+    ap.add_argument("--seconds", type=float, default=240.0,
+                    help="extra legs begin only within this time of the start; the others are named in "
+                         "\"skipped\"")
     ap.add_argument("--copy-calib", type=int, default=0,
                     help="also run one device-to-device copy of this many MiB (PMC byte-counter scale)")
     args = ap.parse_args()
@@ -557,31 +579,32 @@ def main() -> int:
         "one_at_a_time_gcups": None if single is None else round(single, 3),
         "batched_over_one_at_a_time": None if not single else round(gcups / single, 1),
     }
-    if args.single_pair:
-        out["single_pair"] = single_pair_leg(args)
-    if args.singletrack:
-        out["singletrack"] = singletrack_leg(args, pairs, cells)
-    if args.threads_leg > 0:
-        out["threads"] = threads_leg(args, pairs)
-    if args.general > 0:
-        out["general"] = general_leg(args, pairs)
-    if args.banded > 0:
-        out["banded"] = banded_leg(args)
-    if args.uneven > 0:
-        out["uneven"] = uneven_leg(args)
-    if args.serve > 0:
-        out["serving"] = serving_leg(args)
     if not args.no_cpu:
         threads = args.cpu_threads or min(os.cpu_count() or 1, 16)
         log(f"[bench] CPU baseline on {threads} threads")
-        kind, dt, cpu_res = cpu_baseline(pairs, threads)
-        exact = sum(1 for g, c in zip(gpu_res, cpu_res) if g.__dict__ == c.__dict__)
-        out["cpu_baseline"] = {"value": round(cells / dt / 1e9, 3), "unit": "GCUPS", "cores": threads,
+        kind, rate, cpu_res = cpu_baseline(pairs, threads)
+        out["exact"] = agreement(gpu_res, cpu_res)
+        out["cpu_baseline"] = {"value": round(rate, 3), "unit": "GCUPS", "cores": threads,
                                "kind": kind, **host_cpu(),
-                               "sample": f"the full fixed batch ({len(pairs)} pairs, {cells:.3g} cells), "
-                                         "ksw_extd2_avx512 one pair per task, largest first"}
-        out["exact"] = {"agree": exact, "of": len(pairs), "frac": exact / len(pairs)}
-        log(f"[bench] CPU {cells / dt / 1e9:.2f} GCUPS; exact {exact}/{len(pairs)}")
+                               "sample": f"{out['exact']['of']} of the fixed batch's {len(pairs)} pairs, "
+                                         + ("ksw_extd2_avx512" if kind == "reference" else "the C restatement")
+                                         + " one pair per task, largest first"}
+        log(f"[bench] CPU {rate:.2f} GCUPS; exact {out['exact']}")
+    legs = [("single_pair", args.single_pair, lambda: single_pair_leg(args)),
+            ("singletrack", args.singletrack, lambda: singletrack_leg(args, pairs, cells)),
+            ("threads", args.threads_leg, lambda: threads_leg(args, pairs)),
+            ("general", args.general, lambda: general_leg(args, pairs)),
+            ("banded", args.banded, lambda: banded_leg(args)),
+            ("uneven", args.uneven, lambda: uneven_leg(args)),
+            ("serving", args.serve, lambda: serving_leg(args))]
+    for name, on, leg in legs:
+        if on <= 0:
+            continue
+        if time.perf_counter() - T_START > args.seconds:
+            out.setdefault("skipped", []).append(name)
+            log(f"[bench] {name}: skipped, {args.seconds:.0f} s are over")
+            continue
+        out[name] = leg()
     print(json.dumps(out), flush=True)
     return 0
 
