@@ -35,15 +35,21 @@ def test_short_tasks_pass_two_long_flights():
     for pair in long:
         server.submit(*pair, flag=ksw2.KSW_EZ_SCORE_ONLY)
         drain(1)
-    for pair in long:
-        server.submit(*pair, flag=ksw2.KSW_EZ_SCORE_ONLY)
-        time.sleep(0.002)
-    tickets = {server.submit(*task[:2], flag=task[2], w=task[3]): task for task in tasks}
-    done = drain(len(long) + len(tasks))
+    # (three tries: a host that is held up for the flights' milliseconds
+    # submits the tasks too late)
+    for _ in range(3):
+        for pair in long:
+            server.submit(*pair, flag=ksw2.KSW_EZ_SCORE_ONLY)
+            time.sleep(0.002)
+        tickets = {server.submit(*task[:2], flag=task[2], w=task[3]): task for task in tasks}
+        done = drain(len(long) + len(tasks))
+        for ticket, got in done:
+            if ticket in tickets:
+                q, t, f, w = tickets[ticket]
+                r = O.run_oracle(q, t, flag=f, w=w)
+                assert same(got, r), diff(got, r)
+        first = {ticket for ticket, _ in done[: len(tasks)]}
+        if first == set(tickets):
+            break
     server.close()
-    for ticket, got in done:
-        if ticket in tickets:
-            q, t, f, w = tickets[ticket]
-            r = O.run_oracle(q, t, flag=f, w=w)
-            assert same(got, r), diff(got, r)
-    assert {ticket for ticket, _ in done[: len(tasks)]} == set(tickets), [ticket for ticket, _ in done]
+    assert first == set(tickets), [ticket for ticket, _ in done]
