@@ -88,6 +88,7 @@ using cell::sub2;
 constexpr int SR = kBandStripe;                 // positions per stripe
 constexpr int kBlock = 16;                      // anti-diagonals per block
 constexpr uint64_t kWaitTicks = 1000000000ull;  // 10 s of the 100 MHz real-time clock
+constexpr int kDeviceLooks = 1024, kRingLooks = 16384;  // at an entry or a count, between two at the stop flag
 
 struct Band {
     int st0, en0, st16, en16, stB, sc_end;
@@ -226,9 +227,10 @@ __global__ void __launch_bounds__(kWave * kBandGroup) __attribute__((amdgpu_wave
             stop = __builtin_amdgcn_readfirstlane(__hip_atomic_load(a.stop, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM));
         return stop != 0;
     };
-    // (while waiting it is looked at now and then: the load goes over the bus)
+    // (while waiting it is looked at now and then, every millisecond or two:
+    // the load goes over the bus)
     int spins = 0;
-    auto stopped_waiting = [&]() { return (++spins & 1023) == 0 ? stopped() : stop != 0; };
+    auto stopped_waiting = [&](int looks) { return (++spins & (looks - 1)) == 0 ? stopped() : stop != 0; };
     // one workgroup of as many waves as stripes in flight: the last hands on to
     // the first through the first's ring (with fewer, each would wait for room
     // in the next one's ring, the last for a stripe that the first has yet to
@@ -288,7 +290,7 @@ __global__ void __launch_bounds__(kWave * kBandGroup) __attribute__((amdgpu_wave
                     const uint64_t t_start = wall_clock64();
                     for (;;) {
                         if (have) na = load_half(buf, c - wofs, 0), nh = load_half(buf, c - wofs, 1);
-                        if (!missing() || stopped_waiting()) break;
+                        if (!missing() || stopped_waiting(kDeviceLooks)) break;
                         if (wall_clock64() - t_start > kWaitTicks) {
                             late = 1;
                             break;
@@ -307,7 +309,7 @@ __global__ void __launch_bounds__(kWave * kBandGroup) __attribute__((amdgpu_wave
             constexpr int WHAT = decltype(what)::value;
             if (FED && (WHAT & 7) && __builtin_expect(known < in_base + min(c + 4, p_end), 0)) {
                 while ((known = ring_load(&in.filled)) < in_base + min(c + 4, p_end)) {
-                    if (stopped_waiting()) break;
+                    if (stopped_waiting(kRingLooks)) break;
                     __builtin_amdgcn_s_sleep(1);
                 }
             }
@@ -377,7 +379,7 @@ __global__ void __launch_bounds__(kWave * kBandGroup) __attribute__((amdgpu_wave
                 // after this one, or that wave's stripe before)
                 const int need = nb - kRing > n_lo ? base + nb - kRing : base;
                 while (__builtin_expect(room < need, 0)) {
-                    if (stopped_waiting()) break;
+                    if (stopped_waiting(kRingLooks)) break;
                     __builtin_amdgcn_s_sleep(1);
                     room = ring_load(&out.taken);
                 }

@@ -68,6 +68,7 @@ using cell::splat;
 constexpr int kSkew = 2 * kWave;                 // the bottom row's column is handed on this many steps after
 constexpr int kBlock = 16;                       // columns per hand-off
 constexpr uint64_t kWaitTicks = 1000000000ull;  // 10 s of the 100 MHz real-time clock
+constexpr int kDeviceLooks = 1024, kRingLooks = 16384;  // at an entry or a count, between two at the stop flag
 
 __device__ __forceinline__ uint64_t load_entry(const int32_t *bnd, int col)
 {
@@ -183,11 +184,14 @@ __device__ __forceinline__ void thin_run(const StripeArgs &a, const typename Cel
             stop = __builtin_amdgcn_readfirstlane(__hip_atomic_load(a.stop, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM));
         return stop != 0;
     };
-    // while waiting it is looked at now and then: a load over the bus on every
-    // look at a count made each wait last one, and a thousand waves' loads
-    // filled the bus (38 pairs of 5 kbp in a server's flight: 50 ms, 2.5 so)
+    // while waiting it is looked at now and then, every millisecond or two: a
+    // load over the bus on every look at a count made each wait last one, and a
+    // thousand waves' loads filled the bus (38 pairs of 5 kbp in a server's
+    // flight: 50 ms, 2.5 so).  A look at a ring takes a tenth of one at device
+    // memory: with the same number between two loads, flights of 22 and 39
+    // such pairs together still took 6-9 ms or 23-26, from run to run.
     int spins = 0;
-    auto stopped_waiting = [&]() { return (++spins & 1023) == 0 ? stopped() : stop != 0; };
+    auto stopped_waiting = [&](int looks) { return (++spins & (looks - 1)) == 0 ? stopped() : stop != 0; };
 
     // ---- wave 0: column-buffer entries of a block, asked for 16 steps before
     // they are put into the ring and 20 before the first is used.  One set of
@@ -214,7 +218,7 @@ __device__ __forceinline__ void thin_run(const StripeArgs &a, const typename Cel
                 const uint64_t t_start = wall_clock64();
                 for (;;) {
                     if (have) ne = load_entry(bnd, col);
-                    if (__ballot(have && (uint32_t)(ne >> 32 & 0xffffu) != tag) == 0 || stopped_waiting()) break;
+                    if (__ballot(have && (uint32_t)(ne >> 32 & 0xffffu) != tag) == 0 || stopped_waiting(kDeviceLooks)) break;
                     if (wall_clock64() - t_start > kWaitTicks) {
                         late = 1;
                         break;
@@ -234,7 +238,7 @@ __device__ __forceinline__ void thin_run(const StripeArgs &a, const typename Cel
     auto read4 = [&](int c, uint4 (&e)[4]) {
         if (__builtin_expect(known < base + min(c + 4, qlen), 0)) {
             while ((known = __builtin_amdgcn_readfirstlane(ring_load(&in.filled))) < base + min(c + 4, qlen)) {
-                if (stopped_waiting()) break;
+                if (stopped_waiting(kRingLooks)) break;
                 __builtin_amdgcn_s_sleep(1);
             }
         }
@@ -354,7 +358,7 @@ __device__ __forceinline__ void thin_run(const StripeArgs &a, const typename Cel
             // reading its pass before)
             const int need = max(FEEDS ? base + nb - kSkew - kRing : base, base);
             while (__builtin_expect(room < need, 0)) {
-                if (stopped_waiting()) return;
+                if (stopped_waiting(kRingLooks)) return;
                 __builtin_amdgcn_s_sleep(1);
                 room = __builtin_amdgcn_readfirstlane(ring_load(&out.taken));
             }
