@@ -789,10 +789,11 @@ bool Engine::admit_locked(std::unique_lock<std::mutex> &lk)
         // if the first of them to end, and the task's own time on the thin
         // kernel, come before its team would be done, or if that is wide and
         // waits for a share of the device itself; otherwise it runs on its team
-        // now.  Either way the tasks behind it get their turn (the other
-        // classes have streams of their own).  The burst of 256 tasks takes 16-19
-        // ms on four hardware queues and 13-16 on sixteen, 17-24 and 16-21 when
-        // the stream's whole class waited for a third flight's turn.
+        // now.  Either way the tasks behind it get their turn, then the
+        // stream's other classes.  Three bursts of 256 tasks take 21-24, 18
+        // and 18-20 ms on four hardware queues and 16, 13-14 and 14-15 on
+        // sixteen; 28, 15-18 and 18-22, and 20, 12-20 and 17-22, when the
+        // stream's whole class waited for a third flight's turn.
         const double now = now_s();
         int thin_running = 0;
         double thin_wait = 0;  // seconds until one of them ends, as predicted (one that is late: as late again)
@@ -807,16 +808,13 @@ bool Engine::admit_locked(std::unique_lock<std::mutex> &lk)
         };
         int cls = -1;
         Task *head = nullptr;
-        for (int k = 0; k < kClasses && pref[own][k] >= 0; ++k)
-            if (!queue_[pref[own][k]].empty()) {
-                cls = pref[own][k];
-                break;
+        for (int k = 0; k < kClasses && pref[own][k] >= 0 && !head; ++k) {
+            cls = pref[own][k];
+            int passed = 0;
+            for (Task *t : queue_[cls]) {
+                if (!held_back(t)) head = t;
+                if (head || ++passed > backfill_) break;
             }
-        if (cls < 0) continue;
-        int passed = 0;
-        for (Task *t : queue_[cls]) {
-            if (!held_back(t)) head = t;
-            if (head || ++passed > backfill_) break;
         }
         if (!head) continue;
         std::deque<Task *> &q = queue_[cls];
