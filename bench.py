@@ -357,7 +357,7 @@ def serving_leg(args) -> dict:
         return time.perf_counter() - t0, lat
 
     run(None)  # warm-up: device buffers, code objects
-    wall, lat = run(None)
+    wall = sorted(run(None)[0] for _ in range(3))[1]
     cap = len(tasks) / wall
     log(f"[bench] serving batch capacity (every task submitted at once): {cap:.0f} tasks/s, "
         f"{cells.sum() / wall / 1e9:.1f} GCUPS")
@@ -367,6 +367,7 @@ def serving_leg(args) -> dict:
         arr = np.cumsum(rng.exponential(1.0 / rate, len(tasks)))
         wall, lat = run(arr)
         lv = {"load": load, "offered_tasks_per_s": round(rate, 1),
+              "arrived_tasks_per_s": round(len(tasks) / float(arr[-1]), 1),
               "achieved_tasks_per_s": round(len(tasks) / wall, 1),
               "gcups": round(float(cells.sum() / wall / 1e9), 2),
               "p50_ms": round(float(np.percentile(lat, 50)) * 1e3, 3),
@@ -377,15 +378,22 @@ def serving_leg(args) -> dict:
         return lv
 
     # sustained capacity: the highest offered Poisson rate (fractions of the
-    # batch capacity) that the server keeps up with, achieved >= 0.98 offered
+    # batch capacity) that the server keeps up with: achieved >= 0.98 of the
+    # rate at which the drawn arrivals came (a draw of 12,000 gaps may last 3 %
+    # longer than its mean)
     search = []
+
+    def kept_up(lv):
+        return lv["achieved_tasks_per_s"] >= 0.98 * lv["arrived_tasks_per_s"]
+
     for f in [float(x) for x in args.search.split(",") if x]:
         lv = level(f * cap, None)
-        search.append({k: lv[k] for k in ("offered_tasks_per_s", "achieved_tasks_per_s", "p50_ms", "p99_ms")})
+        search.append({k: lv[k] for k in ("offered_tasks_per_s", "arrived_tasks_per_s", "achieved_tasks_per_s",
+                                          "p50_ms", "p99_ms")})
         log(f"[bench] serving capacity search {f:.2f} of batch capacity: {search[-1]}")
-        if lv["achieved_tasks_per_s"] < 0.98 * lv["offered_tasks_per_s"]:
+        if not kept_up(lv):
             break
-    kept = [lv for lv in search if lv["achieved_tasks_per_s"] >= 0.98 * lv["offered_tasks_per_s"]]
+    kept = [lv for lv in search if kept_up(lv)]
     sustained = max(lv["offered_tasks_per_s"] for lv in kept) if kept else search[0]["achieved_tasks_per_s"]
     log(f"[bench] serving sustained capacity: {sustained:.0f} tasks/s ({sustained / cap:.2f} of batch capacity)")
     # the sweep: fractions of the sustained capacity
@@ -413,7 +421,7 @@ def serving_leg(args) -> dict:
             "capacity_search": search,
             "sustained_tasks_per_s": round(sustained, 1),
             "sustained": "highest offered Poisson rate (fractions of the batch capacity, every task submitted "
-                         "at once) with achieved >= 0.98 offered; the sweep's loads are fractions of it",
+                         "at once) with achieved >= 0.98 of the rate that arrived; the sweep's loads are fractions of it",
             "admission_budget_bytes": SERVE_BUDGET,
             "sequences": {"where": "device arena, uploaded at submission", "arena_bytes": ld["seq_arena_bytes"],
                           "resident_tasks": ld["resident_tasks"], "staged_flights": ld["staged_flights"]},
