@@ -57,9 +57,21 @@ uint64_t mem_budget(bool with_cache)
     return with_cache ? std::max<uint64_t>(own, Engine::cached_block_bytes()) : own;
 }
 
-namespace {
+bool device_alloc(uint8_t **p, uint64_t bytes)
+{
+    if (hipMalloc((void **)p, bytes) == hipSuccess) return true;
+    (void)hipGetLastError();
+    *p = nullptr;
+    return false;
+}
 
-}  // namespace
+bool pinned_alloc(void **p, uint64_t bytes, unsigned flags)
+{
+    if (hipHostMalloc(p, bytes, flags) == hipSuccess) return true;
+    (void)hipGetLastError();
+    *p = nullptr;
+    return false;
+}
 
 namespace {
 // Launches whose workgroups wait on one another (band kernel, wide stripe
@@ -908,7 +920,7 @@ int plan_create(Plan **out, const ksw2_pair_t *pairs, const int *idx, int nidx, 
         p->pool = env->pool;
         base = env->pool->base + p->pool_off;
     } else {
-        if (hipMalloc(&p->block, p->block_bytes) != hipSuccess) return fail(KSW2_HIP_ENOMEM);
+        if (!device_alloc(&p->block, p->block_bytes)) return fail(KSW2_HIP_ENOMEM);
         base = p->block;
     }
     p->d_seq = resident ? env->seq_dev : base + o_seq;
@@ -932,8 +944,7 @@ int plan_create(Plan **out, const ksw2_pair_t *pairs, const int *idx, int nidx, 
         p->h_stop = env->h_stop, p->d_stop = env->d_stop, p->own_stop = false;
         p->poll_stop = env->poll_stop;
     } else if (p->n > 0) {
-        if (hipHostMalloc((void **)&p->h_stop, sizeof(int32_t), hipHostMallocMapped) != hipSuccess)
-            return fail(KSW2_HIP_ENOMEM);
+        if (!pinned_alloc((void **)&p->h_stop, sizeof(int32_t), hipHostMallocMapped)) return fail(KSW2_HIP_ENOMEM);
         *p->h_stop = 0;
         if (hipHostGetDevicePointer((void **)&p->d_stop, p->h_stop, 0) != hipSuccess) return fail(KSW2_HIP_EDEVICE);
     }
@@ -977,7 +988,7 @@ int plan_create(Plan **out, const ksw2_pair_t *pairs, const int *idx, int nidx, 
             h_seq = env->staging, p->own_seq = false;
         } else if (p->pinned && p->pinned->grow(p->upload_bytes)) {
             h_seq = p->pinned->base, p->own_seq = false, whole = true;
-        } else if (hipHostMalloc((void **)&h_seq, p->upload_bytes, hipHostMallocDefault) != hipSuccess) {
+        } else if (!pinned_alloc((void **)&h_seq, p->upload_bytes, hipHostMallocDefault)) {
             return fail(KSW2_HIP_ENOMEM);
         } else {
             whole = true;
@@ -1584,11 +1595,7 @@ struct GrowPool : DevicePool {
         if (n > bytes) {
             drop();
             const char *fb = getenv("KSW2_HIP_FAIL_BLOCK");  // tests: blocks of this many bytes cannot be had
-            if (hipMalloc(&base, fb && n >= strtoull(fb, nullptr, 10) ? 1ull << 60 : n) != hipSuccess) {
-                (void)hipGetLastError();
-                base = nullptr;
-                return false;
-            }
+            if (!device_alloc(&base, fb && n >= strtoull(fb, nullptr, 10) ? 1ull << 60 : n)) return false;
             bytes = n, g_blocks += n;
         }
         if (lone) single = std::max(single, n);
@@ -1620,7 +1627,7 @@ struct CallContext {
             if (!stream && hipStreamCreateWithFlags(&stream, hipStreamNonBlocking) != hipSuccess) return false;
             for (auto &e : ev)
                 if (!e && hipEventCreate(&e) != hipSuccess) return false;
-            if (!h_stop && hipHostMalloc((void **)&h_stop, sizeof(int32_t), hipHostMallocMapped) != hipSuccess) return false;
+            if (!h_stop && !pinned_alloc((void **)&h_stop, sizeof(int32_t), hipHostMallocMapped)) return false;
             if (hipHostGetDevicePointer((void **)&d_stop, h_stop, 0) != hipSuccess) return false;
             ready = true;
         }
@@ -1670,12 +1677,7 @@ bool PinnedBuffer::grow(uint64_t want)
     drop();
     uint64_t n = std::max<uint64_t>(want < kPinnedKeep / 2 ? want + want / 4 : want, 1u << 16);
     if (getenv("KSW2_HIP_FAIL_PINNED")) n = 1ull << 60;  // tests: more than there is
-    if (hipHostMalloc((void **)&base, n, hipHostMallocDefault) != hipSuccess) {
-        // (the callers do without: the launches that follow read this error)
-        (void)hipGetLastError();
-        base = nullptr;
-        return false;
-    }
+    if (!pinned_alloc((void **)&base, n, hipHostMallocDefault)) return false;  // (the callers do without)
     bytes = n, g_pinned += n;
     return true;
 }
@@ -1771,11 +1773,9 @@ int run_batch_host(int n, const ksw2_pair_t *pairs, int8_t m, const int8_t *mat,
         int st = one_plan();
         if (no_memory) {
             // what the library keeps may be in the way
-            (void)hipGetLastError();
             release_call_context();
             Engine::release_cached_block();
             st = one_plan();
-            if (no_memory) (void)hipGetLastError();
         }
         if (st == KSW2_HIP_OK) return status;
         // (a batch that still finds no memory is streamed through what there is)

@@ -80,8 +80,7 @@ public:
                 g_cached.base = nullptr, g_cached.bytes = 0;
             }
             if (!g_cached.busy && !g_cached.base) {
-                if (hipMalloc(&g_cached.base, bytes) != hipSuccess) g_cached.base = nullptr;
-                else g_cached.bytes = bytes;
+                if (device_alloc(&g_cached.base, bytes)) g_cached.bytes = bytes;
             }
             if (!g_cached.busy && g_cached.base) {
                 g_cached.busy = true, cached_ = true;
@@ -90,10 +89,7 @@ public:
                 return KSW2_HIP_OK;
             }
         }
-        if (hipMalloc(&base, bytes) != hipSuccess) {
-            base = nullptr;
-            return KSW2_HIP_ENOMEM;
-        }
+        if (!device_alloc(&base, bytes)) return KSW2_HIP_ENOMEM;
         carve_.reset(bytes);
         return KSW2_HIP_OK;
     }
@@ -240,7 +236,7 @@ int Engine::start(bool cached, bool resident_seq)
         A.bytes = std::min<uint64_t>(budget_ / 16, 512ull << 20) / 256 * 256;
         if (A.bytes >= (1u << 20)) {
             if (!pool->alloc(A.bytes, &A.pool_off)) return KSW2_HIP_ENOMEM;
-            if (hipHostMalloc((void **)&A.ring, A.bytes, hipHostMallocDefault) != hipSuccess) return KSW2_HIP_ENOMEM;
+            if (!pinned_alloc((void **)&A.ring, A.bytes, hipHostMallocDefault)) return KSW2_HIP_ENOMEM;
             if (hipStreamCreateWithFlags(&A.up, hipStreamNonBlocking) != hipSuccess) return KSW2_HIP_EDEVICE;
             for (auto &ev : A.ev)
                 if (hipEventCreateWithFlags(&ev, hipEventDisableTiming) != hipSuccess) return KSW2_HIP_EDEVICE;
@@ -258,7 +254,7 @@ int Engine::start(bool cached, bool resident_seq)
         if (hipStreamCreateWithFlags(&streams_[s], hipStreamNonBlocking) != hipSuccess) return KSW2_HIP_EDEVICE;
     resident_waves_ = std::max(1, stripe_resident_waves(kGroupLeft));
     if (stats_) fprintf(stderr, "[ksw2 engine] streams %d resident waves %d\n", nstreams_, resident_waves_);
-    if (hipHostMalloc((void **)&h_stop_, sizeof(int32_t), hipHostMallocMapped) != hipSuccess) return KSW2_HIP_ENOMEM;
+    if (!pinned_alloc((void **)&h_stop_, sizeof(int32_t), hipHostMallocMapped)) return KSW2_HIP_ENOMEM;
     *h_stop_ = 0;
     if (hipHostGetDevicePointer((void **)&d_stop_, h_stop_, 0) != hipSuccess) return KSW2_HIP_EDEVICE;
     worker_ = std::thread([this] { loop(); });
@@ -899,22 +895,22 @@ bool Engine::admit_locked(std::unique_lock<std::mutex> &lk)
             for (Task *t : pick) t->held *= 2;
         }
         // pinned upload buffer of this stream, grown to the flight's sequences
+        const bool no_pinned = getenv("KSW2_HIP_FAIL_PINNED") != nullptr;  // tests: there is none
         if (staging_bytes_[s] < seq) {
             if (staging_[s]) (void)hipHostFree(staging_[s]);
             staging_[s] = nullptr, staging_bytes_[s] = 0;
-            const uint64_t want = std::max<uint64_t>(seq * 2, 1 << 20);
-            if (hipHostMalloc((void **)&staging_[s], want, hipHostMallocDefault) == hipSuccess) staging_bytes_[s] = want;
+            const uint64_t want = no_pinned ? 1ull << 60 : std::max<uint64_t>(seq * 2, 1 << 20);
+            if (pinned_alloc((void **)&staging_[s], want, hipHostMallocDefault)) staging_bytes_[s] = want;
         }
         // host mirror of this stream: result slots, CIGAR words, flags
         Mirror &mr = mirror_[s];
         if (mr.slots < pick.size() || mr.words < cigw) {
             mr.release();
-            const uint64_t slots = std::max<uint64_t>(pick.size() * 2, 4096);
+            const uint64_t slots = no_pinned ? 1ull << 50 : std::max<uint64_t>(pick.size() * 2, 4096);
             const uint64_t words = std::max<uint64_t>(cigw * 2, 1 << 20);
             const unsigned fl = hipHostMallocMapped | hipHostMallocCoherent;
-            if (hipHostMalloc((void **)&mr.out, slots * sizeof(KswOut), fl) == hipSuccess &&
-                hipHostMalloc((void **)&mr.cig, words * 4, fl) == hipSuccess &&
-                hipHostMalloc((void **)&mr.flag, slots * 4, fl) == hipSuccess &&
+            if (pinned_alloc((void **)&mr.out, slots * sizeof(KswOut), fl) &&
+                pinned_alloc((void **)&mr.cig, words * 4, fl) && pinned_alloc((void **)&mr.flag, slots * 4, fl) &&
                 hipHostGetDevicePointer((void **)&mr.out_dev, mr.out, 0) == hipSuccess &&
                 hipHostGetDevicePointer((void **)&mr.cig_dev, mr.cig, 0) == hipSuccess &&
                 hipHostGetDevicePointer((void **)&mr.flag_dev, mr.flag, 0) == hipSuccess) {

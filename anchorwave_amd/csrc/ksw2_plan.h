@@ -90,6 +90,11 @@ int band_r_end(int qlen, int tlen, int w);
 // the cached engine block counted as free when with_cache.
 uint64_t mem_budget(bool with_cache);
 
+// Device and pinned memory; false when there is none, with HIP's last error
+// cleared: the launches that follow would report it as theirs.
+bool device_alloc(uint8_t **p, uint64_t bytes);
+bool pinned_alloc(void **p, uint64_t bytes, unsigned flags);
+
 struct DevicePool;
 // A pool over the process's cached device block (the batch engine's, kept
 // between calls), of `bytes` when it must be allocated; null when the block

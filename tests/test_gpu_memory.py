@@ -85,3 +85,35 @@ def test_threads_keep_a_bounded_sum():
         t.join()
     assert not bad
     assert 1 << 30 < kept < (8 << 30) + (1 << 28), kept / 2**30
+
+
+def test_plan_after_one_that_found_no_memory():
+    """A plan of some 420 GB of direction bytes is refused, and the next one's
+    launches do not report its error."""
+    t = random_pairs(763, 1, 400, 400, 1.0)[0][1]
+    long = t.repeat(1000)
+    with pytest.raises(ksw2.KswError):
+        ksw2.Plan([(long, long)] * 3)
+    pairs = random_pairs(764, 20, 100, 900)
+    plan = ksw2.Plan(pairs)
+    plan.run()
+    got = plan.fetch()
+    plan.close()
+    for (q, t), g in zip(pairs, got):
+        r = O.run_oracle(q, t)
+        assert same(g, r), diff(g, r)
+
+
+def test_server_without_pinned_memory(monkeypatch):
+    """A server's flights that get no pinned staging and no mirror run without."""
+    monkeypatch.setenv("KSW2_HIP_FAIL_PINNED", "1")
+    server = ksw2.Server(device_bytes=2 << 30)
+    tasks = {server.submit(q, t, flag=f, w=w): (q, t, f, w) for q, t, f, w in _tuples(765, 40, 900)}
+    left = len(tasks)
+    while left:
+        for ticket, got, _ in server.poll(64, -1):
+            q, t, f, w = tasks[ticket]
+            r = O.run_oracle(q, t, flag=f, w=w)
+            assert same(got, r), diff(got, r)
+            left -= 1
+    server.close()
