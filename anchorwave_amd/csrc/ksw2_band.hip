@@ -659,8 +659,9 @@ __global__ void __launch_bounds__(256) ksw_band_ctl_kernel(int32_t *bnd, const G
 {
     const GenJob &jb = jobs[order[blockIdx.y]];
     int32_t *ctl = bnd + jb.bnd_off;
-    const int n = kBandCtl + 4 * (jb.qlen + jb.tlen);
-    for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += gridDim.x * blockDim.x) ctl[k] = 0;
+    // (64 bits: 536 million letters of both are 2^31 dwords)
+    const int64_t n = kBandCtl + 4 * ((int64_t)jb.qlen + jb.tlen);
+    for (int64_t k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += gridDim.x * blockDim.x) ctl[k] = 0;
 }
 
 namespace {

@@ -26,3 +26,20 @@ def test_long_pair(sc, flag):
     assert (facts["band_pairs"], facts["redone"]) == (1, 0)
     r = O.run_oracle(q, t, w=64, flag=flag, **sc)
     assert same(got, r), diff(got, r)
+
+
+def test_buffer_of_more_than_two_billion_dwords():
+    """600 letters against 540 million, of which the band reaches some 1,700:
+    the buffer's clearing counts past 2^31, on two workgroups."""
+    rng = np.random.default_rng(721)
+    t = W.random_seq(rng, 600)
+    q = np.zeros(540_000_000, dtype=np.uint8)
+    head = W.mutate(rng, t, 0.1, 0.02)
+    q[: len(head)] = head
+    plan = ksw2.Plan([(q, t)], w=500, flag=ksw2.KSW_EZ_SCORE_ONLY)
+    plan.run()
+    got, facts = plan.fetch()[0], plan.facts()
+    plan.close()
+    assert (facts["band_pairs"], facts["waiting"], facts["redone"]) == (1, 2, 0)
+    r = O.run_oracle(q[:4000], t, w=500, flag=ksw2.KSW_EZ_SCORE_ONLY)
+    assert same(got, r), diff(got, r)
